@@ -14,7 +14,7 @@ import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libcrystalframer_hip.so")
-ABI_VERSION = 13
+ABI_VERSION = 14
 
 CFH_WINDOW_REFERENCE = 0
 CFH_WINDOW_WIDE = 1
@@ -88,6 +88,42 @@ class CfhAdamWJob(ctypes.Structure):
                 ("exp_avg_sq", ctypes.c_void_p), ("n", ctypes.c_int64)]
 
 
+class CfhModelLayer(ctypes.Structure):
+    """Mirror of ``cfh_model_layer`` in include/crystalframer_hip.h."""
+    _fields_ = ([("core", CfhParams)]
+                + [(n, ctypes.c_void_p) for n in ("Wqkv", "bqkv", "lattice_w", "gauss_scale_dev", "W_dist", "W_axis1",
+                                                  "W_axis2", "W_axis3", "Wo", "bo", "W1", "b1", "W2", "b2")]
+                + [("c1", ctypes.c_float), ("lb", ctypes.c_float), ("c2", ctypes.c_float), ("q_scale", ctypes.c_float),
+                   ("adaptive", ctypes.c_int32), ("reserved0", ctypes.c_int32)])
+
+
+class CfhModelLinear(ctypes.Structure):
+    """Mirror of ``cfh_model_linear`` in include/crystalframer_hip.h."""
+    _fields_ = [("W", ctypes.c_void_p), ("b", ctypes.c_void_p), ("K", ctypes.c_int32), ("O", ctypes.c_int32),
+                ("relu", ctypes.c_int32), ("reserved0", ctypes.c_int32)]
+
+
+MODEL_MAX_LINEARS = 6        # CFH_MODEL_MAX_LINEARS, CFH_MODEL_MAX_WIDTH
+MODEL_MAX_WIDTH = 480
+
+
+class CfhModel(ctypes.Structure):
+    """Mirror of ``cfh_model`` in include/crystalframer_hip.h."""
+    _fields_ = [("struct_size", ctypes.c_int32), ("layers", ctypes.c_int32), ("heads", ctypes.c_int32), ("D", ctypes.c_int32),
+                ("F", ctypes.c_int32), ("feat", ctypes.c_int32), ("linears", ctypes.c_int32), ("reserved0", ctypes.c_int32),
+                ("We", ctypes.c_void_p), ("layer", ctypes.POINTER(CfhModelLayer)),
+                ("head", CfhModelLinear * MODEL_MAX_LINEARS)]
+
+
+class CfhModelBatch(ctypes.Structure):
+    """Mirror of ``cfh_model_batch`` in include/crystalframer_hip.h."""
+    _fields_ = [("x", ctypes.c_void_p), ("pos", ctypes.c_void_p), ("batch", ctypes.c_void_p), ("tvecs", ctypes.c_void_p),
+                ("sizes", ctypes.c_void_p), ("N", ctypes.c_int64), ("B", ctypes.c_int64), ("E", ctypes.c_int64),
+                ("x0", ctypes.c_void_p), ("qkv0", ctypes.c_void_p), ("noise_seeds", ctypes.POINTER(ctypes.c_uint64)), ("arena", ctypes.c_void_p),
+                ("arena_bytes", ctypes.c_size_t), ("workspace", ctypes.c_void_p), ("workspace_bytes", ctypes.c_size_t),
+                ("stream", ctypes.c_void_p), ("keep", ctypes.c_int32), ("reserved0", ctypes.c_int32)]
+
+
 EXPORTS = ("cfh_abi_version", "cfh_last_error", "cfh_workspace_bytes", "cfh_frame_axis1",
            "cfh_frame_axis2", "cfh_frame_axes", "cfh_framed_pe_forward", "cfh_framed_pe_forward_static", "cfh_frame_axes_framed_pe_forward",
            "cfh_framed_pe_backward", "cfh_framed_pe_backward_pairwise",
@@ -98,7 +134,8 @@ EXPORTS = ("cfh_abi_version", "cfh_last_error", "cfh_workspace_bytes", "cfh_fram
            "cfh_second_stream_fork", "cfh_second_stream_get", "cfh_second_stream_join",
            "cfh_fused_core_workspace_bytes", "cfh_fused_core_hist_words", "cfh_fused_core_forward",
            "cfh_fused_core_backward", "cfh_adamw_step_batch",
-           "cfh_fused_core_weight_gradients_workspace_bytes", "cfh_fused_core_weight_gradients")
+           "cfh_fused_core_weight_gradients_workspace_bytes", "cfh_fused_core_weight_gradients",
+           "cfh_model_sizes", "cfh_model_forward", "cfh_model_backward")
 
 _lib = None
 _lock = threading.Lock()
@@ -200,6 +237,13 @@ def load():
         lib.cfh_timing_enable.argtypes = [ctypes.c_int]
         lib.cfh_timing_read.restype = ctypes.c_int
         lib.cfh_timing_read.argtypes = [ctypes.c_char_p, ctypes.POINTER(ctypes.c_double), ctypes.POINTER(_I64)]
+        pm, pb = ctypes.POINTER(CfhModel), ctypes.POINTER(CfhModelBatch)
+        lib.cfh_model_sizes.restype = _I64
+        lib.cfh_model_sizes.argtypes = [pm, pb, ctypes.POINTER(ctypes.c_size_t * 4)]
+        lib.cfh_model_forward.restype = ctypes.c_int
+        lib.cfh_model_forward.argtypes = [pm, pb, _P]
+        lib.cfh_model_backward.restype = ctypes.c_int
+        lib.cfh_model_backward.argtypes = [pm, pb, _P, _P, ctypes.c_size_t, _P]
         lib.cfh_second_stream_fork.restype = ctypes.c_int
         lib.cfh_second_stream_fork.argtypes = [_P, ctypes.POINTER(_P)]
         lib.cfh_second_stream_get.restype = ctypes.c_int
@@ -235,6 +279,11 @@ def require_gpu(*tensors: torch.Tensor):
                 f"{t.device}); there is no CPU path")
 
 
+def raw_stream(device: torch.device) -> int:
+    """The framework's current stream of ``device`` as a plain address (without the stream object around it)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
+
+
 _workspaces = {}
 _superseded = []      # outgrown workspaces, kept for captured graphs that still point at them
 
@@ -242,7 +291,7 @@ _superseded = []      # outgrown workspaces, kept for captured graphs that still
 def workspace(device: torch.device, nbytes: int) -> torch.Tensor:
     """Scratch buffer handed to the library, one per (device, stream): kernels of one stream run
     in order, so they can share it; grown on demand, reused across calls."""
-    key = (device.type, device.index, torch.cuda.current_stream(device).cuda_stream)
+    key = (device.type, device.index, raw_stream(device))
     buf = _workspaces.get(key)
     if buf is None or buf.numel() < nbytes:
         if buf is not None:
@@ -299,7 +348,7 @@ def read_status(device: torch.device, reset: bool = False) -> int:
 
 
 def current_stream_ptr(device: torch.device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    return ctypes.c_void_p(raw_stream(device))
 
 
 def kernel_timing(enable: bool):

@@ -30,8 +30,17 @@ struct AttnInArgs {
     float c1, lb, c2, q_scale;
 };
 
+// q . w of a head, 16 lanes one channel each.  The first step of the row sum as one fused multiply-add, spelled out: the
+// compiler makes one of it or not depending on the code around, and the kernels that share this sum agree to the last bit.
+__device__ __forceinline__ float head_dot(float q, float w) {
+    float x = fmaf(q, w, dpp_move<0xB1>(q * w));
+    x += dpp_move<0x4E>(x);
+    x += dpp_move<0x141>(x);
+    x += dpp_move<0x140>(x);
+    return x;
+}
 __device__ __forceinline__ float gauss_alpha(const AttnInArgs& P, float q, float wc, float& slope) {
-    float alpha = row_sum(q * wc);
+    float alpha = head_dot(q, wc);
     float scale = 1.0f;
     if (P.gauss) {
         scale = P.gauss[0];

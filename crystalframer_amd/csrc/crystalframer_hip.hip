@@ -27,6 +27,7 @@
 #include "small_gemm.hpp"
 #include "layer_bridge.hpp"
 #include "adamw.hpp"
+#include "model_tail.hpp"
 
 namespace {
 
@@ -1049,7 +1050,8 @@ int check_wgrad_jobs(const cfh_linear_grad_job* jobs, int32_t njobs) {
 }
 // The launch of the jobs [first, last): slices and workgroup numbers of every job; returns the number of tiles that
 // several slices share.
-int plan_wgrad(const cfh_linear_grad_job* jobs, int32_t first, int32_t last, cfh::WgradJobs& T) {
+// `group` (null: all jobs are one): the slices of a job are chosen as if its group had a launch of its own.
+int plan_wgrad(const cfh_linear_grad_job* jobs, int32_t first, int32_t last, cfh::WgradJobs& T, const int32_t* group = nullptr) {
     // a job whose shape and alignment allow it takes the variant with 16-byte loads
     auto wide = [](const cfh_linear_grad_job& J) {
         return J.dW && J.O % 64 == 0 && J.I % 64 == 0 && J.ldx % 4 == 0 && J.ldy % 4 == 0 &&
@@ -1060,11 +1062,16 @@ int plan_wgrad(const cfh_linear_grad_job* jobs, int32_t first, int32_t last, cfh
         by = (J.O + 63) / 64;
     };
     long tiles = 0;
+    std::vector<long> group_tiles;
     for (int32_t j = first; j < last; j++)
         if (jobs[j].N > 0) {
             long bx, by;
             tiles_of(jobs[j], bx, by);
             tiles += bx * by;
+            if (group) {
+                if ((size_t)group[j] >= group_tiles.size()) group_tiles.resize(group[j] + 1, 0);
+                group_tiles[group[j]] += bx * by;
+            }
         }
     T = cfh::WgradJobs{};
     if (tiles == 0) return 0;
@@ -1073,7 +1080,6 @@ int plan_wgrad(const cfh_linear_grad_job* jobs, int32_t first, int32_t last, cfh
     int cus = device_cus();
     if (cus <= 0) cus = 256;
     const long target = 4L * cus - 24;
-    const int want = (int)(target / tiles > 0 ? target / tiles : 1);
     int blocks = 0, tile0 = 0;
     for (int32_t j = first; j < last; j++) {
         const cfh_linear_grad_job& J = jobs[j];
@@ -1084,7 +1090,8 @@ int plan_wgrad(const cfh_linear_grad_job* jobs, int32_t first, int32_t last, cfh
         long bx, by;
         tiles_of(J, bx, by);
         W.bx = (int)bx; W.by = (int)by; W.wide = wide(J) ? 1 : 0;
-        int slices = want;
+        const long share = target / (group ? group_tiles[group[j]] : tiles);
+        int slices = (int)(share > 0 ? share : 1);
         const int max_slices = (int)((J.N + 31) / 32);
         if (slices > max_slices) slices = max_slices;
         if (slices < 1) slices = 1;
@@ -1156,18 +1163,19 @@ size_t cfh_linear_weight_bias_grad_batch_workspace_bytes(const cfh_linear_grad_j
     return need;
 }
 
-int cfh_linear_weight_bias_grad_batch(const cfh_linear_grad_job* jobs, int32_t njobs, void* workspace,
-                                      size_t workspace_bytes, void* stream) {
+static int linear_wgrad_batch_impl(const cfh_linear_grad_job* jobs, int32_t njobs, void* workspace, size_t workspace_bytes,
+                                   void* stream, bool overwrite, const int32_t* group = nullptr) {
     int rc = check_wgrad_jobs(jobs, njobs);
     if (rc) return rc;
     hipStream_t st = (hipStream_t)stream;
     std::vector<cfh_linear_grad_job> ordered;
     std::vector<int32_t> ends;
     wgrad_launches(jobs, njobs, workspace != nullptr, ordered, ends);
+    if (ends.size() > 1) group = nullptr;      // (the jobs of a grouped call fit one launch and keep their order)
     int32_t first = 0;
     for (int32_t last : ends) {
         cfh::WgradJobs T;
-        plan_wgrad(ordered.data(), first, last, T);
+        plan_wgrad(ordered.data(), first, last, T, group);
         first = last;
         if (T.blocks == 0) continue;
         if (workspace) {
@@ -1176,12 +1184,18 @@ int cfh_linear_weight_bias_grad_batch(const cfh_linear_grad_job* jobs, int32_t n
             if ((rc = check_workspace(workspace, workspace_bytes, (size_t)T.blocks * cfh::WG_PART * sizeof(float))))
                 return rc;
             T.scratch.partials = reinterpret_cast<float*>(workspace);
+            T.scratch.overwrite = overwrite ? 1 : 0;
         }
         hipLaunchKernelGGL(cfh::linear_wgrad_batch_kernel, dim3((T.blocks + 7) & ~7), dim3(256), 0, st, T);
         if (workspace && T.split_tiles > 0)
             hipLaunchKernelGGL(cfh::linear_wgrad_sum_kernel, dim3(4 * T.split_tiles), dim3(256), 0, st, T);
     }
     return finish_launch("linear_weight_bias_grad_batch");
+}
+
+int cfh_linear_weight_bias_grad_batch(const cfh_linear_grad_job* jobs, int32_t njobs, void* workspace,
+                                      size_t workspace_bytes, void* stream) {
+    return linear_wgrad_batch_impl(jobs, njobs, workspace, workspace_bytes, stream, false);
 }
 
 int cfh_layer_bridge_forward(const float* attn, const float* x_res, int64_t N, int32_t D, int32_t F, const float* Wo,
@@ -1195,10 +1209,10 @@ int cfh_layer_bridge_forward(const float* attn, const float* x_res, int64_t N, i
     if (H < 1 || H * cfh::DH != D || cfh::BR_ROWS * H > 64 * cfh::BR_WAVES)
         return fail(CFH_EINVAL, "layer bridge: D=%d must be 16 x H=%d, H at most %d", (int)D, (int)H, 64 * cfh::BR_WAVES / cfh::BR_ROWS);
     if (N == 0) return CFH_OK;
-    if (!attn || !x_res || !Wo || !W1 || !W2 || !x1 || !h || !x2)
-        return fail(CFH_EINVAL, "layer bridge: attn, x_res, the weights and x1, h, x2 must not be NULL");
-    if (Wqkv && (!lattice_w || !qkv || !qs || !k || !v || !a))
-        return fail(CFH_EINVAL, "layer bridge: with Wqkv, lattice_w and qkv, qs, k, v, a must not be NULL");
+    if (!attn || !x_res || !Wo || !W1 || !W2 || !x2)
+        return fail(CFH_EINVAL, "layer bridge: attn, x_res, the weights and x2 must not be NULL");
+    if (Wqkv && (!lattice_w || !qs || !k || !v || !a))
+        return fail(CFH_EINVAL, "layer bridge: with Wqkv, lattice_w and qs, k, v, a must not be NULL");
     const int wide = F > 3 * D ? F : 3 * D;
     const size_t lds = ((size_t)cfh::BR_ROWS * (2 * (D + cfh::BR_PAD) + wide + cfh::BR_PAD) +
                         (size_t)cfh::BR_WAVES * cfh::BR_STAGE_FLOATS) * sizeof(float);
@@ -1311,7 +1325,7 @@ int cfh_small_linear_dx(const float* dy, const float* W, int64_t M, int64_t N, i
         return finish_launch("small_linear_dx");
     }
     hipLaunchKernelGGL(cfh::small_linear_dx_kernel, dim3((unsigned)((M + 63) / 64), (unsigned)((K + 63) / 64)), dim3(256), 0,
-                       (hipStream_t)stream, dy, W, dx, (int)M, (int)N, (int)K);
+                       (hipStream_t)stream, dy, W, (const float*)nullptr, dx, (int)M, (int)N, (int)K);
     return finish_launch("small_linear_dx");
 }
 
@@ -1756,8 +1770,8 @@ size_t cfh_fused_core_weight_gradients_workspace_bytes(const cfh_params* p, int3
            align256((size_t)cfh::CORE_GW_SLICES * p->num_heads * cfh::DH * hw * sizeof(float)) * (size_t)(njobs > 0 ? njobs : 1);
 }
 
-int cfh_fused_core_weight_gradients(const cfh_params* p, const cfh_core_wgrad_job* jobs, int32_t njobs,
-                                    void* workspace, size_t workspace_bytes, void* stream) {
+static int core_weight_gradients_impl(const cfh_params* p, const cfh_core_wgrad_job* jobs, int32_t njobs, void* workspace,
+                                      size_t workspace_bytes, void* stream, bool overwrite) {
     int rc = check_core_params(p);
     if (rc) return rc;
     if (njobs < 0 || (njobs > 0 && !jobs)) return fail(CFH_EINVAL, "jobs is NULL or njobs negative");
@@ -1781,6 +1795,7 @@ int cfh_fused_core_weight_gradients(const cfh_params* p, const cfh_core_wgrad_jo
         const int32_t last = njobs < first + cfh::CORE_WG_MAX_JOBS ? njobs : first + cfh::CORE_WG_MAX_JOBS;
         cfh::CoreWgradJobs T{};
         T.H = p->num_heads; T.hw = hw;
+        T.overwrite = overwrite ? 1 : 0;
         T.dist_coef = p->dist_coef; T.angle_coef = p->angle_coef; T.ws = p->angle_wscale;
         int slices = 0;
         for (int32_t j = first; j < last; j++) {
@@ -1811,8 +1826,11 @@ int cfh_fused_core_weight_gradients(const cfh_params* p, const cfh_core_wgrad_jo
     return finish_launch("fused_core_weight_gradients");
 }
 
+int cfh_fused_core_weight_gradients(const cfh_params* p, const cfh_core_wgrad_job* jobs, int32_t njobs,
+                                    void* workspace, size_t workspace_bytes, void* stream) {
+    return core_weight_gradients_impl(p, jobs, njobs, workspace, workspace_bytes, stream, false);
+}
+
 }  // extern "C"
 
-
-
-
+#include "model_pass.hpp"

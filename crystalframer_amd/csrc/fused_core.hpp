@@ -295,12 +295,11 @@ __global__ __launch_bounds__(256) void core_prepare_wcat_kernel(const KernelArgs
     else core_wcat_block(A, (int)blockIdx.x - prep_blocks);
 }
 // The way back: gW_dist = dist_coef gwcat[.., 0:64];  gW_ax[c,m] = angle_coef sum_{o,m'} gwcat[.., ax,o,m'] D_o(m - m').
-// Block hc = (head, channel), 256 threads = (enc 0..3, bin m).  ACC: added to what the destinations hold.
-template <bool ACC>
+// Block hc = (head, channel), 256 threads = (enc 0..3, bin m).  acc_dst: added to what the destinations hold.
 __device__ __forceinline__ void core_gw_finish_block(const float* __restrict__ gwcat, int nslices, size_t slice_stride,
                                                      int hw, float dist_coef, float angle_coef, float ws,
                                                      float* __restrict__ gWd, float* __restrict__ gW1,
-                                                     float* __restrict__ gW2, float* __restrict__ gW3, int hc) {
+                                                     float* __restrict__ gW2, float* __restrict__ gW3, int hc, bool acc_dst) {
     __shared__ float dtab[NORD * 128];
     __shared__ float grow[3 * NORD * NBINS];
     const int enc = threadIdx.x >> 6, m = threadIdx.x & 63;
@@ -314,7 +313,7 @@ __device__ __forceinline__ void core_gw_finish_block(const float* __restrict__ g
         float sum = 0.0f;
         for (int sl = 0; sl < nslices; sl++) sum += g[sl * slice_stride + word];      // fixed order
         float* d = dst + (size_t)hc * (enc == 0 ? NBINS : SMALL_A) + m;
-        *d = (ACC ? *d : 0.0f) + (enc == 0 ? dist_coef : angle_coef) * sum;
+        *d = (acc_dst ? *d : 0.0f) + (enc == 0 ? dist_coef : angle_coef) * sum;
         return;
     }
     if (hw > HW_DIST) {
@@ -330,7 +329,7 @@ __device__ __forceinline__ void core_gw_finish_block(const float* __restrict__ g
             float sum = 0.0f;
             for (int sl = 0; sl < nslices; sl++) sum += g[sl * slice_stride + m];
             float* d = gWd + (size_t)hc * NBINS + m;
-            *d = (ACC ? *d : 0.0f) + dist_coef * sum;
+            *d = (acc_dst ? *d : 0.0f) + dist_coef * sum;
         }
         return;
     }
@@ -345,15 +344,15 @@ __device__ __forceinline__ void core_gw_finish_block(const float* __restrict__ g
         for (int mp = 0; mp < NBINS; mp++) acc = fmaf(gr[mp], dt[-mp], acc);
     }
     float* d = dst + (size_t)hc * NBINS + m;
-    *d = (ACC ? *d : 0.0f) + angle_coef * acc;
+    *d = (acc_dst ? *d : 0.0f) + angle_coef * acc;
 }
 // grid: H*16 blocks.
 __global__ __launch_bounds__(256) void core_gw_finish_kernel(const float* __restrict__ gwcat, int nslices, int H, int hw,
                                                              float dist_coef, float angle_coef, float ws,
                                                              float* __restrict__ gWd, float* __restrict__ gW1,
                                                              float* __restrict__ gW2, float* __restrict__ gW3) {
-    core_gw_finish_block<false>(gwcat, nslices, (size_t)H * DH * hw, hw, dist_coef, angle_coef, ws, gWd, gW1, gW2, gW3,
-                                (int)blockIdx.x);
+    core_gw_finish_block(gwcat, nslices, (size_t)H * DH * hw, hw, dist_coef, angle_coef, ws, gWd, gW1, gW2, gW3,
+                         (int)blockIdx.x, false);
 }
 
 // Weight gradients of several calls of the core (the layers of a backward pass) in one launch each way.
@@ -370,6 +369,7 @@ struct CoreWgradJobs {
     CoreWgradJob job[CORE_WG_MAX_JOBS];
     int njobs, H, hw;
     float dist_coef, angle_coef, ws;
+    int overwrite;         // the destinations are written, not added to
 };
 // ---- distance window with round-to-nearest fixed-point adds ---------------------------------------------------
 template <int W>
@@ -1123,11 +1123,11 @@ __global__ __launch_bounds__(WAVE * GW_WPB) void core_gwcat_multi_kernel(const C
     const CoreWgradJob& J = T.job[j];
     core_gwcat_block(J.go, J.hist, J.gwcat, J.N, T.H, T.hw, J.per_slice, (int)blockIdx.z - J.slice0);
 }
-// grid (H*16, jobs): added to the destinations
+// grid (H*16, jobs): added to the destinations (or written)
 __global__ __launch_bounds__(256) void core_gw_finish_multi_kernel(const CoreWgradJobs T) {
     const CoreWgradJob& J = T.job[blockIdx.y];
-    core_gw_finish_block<true>(J.gwcat, J.nslices, (size_t)T.H * DH * T.hw, T.hw, T.dist_coef, T.angle_coef, T.ws,
-                               J.gW[0], J.gW[1], J.gW[2], J.gW[3], (int)blockIdx.x);
+    core_gw_finish_block(J.gwcat, J.nslices, (size_t)T.H * DH * T.hw, T.hw, T.dist_coef, T.angle_coef, T.ws,
+                         J.gW[0], J.gW[1], J.gW[2], J.gW[3], (int)blockIdx.x, T.overwrite == 0);
 }
 
 

@@ -13,6 +13,7 @@
 // stage, 16 at a time, and stream the weights from the L2.  Every intermediate is also written out:
 // the backward pass needs all of them.
 #pragma once
+#include "attention_inputs.hpp"
 #include "device_common.hpp"
 
 namespace cfh {
@@ -31,7 +32,7 @@ struct BridgeArgs {
     const float* W2; const float* b2;             // (D, F), (D)
     const float* Wq; const float* bq;             // (3 D, D), (3 D); Wq null: the chain ends with x2
     const float* lattice_w; const float* gauss;   // (D); device {scale, shift} or null
-    float* x1; float* h; float* x2; float* qkv;   // (N, D), (N, F), (N, D), (N, 3 D)
+    float* x1; float* h; float* x2; float* qkv;   // (N, D), (N, F), (N, D), (N, 3 D); x1, h, qkv null: not written
     float* qs; float* k; float* v; float* a;      // (N, D) x 3, (N, H)
     int N, D, F, H;
     float c1, lb, c2, q_scale;
@@ -127,7 +128,7 @@ __device__ __forceinline__ void bridge_tiles(const float* in, int K, const float
             if (res_lds) val += res_lds[m * ldout + n];
             if (RELU) val = fmaxf(val, 0.f);
             if (out_lds) out_lds[m * ldout + n] = val;
-            if (m < nrows) out_g[(size_t)(r0 + m) * O + n] = val;
+            if (out_g && m < nrows) out_g[(size_t)(r0 + m) * O + n] = val;
         }
     }
 }
@@ -199,6 +200,73 @@ __global__ __launch_bounds__(64 * BR_WAVES) void layer_bridge_fwd_kernel(const B
     }
 }
 
+// The start of the chain: x0 = x We^T (embedding, (N, feat) features), then the first layer's inputs as above.  The
+// arguments of the bridge with attn = x, Wo = We and x2 = x0.  The features are one-hot or a few dozen columns, not a
+// multiple of the matrix instruction's operands, and their rows are not 16-byte aligned: the operands are single words,
+// zero past the last feature.  dynamic LDS: 16 (D + 4 + 3 D + 4 + feat rounded up to 4, + 4) floats and the stages.
+__host__ __device__ inline size_t bridge_front_lds_floats(int D, int feat) {
+    return (size_t)BR_ROWS * ((D + BR_PAD) + (3 * D + BR_PAD) + ((feat + 3) / 4 * 4 + BR_PAD)) + (size_t)BR_WAVES * BR_STAGE_FLOATS;
+}
+__global__ __launch_bounds__(64 * BR_WAVES) void layer_front_fwd_kernel(const BridgeArgs P, int feat) {
+    extern __shared__ __attribute__((aligned(16))) float bridge_lds[];
+    const int D = P.D, Q = 3 * D, steps = (feat + 3) / 4, ldx = 4 * steps + BR_PAD;
+    float* const s_a = bridge_lds;                            // [16][D+4]  x0
+    float* const s_c = s_a + BR_ROWS * (D + BR_PAD);          // [16][3D+4] qkv
+    float* const s_x = s_c + BR_ROWS * (Q + BR_PAD);          // [16][feat+]
+    float* const stage = s_x + BR_ROWS * ldx + (threadIdx.x >> 6) * BR_STAGE_FLOATS;
+    const int r0 = blockIdx.x * BR_ROWS;
+    const int nrows = min(BR_ROWS, P.N - r0);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, kk = lane >> 4;
+    for (int idx = threadIdx.x; idx < BR_ROWS * 4 * steps; idx += 64 * BR_WAVES) {
+        const int m = idx / (4 * steps), c = idx - m * 4 * steps;
+        s_x[m * ldx + c] = m < nrows && c < feat ? P.attn[(size_t)(r0 + m) * feat + c] : 0.0f;
+    }
+    __syncthreads();
+    for (int t = wave; t < D / 16; t += BR_WAVES) {
+        const float* const wrow = P.Wo + (size_t)(16 * t + col) * feat;
+        v4f_b2 acc = {0.f, 0.f, 0.f, 0.f};
+        constexpr int UN = 8;                                 // steps whose loads are in flight
+        for (int s0 = 0; s0 < steps; s0 += UN) {
+            float w[UN];
+#pragma unroll
+            for (int u = 0; u < UN; u++) {                    // (past the end: the last word again, its feature is zero)
+                const int k = 4 * min(s0 + u, steps - 1) + kk;
+                w[u] = wrow[min(k, feat - 1)];
+            }
+#pragma unroll
+            for (int u = 0; u < UN; u++)
+                if (s0 + u < steps) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(s_x[col * ldx + 4 * (s0 + u) + kk], w[u], acc, 0, 0, 0);
+        }
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const int m = 4 * kk + c, n = 16 * t + col;
+            s_a[m * (D + BR_PAD) + n] = acc[c];
+            if (m < nrows) P.x2[(size_t)(r0 + m) * D + n] = acc[c];
+        }
+    }
+    __syncthreads();
+    bridge_stage<false>(s_a, D, P.Wq, P.bq, Q, nullptr, nullptr, r0, nrows, s_c, P.qkv, stage);
+    __syncthreads();
+    // the inputs of the first layer as attention_inputs_fwd_kernel makes them: a thread per (row, channel), alpha as a row
+    // sum over the 16 lanes of a head (64 BR_WAVES is a multiple of 16, and D of 128: no head is split over wavefronts)
+    for (int idx = threadIdx.x; idx < BR_ROWS * D; idx += 64 * BR_WAVES) {
+        const int m = idx / D, c = idx - m * D;
+        const float* const row = s_c + m * (Q + BR_PAD);
+        const float q = m < nrows ? row[c] : 0.0f;
+        float alpha = head_dot(q, P.lattice_w[c]);
+        if (P.gauss) alpha = (alpha + P.gauss[1]) * P.gauss[0];
+        const float u = alpha * P.c1;
+        const float e = u > 0.0f ? u : expm1f(u);
+        const float a = ((1.0f - P.lb) * e + 1.0f) * P.c2;
+        if (m >= nrows) continue;
+        const size_t o = (size_t)(r0 + m) * D + c;
+        P.qs[o] = q * P.q_scale;
+        P.k[o] = row[D + c];
+        P.v[o] = row[2 * D + c];
+        if ((c & 15) == 0) P.a[(size_t)(r0 + m) * P.H + (c >> 4)] = a;
+    }
+}
+
 
 // ---- backward: the input gradients of the same chain ------------------------------------------------
 //     g2 = g_x2 + gqkv Wqkv;   gh = (g2 W2) [h > 0];   g1 = g2 + gh W1;   g_attn = g1 Wo
@@ -207,6 +275,8 @@ __global__ __launch_bounds__(64 * BR_WAVES) void layer_bridge_fwd_kernel(const B
 // launch at the end of the backward pass multiplies them with the saved activations.
 struct BridgeBwdArgs {
     const float* g_x2;            // (N, D) or null (zero)
+    const int64_t* batch;         // optional: g_x2 is (B, D) per crystal, a row takes that of its crystal over the
+    const int64_t* atom_start;    // crystal's atoms (the mean over a crystal behind the last layer); no next layer
     const float* gqkv;            // (N, 3 D) or null: no next layer, g2 = g_x2 (g2 is then not written)
     const float* h;               // (N, F) forward activations (the rectifier's mask)
     const float* Wq; const float* W2; const float* W1; const float* Wo;     // (3D, D), (D, F), (F, D), (D, D)
@@ -397,7 +467,13 @@ __global__ __launch_bounds__(64 * BR_WAVES) void layer_bridge_bwd_kernel(const B
         for (int idx = threadIdx.x * 4; idx < BR_ROWS * D; idx += 64 * BR_WAVES * 4) {
             const int m = idx / D, c = idx - m * D;
             float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (m < nrows && P.g_x2) v = *reinterpret_cast<const float4*>(P.g_x2 + (size_t)(r0 + m) * D + c);
+            if (m < nrows && P.batch) {
+                const int64_t b = P.batch[r0 + m];
+                const float inv = 1.0f / (float)(P.atom_start[b + 1] - P.atom_start[b]);
+                v = *reinterpret_cast<const float4*>(P.g_x2 + (size_t)b * D + c);
+                v.x *= inv; v.y *= inv; v.z *= inv; v.w *= inv;
+                *reinterpret_cast<float4*>(P.g2 + (size_t)(r0 + m) * D + c) = v;
+            } else if (m < nrows && P.g_x2) v = *reinterpret_cast<const float4*>(P.g_x2 + (size_t)(r0 + m) * D + c);
             *reinterpret_cast<float4*>(s_g2 + m * (D + BR_PAD) + c) = v;
         }
     }

@@ -231,6 +231,7 @@ __device__ __forceinline__ void wgrad_block_wide(const float* __restrict__ x, co
 // workgroups computed them, WG_PART floats each, in the order of the workgroups' numbers.
 struct WgradScratch {
     float* partials;
+    int overwrite;      // with partials: the outputs are written, not added to (their memory need not be cleared)
 };
 constexpr int WG_PART = 64 * 64 + 64;      // floats a workgroup stores: its tile and its 64 column sums
 
@@ -253,9 +254,13 @@ __device__ __forceinline__ void wgrad_output(const float* block, const float* co
         if (dW)
             for (int idx = threadIdx.x; idx < 64 * 64; idx += 256) {
                 const int m = idx >> 6, n = idx & 63;
-                if (o0 + m < O && i0 + n < I) dW[(size_t)(o0 + m) * I + i0 + n] += block[m * WG_LDS_ROW + n];
+                if (o0 + m < O && i0 + n < I) {
+                    float* const d = dW + (size_t)(o0 + m) * I + i0 + n;
+                    *d = (S.overwrite ? 0.0f : *d) + block[m * WG_LDS_ROW + n];
+                }
             }
-        if (bias && threadIdx.x < 64 && o0 + (int)threadIdx.x < O) db[o0 + threadIdx.x] += colsum[threadIdx.x];
+        if (bias && threadIdx.x < 64 && o0 + (int)threadIdx.x < O)
+            db[o0 + threadIdx.x] = (S.overwrite ? 0.0f : db[o0 + threadIdx.x]) + colsum[threadIdx.x];
         return;
     }
     // stored for linear_wgrad_sum_kernel: the 16-byte pieces q = threadIdx.x + 256 j (row q / 16, columns 4 (q % 16) ...)
@@ -296,7 +301,7 @@ __device__ __forceinline__ void wgrad_tile(const float* __restrict__ x, const fl
 __global__ __launch_bounds__(256) void linear_wgrad_kernel(const float* __restrict__ x, const float* __restrict__ dy,
                                                            int N, int I, int O, int rows_per_slice,
                                                            float* dW, float* db) {
-    const WgradScratch none{nullptr};
+    const WgradScratch none{nullptr, 0};
     wgrad_tile(x, dy, N, I, O, I, O, rows_per_slice, blockIdx.x, blockIdx.y, blockIdx.z, (int)gridDim.z, dW, db, false, 0,
                none);
 }
@@ -363,8 +368,9 @@ __global__ __launch_bounds__(256) void linear_wgrad_sum_kernel(const WgradJobs T
     const bool vec = row_ok && (J.I & 3) == 0 && (reinterpret_cast<uintptr_t>(J.dW) & 15) == 0 && i0 + n + 3 < J.I;
     // what the outputs hold is asked for before the stored tiles, not after them
     v4f_l sum = {0.f, 0.f, 0.f, 0.f};
-    if (vec) sum = *reinterpret_cast<const v4f_l*>(dst);
-    float bsum = do_bias ? J.db[o0 + threadIdx.x] : 0.0f;
+    const bool keep = T.scratch.overwrite == 0;
+    if (vec && keep) sum = *reinterpret_cast<const v4f_l*>(dst);
+    float bsum = do_bias && keep ? J.db[o0 + threadIdx.x] : 0.0f;
     v4f_l add = {0.f, 0.f, 0.f, 0.f};
     float badd = 0.0f;
     for (int sl = 0; sl < slices; sl += 8) {
@@ -385,7 +391,7 @@ __global__ __launch_bounds__(256) void linear_wgrad_sum_kernel(const WgradJobs T
     } else if (row_ok) {
 #pragma unroll
         for (int e = 0; e < 4; e++)
-            if (i0 + n + e < J.I) dst[e] += add[e];
+            if (i0 + n + e < J.I) dst[e] = (keep ? dst[e] : 0.0f) + add[e];
     }
     if (do_bias) J.db[o0 + threadIdx.x] = bsum + badd;
 }

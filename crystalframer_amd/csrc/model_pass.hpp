@@ -1,0 +1,468 @@
+// Host side of cfh_model_forward / cfh_model_backward: the launches of a whole pass, one after the other, with every
+// intermediate in the caller's arena.  Included by crystalframer_hip.hip behind the entry points it calls.
+//
+// What bounds a pass over a small batch is not any kernel but the host between them: the same launches made from Python,
+// one autograd function per operator with its allocations, took 755 us per inference pass and 2330 us per training step
+// against 250 and 730 us of kernels (4 layers, 1 and 13 crystals).
+namespace {
+
+struct ModelLayerBuffers {
+    float *x1, *h, *qkv, *qs, *k, *v, *a;      // qkv .. a: inputs of this layer; x1, h: behind its core
+    float *x2;                                 // output of this layer
+    float *frames, *z, *prob, *hist, *out, *wcat;
+    uint32_t* records;
+};
+constexpr int MODEL_MAX_LAYERS = 64;
+struct ModelBuffers {
+    int64_t *edges, *e_start, *atom_start;
+    int32_t* order;
+    float *rpos, *recip, *rvlen, *vcell, *near_, *x0, *pooled;
+    float4* table;
+    char* geo_ws;
+    float* y[CFH_MODEL_MAX_LINEARS];           // results of the head's linear layers but the last
+    ModelLayerBuffers layer[MODEL_MAX_LAYERS];
+    size_t total;
+};
+struct Carver {
+    char* base;
+    size_t off = 0;
+    template <typename T>
+    T* take(size_t n) {
+        T* p = base ? reinterpret_cast<T*>(base + off) : nullptr;
+        off += align256((n > 0 ? n : 1) * sizeof(T));
+        return p;
+    }
+};
+
+int check_model(const cfh_model* m, const cfh_model_batch* b) {
+    if (!m || !b) return fail(CFH_EINVAL, "model and batch must not be NULL");
+    if (m->struct_size != (int32_t)sizeof(cfh_model))
+        return fail(CFH_EINVAL, "cfh_model.struct_size %d != %zu (header/library mismatch)", m->struct_size, sizeof(cfh_model));
+    if (m->layers < 1 || m->layers > MODEL_MAX_LAYERS || !m->layer || !m->We)
+        return fail(CFH_EINVAL, "model: 1 to %d layers with their weights and an embedding are needed", MODEL_MAX_LAYERS);
+    if (m->heads < 1 || m->heads > 32 || m->D != m->heads * cfh::DH || m->D % 128 != 0 || 256 % m->D != 0 ||
+        m->F < 128 || m->F % 128 != 0 || m->feat < 1 || m->feat > 512)
+        return fail(CFH_EINVAL, "model: D=%d (16 x H=%d), F=%d, feat=%d not supported", m->D, m->heads, m->F, m->feat);
+    if (m->linears < 1 || m->linears > CFH_MODEL_MAX_LINEARS)
+        return fail(CFH_EINVAL, "model: %d linear layers in the head (1 to %d)", m->linears, CFH_MODEL_MAX_LINEARS);
+    for (int i = 0; i < m->linears; i++) {
+        const cfh_model_linear& T = m->head[i];
+        if (!T.W || T.in % 16 != 0 || T.in != (i ? m->head[i - 1].out : m->D) || T.in > CFH_MODEL_MAX_WIDTH || T.out < 1 ||
+            T.out > CFH_MODEL_MAX_WIDTH)
+            return fail(CFH_EINVAL, "model: head layer %d (%d -> %d) not supported", i, T.in, T.out);
+    }
+    for (int l = 0; l < m->layers; l++) {
+        const cfh_model_layer& L = m->layer[l];
+        if (int rc = check_core_params(&L.core)) return rc;
+        if (L.core.num_heads != m->heads || L.core.angle_bins != m->layer[0].core.angle_bins)
+            return fail(CFH_EINVAL, "model: layer %d differs from layer 0 in heads or angle bins", l);
+        if (!L.Wqkv || !L.bqkv || !L.lattice_w || !L.W_dist || !L.Wo || !L.bo || !L.W1 || !L.b1 || !L.W2 || !L.b2 ||
+            (L.core.angle_bins > 0 && (!L.W_axis1 || !L.W_axis2 || !L.W_axis3)))
+            return fail(CFH_EINVAL, "model: a weight of layer %d is NULL", l);
+    }
+    if (b->N < 1 || b->B < 1 || b->E < 1 || b->B > 0x7fffffffLL / 64)
+        return fail(CFH_EINVAL, "model: N=%lld B=%lld E=%lld", (long long)b->N, (long long)b->B, (long long)b->E);
+    return check_core_sizes(&m->layer[0].core, b->N, b->E);
+}
+
+// The tables of the geometry (sorted shifts, nearest images) are shared by the layers whose box rule agrees.
+bool same_tables(const cfh_model_layer& a, const cfh_model_layer& b) {
+    auto R0 = [](const cfh_model_layer& L) {
+        return L.adaptive && L.core.cutoff_radius != 0.0f ? L.core.minimum_range : L.core.lattice_range;
+    };
+    return R0(a) == R0(b);
+}
+
+// Layout of the arena.  keep: every layer its own buffers, for the backward pass; else the layers share one set (a layer
+// reads its inputs before the next one's are written: the inputs of a layer alternate between two sets).
+void model_buffers(const cfh_model* m, const cfh_model_batch* b, ModelBuffers& M) {
+    Carver c{reinterpret_cast<char*>(b->arena)};
+    const size_t N = b->N, E = b->E, B = b->B, D = m->D, F = m->F, H = m->heads;
+    const size_t hw = cfh::core_hist_words(m->layer[0].core.angle_bins);
+    M.edges = c.take<int64_t>(2 * E);
+    M.e_start = c.take<int64_t>(N + 1);
+    M.atom_start = c.take<int64_t>(B + 1);
+    M.order = c.take<int32_t>(N);
+    M.rpos = c.take<float>(3 * E);
+    M.recip = c.take<float>(9 * B);
+    M.rvlen = c.take<float>(3 * B);
+    M.vcell = c.take<float>(B);
+    M.geo_ws = c.take<char>((2 * B + 1) * sizeof(int64_t));
+    M.table = c.take<float4>(B * cfh::FC_TCAP);
+    M.near_ = c.take<float>(2 * E);
+    M.x0 = c.take<float>(N * D);
+    M.pooled = c.take<float>(B * D);
+    for (int i = 0; i + 1 < m->linears; i++) M.y[i] = c.take<float>(B * (size_t)m->head[i].out);
+    ModelLayerBuffers set[2];
+    for (int l = 0; l < m->layers; l++) {
+        ModelLayerBuffers& L = M.layer[l];
+        if (b->keep || l < 2) {
+            L.qs = c.take<float>(N * D); L.k = c.take<float>(N * D); L.v = c.take<float>(N * D); L.a = c.take<float>(N * H);
+            L.x2 = c.take<float>(N * D);
+            L.qkv = b->keep ? c.take<float>(N * 3 * D) : nullptr;
+            if (b->keep || l == 0) {
+                L.x1 = b->keep ? c.take<float>(N * D) : nullptr;
+                L.h = b->keep ? c.take<float>(N * F) : nullptr;
+                L.frames = c.take<float>(9 * N * H);
+                L.z = c.take<float>(E * H); L.prob = c.take<float>(E * H);
+                L.hist = c.take<float>(H * N * hw);
+                L.out = c.take<float>(N * D);
+                L.wcat = c.take<float>(D * hw);
+                L.records = c.take<uint32_t>(N * H * cfh::REC_WORDS);
+            }
+            if (l < 2) set[l] = L;
+        }
+        if (!b->keep && l > 0) {
+            L = set[0];
+            L.qs = set[l & 1].qs; L.k = set[l & 1].k; L.v = set[l & 1].v; L.a = set[l & 1].a; L.x2 = set[l & 1].x2;
+        }
+    }
+    M.total = c.off;
+    if (b->x0 && b->qkv0 && b->keep) {        // (only read)
+        M.x0 = const_cast<float*>(b->x0);
+        M.layer[0].qkv = const_cast<float*>(b->qkv0);
+    }
+}
+
+// Rows of the per-block partial sums of a layer's lattice-weight gradient: the first layer's come from
+// attention_inputs_bwd_kernel, the others' from the bridge.
+int64_t model_partial_rows(const cfh_model* m, int l, int64_t N) {
+    const int rows = l == 0 ? 4 * (256 / m->D) : cfh::BR_ROWS;
+    return (N + rows - 1) / rows;
+}
+struct ModelGrads {
+    float *gx0, *gpooled, *gy[CFH_MODEL_MAX_LINEARS], *glogit, *gq, *gk, *gv, *ga;
+    struct { float *g2, *gh, *g1, *g_attn, *gqkv, *gw_partial; } layer[MODEL_MAX_LAYERS];
+    void* wgrad_ws;
+    size_t wgrad_bytes, total;
+};
+size_t model_wgrad_bytes(const cfh_model* m, const cfh_model_batch* b);
+void model_grads(const cfh_model* m, const cfh_model_batch* b, void* scratch, ModelGrads& G) {
+    Carver c{reinterpret_cast<char*>(scratch)};
+    const size_t N = b->N, E = b->E, B = b->B, D = m->D, F = m->F, H = m->heads;
+    G.gx0 = c.take<float>(N * D);
+    G.gpooled = c.take<float>(B * D);
+    for (int i = 0; i < m->linears; i++) G.gy[i] = c.take<float>(B * (size_t)m->head[i].out);
+    G.glogit = c.take<float>(E * H);
+    G.gq = c.take<float>(N * D); G.gk = c.take<float>(N * D); G.gv = c.take<float>(N * D); G.ga = c.take<float>(N * H);
+    for (int l = 0; l < m->layers; l++) {
+        auto& L = G.layer[l];
+        L.g2 = c.take<float>(N * D); L.gh = c.take<float>(N * F); L.g1 = c.take<float>(N * D);
+        L.g_attn = c.take<float>(N * D); L.gqkv = c.take<float>(N * 3 * D);
+        L.gw_partial = c.take<float>(model_partial_rows(m, l, b->N) * D);
+    }
+    G.wgrad_bytes = model_wgrad_bytes(m, b);
+    G.wgrad_ws = c.take<char>(G.wgrad_bytes);
+    G.total = c.off;
+}
+
+int64_t model_gradient_floats(const cfh_model* m) {
+    const int64_t D = m->D, F = m->F, A = m->layer[0].core.angle_bins;
+    int64_t n = D * m->feat + m->layers * (4 * D * D + 2 * D * F + D * (64 + 3 * A) + 3 * D + D + D + F + D);
+    for (int i = 0; i < m->linears; i++) n += (int64_t)m->head[i].out * (m->head[i].in + 1);
+    return n;
+}
+
+// The products that make the weight and bias gradients of the projections (pointers filled in from M, G and grads; with
+// null buffers the list has the right sizes).
+std::vector<cfh_linear_grad_job> model_wgrad_jobs(const cfh_model* m, const cfh_model_batch* b, const ModelBuffers& M,
+                                                  const ModelGrads& G, float* grads, float** core_grads) {
+    std::vector<cfh_linear_grad_job> jobs;
+    const int64_t N = b->N, D = m->D, F = m->F, A = m->layer[0].core.angle_bins;
+    float* g = grads;
+    auto next = [&](int64_t n) { float* p = g; g += n; return p; };
+    auto job = [&](const float* x, const float* dy, float* dW, float* db, int64_t rows, int64_t I, int64_t O) {
+        jobs.push_back(cfh_linear_grad_job{x, dy, dW, db, rows, I, O, I, O});
+    };
+    job(b->x, G.gx0, next(D * m->feat), nullptr, N, m->feat, D);
+    for (int l = 0; l < m->layers; l++) {
+        const ModelLayerBuffers& L = M.layer[l];
+        float* const gWqkv = next(3 * D * D);
+        job(l ? M.layer[l - 1].x2 : M.x0, G.layer[l].gqkv, gWqkv, next(3 * D), N, D, 3 * D);
+        float* const gWo = next(D * D);
+        job(L.out, G.layer[l].g1, gWo, next(D), N, D, D);
+        // (column sums of the per-block partial sums)
+        jobs.push_back(cfh_linear_grad_job{nullptr, G.layer[l].gw_partial, nullptr, next(D), model_partial_rows(m, l, N), 1, D, 1, D});
+        for (int e = 0; e < (A > 0 ? 4 : 1); e++) {
+            float* const p = next(D * (e == 0 ? 64 : A));
+            if (core_grads) core_grads[4 * l + e] = p;
+        }
+        float* const gW1 = next(F * D);
+        job(L.x1, G.layer[l].gh, gW1, next(F), N, D, F);
+        float* const gW2 = next(D * F);
+        job(L.h, G.layer[l].g2, gW2, next(D), N, F, D);
+    }
+    for (int i = 0; i < m->linears; i++) {
+        const cfh_model_linear& T = m->head[i];
+        float* const gW = next((int64_t)T.out * T.in);
+        job(i ? M.y[i - 1] : M.pooled, G.gy[i], gW, next(T.out), b->B, T.in, T.out);
+    }
+    return jobs;
+}
+// Which jobs of that list share the slicing of their rows.  With the 64-bin and without the angle encoding all of them
+// (empty: one group); with the 16-bin encoding, whose small histograms leave the layers short, the jobs that become
+// ready together while the pass walks down the layers, so that each group spreads over the whole chip.
+std::vector<int32_t> model_wgrad_groups(const cfh_model* m) {
+    std::vector<int32_t> g;
+    const int L = m->layers;
+    if (m->layer[0].core.angle_bins != cfh::SMALL_A) return g;
+    g.push_back(L);                                          // embedding
+    for (int l = 0; l < L; l++) {
+        g.push_back(L - l);                                  // input projection
+        g.push_back(L - 1 - l);                              // output projection
+        g.push_back(L - l);                                  // lattice weights
+        g.push_back(L - 1 - l);
+        g.push_back(L - 1 - l);                              // feed-forward block
+    }
+    for (int i = 0; i < m->linears; i++) g.push_back(0);
+    return g;
+}
+size_t model_wgrad_bytes(const cfh_model* m, const cfh_model_batch* b) {
+    // (sizes and alignment are all that counts here: the pointers stand for the 256-byte aligned buffers of the pass)
+    static float dummy;
+    ModelBuffers M{};
+    ModelGrads G{};
+    std::vector<cfh_linear_grad_job> jobs = model_wgrad_jobs(m, b, M, G, nullptr, nullptr);
+    float* d = reinterpret_cast<float*>(((uintptr_t)&dummy) & ~(uintptr_t)255);
+    for (size_t j = 0; j < jobs.size(); j++) {
+        // (distinct destinations: none of them overlap)
+        if (jobs[j].I > 1 || jobs[j].x) jobs[j].x = d;
+        const bool has_w = jobs[j].I > 1;
+        jobs[j].dy = d;
+        jobs[j].dW = has_w ? d + (j << 24) : nullptr;
+        jobs[j].db = has_w ? nullptr : d + (j << 24);
+    }
+    if ((int)jobs.size() > cfh::WGRAD_MAX_JOBS)
+        return cfh_linear_weight_bias_grad_batch_workspace_bytes(jobs.data(), (int32_t)jobs.size());
+    const std::vector<int32_t> group = model_wgrad_groups(m);
+    cfh::WgradJobs T;
+    plan_wgrad(jobs.data(), 0, (int32_t)jobs.size(), T, group.empty() ? nullptr : group.data());
+    return 256 + (size_t)T.blocks * cfh::WG_PART * sizeof(float);
+}
+
+void tail_args(const cfh_model* m, const cfh_model_batch* b, const ModelBuffers& M, cfh::TailArgs& T) {
+    std::memset(&T, 0, sizeof(T));
+    T.atom_start = M.atom_start; T.pooled = M.pooled;
+    T.B = (int)b->B; T.D = m->D; T.nlin = m->linears;
+    // (with 256 crystals and more every compute unit has a workgroup of its own already)
+    T.per_wg = b->B <= 512 ? 1 : (b->B <= 2048 ? 4 : cfh::TAIL_ROWS);
+    int widest = m->D;
+    for (int i = 0; i < m->linears; i++) {
+        cfh::TailLinear& L = T.lin[i];
+        L.W = m->head[i].W; L.b = m->head[i].b; L.K = m->head[i].in; L.O = m->head[i].out; L.relu = m->head[i].relu;
+        L.y = i + 1 < m->linears ? M.y[i] : nullptr;
+        if (L.O > widest) widest = L.O;
+    }
+    T.ld = (widest + 3) / 4 * 4 + cfh::TAIL_PAD;
+}
+int tail_launch(const cfh::TailArgs& T, const float* gout, hipStream_t st) {
+    const dim3 grid((unsigned)((T.B + T.per_wg - 1) / T.per_wg)), block(64 * cfh::TAIL_WAVES);
+    const size_t lds = 2 * (size_t)cfh::TAIL_ROWS * T.ld * sizeof(float);
+    if (gout) hipLaunchKernelGGL(cfh::model_tail_bwd_kernel, grid, block, lds, st, T, gout);
+    else hipLaunchKernelGGL(cfh::model_tail_fwd_kernel, grid, block, lds, st, T);
+    return finish_launch("model_tail");
+}
+int set_dynamic_lds(const void* kernel, int* set, size_t lds, const char* what) {
+    int dev = 0;
+    if (lds > 160 * 1024) return fail(CFH_EINVAL, "%s: %zu bytes of LDS needed", what, lds);
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return fail(CFH_ELAUNCH, "%s: no current device", what);
+    if (set[dev] < (int)lds) {
+        if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+            return fail(CFH_ELAUNCH, "%s: %zu bytes of LDS refused", what, lds);
+        set[dev] = (int)lds;
+    }
+    return CFH_OK;
+}
+}  // namespace
+
+extern "C" {
+
+int64_t cfh_model_sizes(const cfh_model* m, const cfh_model_batch* b, size_t bytes[4]) {
+    if (int rc = check_model(m, b)) return rc;
+    if (!bytes) return fail(CFH_EINVAL, "bytes must not be NULL");
+    cfh_model_batch q = *b;
+    q.arena = nullptr;
+    ModelBuffers M{};
+    model_buffers(m, &q, M);
+    bytes[0] = M.total;
+    bytes[1] = core_layout(&m->layer[0].core, b->N, b->E, b->B, false).total;
+    bytes[2] = bytes[3] = 0;
+    if (b->keep) {
+        ModelGrads G{};
+        model_grads(m, &q, nullptr, G);
+        bytes[2] = G.total;
+        bytes[3] = core_layout(&m->layer[0].core, b->N, b->E, b->B, true).total;
+        const size_t wg = cfh_fused_core_weight_gradients_workspace_bytes(&m->layer[0].core, m->layers);
+        if (wg > bytes[3]) bytes[3] = wg;
+    }
+    return model_gradient_floats(m);
+}
+
+int cfh_model_forward(const cfh_model* m, const cfh_model_batch* b, float* out) {
+    int rc = check_model(m, b);
+    if (rc) return rc;
+    if (!b->x || !b->pos || !b->batch || !b->tvecs || !b->sizes || !out)
+        return fail(CFH_EINVAL, "model: x, pos, batch, tvecs, sizes and out must not be NULL");
+    ModelBuffers M{};
+    model_buffers(m, b, M);
+    if (!b->arena || b->arena_bytes < M.total || ((uintptr_t)b->arena & 255))
+        return fail(CFH_EWORKSPACE, "model: arena of %zu bytes (256-byte aligned) needed, %zu given", M.total, b->arena_bytes);
+    hipStream_t st = (hipStream_t)b->stream;
+    const int64_t N = b->N, E = b->E, B = b->B;
+    const int D = m->D, F = m->F, H = m->heads;
+    if ((rc = cfh_crystal_geometry(b->pos, b->batch, b->tvecs, b->sizes, N, B, E, M.edges, M.rpos, M.recip, M.rvlen, M.vcell,
+                                   M.e_start, M.atom_start, M.order, M.geo_ws, (2 * (size_t)B + 1) * sizeof(int64_t), b->stream)))
+        return rc;
+    {   // embedding and the inputs of the first layer
+        const cfh_model_layer& L = m->layer[0];
+        const ModelLayerBuffers& Y = M.layer[0];
+        if (b->x0 && b->qkv0) {
+            if (!b->keep) return fail(CFH_EINVAL, "model: x0 and qkv0 are taken with keep only");
+            if ((rc = cfh_attention_inputs_forward(Y.qkv, L.lattice_w, L.gauss_scale_dev, L.c1, L.lb, L.c2, L.q_scale, N, H,
+                                                   cfh::DH, Y.qs, Y.k, Y.v, Y.a, b->stream)))
+                return rc;
+        } else {
+            static int lds_set[64] = {0};
+            const size_t lds = cfh::bridge_front_lds_floats(D, m->feat) * sizeof(float);
+            if ((rc = set_dynamic_lds((const void*)cfh::layer_front_fwd_kernel, lds_set, lds, "layer front"))) return rc;
+            cfh::BridgeArgs A{};
+            A.attn = b->x; A.Wo = m->We; A.x2 = M.x0;
+            A.Wq = L.Wqkv; A.bq = L.bqkv; A.lattice_w = L.lattice_w; A.gauss = L.gauss_scale_dev;
+            A.qkv = Y.qkv; A.qs = Y.qs; A.k = Y.k; A.v = Y.v; A.a = Y.a;
+            A.N = (int)N; A.D = D; A.H = H;
+            A.c1 = L.c1; A.lb = L.lb; A.c2 = L.c2; A.q_scale = L.q_scale;
+            hipLaunchKernelGGL(cfh::layer_front_fwd_kernel, dim3((unsigned)((N + cfh::BR_ROWS - 1) / cfh::BR_ROWS)),
+                               dim3(64 * cfh::BR_WAVES), lds, st, A, m->feat);
+            if ((rc = finish_launch("layer_front_forward"))) return rc;
+        }
+    }
+    for (int l = 0; l < m->layers; l++) {
+        const cfh_model_layer& L = m->layer[l];
+        const ModelLayerBuffers& Y = M.layer[l];
+        cfh_params p = L.core;
+        if (b->noise_seeds) p.noise_seed = b->noise_seeds[l];
+        const bool ready = l > 0 && same_tables(m->layer[l - 1], L);
+        const cfh_core_cache cache{reinterpret_cast<float*>(M.table), M.near_, Y.wcat, Y.records, ready ? 1 : 0, 0, 0, 0};
+        const bool ang = p.angle_bins > 0;
+        if ((rc = cfh_fused_core_forward(&p, Y.qs, Y.k, Y.v, Y.a, M.rpos, b->tvecs, L.adaptive ? M.rvlen : nullptr, b->batch,
+                                         M.edges, M.e_start, M.order, L.W_dist, ang ? L.W_axis1 : nullptr,
+                                         ang ? L.W_axis2 : nullptr, ang ? L.W_axis3 : nullptr, N, E, B,
+                                         ang ? Y.frames : nullptr, ang ? 1 : 0, Y.z, Y.prob, Y.hist, Y.out, &cache,
+                                         b->workspace, b->workspace_bytes, b->stream)))
+            return rc;
+        const bool next = l + 1 < m->layers;
+        const cfh_model_layer& Ln = m->layer[next ? l + 1 : l];
+        const ModelLayerBuffers& Yn = M.layer[next ? l + 1 : l];
+        if ((rc = cfh_layer_bridge_forward(Y.out, l ? M.layer[l - 1].x2 : M.x0, N, D, F, L.Wo, L.bo, L.W1, L.b1, L.W2, L.b2,
+                                           next ? Ln.Wqkv : nullptr, Ln.bqkv, Ln.lattice_w, Ln.gauss_scale_dev, Ln.c1, Ln.lb,
+                                           Ln.c2, Ln.q_scale, H, Y.x1, Y.h, Y.x2, Yn.qkv, Yn.qs, Yn.k, Yn.v, Yn.a, b->stream)))
+            return rc;
+    }
+    cfh::TailArgs T;
+    tail_args(m, b, M, T);
+    T.x = M.layer[m->layers - 1].x2;
+    T.lin[m->linears - 1].y = out;
+    return tail_launch(T, nullptr, st);
+}
+
+int cfh_model_backward(const cfh_model* m, const cfh_model_batch* b, const float* gout, void* scratch,
+                       size_t scratch_bytes, float* grads) {
+    int rc = check_model(m, b);
+    if (rc) return rc;
+    if (!b->x || !b->pos || !b->batch || !b->tvecs || !b->sizes || !gout || !grads || !b->keep)
+        return fail(CFH_EINVAL, "model backward: the forward's inputs (with keep), gout and grads must not be NULL");
+    ModelBuffers M{};
+    model_buffers(m, b, M);
+    if (!b->arena || b->arena_bytes < M.total || ((uintptr_t)b->arena & 255))
+        return fail(CFH_EWORKSPACE, "model: arena of %zu bytes (256-byte aligned) needed, %zu given", M.total, b->arena_bytes);
+    ModelGrads G{};
+    model_grads(m, b, scratch, G);
+    if (!scratch || scratch_bytes < G.total || ((uintptr_t)scratch & 255))
+        return fail(CFH_EWORKSPACE, "model: scratch of %zu bytes (256-byte aligned) needed, %zu given", G.total, scratch_bytes);
+    if (m->head[m->linears - 1].relu) return fail(CFH_EINVAL, "model: a rectifier behind the last linear layer");
+    hipStream_t st = (hipStream_t)b->stream;
+    const int64_t N = b->N, E = b->E, B = b->B;
+    const int D = m->D, F = m->F, H = m->heads;
+    cfh::TailArgs T;
+    tail_args(m, b, M, T);
+    for (int i = 0; i < m->linears; i++) T.lin[i].gy = G.gy[i];
+    T.gpooled = G.gpooled;
+    if ((rc = tail_launch(T, gout, st))) return rc;
+
+    static int lds_set[64] = {0};
+    const size_t lds = cfh::bridge_bwd_lds_floats(D, F) * sizeof(float);
+    if ((rc = set_dynamic_lds((const void*)cfh::layer_bridge_bwd_kernel, lds_set, lds, "layer bridge backward"))) return rc;
+    const dim3 bridge_grid((unsigned)((N + cfh::BR_ROWS - 1) / cfh::BR_ROWS)), bridge_block(64 * cfh::BR_WAVES);
+    for (int l = m->layers - 1; l >= 0; l--) {
+        // the projections between the core of layer l and the inputs of layer l + 1
+        cfh::BridgeBwdArgs A{};
+        A.N = (int)N; A.D = D; A.F = F; A.H = H;
+        if (l + 1 < m->layers) {
+            const cfh_model_layer& Ln = m->layer[l + 1];
+            A.g_x2 = G.layer[l + 1].g1;
+            A.Wq = Ln.Wqkv; A.ai_w = Ln.lattice_w; A.ai_gauss = Ln.gauss_scale_dev;
+            A.ai_qkv = M.layer[l + 1].qkv;
+            A.ai_gqs = G.gq; A.ai_gk = G.gk; A.ai_gv = G.gv; A.ai_ga = G.ga;
+            A.gqkv_out = G.layer[l + 1].gqkv; A.gw_partial = G.layer[l + 1].gw_partial;
+            A.c1 = Ln.c1; A.lb = Ln.lb; A.c2 = Ln.c2; A.q_scale = Ln.q_scale;
+        } else {
+            A.g_x2 = G.gpooled; A.batch = b->batch; A.atom_start = M.atom_start;
+        }
+        const cfh_model_layer& L = m->layer[l];
+        const ModelLayerBuffers& Y = M.layer[l];
+        A.g2 = G.layer[l].g2;
+        A.h = Y.h; A.W2 = L.W2; A.W1 = L.W1; A.Wo = L.Wo;
+        A.gh = G.layer[l].gh; A.g1 = G.layer[l].g1; A.g_attn = G.layer[l].g_attn;
+        hipLaunchKernelGGL(cfh::layer_bridge_bwd_kernel, bridge_grid, bridge_block, lds, st, A);
+        if ((rc = finish_launch("layer_bridge_backward"))) return rc;
+        cfh_params p = L.core;
+        p.flags |= CFH_FLAG_NO_WEIGHT_GRADS;
+        // (the table in the arena is that of the last layer whose box rule differs from its predecessor's)
+        bool table_ready = true;
+        for (int u = l + 1; u < m->layers; u++) table_ready = table_ready && same_tables(L, m->layer[u]);
+        const cfh_core_cache cache{reinterpret_cast<float*>(M.table), nullptr, Y.wcat, Y.records, table_ready ? 1 : 0, 1, 1, 0};
+        const bool ang = p.angle_bins > 0;
+        if ((rc = cfh_fused_core_backward(&p, Y.qs, Y.k, Y.v, Y.a, M.rpos, b->tvecs, L.adaptive ? M.rvlen : nullptr, b->batch,
+                                          M.edges, M.e_start, M.order, L.W_dist, ang ? L.W_axis1 : nullptr,
+                                          ang ? L.W_axis2 : nullptr, ang ? L.W_axis3 : nullptr, ang ? Y.frames : nullptr, Y.z,
+                                          Y.prob, Y.hist, Y.out, G.layer[l].g_attn, N, E, B, G.gq, G.gk, G.gv, G.ga, G.glogit,
+                                          nullptr, nullptr, nullptr, nullptr, &cache, b->workspace, b->workspace_bytes,
+                                          b->stream)))
+            return rc;
+    }
+    {   // the inputs of the first layer: gradient of its projection, of the embedded atoms (projection + residual)
+        const cfh_model_layer& L = m->layer[0];
+        auto& g = G.layer[0];
+        if ((rc = cfh_attention_inputs_backward(M.layer[0].qkv, L.lattice_w, L.gauss_scale_dev, L.c1, L.lb, L.c2, L.q_scale, G.gq,
+                                                G.gk, G.gv, G.ga, N, H, cfh::DH, g.gqkv, nullptr, g.gw_partial,
+                                                (size_t)model_partial_rows(m, 0, N) * D * sizeof(float), b->stream)))
+            return rc;
+        hipLaunchKernelGGL(cfh::small_linear_dx_kernel, dim3((unsigned)((N + 63) / 64), (unsigned)((D + 63) / 64)), dim3(256), 0,
+                           st, g.gqkv, L.Wqkv, g.g1, G.gx0, (int)N, 3 * D, D);
+        if ((rc = finish_launch("layer_front_backward"))) return rc;
+    }
+    // the weight gradients of the whole pass: the projections, then the cores
+    std::vector<float*> core_grads(4 * (size_t)m->layers, nullptr);
+    const std::vector<cfh_linear_grad_job> jobs = model_wgrad_jobs(m, b, M, G, grads, core_grads.data());
+    const std::vector<int32_t> group = model_wgrad_groups(m);
+    if ((rc = linear_wgrad_batch_impl(jobs.data(), (int32_t)jobs.size(), G.wgrad_ws, G.wgrad_bytes, b->stream, true,
+                                      group.empty() ? nullptr : group.data())))
+        return rc;
+    std::vector<cfh_core_wgrad_job> cj;
+    for (int l = 0; l < m->layers; l++) {
+        cj.push_back(cfh_core_wgrad_job{G.layer[l].g_attn, M.layer[l].hist, N, core_grads[4 * l], core_grads[4 * l + 1],
+                                        core_grads[4 * l + 2], core_grads[4 * l + 3]});
+        // (layers whose encodings have the same constants go together)
+        const bool last = l + 1 == m->layers;
+        const cfh_params &p = m->layer[l].core, &q = m->layer[last ? l : l + 1].core;
+        if (last || p.dist_coef != q.dist_coef || p.angle_coef != q.angle_coef || p.angle_wscale != q.angle_wscale) {
+            if ((rc = core_weight_gradients_impl(&p, cj.data(), (int32_t)cj.size(), b->workspace, b->workspace_bytes, b->stream,
+                                                 true)))
+                return rc;
+            cj.clear();
+        }
+    }
+    return CFH_OK;
+}
+
+}  // extern "C"

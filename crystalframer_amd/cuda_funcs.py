@@ -103,7 +103,8 @@ def _fused_core_default() -> bool:
 
 # --------------------------------------------------------------------------------------------------
 def _params(H: int, Dh: int, K: int, A: int, cos_abs: int, dist_max: float, wscale: float,
-            angle_wscale: float, dist_coef: float, angle_coef: float, cutoff_radius) -> _lib.CfhParams:
+            angle_wscale: float, dist_coef: float, angle_coef: float, cutoff_radius,
+            noise_seed: Optional[int] = None) -> _lib.CfhParams:
     p = _lib.CfhParams()
     p.struct_size = ctypes.sizeof(_lib.CfhParams)
     p.num_heads, p.head_dim, p.dist_bins, p.angle_bins = H, Dh, K, A
@@ -116,7 +117,9 @@ def _params(H: int, Dh: int, K: int, A: int, cos_abs: int, dist_max: float, wsca
     p.cutoff_radius = 0.0 if cutoff_radius is None else float(cutoff_radius)
     p.prune_log2 = float(KernelManager.PRUNE_LOG2)
     p.symm_break_noise = float(KernelManager.SYMM_BREAK_NOISE)
-    if KernelManager.NOISE_SEED is None:
+    if noise_seed is not None:
+        p.noise_seed = int(noise_seed)
+    elif KernelManager.NOISE_SEED is None:
         p.noise_seed = int(torch.randint(0, 2 ** 62, (1,)).item()) if p.symm_break_noise > 0 else 0
     else:
         p.noise_seed = int(KernelManager.NOISE_SEED)

@@ -11,7 +11,7 @@ import copy
 import torch
 from torch import nn
 
-from . import cuda_funcs
+from . import cuda_funcs, model_pass
 from .encoder import CrystalformerEncoderCUDA
 from .params import LatticeformerParams, ModelParams
 
@@ -106,6 +106,9 @@ class Latticeformer(nn.Module):
 
     def forward(self, data, this_epoch=None):
         """``data`` carries x (N,98), pos (N,3), batch (N), trans_vec (B,3,3), sizes (B)."""
+        out = model_pass.run(self, data)         # the whole pass as one library call, where that covers it
+        if out is not None:
+            return out
         x = cuda_funcs.linear(data.x, self.input_embeddings.weight, self.input_embeddings.bias)
         num_pairs = getattr(data, "num_pairs", -1)
         x = self.encoder(x, data.pos, data.batch, data.trans_vec, data.sizes, this_epoch=this_epoch,

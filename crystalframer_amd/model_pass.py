@@ -1,0 +1,371 @@
+"""The whole model in one library call per direction (cfh_model_forward / cfh_model_backward).
+
+``Latticeformer.forward`` comes here first.  When the model and the batch are of the kind the library call covers (the
+default architecture: no layer norm, no dropout, ReLU, "max" frames, mean pooling, a head of linear layers; float32
+batches whose pair count is known on the host), the pass is ONE autograd function: embedding, geometry, layers, pooling and head
+are enqueued by native code, the backward pass with all parameter gradients likewise.  Everything else takes the modules'
+own forward: same kernels, one autograd function per operator.
+
+The modules' path makes some thirty (inference) to eighty (training) calls from Python, each with its own allocations,
+argument structures and autograd nodes: 755 us of host time per inference pass and 2330 us per training step of the
+4-layer model, whatever the batch, where the GPU needs 250 us for one crystal and 730 us for a training step on 13.
+"""
+from __future__ import annotations
+
+import ctypes
+import math
+
+import torch
+from torch import nn
+
+from . import _lib
+
+ENABLED = True
+
+
+def _no_plan():
+    return None
+
+
+class _Plan:
+    """What a model's passes share: its parameters in the library's order, the structures that hold their addresses, and
+    the objects all of it was derived from.  ``current()`` is False as soon as a module or parameter was exchanged or a
+    parameter got another storage; the plan is then made again.  The plan keeps the storages it points at alive."""
+
+    def __init__(self, model):
+        self.links = []          # (dict, key, value): the plan holds while dict[key] is value
+        self.params = []         # in the order of the library's gradients
+        self.ok = False
+        self.tables = {}         # kernel constants -> (layer structures, objects kept alive)
+        self.hooked = []         # modules whose hooks the library call would pass over
+        self.attn = []
+        self._collect(model)
+        self.ptrs = [p.data_ptr() for p in self.params]
+        if self.ok:
+            self.alive = [p.detach() for p in self.params]
+
+    def __reduce_ex__(self, protocol):       # copies and pickles of a model carry no plan (addresses of the original)
+        return _no_plan, ()
+
+    def current(self) -> bool:
+        for d, k, v in self.links:
+            if d.get(k) is not v:
+                return False
+        return [p.data_ptr() for p in self.params] == self.ptrs
+
+    def _child(self, module, *names):
+        for n in names:
+            child = module._modules.get(n)
+            self.links.append((module._modules, n, child))
+            module = child
+            if module is None:
+                return None
+        return module
+
+    def _param(self, module, name):
+        p = module._parameters.get(name)
+        self.links.append((module._parameters, name, p))
+        return p
+
+    def _collect(self, model):
+        from . import cuda_funcs
+        from .latticeformer import avr_pool
+        enc = self._child(model, "encoder")
+        emb = self._child(model, "input_embeddings")
+        mlp = self._child(model, "mlp")
+        pre = self._child(model, "proj_before_pooling")
+        self.links.append((model.__dict__, "pooling_layer", model.__dict__.get("pooling_layer")))
+        if not (isinstance(emb, nn.Linear) and isinstance(mlp, nn.Sequential) and isinstance(pre, nn.Identity)
+                and model.__dict__.get("pooling_layer") is avr_pool and enc is not None and enc._modules.get("norm") is None):
+            return
+        self.links.append((enc._modules, "norm", enc._modules.get("norm")))
+        self.hooked.append(enc)
+        layers = self._child(enc, "layers")
+        We = self._param(emb, "weight")
+        if self._param(emb, "bias") is not None or len(layers) < 1:
+            return
+        self.params.append(We)
+        self.layers = []
+        for name in layers._modules:
+            layer = self._child(layers, name)
+            at = self._child(layer, "self_attn")
+            out_proj = self._child(at, "out_proj")
+            l1, l2 = self._child(layer, "linear1"), self._child(layer, "linear2")
+            for n in ("norm1", "norm2", "dropout", "dropout1", "dropout2"):
+                if not isinstance(self._child(layer, n), nn.Identity):
+                    return
+            self.links.append((layer.__dict__, "activation", layer.activation))
+            P = at.params
+            A = P.value_pe_angle_real
+            if not (layer.activation is torch.nn.functional.relu and P.frame_method == "max" and at.kdim == at.vdim == enc.d_model
+                    and P.value_pe_dist_real > 0 and at.head_dim == 16
+                    and cuda_funcs.AttentionInputsHIP.supported(at.num_heads, at.head_dim)):
+                return
+            names = ["q_proj_weight", "k_proj_weight", "v_proj_weight", "in_proj_bias"]
+            ps = [self._param(at, n) for n in names] + [self._param(out_proj, "weight"), self._param(out_proj, "bias"),
+                                                        self._param(at, "lattice_pos_weights"), self._param(at, "pe_dist_proj")]
+            if A > 0:
+                ps += [self._param(at, f"proj_angle{n}") for n in (1, 2, 3)]
+            ps += [self._param(l1, "weight"), self._param(l1, "bias"), self._param(l2, "weight"), self._param(l2, "bias")]
+            gauss = self._param(at, "gauss_scale")
+            if any(p is None for p in ps):
+                return
+            if not (cuda_funcs.LayerBridgeHIP.supported(enc.d_model, l1.out_features, at.num_heads)
+                    and cuda_funcs.LayerBridgeHIP.backward_supported(enc.d_model, l1.out_features)
+                    and cuda_funcs.PeriodicAttentionCoreHIP.supported(
+                        P.value_pe_dist_real, A, P.value_pe_dist_wscale, P.value_pe_angle_wscale, at.pe_dist_proj,
+                        at.proj_angle1 if A > 0 else None)):
+                return
+            self.params += ps
+            self.attn.append(at)
+            self.layers.append((at, ps, gauss, A))
+        self.head = []
+        mods = []
+        for name in mlp._modules:
+            m = self._child(mlp, name)
+            if isinstance(m, nn.Linear):
+                W, b = self._param(m, "weight"), self._param(m, "bias")
+                if b is None:
+                    return
+                mods.append([m, W, b, 0])
+            elif isinstance(m, nn.ReLU) and mods and not mods[-1][3]:
+                mods[-1][3] = 1
+            elif not isinstance(m, nn.Identity):
+                return
+        D = enc.d_model
+        if not 1 <= len(mods) <= _lib.MODEL_MAX_LINEARS or mods[-1][3] or D > _lib.MODEL_MAX_WIDTH or len(self.attn) > 64:
+            return
+        width = D
+        for m, W, b, relu in mods:
+            if m.in_features != width or width % 16 or m.out_features > _lib.MODEL_MAX_WIDTH:
+                return
+            width = m.out_features
+            self.params += [W, b]
+        self.head, self.out_features = mods, width
+        self.D, self.F, self.H, self.feat = D, self.layers[0][1][-4].shape[0], self.attn[0].num_heads, We.shape[1]
+        dev = We.device
+        if not We.is_cuda or not 1 <= self.feat <= 512 or We.shape[0] != D:
+            return
+        for p in self.params:
+            if p.dtype != torch.float32 or p.device != dev or not p.is_contiguous():
+                return
+        for at, ps, gauss, A in self.layers:
+            if (ps[-4].shape[0] != self.F or at.num_heads != self.H or A != self.layers[0][3]
+                    or gauss.device != dev or gauss.dtype != torch.float32
+                    or any(w.dim() == 4 and w.shape[0] != 1 for w in ps)):
+                return
+            stack = at._stacked_in_proj()    # query, key and value weights as adjacent rows of one storage
+            if at is self.attn[0]:
+                self.in_proj = stack.detach()
+        # the gradients lie one behind the other: every one but the last starts on 16 bytes
+        if any(p.numel() % 4 for p in self.params[:-1]):
+            return
+        self.gauss = [g for _, _, g, _ in self.layers]
+        self.embedding, self.in_proj_bias = We.detach(), self.layers[0][1][3].detach()
+        self.device = dev
+        self.ok = True
+
+    # ---- structures of the library call
+    def constants(self):
+        """What the attention cores take from KernelManager, as a key of ``tables``."""
+        from .cuda_funcs import KernelManager as K
+        sd = K.NOISE_SEED_DEVICE
+        return (K.LATTICE_RANGE, K.MINIMUM_RANGE, K.CORE_WINDOW_MODE, K.PRUNE_LOG2, K.SYMM_BREAK_NOISE, K.NOISE_SEED,
+                None if sd is None else sd.data_ptr(), bool(K.COLLECT_STATS), tuple([g.data_ptr() for g in self.gauss]))
+
+    def table(self):
+        key = self.constants()
+        got = self.tables.get(key)
+        if got is None:
+            if len(self.tables) >= 8:
+                self.tables.clear()
+            got = self.tables[key] = self._build_table()
+        return got
+
+    def _build_table(self):
+        from . import cuda_funcs
+        K = cuda_funcs.KernelManager
+        arr = (_lib.CfhModelLayer * len(self.layers))()
+        seed = K.NOISE_SEED
+        for S, (at, ps, gauss, A) in zip(arr, self.layers):
+            P = at.params
+            dist_max = P.value_pe_dist_max if P.value_pe_dist_max >= 0 else -P.value_pe_dist_max * P.scale_real
+            cutoff = None
+            if P.adaptive_cutoff_sigma != 0:
+                cutoff = (P.adaptive_cutoff_sigma if P.adaptive_cutoff_sigma < 0
+                          else P.scale_real * P.gauss_lb_real ** (-0.5) * P.adaptive_cutoff_sigma)
+            p = cuda_funcs._params(at.num_heads, at.head_dim, P.value_pe_dist_real, A, P.cos_abs, dist_max,
+                                   P.value_pe_dist_wscale, P.value_pe_angle_wscale, P.value_pe_dist_coef,
+                                   P.value_pe_angle_coef, cutoff, noise_seed=0 if seed is None else seed)
+            p.window_mode = int(K.CORE_WINDOW_MODE)
+            S.core = p
+            q, _, _, bq, Wo, bo, lw, Wd = ps[:8]
+            S.Wqkv, S.bqkv, S.lattice_w = q.data_ptr(), bq.data_ptr(), lw.data_ptr()
+            S.gauss_scale_dev = gauss.data_ptr() if P.normalize_gauss else None
+            S.W_dist, S.Wo, S.bo = Wd.data_ptr(), Wo.data_ptr(), bo.data_ptr()
+            if A > 0:
+                S.W_axis1, S.W_axis2, S.W_axis3 = (w.data_ptr() for w in ps[8:11])
+            S.W1, S.b1, S.W2, S.b2 = (w.data_ptr() for w in ps[-4:])
+            S.c1, S.lb, S.c2 = at._gauss_constants()
+            S.q_scale = 1.0 / math.sqrt(at.head_dim)
+            S.adaptive = 1 if cutoff is not None else 0
+        m = _lib.CfhModel()
+        m.struct_size = ctypes.sizeof(_lib.CfhModel)
+        m.layers, m.heads, m.D, m.F, m.feat, m.linears = len(self.layers), self.H, self.D, self.F, self.feat, len(self.head)
+        m.We = self.params[0].data_ptr()
+        m.layer = ctypes.cast(arr, ctypes.POINTER(_lib.CfhModelLayer))
+        for T, (mod, W, b, relu) in zip(m.head, self.head):
+            T.W, T.b, T.K, T.O, T.relu = W.data_ptr(), b.data_ptr(), mod.in_features, mod.out_features, relu
+        return m, arr, K.NOISE_SEED_DEVICE, list(self.gauss)
+
+
+def _switches_default() -> bool:
+    """The switches that choose between the kernels' variants from Python stand where this path stands."""
+    from . import attention, cuda_funcs, encoder, geometry
+    K = cuda_funcs.KernelManager
+    return (ENABLED and attention.FUSED_CORE and attention.FUSED_INPUTS and encoder.FUSED_LAYER_BRIDGE and geometry.USE_LIBRARY
+            and cuda_funcs.LayerBridgeHIP.FUSED_BACKWARD and K.DEFER_WEIGHT_GRADS and K.DEFER_CORE_WEIGHT_GRADS
+            and K.DETERMINISTIC_WEIGHT_GRADIENTS and not K.GRAD_COEF_QUIRK and K.EVENT_LOG is None)
+
+
+def _arena(nbytes: int, dev) -> torch.Tensor:
+    """Memory of a pass.  Sizes are rounded up to an eighth of their power of two: the batches of an epoch differ a little from each
+    other, and the framework's allocator then finds a block to use again."""
+    step = max(1 << 9, 1 << max(nbytes.bit_length() - 4, 0))
+    return torch.empty((nbytes + step - 1) // step * step, dtype=torch.uint8, device=dev)
+
+
+def _sizes(m, b):
+    out = (ctypes.c_size_t * 4)()
+    n = _lib.load().cfh_model_sizes(m, b, out)
+    if n < 0:
+        _lib.check(int(n), "cfh_model_sizes")
+    return n, out
+
+
+def _forward(plan, data, keep: bool):
+    """(out, what the backward pass needs)."""
+    from .cuda_funcs import KernelManager as K, LinearHIP
+    lib = _lib.load()
+    m, arr, seed_dev, gauss = plan.table()
+    dev = plan.device
+    x, pos, batch, trans, sizes, E = data
+    N, B = x.shape[0], trans.shape[0]
+    b = _lib.CfhModelBatch(x.data_ptr(), pos.data_ptr(), batch.data_ptr(), trans.data_ptr(), sizes.data_ptr(), N, B, E)
+    b.keep = 1 if keep else 0
+    first = None
+    if keep and N > LinearHIP.SMALL_ROWS:
+        # the embedding and the first projection of a long batch as the modules' path makes them, by the framework's
+        # GEMM: a training step is then the same to the last bit whichever path makes it
+        x0 = torch.nn.functional.linear(x, plan.embedding)
+        first = (x0, torch.nn.functional.linear(x0, plan.in_proj, plan.in_proj_bias))
+        b.x0, b.qkv0 = first[0].data_ptr(), first[1].data_ptr()
+    seeds = None
+    if K.NOISE_SEED is None and K.SYMM_BREAK_NOISE > 0:
+        seeds = (ctypes.c_uint64 * len(arr))(*[int(torch.randint(0, 2 ** 62, (1,)).item()) for _ in arr])
+        b.noise_seeds = seeds
+    total, nbytes = _sizes(m, b)
+    arena = _arena(nbytes[0], dev)
+    ws = _lib.workspace(dev, nbytes[1])
+    out = torch.empty((B, plan.out_features), dtype=torch.float32, device=dev)
+    b.arena, b.arena_bytes = arena.data_ptr(), arena.numel()
+    b.workspace, b.workspace_bytes = ws.data_ptr(), ws.numel()
+    b.stream = _lib.raw_stream(dev)
+    rc = lib.cfh_model_forward(m, b, out.data_ptr())
+    if rc:
+        _lib.check(rc, "cfh_model_forward")
+    return out, (m, arr, seed_dev, gauss, b, seeds, total, tuple(nbytes), arena, first)
+
+
+class ModelPassHIP(torch.autograd.Function):
+    """The model's forward pass as one node; see the module's docstring.  ``params``: the plan's parameters."""
+
+    @staticmethod
+    def forward(ctx, plan, data, *params):
+        out, kept = _forward(plan, data, True)
+        ctx.plan, ctx.kept, ctx.device = plan, kept[:-2], plan.device
+        ctx.versions = [p._version for p in params] + [g._version for g in plan.gauss]
+        ctx.save_for_backward(kept[-2], *data[:5], *(kept[-1] or ()))
+        ctx.set_materialize_grads(False)
+        return out
+
+    @staticmethod
+    def backward(ctx, gout):
+        plan = ctx.plan
+        arena, *_ = ctx.saved_tensors
+        if gout is None:
+            return (None,) * (2 + len(plan.params))
+        if [p._version for p in plan.params] + [g._version for g in plan.gauss] != ctx.versions:
+            raise RuntimeError("one of the variables needed for gradient computation has been modified by an inplace operation: "
+                               "a parameter of the model changed between its forward and its backward pass")
+        m, arr, seed_dev, gauss, b, seeds, total, nbytes = ctx.kept
+        dev = ctx.device
+        lib = _lib.load()
+        gout = gout.detach().to(torch.float32).contiguous()
+        grads = torch.empty(total, dtype=torch.float32, device=dev)
+        scratch = _arena(nbytes[2], dev)
+        with torch.cuda.device(dev):
+            ws = _lib.workspace(dev, nbytes[3])
+            q = _lib.CfhModelBatch.from_buffer_copy(b)
+            q.workspace, q.workspace_bytes, q.stream = ws.data_ptr(), ws.numel(), _lib.raw_stream(dev)
+            rc = lib.cfh_model_backward(m, q, gout.data_ptr(), scratch.data_ptr(), scratch.numel(), grads.data_ptr())
+        _lib.check(rc, "cfh_model_backward")
+        views = torch._C._nn.unflatten_dense_tensors(grads, plan.params)
+        del grads            # autograd adopts a view as .grad only if nobody else holds it
+        return (None, None, *views)
+
+
+def run(model, data):
+    """The model's output for ``data``, or None when the pass is not one this path covers."""
+    if not _switches_default():
+        return None
+    plan = model.__dict__.get("_pass_plan")
+    if plan is None or not plan.current():
+        plan = model.__dict__["_pass_plan"] = _Plan(model)
+    if not plan.ok:
+        return None
+    x, pos, batch, trans, sizes = data.x, data.pos, data.batch, data.trans_vec, data.sizes
+    if sizes is None or torch.is_autocast_enabled():
+        return None
+    dev = plan.device
+    f32, i64 = torch.float32, torch.int64
+    if not (x.dtype is f32 and pos.dtype is f32 and trans.dtype is f32 and batch.dtype is i64 and sizes.dtype is i64
+            and x.dim() == 2 and x.shape[1] == plan.feat and x.shape[0] > 0
+            and x.device == dev and pos.device == dev and trans.device == dev and batch.device == dev and sizes.device == dev
+            and x.is_contiguous() and pos.is_contiguous() and trans.is_contiguous() and batch.is_contiguous()
+            and sizes.is_contiguous()):
+        return None
+    for at in plan.attn:
+        if at.frame_sink is not None or at.grad_sink is not None:
+            return None
+        if at.params.normalize_gauss and not at._gauss_scale_ready():
+            return None
+    for mod in plan.hooked:
+        if mod._forward_hooks or mod._forward_pre_hooks or mod._backward_hooks or mod._backward_pre_hooks:
+            return None
+    if not getattr(data, "zero_based", False):       # the reference subtracts batch[0]
+        batch = batch - batch[0]
+    E = getattr(data, "num_pairs", -1)
+    if E is None or E < 0:                           # not known on the host: read back, as the modules' path does
+        E = int((sizes * sizes).sum().item())
+    if E < 1:
+        return None
+    lim = 1 << 30
+    if x.shape[0] * plan.D >= lim or E * max(plan.H, 3) >= lim:
+        return None
+    args = (x, pos, batch, trans, sizes, int(E))
+    if torch.is_grad_enabled():
+        if x.requires_grad or pos.requires_grad or trans.requires_grad:
+            return None
+        wants = [p.requires_grad for p in plan.params]
+        if all(wants):
+            if torch.cuda.current_device() != dev.index:
+                with torch.cuda.device(dev):
+                    return ModelPassHIP.apply(plan, args, *plan.params)
+            return ModelPassHIP.apply(plan, args, *plan.params)
+        if any(wants):
+            return None
+    if torch.cuda.current_device() != dev.index:
+        with torch.cuda.device(dev):
+            return _forward(plan, args, False)[0]
+    return _forward(plan, args, False)[0]

@@ -28,7 +28,7 @@
 extern "C" {
 #endif
 
-#define CFH_ABI_VERSION 13
+#define CFH_ABI_VERSION 14
 
 enum {
     CFH_OK = 0,
@@ -597,6 +597,64 @@ int cfh_attention_inputs_backward(const float* qkv, const float* lattice_w, cons
                                   const float* gv, const float* ga, int64_t N, int32_t H, int32_t Dh,
                                   float* gqkv, float* g_lattice_w, void* workspace, size_t workspace_bytes,
                                   void* stream);
+
+/*
+ * The whole property regressor in one call per direction: atom embedding, batch geometry, the encoder layers (attention
+ * core and the projections between two cores), mean over the atoms of a crystal, and a head of linear layers
+ * (models/latticeformer.py:150-287 with models/indexed_latticeformer_encoder.py:644-901, for layers without layer norm
+ * and dropout and with ReLU).  The same kernels as the single entry points, enqueued without a host round trip between
+ * them; every intermediate lives in memory the caller provides.
+ *   x (N, feat) atom features, pos (N,3), batch (N) ascending from 0, tvecs (B,3,3), sizes (B); E = sum of sizes^2.
+ *   out (B, out features of the last linear layer).
+ * Sizes: D = 16 H (128 or 256) and F a multiple of 128 as for cfh_layer_bridge_forward; the input features of every linear layer of
+ * the head a multiple of 16, all its widths at most CFH_MODEL_MAX_WIDTH; 1 <= feat <= 512.
+ * All weights float32; Wqkv (3D, D) is the row-wise stack of the query, key and value projections.
+ */
+#define CFH_MODEL_MAX_LINEARS 6
+#define CFH_MODEL_MAX_WIDTH 480
+typedef struct cfh_model_layer {
+    cfh_params core;                      /* constants of the layer's attention core                     */
+    const float* Wqkv; const float* bqkv; /* input projection; bqkv (3D)                                  */
+    const float* lattice_w;               /* (D)                                                         */
+    const float* gauss_scale_dev;         /* {scale, shift} or NULL                                      */
+    const float* W_dist; const float* W_axis1; const float* W_axis2; const float* W_axis3;
+    const float* Wo; const float* bo; const float* W1; const float* b1; const float* W2; const float* b2;
+    float c1, lb, c2, q_scale;            /* see cfh_attention_inputs_forward                            */
+    int32_t adaptive;                     /* 1: the translation boxes follow the reciprocal lattice       */
+    int32_t reserved0;
+} cfh_model_layer;
+typedef struct cfh_model_linear {
+    const float* W; const float* b;       /* (out, in), (out)                                            */
+    int32_t in, out, relu, reserved0;
+} cfh_model_linear;
+typedef struct cfh_model {
+    int32_t struct_size;                  /* = sizeof(cfh_model)                                         */
+    int32_t layers, heads, D, F, feat, linears, reserved0;
+    const float* We;                      /* (D, feat) embedding                                         */
+    const cfh_model_layer* layer;         /* (layers)                                                    */
+    cfh_model_linear head[CFH_MODEL_MAX_LINEARS];
+} cfh_model;
+typedef struct cfh_model_batch {
+    const float* x; const float* pos; const int64_t* batch; const float* tvecs; const int64_t* sizes;
+    int64_t N, B, E;
+    const float* x0; const float* qkv0;   /* optional: the embedded atoms (N, D) and the first layer's projection (N, 3D),
+                                             made by the caller (both, with keep, or neither)              */
+    const uint64_t* noise_seeds;          /* (layers) seeds of the frame searches, or NULL: core.noise_seed */
+    void* arena; size_t arena_bytes;      /* intermediates of the forward pass (256-byte aligned)        */
+    void* workspace; size_t workspace_bytes;
+    void* stream;
+    int32_t keep;                         /* 1: the arena holds what cfh_model_backward needs            */
+    int32_t reserved0;
+} cfh_model_batch;
+/* Bytes the passes need: [0] arena and [1] workspace of the forward, [2] scratch and [3] workspace of the backward
+ * (0 with keep == 0); returns the floats of all parameter gradients, or a negative CFH_E* code. */
+int64_t cfh_model_sizes(const cfh_model* m, const cfh_model_batch* b, size_t bytes[4]);
+int cfh_model_forward(const cfh_model* m, const cfh_model_batch* b, float* out);
+/* gout (B, out); grads: every parameter's gradient, one after the other (written, not added to): We; per layer
+ * Wqkv, bqkv, Wo, bo, lattice_w, W_dist, W_axis1..3 (with the angle encoding), W1, b1, W2, b2; per linear layer of the
+ * head W, b.  `b` is the forward's (same arena, untouched since). */
+int cfh_model_backward(const cfh_model* m, const cfh_model_batch* b, const float* gout, void* scratch,
+                       size_t scratch_bytes, float* grads);
 
 #ifdef __cplusplus
 }

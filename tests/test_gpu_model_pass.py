@@ -1,0 +1,92 @@
+"""The whole-model library call (cfh_model_forward / cfh_model_backward) against the modules' own path, which makes the
+same kernels' calls one operator at a time: the same bits where both use the library's kernels throughout, float32
+rounding where the modules' path hands a product to the framework's GEMM."""
+import copy
+
+import pytest
+import torch
+
+import helpers as Hh
+
+pytestmark = pytest.mark.gpu
+
+
+def _both(mp, cb, seed=1):
+    from crystalframer_amd import latticeformer, model_pass
+    dev = torch.device("cuda:0")
+    torch.manual_seed(seed)
+    model = latticeformer.Latticeformer(mp).to(dev)
+    cb = cb.to(dev)
+    model.train()
+    model(cb)                                   # stores the normalisation of alpha (modules' path)
+    target = torch.linspace(-1, 1, cb.num_crystals * model.mlp[-1].out_features, device=dev).view(cb.num_crystals, -1)
+    results = []
+    for on in (True, False):
+        model_pass.ENABLED = on
+        try:
+            model.zero_grad(set_to_none=True)
+            out = model(cb)
+            torch.nn.functional.mse_loss(out, target).backward()
+            with torch.no_grad():
+                ev = model(cb)
+        finally:
+            model_pass.ENABLED = True
+        assert (type(out.grad_fn).__name__ == "ModelPassHIPBackward") == on
+        results.append((out.detach(), ev, {n: p.grad.clone() for n, p in model.named_parameters() if p.grad is not None}))
+    return model, cb, results
+
+
+# one atom; a tile of 16 atoms and its edges; one crystal; more crystals than a workgroup of the tail takes (1, 4, 16);
+# around the 512 rows where the modules' path hands the first projection to the framework's GEMM
+@pytest.mark.parametrize("B,hi,bins,layers", [(1, 1, 64, 1), (1, 16, 64, 2), (3, 6, 16, 2), (16, 2, 0, 1), (17, 9, 64, 4),
+                                              (97, 9, 0, 4), (120, 9, 16, 3), (513, 3, 64, 2), (2050, 1, 0, 1)])
+def test_one_call_equals_the_modules_path(B, hi, bins, layers):
+    from crystalframer_amd import params, synthetic
+    kw = dict(value_pe_angle_wscale=1.0, value_pe_dist_coef=1.5, value_pe_angle_coef=6.0) if bins == 16 else {}
+    mp = params.ModelParams(num_layers=layers, value_pe_angle_real=bins, symm_break_noise=0.0, **kw)
+    cb = synthetic.make_batch(B, atoms="uniform", atoms_lo=1, atoms_hi=hi, len_lo=3.0, len_hi=9.0, ang_lo=65.0, ang_hi=115.0,
+                              seed=B)
+    model, cb, ((o1, e1, g1), (o2, e2, g2)) = _both(mp, cb)
+    assert g1.keys() == g2.keys() and len(g1) == (4 + 15 * layers if bins else 4 + 12 * layers) + 1
+    if B <= 512:                                # (above, the modules' head goes through the framework's GEMM)
+        assert torch.equal(o1, o2)
+        for n in g1:
+            assert torch.equal(g1[n], g2[n]), n
+    assert Hh.rel_err(o1, o2.double()) < 1e-6 and Hh.rel_err(e1, e2.double()) < 1e-6
+    for n in g1:
+        assert Hh.rel_err(g1[n], g2[n].double()) < 1e-5, n
+
+
+def test_head_of_several_layers_and_targets():
+    from crystalframer_amd import params, synthetic
+    mp = params.ModelParams(num_layers=1, symm_break_noise=0.0, embedding_dim=[64, 208], targets=["a", "b", "c"])
+    cb = synthetic.make_batch(21, atoms="uniform", atoms_lo=1, atoms_hi=5, len_lo=3.0, len_hi=9.0, ang_lo=65.0, ang_hi=115.0,
+                              seed=4)
+    model, cb, ((o1, e1, g1), (o2, e2, g2)) = _both(mp, cb)
+    assert o1.shape == (21, 3)
+    assert Hh.rel_err(o1, o2.double()) < 1e-6 and Hh.rel_err(e1, e2.double()) < 1e-6
+    for n in g1:
+        assert Hh.rel_err(g1[n], g2[n].double()) < 1e-5, n
+
+
+def test_copies_exchanged_weights_and_changes_before_the_backward_pass():
+    from crystalframer_amd import params, synthetic
+    mp = params.ModelParams(num_layers=1, symm_break_noise=0.0)
+    cb = synthetic.make_batch(5, atoms="uniform", atoms_lo=1, atoms_hi=5, len_lo=3.0, len_hi=9.0, ang_lo=65.0, ang_hi=115.0,
+                              seed=6)
+    model, cb, _ = _both(mp, cb)
+    with torch.no_grad():
+        ref = model(cb)
+        assert torch.equal(copy.deepcopy(model)(cb), ref)
+        layer = model.encoder.layers[0]
+        old = layer.linear1.weight
+        layer.linear1.weight = torch.nn.Parameter(old * 2.0)           # another parameter
+        changed = model(cb)
+        assert not torch.equal(changed, ref)
+        layer.linear1.weight.data = old.detach().clone()               # another storage
+        assert torch.equal(model(cb), ref)
+    out = model(cb)
+    with torch.no_grad():
+        layer.linear1.weight.mul_(1.5)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        out.sum().backward()
