@@ -79,32 +79,58 @@ class AdamW(torch.optim.Optimizer):
             st = self._group_state(group)
             if st is None:
                 continue
-            jobs = []
-            for p in group["params"]:
+            plan = self._plan(group, st)
+            jobs, offs = plan["jobs"], plan["offs"]
+            m0, v0 = st["exp_avg"].data_ptr(), st["exp_avg_sq"].data_ptr()
+            n, keep = 0, None
+            for p, off in zip(plan["params"], offs):
                 g = p.grad
                 if g is None:
                     continue
+                if off is None:
+                    raise RuntimeError("a parameter that did not require a gradient at the first step has one now")
                 if g.is_sparse:
                     raise RuntimeError("sparse gradients are not supported")
                 if not p.is_contiguous():
                     raise RuntimeError("AdamW of crystalframer_amd needs contiguous parameters")
                 if not g.is_contiguous():
                     g = g.contiguous()
-                o = st["offset"][id(p)]
-                jobs.append((p, g, o))
-            if not jobs:
+                    keep = (keep, g)
+                # a slot of the job table holds a parameter's addresses from the step before as long as the same
+                # parameters have gradients; only what differs is written (a ctypes field costs as much as a launch
+                # argument check, and there are five per parameter)
+                a = jobs[n]
+                known = plan["slot"][n]
+                pp = p.data_ptr()
+                if known[0] != off or known[1] != pp:
+                    a.param, a.exp_avg, a.exp_avg_sq, a.n = pp, m0 + 4 * off, v0 + 4 * off, p.numel()
+                    plan["slot"][n] = (off, pp)
+                a.grad = g.data_ptr()
+                n += 1
+            if n == 0:
                 continue
-            dev = jobs[0][0].device
-            arr = (_lib.CfhAdamWJob * len(jobs))()
-            m0, v0 = st["exp_avg"].data_ptr(), st["exp_avg_sq"].data_ptr()
-            for a, (p, g, o) in zip(arr, jobs):
-                a.param, a.grad = p.data_ptr(), g.data_ptr()
-                a.exp_avg, a.exp_avg_sq, a.n = m0 + 4 * o, v0 + 4 * o, p.numel()
+            dev = plan["device"]
             b1, b2 = group["betas"]
-            with torch.cuda.device(dev):
-                rc = lib.cfh_adamw_step_batch(arr, len(jobs), float(group["lr"]), float(b1), float(b2),
-                                              float(group["eps"]), float(group["weight_decay"]),
-                                              _lib.ptr(st["step"]), _lib.current_stream_ptr(dev))
+            if torch.cuda.current_device() != dev.index:
+                with torch.cuda.device(dev):
+                    rc = self._launch(lib, jobs, n, group, b1, b2, st, dev)
+            else:
+                rc = self._launch(lib, jobs, n, group, b1, b2, st, dev)
             _lib.check(rc, "cfh_adamw_step_batch")
-            del jobs      # the gradients stay alive through p.grad (or, made contiguous here, through the stream order)
+            del keep      # the gradients stay alive through p.grad (or, made contiguous here, through the stream order)
         return loss
+
+    @staticmethod
+    def _launch(lib, jobs, n, group, b1, b2, st, dev):
+        return lib.cfh_adamw_step_batch(jobs, n, float(group["lr"]), float(b1), float(b2), float(group["eps"]),
+                                        float(group["weight_decay"]), st["step"].data_ptr(), _lib.raw_stream(dev))
+
+    def _plan(self, group, st):
+        """Job table of the group's launch, kept from step to step (made again when the group's parameters changed)."""
+        plan = st.get("plan")
+        if plan is None or plan["count"] != len(group["params"]) or plan["moments"] != st["exp_avg"].data_ptr():
+            ps = list(group["params"])
+            plan = st["plan"] = dict(params=ps, offs=[st["offset"].get(id(p)) for p in ps], count=len(group["params"]),
+                                     moments=st["exp_avg"].data_ptr(), jobs=(_lib.CfhAdamWJob * max(len(ps), 1))(),
+                                     slot=[(None, None)] * max(len(ps), 1), device=st["exp_avg"].device)
+        return plan
