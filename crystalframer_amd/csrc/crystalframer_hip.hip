@@ -1198,82 +1198,194 @@ int cfh_linear_weight_bias_grad_batch(const cfh_linear_grad_job* jobs, int32_t n
     return linear_wgrad_batch_impl(jobs, njobs, workspace, workspace_bytes, stream, false);
 }
 
+}  // extern "C"
+namespace {
+// How the rows of a layer bridge are dealt.  Few tiles of 16 rows: the chain in two launches of several workgroups per tile,
+// as long as each of those finds a compute unit of its own (and the rows of the feed-forward block's inside fit LDS).
+bool bridge_split(int64_t N, int F) {
+    int cus = device_cus();
+    if (cus <= 0) cus = 256;
+    return ((N + 15) / 16) * (F / 128) <= cus && F <= 1024;
+}
+// Many: 32 rows per workgroup in the forward direction (the weights read half as often) once there are two of those per
+// compute unit.  The backward kernel with 32 rows leaves a compute unit one workgroup (84 KB of LDS): 140 us against 128 at 22 528.
+bool bridge_rows32(int64_t N, int D) {
+    int cus = device_cus();
+    if (cus <= 0) cus = 256;
+    return D == 128 && (N + 31) / 32 >= 2 * (int64_t)cus;
+}
+// The slices in which the sum over k of an input gradient is made: eight units of (64 columns, slice).
+int bridge_klen(int K, int O) {
+    const int groups = O >> 6;
+    return K / (groups >= 8 ? 1 : 8 / groups);
+}
+int check_bridge(int64_t N, int32_t D, int32_t F) {
+    if (N < 0 || N > 0x7fffffffLL / 1024 || (D != 128 && D != 256) || F < 128 || F % 128 != 0 || F > 65536)
+        return fail(CFH_EINVAL, "layer bridge: N=%lld, D=%d (128 or 256) and F=%d (a multiple of 128)", (long long)N, (int)D, (int)F);
+    return CFH_OK;
+}
+// Floats of a weight stream (a group of eight steps behind its end is read, not used).
+size_t bridge_stream_floats(int kind, int D, int F, bool next, int feat = 0) {
+    return (size_t)(cfh::BR_WAVES * cfh::bridge_stream_steps(kind, D, F, next, feat) + cfh::BR_RING) * 64 * 4;
+}
+// Collects weight streams and makes them in as few launches as the argument table allows.
+struct StreamList {
+    cfh::BridgeStreams T{};
+    int blocks = 0;
+    hipStream_t st;
+    StreamList(int D, int F, hipStream_t stream, int feat = 0) : st(stream) { T.D = D; T.F = F; T.feat = feat; }
+    int add(int kind, const float* Wo, const float* W1, const float* W2, const float* Wq, float* dst) {
+        if (T.n == cfh::BR_MAX_STREAMS) flush();
+        cfh::BridgeStream& S = T.s[T.n++];
+        S.Wo = Wo; S.W1 = W1; S.W2 = W2; S.Wq = Wq; S.dst = dst; S.kind = kind;
+        S.steps = cfh::bridge_stream_steps(kind, T.D, T.F, Wq != nullptr, T.feat);
+        S.block0 = blocks;
+        blocks += (cfh::BR_WAVES * S.steps * 64 + 255) / 256;
+        return S.steps;
+    }
+    void flush() {
+        if (T.n) hipLaunchKernelGGL(cfh::bridge_stream_kernel, dim3((unsigned)blocks), dim3(256), 0, st, T);
+        T.n = 0;
+        blocks = 0;
+    }
+};
+// Dynamic LDS of more than 64 KB has to be asked for, once per kernel and device.
+template <typename Kern>
+int allow_lds(Kern kern, size_t lds) {
+    static int lds_set[64] = {0};
+    if (lds <= 64 * 1024) return CFH_OK;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return fail(CFH_ELAUNCH, "layer bridge: no current device");
+    if (lds_set[dev] < (int)lds) {
+        if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+            return fail(CFH_ELAUNCH, "layer bridge: %zu bytes of LDS refused", lds);
+        lds_set[dev] = (int)lds;
+    }
+    return CFH_OK;
+}
+// A.x1 and A.h: needed as memory between the two launches of the split form, else optional.
+int bridge_forward(const cfh::BridgeArgs& A, int D, hipStream_t st) {
+    const unsigned tiles = (unsigned)((A.N + 15) / 16);
+    const dim3 block(64 * cfh::BR_WAVES);
+    if (bridge_split(A.N, A.F) && A.x1 && A.h) {
+        const dim3 g1(tiles, (unsigned)(A.F / 128)), g2(tiles, A.qs ? 3u : 1u);
+        const size_t lds = 16 * (size_t)(A.F + cfh::BR_PAD) * sizeof(float);
+        if (D == 128) {
+            if (int rc = allow_lds(cfh::layer_bridge_fwd_split2_kernel<1>, lds)) return rc;
+            hipLaunchKernelGGL(cfh::layer_bridge_fwd_split1_kernel<1>, g1, block, 0, st, A);
+            hipLaunchKernelGGL(cfh::layer_bridge_fwd_split2_kernel<1>, g2, block, lds, st, A);
+        } else {
+            if (int rc = allow_lds(cfh::layer_bridge_fwd_split2_kernel<2>, lds)) return rc;
+            hipLaunchKernelGGL(cfh::layer_bridge_fwd_split1_kernel<2>, g1, block, 0, st, A);
+            hipLaunchKernelGGL(cfh::layer_bridge_fwd_split2_kernel<2>, g2, block, lds, st, A);
+        }
+    } else if (D == 256) {
+        hipLaunchKernelGGL((cfh::layer_bridge_fwd_kernel<1, 2>), dim3(tiles), block, 0, st, A);
+    } else if (bridge_rows32(A.N, D)) {
+        hipLaunchKernelGGL((cfh::layer_bridge_fwd_kernel<2, 1>), dim3((tiles + 1) / 2), block, 0, st, A);
+    } else {
+        hipLaunchKernelGGL((cfh::layer_bridge_fwd_kernel<1, 1>), dim3(tiles), block, 0, st, A);
+    }
+    return finish_launch("layer_bridge_forward");
+}
+int bridge_front(const cfh::BridgeArgs& A, int D, hipStream_t st) {
+    const unsigned tiles = (unsigned)((A.N + 15) / 16), parts = bridge_split(A.N, A.F) ? 3u : 1u;
+    const dim3 block(64 * cfh::BR_WAVES);
+    const size_t lds = 16 * (size_t)(16 * cfh::bridge_feat_steps(A.feat) + cfh::BR_PAD) * sizeof(float);
+    if (D == 256) hipLaunchKernelGGL(cfh::layer_front_fwd_kernel<2>, dim3(tiles, parts), block, lds, st, A);
+    else hipLaunchKernelGGL(cfh::layer_front_fwd_kernel<1>, dim3(tiles, parts), block, lds, st, A);
+    return finish_launch("layer_front_forward");
+}
+int bridge_backward(cfh::BridgeBwdArgs A, int D, hipStream_t st) {
+    A.klen_h = bridge_klen(D, A.F); A.klen_1 = bridge_klen(A.F, D); A.klen_o = bridge_klen(D, D);
+    const unsigned tiles = (unsigned)((A.N + 15) / 16);
+    const dim3 block(64 * cfh::BR_WAVES);
+    if (bridge_split(A.N, A.F) && !A.inputs_only) {
+        const dim3 g1(tiles, (unsigned)(A.F / 128));
+        const size_t lds = 16 * (size_t)(A.F + cfh::BR_PAD) * sizeof(float);
+        if (D == 128) {
+            if (int rc = allow_lds(cfh::layer_bridge_bwd_split2_kernel<1>, lds)) return rc;
+            hipLaunchKernelGGL(cfh::layer_bridge_bwd_split1_kernel<1>, g1, block, 0, st, A);
+            hipLaunchKernelGGL(cfh::layer_bridge_bwd_split2_kernel<1>, dim3(tiles), block, lds, st, A);
+        } else {
+            if (int rc = allow_lds(cfh::layer_bridge_bwd_split2_kernel<2>, lds)) return rc;
+            hipLaunchKernelGGL(cfh::layer_bridge_bwd_split1_kernel<2>, g1, block, 0, st, A);
+            hipLaunchKernelGGL(cfh::layer_bridge_bwd_split2_kernel<2>, dim3(tiles), block, lds, st, A);
+        }
+    } else if (D == 256) {
+        hipLaunchKernelGGL((cfh::layer_bridge_bwd_kernel<1, 2>), dim3(tiles), block, 0, st, A);
+    } else {
+        hipLaunchKernelGGL((cfh::layer_bridge_bwd_kernel<1, 1>), dim3(tiles), block, 0, st, A);
+    }
+    return finish_launch("layer_bridge_backward");
+}
+}  // namespace
+extern "C" {
+
+size_t cfh_layer_bridge_workspace_bytes(int32_t D, int32_t F) {
+    if (check_bridge(0, D, F)) return 0;
+    const size_t f = bridge_stream_floats(cfh::BS_FORWARD, D, F, true), b = bridge_stream_floats(cfh::BS_BACKWARD, D, F, true);
+    return COUNTER_BYTES + (f > b ? f : b) * sizeof(float);
+}
+
 int cfh_layer_bridge_forward(const float* attn, const float* x_res, int64_t N, int32_t D, int32_t F, const float* Wo,
                              const float* bo, const float* W1, const float* b1, const float* W2, const float* b2,
                              const float* Wqkv, const float* bqkv, const float* lattice_w,
                              const float* gauss_scale_dev, float c1, float lb, float c2, float q_scale, int32_t H,
                              float* x1, float* h, float* x2, float* qkv, float* qs, float* k, float* v, float* a,
-                             void* stream) {
-    if (N < 0 || N > 0x7fffffffLL / 1024 || D < 128 || F < 128 || D % 128 != 0 || F % 128 != 0 || D > 65536 || F > 65536)
-        return fail(CFH_EINVAL, "layer bridge: N=%lld, D=%d and F=%d must be multiples of 128", (long long)N, (int)D, (int)F);
-    if (H < 1 || H * cfh::DH != D || cfh::BR_ROWS * H > 64 * cfh::BR_WAVES)
-        return fail(CFH_EINVAL, "layer bridge: D=%d must be 16 x H=%d, H at most %d", (int)D, (int)H, 64 * cfh::BR_WAVES / cfh::BR_ROWS);
+                             void* workspace, size_t workspace_bytes, void* stream) {
+    if (int rc = check_bridge(N, D, F)) return rc;
+    if (H < 1 || H * cfh::DH != D) return fail(CFH_EINVAL, "layer bridge: D=%d must be 16 x H=%d", (int)D, (int)H);
     if (N == 0) return CFH_OK;
-    if (!attn || !x_res || !Wo || !W1 || !W2 || !x2)
-        return fail(CFH_EINVAL, "layer bridge: attn, x_res, the weights and x2 must not be NULL");
-    if (Wqkv && (!lattice_w || !qs || !k || !v || !a))
-        return fail(CFH_EINVAL, "layer bridge: with Wqkv, lattice_w and qs, k, v, a must not be NULL");
-    const int wide = F > 3 * D ? F : 3 * D;
-    const size_t lds = ((size_t)cfh::BR_ROWS * (2 * (D + cfh::BR_PAD) + wide + cfh::BR_PAD) +
-                        (size_t)cfh::BR_WAVES * cfh::BR_STAGE_FLOATS) * sizeof(float);
-    if (lds > 160 * 1024) return fail(CFH_EINVAL, "layer bridge: D=%d, F=%d need %zu bytes of LDS", (int)D, (int)F, lds);
-    static int lds_set[64] = {0};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return fail(CFH_ELAUNCH, "layer bridge: no current device");
-    if (lds_set[dev] < (int)lds) {
-        if (hipFuncSetAttribute((const void*)cfh::layer_bridge_fwd_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)lds) != hipSuccess)
-            return fail(CFH_ELAUNCH, "layer bridge: %zu bytes of LDS refused", lds);
-        lds_set[dev] = (int)lds;
-    }
+    if (!attn || !x_res || !Wo || !W1 || !W2 || !x1 || !h || !x2)
+        return fail(CFH_EINVAL, "layer bridge: attn, x_res, the weights and x1, h, x2 must not be NULL");
+    if (Wqkv && (!lattice_w || !qkv || !qs || !k || !v || !a))
+        return fail(CFH_EINVAL, "layer bridge: with Wqkv, lattice_w and qkv, qs, k, v, a must not be NULL");
+    if (int rc = check_workspace(workspace, workspace_bytes, cfh_layer_bridge_workspace_bytes(D, F))) return rc;
+    hipStream_t st = (hipStream_t)stream;
+    float* const ws = reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + COUNTER_BYTES);
     cfh::BridgeArgs A{};
-    A.attn = attn; A.xres = x_res; A.Wo = Wo; A.bo = bo; A.W1 = W1; A.b1 = b1; A.W2 = W2; A.b2 = b2;
-    A.Wq = Wqkv; A.bq = bqkv; A.lattice_w = lattice_w; A.gauss = gauss_scale_dev;
-    A.x1 = x1; A.h = h; A.x2 = x2; A.qkv = qkv; A.qs = qs; A.k = k; A.v = v; A.a = a;
+    StreamList S(D, F, st);
+    A.steps = S.add(cfh::BS_FORWARD, Wo, W1, W2, Wqkv, ws);
+    S.flush();
+    A.attn = attn; A.xres = x_res; A.bo = bo; A.b1 = b1; A.b2 = b2; A.bq = bqkv; A.stream = ws;
+    A.lattice_w = lattice_w; A.gauss = gauss_scale_dev;
+    A.x1 = x1; A.h = h; A.x2 = x2;
+    if (Wqkv) { A.qkv = qkv; A.qs = qs; A.k = k; A.v = v; A.a = a; }
     A.N = (int)N; A.D = D; A.F = F; A.H = H;
     A.c1 = c1; A.lb = lb; A.c2 = c2; A.q_scale = q_scale;
-    hipLaunchKernelGGL(cfh::layer_bridge_fwd_kernel, dim3((unsigned)((N + cfh::BR_ROWS - 1) / cfh::BR_ROWS)),
-                       dim3(64 * cfh::BR_WAVES), lds, (hipStream_t)stream, A);
-    return finish_launch("layer_bridge_forward");
+    return bridge_forward(A, D, st);
 }
 
 int cfh_layer_bridge_backward(const float* g_x2, const float* gqkv, const float* h, const float* Wqkv,
                               const float* W2, const float* W1, const float* Wo, int64_t N, int32_t D, int32_t F,
                               float* g2, float* gh, float* g1, float* g_attn, const cfh_attention_inputs_grad* ai,
-                              void* stream) {
-    if (N < 0 || N > 0x7fffffffLL / 1024 || D < 128 || F < 128 || D % 128 != 0 || F % 128 != 0 || D > 65536 || F > 65536)
-        return fail(CFH_EINVAL, "layer bridge: N=%lld, D=%d and F=%d must be multiples of 128", (long long)N, (int)D, (int)F);
+                              void* workspace, size_t workspace_bytes, void* stream) {
+    if (int rc = check_bridge(N, D, F)) return rc;
     if (N == 0) return CFH_OK;
     if (!h || !W2 || !W1 || !Wo || !gh || !g1 || !g_attn || ((gqkv || ai) && (!Wqkv || !g2)))
         return fail(CFH_EINVAL, "layer bridge backward: h, the weights and gh, g1, g_attn (with gqkv: Wqkv and g2) must not be NULL");
-    if (ai && (gqkv || !ai->qkv || !ai->lattice_w || !ai->gqkv || !ai->gw_partial || ai->H < 1 || ai->H * cfh::DH != D ||
-               cfh::BR_ROWS * ai->H > 64 * cfh::BR_WAVES))
+    if (ai && (gqkv || !ai->qkv || !ai->lattice_w || !ai->gqkv || !ai->gw_partial || ai->H < 1 || ai->H * cfh::DH != D))
         return fail(CFH_EINVAL, "layer bridge backward: attention-input gradients need qkv, lattice_w, gqkv, gw_partial, "
                                 "D = 16 H, and no gqkv argument");
-    const size_t lds = cfh::bridge_bwd_lds_floats(D, F) * sizeof(float);
-    if (lds > 160 * 1024) return fail(CFH_EINVAL, "layer bridge backward: D=%d, F=%d need %zu bytes of LDS", (int)D, (int)F, lds);
-    static int lds_set[64] = {0};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return fail(CFH_ELAUNCH, "layer bridge: no current device");
-    if (lds_set[dev] < (int)lds) {
-        if (hipFuncSetAttribute((const void*)cfh::layer_bridge_bwd_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)lds) != hipSuccess)
-            return fail(CFH_ELAUNCH, "layer bridge backward: %zu bytes of LDS refused", lds);
-        lds_set[dev] = (int)lds;
-    }
+    if (int rc = check_workspace(workspace, workspace_bytes, cfh_layer_bridge_workspace_bytes(D, F))) return rc;
+    hipStream_t st = (hipStream_t)stream;
+    float* const ws = reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + COUNTER_BYTES);
     cfh::BridgeBwdArgs A{};
-    A.g_x2 = g_x2; A.gqkv = gqkv; A.h = h; A.Wq = Wqkv; A.W2 = W2; A.W1 = W1; A.Wo = Wo;
+    StreamList S(D, F, st);
+    A.steps = S.add(cfh::BS_BACKWARD, Wo, W1, W2, gqkv || ai ? Wqkv : nullptr, ws);
+    S.flush();
+    A.g_x2 = g_x2; A.gqkv = gqkv; A.h = h; A.stream = ws;
     A.g2 = g2; A.gh = gh; A.g1 = g1; A.g_attn = g_attn;
-    A.N = (int)N; A.D = D; A.F = F;
+    A.N = (int)N; A.F = F; A.H = D / cfh::DH;
+    A.klen_q = bridge_klen(3 * D, D);
     if (ai) {
         A.ai_qkv = ai->qkv; A.ai_w = ai->lattice_w; A.ai_gauss = ai->gauss_scale_dev;
         A.ai_gqs = ai->gqs; A.ai_gk = ai->gk; A.ai_gv = ai->gv; A.ai_ga = ai->ga;
-        A.gqkv_out = ai->gqkv; A.gw_partial = ai->gw_partial; A.H = ai->H;
+        A.gqkv_out = ai->gqkv; A.gw_partial = ai->gw_partial;
         A.c1 = ai->c1; A.lb = ai->lb; A.c2 = ai->c2; A.q_scale = ai->q_scale;
     }
-    hipLaunchKernelGGL(cfh::layer_bridge_bwd_kernel, dim3((unsigned)((N + cfh::BR_ROWS - 1) / cfh::BR_ROWS)),
-                       dim3(64 * cfh::BR_WAVES), lds, (hipStream_t)stream, A);
-    return finish_launch("layer_bridge_backward");
+    return bridge_backward(A, D, st);
 }
 
 int cfh_crystal_geometry(const float* pos, const int64_t* batch, const float* tvecs, const int64_t* sizes,
@@ -1325,7 +1437,7 @@ int cfh_small_linear_dx(const float* dy, const float* W, int64_t M, int64_t N, i
         return finish_launch("small_linear_dx");
     }
     hipLaunchKernelGGL(cfh::small_linear_dx_kernel, dim3((unsigned)((M + 63) / 64), (unsigned)((K + 63) / 64)), dim3(256), 0,
-                       (hipStream_t)stream, dy, W, (const float*)nullptr, dx, (int)M, (int)N, (int)K);
+                       (hipStream_t)stream, dy, W, dx, (int)M, (int)N, (int)K);
     return finish_launch("small_linear_dx");
 }
 

@@ -9,6 +9,7 @@ namespace {
 struct ModelLayerBuffers {
     float *x1, *h, *qkv, *qs, *k, *v, *a;      // qkv .. a: inputs of this layer; x1, h: behind its core
     float *x2;                                 // output of this layer
+    float *stream, *stream_bwd;                // weights of the bridge behind this layer's core in the order of their use
     float *frames, *z, *prob, *hist, *out, *wcat;
     uint32_t* records;
 };
@@ -19,6 +20,7 @@ struct ModelBuffers {
     float *rpos, *recip, *rvlen, *vcell, *near_, *x0, *pooled;
     float4* table;
     char* geo_ws;
+    float *front_stream, *front_stream_bwd;    // weights of the bridges in the order of their use
     float* y[CFH_MODEL_MAX_LINEARS];           // results of the head's linear layers but the last
     ModelLayerBuffers layer[MODEL_MAX_LAYERS];
     size_t total;
@@ -92,17 +94,23 @@ void model_buffers(const cfh_model* m, const cfh_model_batch* b, ModelBuffers& M
     M.near_ = c.take<float>(2 * E);
     M.x0 = c.take<float>(N * D);
     M.pooled = c.take<float>(B * D);
+    M.front_stream = c.take<float>(bridge_stream_floats(cfh::BS_INPUTS, m->D, m->F, true, m->feat));
+    M.front_stream_bwd = b->keep ? c.take<float>(bridge_stream_floats(cfh::BS_INPUTS_BACKWARD, m->D, m->F, true)) : nullptr;
     for (int i = 0; i + 1 < m->linears; i++) M.y[i] = c.take<float>(B * (size_t)m->head[i].out);
     ModelLayerBuffers set[2];
     for (int l = 0; l < m->layers; l++) {
         ModelLayerBuffers& L = M.layer[l];
+        const bool next = l + 1 < m->layers;
+        float* const stream = c.take<float>(bridge_stream_floats(cfh::BS_FORWARD, m->D, m->F, next));
+        float* const stream_bwd = b->keep ? c.take<float>(bridge_stream_floats(cfh::BS_BACKWARD, m->D, m->F, next)) : nullptr;
         if (b->keep || l < 2) {
             L.qs = c.take<float>(N * D); L.k = c.take<float>(N * D); L.v = c.take<float>(N * D); L.a = c.take<float>(N * H);
             L.x2 = c.take<float>(N * D);
             L.qkv = b->keep ? c.take<float>(N * 3 * D) : nullptr;
             if (b->keep || l == 0) {
-                L.x1 = b->keep ? c.take<float>(N * D) : nullptr;
-                L.h = b->keep ? c.take<float>(N * F) : nullptr;
+                const bool split = bridge_split(b->N, m->F);      // (the bridge in two launches passes them through memory)
+                L.x1 = b->keep || split ? c.take<float>(N * D) : nullptr;
+                L.h = b->keep || split ? c.take<float>(N * F) : nullptr;
                 L.frames = c.take<float>(9 * N * H);
                 L.z = c.take<float>(E * H); L.prob = c.take<float>(E * H);
                 L.hist = c.take<float>(H * N * hw);
@@ -116,6 +124,8 @@ void model_buffers(const cfh_model* m, const cfh_model_batch* b, ModelBuffers& M
             L = set[0];
             L.qs = set[l & 1].qs; L.k = set[l & 1].k; L.v = set[l & 1].v; L.a = set[l & 1].a; L.x2 = set[l & 1].x2;
         }
+        L.stream = stream;
+        L.stream_bwd = stream_bwd;
     }
     M.total = c.off;
     if (b->x0 && b->qkv0 && b->keep) {        // (only read)
@@ -127,11 +137,11 @@ void model_buffers(const cfh_model* m, const cfh_model_batch* b, ModelBuffers& M
 // Rows of the per-block partial sums of a layer's lattice-weight gradient: the first layer's come from
 // attention_inputs_bwd_kernel, the others' from the bridge.
 int64_t model_partial_rows(const cfh_model* m, int l, int64_t N) {
-    const int rows = l == 0 ? 4 * (256 / m->D) : cfh::BR_ROWS;
+    const int rows = l == 0 ? 4 * (256 / m->D) : 16;
     return (N + rows - 1) / rows;
 }
 struct ModelGrads {
-    float *gx0, *gpooled, *gy[CFH_MODEL_MAX_LINEARS], *glogit, *gq, *gk, *gv, *ga;
+    float *gx0, *gy[CFH_MODEL_MAX_LINEARS], *glogit, *gq, *gk, *gv, *ga;
     struct { float *g2, *gh, *g1, *g_attn, *gqkv, *gw_partial; } layer[MODEL_MAX_LAYERS];
     void* wgrad_ws;
     size_t wgrad_bytes, total;
@@ -141,7 +151,6 @@ void model_grads(const cfh_model* m, const cfh_model_batch* b, void* scratch, Mo
     Carver c{reinterpret_cast<char*>(scratch)};
     const size_t N = b->N, E = b->E, B = b->B, D = m->D, F = m->F, H = m->heads;
     G.gx0 = c.take<float>(N * D);
-    G.gpooled = c.take<float>(B * D);
     for (int i = 0; i < m->linears; i++) G.gy[i] = c.take<float>(B * (size_t)m->head[i].out);
     G.glogit = c.take<float>(E * H);
     G.gq = c.take<float>(N * D); G.gk = c.take<float>(N * D); G.gv = c.take<float>(N * D); G.ga = c.take<float>(N * H);
@@ -262,17 +271,6 @@ int tail_launch(const cfh::TailArgs& T, const float* gout, hipStream_t st) {
     else hipLaunchKernelGGL(cfh::model_tail_fwd_kernel, grid, block, lds, st, T);
     return finish_launch("model_tail");
 }
-int set_dynamic_lds(const void* kernel, int* set, size_t lds, const char* what) {
-    int dev = 0;
-    if (lds > 160 * 1024) return fail(CFH_EINVAL, "%s: %zu bytes of LDS needed", what, lds);
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return fail(CFH_ELAUNCH, "%s: no current device", what);
-    if (set[dev] < (int)lds) {
-        if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
-            return fail(CFH_ELAUNCH, "%s: %zu bytes of LDS refused", what, lds);
-        set[dev] = (int)lds;
-    }
-    return CFH_OK;
-}
 }  // namespace
 
 extern "C" {
@@ -313,6 +311,18 @@ int cfh_model_forward(const cfh_model* m, const cfh_model_batch* b, float* out) 
     if ((rc = cfh_crystal_geometry(b->pos, b->batch, b->tvecs, b->sizes, N, B, E, M.edges, M.rpos, M.recip, M.rvlen, M.vcell,
                                    M.e_start, M.atom_start, M.order, M.geo_ws, (2 * (size_t)B + 1) * sizeof(int64_t), b->stream)))
         return rc;
+    {   // the weights of the bridges in the order of their use
+        StreamList S(D, F, st, m->feat);
+        S.add(cfh::BS_INPUTS, m->We, nullptr, nullptr, m->layer[0].Wqkv, M.front_stream);
+        if (b->keep) S.add(cfh::BS_INPUTS_BACKWARD, nullptr, nullptr, nullptr, m->layer[0].Wqkv, M.front_stream_bwd);
+        for (int l = 0; l < m->layers; l++) {
+            const cfh_model_layer& L = m->layer[l];
+            const float* const Wq = l + 1 < m->layers ? m->layer[l + 1].Wqkv : nullptr;
+            S.add(cfh::BS_FORWARD, L.Wo, L.W1, L.W2, Wq, M.layer[l].stream);
+            if (b->keep) S.add(cfh::BS_BACKWARD, L.Wo, L.W1, L.W2, Wq, M.layer[l].stream_bwd);
+        }
+        S.flush();
+    }
     {   // embedding and the inputs of the first layer
         const cfh_model_layer& L = m->layer[0];
         const ModelLayerBuffers& Y = M.layer[0];
@@ -322,18 +332,14 @@ int cfh_model_forward(const cfh_model* m, const cfh_model_batch* b, float* out) 
                                                    cfh::DH, Y.qs, Y.k, Y.v, Y.a, b->stream)))
                 return rc;
         } else {
-            static int lds_set[64] = {0};
-            const size_t lds = cfh::bridge_front_lds_floats(D, m->feat) * sizeof(float);
-            if ((rc = set_dynamic_lds((const void*)cfh::layer_front_fwd_kernel, lds_set, lds, "layer front"))) return rc;
             cfh::BridgeArgs A{};
-            A.attn = b->x; A.Wo = m->We; A.x2 = M.x0;
-            A.Wq = L.Wqkv; A.bq = L.bqkv; A.lattice_w = L.lattice_w; A.gauss = L.gauss_scale_dev;
+            A.attn = b->x; A.x2 = M.x0; A.feat = m->feat;
+            A.stream = M.front_stream; A.steps = cfh::bridge_stream_steps(cfh::BS_INPUTS, D, F, true, m->feat);
+            A.bq = L.bqkv; A.lattice_w = L.lattice_w; A.gauss = L.gauss_scale_dev;
             A.qkv = Y.qkv; A.qs = Y.qs; A.k = Y.k; A.v = Y.v; A.a = Y.a;
-            A.N = (int)N; A.D = D; A.H = H;
+            A.N = (int)N; A.D = D; A.F = F; A.H = H;
             A.c1 = L.c1; A.lb = L.lb; A.c2 = L.c2; A.q_scale = L.q_scale;
-            hipLaunchKernelGGL(cfh::layer_front_fwd_kernel, dim3((unsigned)((N + cfh::BR_ROWS - 1) / cfh::BR_ROWS)),
-                               dim3(64 * cfh::BR_WAVES), lds, st, A, m->feat);
-            if ((rc = finish_launch("layer_front_forward"))) return rc;
+            if ((rc = bridge_front(A, D, st))) return rc;
         }
     }
     for (int l = 0; l < m->layers; l++) {
@@ -353,10 +359,18 @@ int cfh_model_forward(const cfh_model* m, const cfh_model_batch* b, float* out) 
         const bool next = l + 1 < m->layers;
         const cfh_model_layer& Ln = m->layer[next ? l + 1 : l];
         const ModelLayerBuffers& Yn = M.layer[next ? l + 1 : l];
-        if ((rc = cfh_layer_bridge_forward(Y.out, l ? M.layer[l - 1].x2 : M.x0, N, D, F, L.Wo, L.bo, L.W1, L.b1, L.W2, L.b2,
-                                           next ? Ln.Wqkv : nullptr, Ln.bqkv, Ln.lattice_w, Ln.gauss_scale_dev, Ln.c1, Ln.lb,
-                                           Ln.c2, Ln.q_scale, H, Y.x1, Y.h, Y.x2, Yn.qkv, Yn.qs, Yn.k, Yn.v, Yn.a, b->stream)))
-            return rc;
+        cfh::BridgeArgs A{};
+        A.attn = Y.out; A.xres = l ? M.layer[l - 1].x2 : M.x0;
+        A.bo = L.bo; A.b1 = L.b1; A.b2 = L.b2;
+        A.stream = Y.stream; A.steps = cfh::bridge_stream_steps(cfh::BS_FORWARD, D, F, next);
+        A.x1 = Y.x1; A.h = Y.h; A.x2 = Y.x2;
+        A.N = (int)N; A.D = D; A.F = F; A.H = H;
+        if (next) {
+            A.bq = Ln.bqkv; A.lattice_w = Ln.lattice_w; A.gauss = Ln.gauss_scale_dev;
+            A.qkv = Yn.qkv; A.qs = Yn.qs; A.k = Yn.k; A.v = Yn.v; A.a = Yn.a;
+            A.c1 = Ln.c1; A.lb = Ln.lb; A.c2 = Ln.c2; A.q_scale = Ln.q_scale;
+        }
+        if ((rc = bridge_forward(A, D, st))) return rc;
     }
     cfh::TailArgs T;
     tail_args(m, b, M, T);
@@ -386,35 +400,29 @@ int cfh_model_backward(const cfh_model* m, const cfh_model_batch* b, const float
     cfh::TailArgs T;
     tail_args(m, b, M, T);
     for (int i = 0; i < m->linears; i++) T.lin[i].gy = G.gy[i];
-    T.gpooled = G.gpooled;
+    T.gx = G.layer[m->layers - 1].g2;
     if ((rc = tail_launch(T, gout, st))) return rc;
 
-    static int lds_set[64] = {0};
-    const size_t lds = cfh::bridge_bwd_lds_floats(D, F) * sizeof(float);
-    if ((rc = set_dynamic_lds((const void*)cfh::layer_bridge_bwd_kernel, lds_set, lds, "layer bridge backward"))) return rc;
-    const dim3 bridge_grid((unsigned)((N + cfh::BR_ROWS - 1) / cfh::BR_ROWS)), bridge_block(64 * cfh::BR_WAVES);
     for (int l = m->layers - 1; l >= 0; l--) {
         // the projections between the core of layer l and the inputs of layer l + 1
+        const cfh_model_layer& L = m->layer[l];
+        const ModelLayerBuffers& Y = M.layer[l];
+        auto& g = G.layer[l];
+        const bool next = l + 1 < m->layers;
         cfh::BridgeBwdArgs A{};
-        A.N = (int)N; A.D = D; A.F = F; A.H = H;
-        if (l + 1 < m->layers) {
+        A.h = Y.h; A.stream = Y.stream_bwd; A.steps = cfh::bridge_stream_steps(cfh::BS_BACKWARD, D, F, next);
+        A.g_x2 = next ? G.layer[l + 1].g1 : g.g2;
+        A.g2 = g.g2; A.gh = g.gh; A.g1 = g.g1; A.g_attn = g.g_attn;
+        A.N = (int)N; A.F = F; A.H = H;
+        A.klen_q = bridge_klen(3 * D, D);
+        if (next) {
             const cfh_model_layer& Ln = m->layer[l + 1];
-            A.g_x2 = G.layer[l + 1].g1;
-            A.Wq = Ln.Wqkv; A.ai_w = Ln.lattice_w; A.ai_gauss = Ln.gauss_scale_dev;
-            A.ai_qkv = M.layer[l + 1].qkv;
+            A.ai_qkv = M.layer[l + 1].qkv; A.ai_w = Ln.lattice_w; A.ai_gauss = Ln.gauss_scale_dev;
             A.ai_gqs = G.gq; A.ai_gk = G.gk; A.ai_gv = G.gv; A.ai_ga = G.ga;
             A.gqkv_out = G.layer[l + 1].gqkv; A.gw_partial = G.layer[l + 1].gw_partial;
             A.c1 = Ln.c1; A.lb = Ln.lb; A.c2 = Ln.c2; A.q_scale = Ln.q_scale;
-        } else {
-            A.g_x2 = G.gpooled; A.batch = b->batch; A.atom_start = M.atom_start;
         }
-        const cfh_model_layer& L = m->layer[l];
-        const ModelLayerBuffers& Y = M.layer[l];
-        A.g2 = G.layer[l].g2;
-        A.h = Y.h; A.W2 = L.W2; A.W1 = L.W1; A.Wo = L.Wo;
-        A.gh = G.layer[l].gh; A.g1 = G.layer[l].g1; A.g_attn = G.layer[l].g_attn;
-        hipLaunchKernelGGL(cfh::layer_bridge_bwd_kernel, bridge_grid, bridge_block, lds, st, A);
-        if ((rc = finish_launch("layer_bridge_backward"))) return rc;
+        if ((rc = bridge_backward(A, D, st))) return rc;
         cfh_params p = L.core;
         p.flags |= CFH_FLAG_NO_WEIGHT_GRADS;
         // (the table in the arena is that of the last layer whose box rule differs from its predecessor's)
@@ -437,9 +445,13 @@ int cfh_model_backward(const cfh_model* m, const cfh_model_batch* b, const float
                                                 G.gk, G.gv, G.ga, N, H, cfh::DH, g.gqkv, nullptr, g.gw_partial,
                                                 (size_t)model_partial_rows(m, 0, N) * D * sizeof(float), b->stream)))
             return rc;
-        hipLaunchKernelGGL(cfh::small_linear_dx_kernel, dim3((unsigned)((N + 63) / 64), (unsigned)((D + 63) / 64)), dim3(256), 0,
-                           st, g.gqkv, L.Wqkv, g.g1, G.gx0, (int)N, 3 * D, D);
-        if ((rc = finish_launch("layer_front_backward"))) return rc;
+        cfh::BridgeBwdArgs A{};
+        A.g_x2 = g.g1; A.gqkv = g.gqkv; A.g2 = G.gx0;
+        A.stream = M.front_stream_bwd; A.steps = cfh::bridge_stream_steps(cfh::BS_INPUTS_BACKWARD, D, F, true);
+        A.N = (int)N; A.F = F; A.H = H;
+        A.inputs_only = 1;
+        A.klen_q = 3 * D;                      // (one sum, as small_linear_dx_kernel makes it)
+        if ((rc = bridge_backward(A, D, st))) return rc;
     }
     // the weight gradients of the whole pass: the projections, then the cores
     std::vector<float*> core_grads(4 * (size_t)m->layers, nullptr);

@@ -24,7 +24,7 @@ struct TailArgs {
     const float* x;                      // (N, D)
     const int64_t* atom_start;           // (B + 1)
     float* pooled;                       // (B, D)
-    float* gpooled;                      // (B, D) backward
+    float* gx;                           // (N, D) backward: gradient of x, every atom its crystal's over their number
     TailLinear lin[TAIL_MAX_LINEARS];
     int B, D, per_wg, nlin, ld;          // ld: floats of an LDS row (the widest row rounded up to 4, + TAIL_PAD)
 };
@@ -113,7 +113,7 @@ __global__ __launch_bounds__(64 * TAIL_WAVES) void model_tail_fwd_kernel(const T
 }
 
 // Gradients of the head's inputs: gy of the last layer is given (its rectifier, if it has one, is applied here and the
-// result written to gy), the others and gpooled are made here.  Dynamic LDS as in the forward kernel.
+// result written to gy), the others and the atoms' are made here.  Dynamic LDS as in the forward kernel.
 __global__ __launch_bounds__(64 * TAIL_WAVES) void model_tail_bwd_kernel(const TailArgs P, const float* __restrict__ gout) {
     extern __shared__ __attribute__((aligned(16))) float tail_lds[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, kk = lane >> 4;
@@ -140,7 +140,7 @@ __global__ __launch_bounds__(64 * TAIL_WAVES) void model_tail_bwd_kernel(const T
         const int K = T.K, O = T.O, steps = (O + 3) / 4;
         const bool mask = li > 0 && P.lin[li > 0 ? li - 1 : 0].relu;
         const float* const ymask = li > 0 ? P.lin[li - 1].y : nullptr;
-        float* const dst = li > 0 ? P.lin[li - 1].gy : P.gpooled;
+        float* const dst = li > 0 ? P.lin[li - 1].gy : nullptr;
         for (int t = wave; 16 * t < K; t += TAIL_WAVES) {
             const int n = 16 * t + col;                       // (K is a multiple of 16)
             v4f_t acc = {0.f, 0.f, 0.f, 0.f};
@@ -167,13 +167,24 @@ __global__ __launch_bounds__(64 * TAIL_WAVES) void model_tail_bwd_kernel(const T
                 float v = acc[c];
                 if (m < nrows) {
                     if (mask && !(ymask[(size_t)(b0 + m) * K + n] > 0.0f)) v = 0.0f;
-                    dst[(size_t)(b0 + m) * K + n] = v;
+                    if (dst) dst[(size_t)(b0 + m) * K + n] = v;
                 }
                 gin[m * ld + n] = v;
             }
         }
         __syncthreads();
         float* const tmp = g; g = gin; gin = tmp;
+    }
+    // the mean over the atoms: Q threads per atom
+    const int Q = P.D >> 2, R = (64 * TAIL_WAVES) / Q;
+    const int rr = (int)threadIdx.x / Q, q = (int)threadIdx.x - rr * Q;
+    if (rr >= R) return;
+    for (int c = 0; c < nrows; c++) {
+        const int64_t s = P.atom_start[b0 + c], t = P.atom_start[b0 + c + 1];
+        const float inv = 1.0f / (float)(t - s);
+        float4 v = *reinterpret_cast<const float4*>(g + c * ld + 4 * q);
+        v.x *= inv; v.y *= inv; v.z *= inv; v.w *= inv;
+        for (int64_t i = s + rr; i < t; i += R) reinterpret_cast<float4*>(P.gx)[(size_t)i * Q + q] = v;
     }
 }
 

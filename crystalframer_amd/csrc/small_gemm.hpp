@@ -69,10 +69,9 @@ __global__ __launch_bounds__(256) void small_linear_fwd_kernel(const float* __re
     }
 }
 
-// dx (M,K) = dy (M,N) W (+ add, (M,K) or null), W (N,K).  grid: (ceil(M/64), ceil(K/64)); N % 16 == 0, rows of dy 16-byte aligned.
+// dx (M,K) = dy (M,N) W, W (N,K).  grid: (ceil(M/64), ceil(K/64)); N % 16 == 0, rows of dy 16-byte aligned.
 __global__ __launch_bounds__(256) void small_linear_dx_kernel(const float* __restrict__ dy, const float* __restrict__ w,
-                                                              const float* __restrict__ add, float* __restrict__ dx, int M,
-                                                              int N, int K) {
+                                                              float* __restrict__ dx, int M, int N, int K) {
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int col = lane & 15, kk = lane >> 4;
     const int m0 = blockIdx.x * 64 + 32 * (wv >> 1), k0 = blockIdx.y * 64 + 32 * (wv & 1);
@@ -115,7 +114,7 @@ __global__ __launch_bounds__(256) void small_linear_dx_kernel(const float* __res
     for (; c + 2 <= chunks; c += 2) step(c, 2);
     if (c < chunks) step(c, 1);
     auto put = [&](int r, int n, float v) {
-        if (r < M && n < K) dx[(size_t)r * K + n] = add ? v + add[(size_t)r * K + n] : v;
+        if (r < M && n < K) dx[(size_t)r * K + n] = v;
     };
 #pragma unroll
     for (int c = 0; c < 4; c++) {

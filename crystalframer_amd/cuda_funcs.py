@@ -1363,16 +1363,8 @@ class LayerBridgeHIP(torch.autograd.Function):
     FUSED_BACKWARD = True     # the four input-gradient products in one launch too (False: framework GEMMs)
 
     @staticmethod
-    def backward_supported(D: int, F: int) -> bool:
-        sl = lambda O: 1 if O // 64 >= 8 else 8 // (O // 64)
-        part = max(sl(D) * 16 * (D + 4), sl(F) * 16 * (F + 4))
-        return (16 * ((3 * D + 4) + 2 * (D + 4) + (F + 4)) + part) * 4 <= 160 * 1024
-
-    @staticmethod
     def supported(D: int, F: int, H: int) -> bool:
-        wide = max(F, 3 * D)
-        return (D % 128 == 0 and F % 128 == 0 and D == 16 * H and H <= 32
-                and (16 * (2 * (D + 4) + wide + 4) + 8 * 64 * 36) * 4 <= 160 * 1024)
+        return D in (128, 256) and F % 128 == 0 and D == 16 * H
 
     @staticmethod
     def forward(ctx, attn, x_res, Wo, bo, W1, b1, W2, b2, stacked, in_bias, lattice_w, gauss_scale, H, c1, lb,
@@ -1402,11 +1394,13 @@ class LayerBridgeHIP(torch.autograd.Function):
             v = torch.empty_like(qs)
             a = torch.empty((N, H), dtype=torch.float32, device=dev)
         with torch.cuda.device(dev), _timed("layer_bridge_forward", dev):
+            ws = _lib.workspace(dev, lib.cfh_layer_bridge_workspace_bytes(D, F))
             rc = lib.cfh_layer_bridge_forward(
                 _lib.ptr(attn_c), _lib.ptr(xres_c), N, D, F, _lib.ptr(Wo_c), _lib.ptr(bo_c), _lib.ptr(W1_c),
                 _lib.ptr(b1_c), _lib.ptr(W2_c), _lib.ptr(b2_c), _lib.ptr(Wq), _lib.ptr(bq), _lib.ptr(w), _lib.ptr(gs),
                 float(c1), float(lb), float(c2), float(q_scale), H, _lib.ptr(x1), _lib.ptr(h), _lib.ptr(x2),
-                _lib.ptr(qkv), _lib.ptr(qs), _lib.ptr(k), _lib.ptr(v), _lib.ptr(a), _lib.current_stream_ptr(dev))
+                _lib.ptr(qkv), _lib.ptr(qs), _lib.ptr(k), _lib.ptr(v), _lib.ptr(a), _lib.ptr(ws), ws.numel(),
+                _lib.current_stream_ptr(dev))
         _lib.check(rc, "cfh_layer_bridge_forward")
         ctx.save_for_backward(attn_c, x1, h, x2, qkv, Wo_c, W1_c, W2_c, Wq, w, gs)
         ctx.params = (Wo, bo, W1, b1, W2, b2, tuple(qkv_weights), in_bias, lattice_w)
@@ -1427,7 +1421,7 @@ class LayerBridgeHIP(torch.autograd.Function):
         N, D = attn.shape
         F = W1_c.shape[0]
         dev = attn.device
-        fused = LayerBridgeHIP.FUSED_BACKWARD and LayerBridgeHIP.backward_supported(D, F)
+        fused = LayerBridgeHIP.FUSED_BACKWARD
         with_inputs = bool(qkv_weights) and any(g is not None for g in (g_qs, g_k, g_v, g_a))
         if with_inputs and not fused:
             gqkv, g_lw = _attention_inputs_grads(qkv, w, gs, ctx.consts, lattice_w, g_qs, g_k, g_v, g_a)
@@ -1452,10 +1446,12 @@ class LayerBridgeHIP(torch.autograd.Function):
             g1 = torch.empty((N, D), dtype=torch.float32, device=dev)
             g_attn = torch.empty((N, D), dtype=torch.float32, device=dev)
             with torch.cuda.device(dev), _timed("layer_bridge_backward", dev):
+                ws = _lib.workspace(dev, lib.cfh_layer_bridge_workspace_bytes(D, F))
                 rc = lib.cfh_layer_bridge_backward(_lib.ptr(g2), None, _lib.ptr(h), _lib.ptr(Wq), _lib.ptr(W2_c),
                                                    _lib.ptr(W1_c), _lib.ptr(Wo_c), N, D, F, _lib.ptr(g2_out), _lib.ptr(gh),
                                                    _lib.ptr(g1), _lib.ptr(g_attn),
-                                                   None if ai is None else ctypes.byref(ai), _lib.current_stream_ptr(dev))
+                                                   None if ai is None else ctypes.byref(ai), _lib.ptr(ws), ws.numel(),
+                                                   _lib.current_stream_ptr(dev))
             _lib.check(rc, "cfh_layer_bridge_backward")
             del keep
             if with_inputs:

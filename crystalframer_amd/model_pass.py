@@ -111,7 +111,6 @@ class _Plan:
             if any(p is None for p in ps):
                 return
             if not (cuda_funcs.LayerBridgeHIP.supported(enc.d_model, l1.out_features, at.num_heads)
-                    and cuda_funcs.LayerBridgeHIP.backward_supported(enc.d_model, l1.out_features)
                     and cuda_funcs.PeriodicAttentionCoreHIP.supported(
                         P.value_pe_dist_real, A, P.value_pe_dist_wscale, P.value_pe_angle_wscale, at.pe_dist_proj,
                         at.proj_angle1 if A > 0 else None)):

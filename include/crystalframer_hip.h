@@ -522,37 +522,38 @@ int cfh_small_linear_dx(const float* dy, const float* W, int64_t M, int64_t N, i
 
 /*
  * The projections between the attention cores of two consecutive encoder layers, which act on every atom
- * separately, in one launch (forward):
+ * separately (forward):
  *   x1 (N,D) = x_res + attn Wo^T + bo;  h (N,F) = relu(x1 W1^T + b1);  x2 (N,D) = x1 + h W2^T + b2;
  *   with Wqkv (3D,D): qkv (N,3D) = x2 Wqkv^T + bqkv and qs, k, v, a as cfh_attention_inputs_forward makes
  *   them from qkv (Wqkv NULL: the chain ends with x2 and the last eight outputs are not touched).
- * Weights as torch.nn.Linear stores them, biases may be NULL; D = 16 H and F multiples of 128.  Every
- * intermediate is an output because the backward pass (framework GEMMs and the entry points above) needs
- * it.  Replaces, for a layer without layer norm and dropout and with the ReLU activation, the out_proj of
+ * Weights as torch.nn.Linear stores them, biases may be NULL; D = 16 H, 128 or 256, and F a multiple of 128.  Every
+ * intermediate is an output because the backward pass needs it.  workspace:
+ * cfh_layer_bridge_workspace_bytes(D, F), for the weights in the order in which the launch reads them; laid out anew by every
+ * call.  Replaces, for a layer without layer norm and dropout and with the ReLU activation, the out_proj of
  * the attention and the residual (models/indexed_lattice_multi_head_attention_cuda.py:734,
  * models/indexed_latticeformer_encoder.py:639-648), the feed-forward block (:606, :644-648) and the
  * input projection, query scaling and Gaussian coefficient of the next layer
  * (models/indexed_lattice_multi_head_attention_cuda.py:399-409, :896-940): seven launches of the framework
  * per layer in the reference's formulation.
  */
+size_t cfh_layer_bridge_workspace_bytes(int32_t D, int32_t F);
 int cfh_layer_bridge_forward(const float* attn, const float* x_res, int64_t N, int32_t D, int32_t F, const float* Wo,
                              const float* bo, const float* W1, const float* b1, const float* W2, const float* b2,
                              const float* Wqkv, const float* bqkv, const float* lattice_w,
                              const float* gauss_scale_dev, float c1, float lb, float c2, float q_scale, int32_t H,
                              float* x1, float* h, float* x2, float* qkv, float* qs, float* k, float* v, float* a,
-                             void* stream);
+                             void* workspace, size_t workspace_bytes, void* stream);
 
 /*
- * Input gradients of the chain of cfh_layer_bridge_forward in one launch:
+ * Input gradients of the chain of cfh_layer_bridge_forward:
  *   g2 (N,D) = g_x2 + gqkv Wqkv;  gh (N,F) = (g2 W2) where h > 0, else 0;  g1 (N,D) = g2 + gh W1  (the
  *   gradient of x_res and of x1);  g_attn (N,D) = g1 Wo.
  * g_x2 may be NULL (zero).  gqkv NULL (no next layer): g2 = g_x2 and g2 is not written.  gqkv is what
  * cfh_attention_inputs_backward returns; with `ai` given instead (gqkv NULL), that backward is made here as
  * well, from the gradients of (qs, k, v, a), and gqkv is an output.  All four results are outputs because the weight gradients are
  * their products with the saved activations (cfh_linear_weight_bias_grad_batch: dWqkv = gqkv^T x2,
- * dW2 = g2^T h, dW1 = gh^T x1, dWo = g1^T attn).  D, F multiples of 128; returns CFH_EINVAL when D and F
- * need more LDS than a CU has (the caller then uses GEMMs).  Replaces the framework's autograd of the same
- * modules (eight launches per layer).
+ * dW2 = g2^T h, dW1 = gh^T x1, dWo = g1^T attn).  Sizes and workspace as for cfh_layer_bridge_forward.  Replaces the
+ * framework's autograd of the same modules (eight launches per layer).
  */
 typedef struct cfh_attention_inputs_grad {
     const float* qkv;              /* (N, 3D) the forward's stacked projection output */
@@ -572,7 +573,7 @@ typedef struct cfh_attention_inputs_grad {
 int cfh_layer_bridge_backward(const float* g_x2, const float* gqkv, const float* h, const float* Wqkv,
                               const float* W2, const float* W1, const float* Wo, int64_t N, int32_t D, int32_t F,
                               float* g2, float* gh, float* g1, float* g_attn, const cfh_attention_inputs_grad* ai,
-                              void* stream);
+                              void* workspace, size_t workspace_bytes, void* stream);
 
 /*
  * What lies between the stacked q/k/v projection of a layer and its kernels, one launch each way.
