@@ -1577,8 +1577,8 @@ int slow_wave_count(int64_t N, int H) {
 }
 // one wavefront (= workgroup) per (item, head); the hardware deals them to the compute units as slots free up
 template <typename Kern>
-int launch_core(Kern kern, const cfh::CoreArgs& C, hipStream_t st, const char* what, unsigned waves = 0) {
-    if (waves == 0) waves = (unsigned)C.K.N * (unsigned)C.K.H + (unsigned)C.slow_wgs;
+int launch_core(Kern kern, const cfh::CoreArgs& C, hipStream_t st, const char* what) {
+    const unsigned waves = (unsigned)C.K.N * (unsigned)C.K.H + (unsigned)C.slow_wgs;
     const unsigned blocks = (waves + cfh::CORE_WPB - 1) / cfh::CORE_WPB;
     {
         TimedScope timed(what, st);
@@ -1586,34 +1586,42 @@ int launch_core(Kern kern, const cfh::CoreArgs& C, hipStream_t st, const char* w
     }
     return finish_launch(what);
 }
-}  // namespace
-
-extern "C" {
-
-size_t cfh_fused_core_workspace_bytes(const cfh_params* p, int64_t N, int64_t E, int64_t B, int32_t backward) {
-    if (check_core_params(p) != CFH_OK) return 0;
-    return core_layout(p, N, E, B, backward != 0).total;
+// The slices of the sum over the words: 256 words per wavefront with all moments, 128 with the nodes of inference.
+void project_launch(int hw, const float* hist, const float* wcat, float* out, int64_t N, int H, hipStream_t st) {
+    const dim3 grid((unsigned)((N + 15) / 16), (unsigned)H);
+    auto launch = [&](auto kern, int waves) {
+        hipLaunchKernelGGL(kern, grid, dim3(cfh::WAVE * waves), 0, st, hist, wcat, out, (int)N, H);
+    };
+    if (hw == cfh::HW_ANG) launch(cfh::core_project_kernel<4, 4>, 4);
+    else if (hw == cfh::HW_LEAN) launch(cfh::core_project_kernel<5, 2>, 5);
+    else if (hw == cfh::HW_ANG16) launch(cfh::core_project_kernel<2, 1>, 2);
+    else launch(cfh::core_project_kernel<1, 1>, 1);
 }
-
-int32_t cfh_fused_core_hist_words(const cfh_params* p) {
-    if (check_core_params(p) != CFH_OK) return 0;
-    return cfh::core_hist_words(p->angle_bins);
-}
-
-int cfh_fused_core_forward(const cfh_params* p, const float* qs, const float* k, const float* v, const float* a_ih,
+#define CFH_CORE_FWD(...) launch_core(cfh::fused_core_fwd_kernel<__VA_ARGS__>, C, st, what)
+#define CFH_CORE_FWD_LEAN(...) launch_core(cfh::fused_core_fwd_kernel<__VA_ARGS__, true>, C, st, what)
+#define CFH_CORE_BWD(...) launch_core(cfh::fused_core_bwd_kernel<__VA_ARGS__>, C, st, what)
+// (a distance window whose width is not one of the compiled ones: 0)
+#define CFH_CORE_WINDOW(LAUNCH, WL)                                                                       \
+    (p->angle_bins == cfh::SMALL_A                                                                        \
+         ? (p->cos_abs ? LAUNCH(WL, cfh::SMALL_A, true) : LAUNCH(WL, cfh::SMALL_A, false))                \
+         : has_ang ? (p->cos_abs ? LAUNCH(WL, cfh::NBINS, true) : LAUNCH(WL, cfh::NBINS, false)) : LAUNCH(WL, 0, false))
+#define CFH_CORE_DISPATCH(LAUNCH)                                                                         \
+    rc = dist_window_dynamic(p) ? CFH_CORE_WINDOW(LAUNCH, 0)                                              \
+         : p->window_mode == CFH_WINDOW_WIDE ? CFH_CORE_WINDOW(LAUNCH, 11) : CFH_CORE_WINDOW(LAUNCH, 9)
+int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k, const float* v, const float* a_ih,
                            const float* rpos, const float* tvecs, const float* rvlen, const int64_t* batch,
                            const int64_t* edges, const int64_t* e_start, const int32_t* order, const float* W_dist,
                            const float* W_axis1, const float* W_axis2, const float* W_axis3, int64_t N, int64_t E,
                            int64_t B, float* frames, int32_t search_frames, float* z, float* prob, float* hist,
                            float* out, const cfh_core_cache* cache, void* workspace, size_t workspace_bytes,
-                           void* stream) {
+                           void* stream, bool lean) {
     int rc = check_core_params(p);
     if (rc) return rc;
     if ((rc = check_geometry(a_ih, rpos, tvecs, batch, edges, e_start, N, E, B))) return rc;
     if ((rc = check_core_sizes(p, N, E))) return rc;
     if (N == 0) return CFH_OK;
     const bool has_ang = p->angle_bins > 0;
-    if (!qs || !k || !v || !W_dist || !z || !prob || !hist || !out)
+    if (!qs || !k || !v || !W_dist || (!lean && (!z || !prob)) || !hist || !out)
         return fail(CFH_EINVAL, "qs, k, v, W_dist, z, prob, hist and out must not be NULL");
     if (has_ang && (!W_axis1 || !W_axis2 || !W_axis3 || !frames))
         return fail(CFH_EINVAL, "the angle encoding needs W_axis1..3 and frames");
@@ -1639,7 +1647,9 @@ int cfh_fused_core_forward(const cfh_params* p, const float* qs, const float* k,
     }
     C.pair_near = buf.near;
     float* wcat = buf.wcat;
-    const cfh::WcatArgs WA{W_dist, W_axis1, W_axis2, W_axis3, L.hw, p->dist_coef, p->angle_coef, p->angle_wscale, wcat};
+    const int hw = cfh::core_hist_words(p->angle_bins, lean);
+    const cfh::WcatArgs WA{W_dist, W_axis1, W_axis2, W_axis3, hw, p->dist_coef, p->angle_coef,
+                           p->angle_wscale, wcat};
     {
         const int prep_blocks = L.prep_blocks;
         // records whose box is not the table's are listed by the launch that makes them and taken first by the main kernel
@@ -1695,34 +1705,48 @@ int cfh_fused_core_forward(const cfh_params* p, const float* qs, const float* k,
         C.slow_wgs = slow_wave_count(N, p->num_heads);
     }
     C.slow_flag = cfh::REC_BOX_LISTED;
-    const bool wide = p->window_mode == CFH_WINDOW_WIDE;
-    const bool dyn = dist_window_dynamic(p);      // a distance window whose width is not one of the compiled ones
     const char* what = "fused_core_forward";
-#define CFH_CORE_DISPATCH(KERNEL)                                                                         \
-    do {                                                                                                  \
-        if (p->angle_bins == cfh::SMALL_A) {                                                              \
-            if (wide) rc = p->cos_abs ? (dyn ? launch_core(KERNEL<0, cfh::SMALL_A, true>, C, st, what) : launch_core(KERNEL<11, cfh::SMALL_A, true>, C, st, what))          \
-                                      : (dyn ? launch_core(KERNEL<0, cfh::SMALL_A, false>, C, st, what) : launch_core(KERNEL<11, cfh::SMALL_A, false>, C, st, what));        \
-            else rc = p->cos_abs ? (dyn ? launch_core(KERNEL<0, cfh::SMALL_A, true>, C, st, what) : launch_core(KERNEL<9, cfh::SMALL_A, true>, C, st, what))                \
-                                 : (dyn ? launch_core(KERNEL<0, cfh::SMALL_A, false>, C, st, what) : launch_core(KERNEL<9, cfh::SMALL_A, false>, C, st, what));              \
-        } else if (has_ang) {                                                                             \
-            if (wide) rc = p->cos_abs ? (dyn ? launch_core(KERNEL<0, cfh::NBINS, true>, C, st, what) : launch_core(KERNEL<11, cfh::NBINS, true>, C, st, what))            \
-                                      : (dyn ? launch_core(KERNEL<0, cfh::NBINS, false>, C, st, what) : launch_core(KERNEL<11, cfh::NBINS, false>, C, st, what));          \
-            else rc = p->cos_abs ? (dyn ? launch_core(KERNEL<0, cfh::NBINS, true>, C, st, what) : launch_core(KERNEL<9, cfh::NBINS, true>, C, st, what))                  \
-                                 : (dyn ? launch_core(KERNEL<0, cfh::NBINS, false>, C, st, what) : launch_core(KERNEL<9, cfh::NBINS, false>, C, st, what));                \
-        } else {                                                                                          \
-            rc = wide ? (dyn ? launch_core(KERNEL<0, 0, false>, C, st, what) : launch_core(KERNEL<11, 0, false>, C, st, what))                                    \
-                      : (dyn ? launch_core(KERNEL<0, 0, false>, C, st, what) : launch_core(KERNEL<9, 0, false>, C, st, what));                                    \
-        }                                                                                                 \
-    } while (0)
-    CFH_CORE_DISPATCH(cfh::fused_core_fwd_kernel);
+    if (lean) {
+        if (p->angle_bins == cfh::NBINS) {      // moments around the nodes of inference, every LEAN_STEP / 3 bins
+            C.K.bc.ang_mu0 += cfh::LEAN_FIRST * C.K.bc.ang_interval;
+            C.K.bc.ang_inv_interval *= 3.0f / cfh::LEAN_STEP;
+        }
+        CFH_CORE_DISPATCH(CFH_CORE_FWD_LEAN);
+    } else {
+        CFH_CORE_DISPATCH(CFH_CORE_FWD);
+    }
     if (rc) return rc;
     {
         TimedScope timed("core_project", st);
-        hipLaunchKernelGGL(cfh::core_project_kernel, dim3((unsigned)((N + 15) / 16), p->num_heads),
-                           dim3(cfh::WAVE * cfh::PROJ_WAVES), 0, st, hist, wcat, out, (int)N, p->num_heads, L.hw);
+        project_launch(hw, hist, wcat, out, N, p->num_heads, st);
     }
     return finish_launch("fused_core_project");
+}
+
+}  // namespace
+
+extern "C" {
+
+size_t cfh_fused_core_workspace_bytes(const cfh_params* p, int64_t N, int64_t E, int64_t B, int32_t backward) {
+    if (check_core_params(p) != CFH_OK) return 0;
+    return core_layout(p, N, E, B, backward != 0).total;
+}
+
+int32_t cfh_fused_core_hist_words(const cfh_params* p) {
+    if (check_core_params(p) != CFH_OK) return 0;
+    return cfh::core_hist_words(p->angle_bins);
+}
+
+int cfh_fused_core_forward(const cfh_params* p, const float* qs, const float* k, const float* v, const float* a_ih,
+                           const float* rpos, const float* tvecs, const float* rvlen, const int64_t* batch,
+                           const int64_t* edges, const int64_t* e_start, const int32_t* order, const float* W_dist,
+                           const float* W_axis1, const float* W_axis2, const float* W_axis3, int64_t N, int64_t E,
+                           int64_t B, float* frames, int32_t search_frames, float* z, float* prob, float* hist,
+                           float* out, const cfh_core_cache* cache, void* workspace, size_t workspace_bytes,
+                           void* stream) {
+    return fused_core_forward_impl(p, qs, k, v, a_ih, rpos, tvecs, rvlen, batch, edges, e_start, order, W_dist, W_axis1, W_axis2,
+                                   W_axis3, N, E, B, frames, search_frames, z, prob, hist, out, cache, workspace,
+                                   workspace_bytes, stream, false);
 }
 
 int cfh_fused_core_backward(const cfh_params* p, const float* qs, const float* k, const float* v, const float* a_ih,
@@ -1846,7 +1870,7 @@ int cfh_fused_core_backward(const cfh_params* p, const float* qs, const float* k
     const bool wide = p->window_mode == CFH_WINDOW_WIDE;
     const bool dyn = dist_window_dynamic(p);      // a distance window whose width is not one of the compiled ones
     const char* what = "fused_core_backward";
-    CFH_CORE_DISPATCH(cfh::fused_core_bwd_kernel);
+    CFH_CORE_DISPATCH(CFH_CORE_BWD);
 #undef CFH_CORE_DISPATCH
     if (!rc) {
         // gk, gv: sums over the pairs that point at an atom

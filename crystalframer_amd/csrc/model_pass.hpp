@@ -80,7 +80,8 @@ bool same_tables(const cfh_model_layer& a, const cfh_model_layer& b) {
 void model_buffers(const cfh_model* m, const cfh_model_batch* b, ModelBuffers& M) {
     Carver c{reinterpret_cast<char*>(b->arena)};
     const size_t N = b->N, E = b->E, B = b->B, D = m->D, F = m->F, H = m->heads;
-    const size_t hw = cfh::core_hist_words(m->layer[0].core.angle_bins);
+    const int ang = m->layer[0].core.angle_bins;
+    const size_t hw = cfh::core_hist_words(ang, !b->keep);
     M.edges = c.take<int64_t>(2 * E);
     M.e_start = c.take<int64_t>(N + 1);
     M.atom_start = c.take<int64_t>(B + 1);
@@ -112,7 +113,7 @@ void model_buffers(const cfh_model* m, const cfh_model_batch* b, ModelBuffers& M
                 L.x1 = b->keep || split ? c.take<float>(N * D) : nullptr;
                 L.h = b->keep || split ? c.take<float>(N * F) : nullptr;
                 L.frames = c.take<float>(9 * N * H);
-                L.z = c.take<float>(E * H); L.prob = c.take<float>(E * H);
+                if (b->keep) { L.z = c.take<float>(E * H); L.prob = c.take<float>(E * H); }
                 L.hist = c.take<float>(H * N * hw);
                 L.out = c.take<float>(N * D);
                 L.wcat = c.take<float>(D * hw);
@@ -350,11 +351,11 @@ int cfh_model_forward(const cfh_model* m, const cfh_model_batch* b, float* out) 
         const bool ready = l > 0 && same_tables(m->layer[l - 1], L);
         const cfh_core_cache cache{reinterpret_cast<float*>(M.table), M.near_, Y.wcat, Y.records, ready ? 1 : 0, 0, 0, 0};
         const bool ang = p.angle_bins > 0;
-        if ((rc = cfh_fused_core_forward(&p, Y.qs, Y.k, Y.v, Y.a, M.rpos, b->tvecs, L.adaptive ? M.rvlen : nullptr, b->batch,
+        if ((rc = fused_core_forward_impl(&p, Y.qs, Y.k, Y.v, Y.a, M.rpos, b->tvecs, L.adaptive ? M.rvlen : nullptr, b->batch,
                                          M.edges, M.e_start, M.order, L.W_dist, ang ? L.W_axis1 : nullptr,
                                          ang ? L.W_axis2 : nullptr, ang ? L.W_axis3 : nullptr, N, E, B,
                                          ang ? Y.frames : nullptr, ang ? 1 : 0, Y.z, Y.prob, Y.hist, Y.out, &cache,
-                                         b->workspace, b->workspace_bytes, b->stream)))
+                                         b->workspace, b->workspace_bytes, b->stream, !b->keep)))
             return rc;
         const bool next = l + 1 < m->layers;
         const cfh_model_layer& Ln = m->layer[next ? l + 1 : l];
