@@ -282,6 +282,27 @@ def require_gpu(*tensors: torch.Tensor):
                 f"{t.device}); there is no CPU path")
 
 
+_host = None
+
+
+def load_host():
+    """The host extension module (csrc/host_module.cpp), bound to the library's entry points; raises if it is absent."""
+    global _host
+    if _host is None:
+        lib = load()
+        try:
+            from . import _host as mod
+        except ImportError as e:
+            raise RuntimeError(f"crystalframer_amd/_host.so is missing or does not load ({e}): build it with "
+                               "`python -m crystalframer_amd.build`. There is no fallback path.") from e
+        if mod.abi != ABI_VERSION:
+            raise RuntimeError(f"ABI version {mod.abi} of crystalframer_amd/_host.so != {ABI_VERSION}")
+        addr = lambda f: ctypes.cast(f, ctypes.c_void_p).value
+        mod.bind(addr(lib.cfh_model_sizes), addr(lib.cfh_model_forward), addr(lib.cfh_model_backward), addr(lib.cfh_last_error))
+        _host = mod
+    return _host
+
+
 def raw_stream(device: torch.device) -> int:
     """The framework's current stream of ``device`` as a plain address (without the stream object around it)."""
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)

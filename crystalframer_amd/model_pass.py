@@ -40,18 +40,21 @@ class _Plan:
         self.hooked = []         # modules whose hooks the library call would pass over
         self.attn = []
         self._collect(model)
-        self.ptrs = [p.data_ptr() for p in self.params]
+        self.native = None
         if self.ok:
             self.alive = [p.detach() for p in self.params]
+            self.native = _lib.load_host().Plan(self.links, self.params, self.gauss, self.feat, self.D, self.H, self.out_features)
+        else:
+            self.ptrs = [p.data_ptr() for p in self.params if p is not None]
 
     def __reduce_ex__(self, protocol):       # copies and pickles of a model carry no plan (addresses of the original)
         return _no_plan, ()
 
     def current(self) -> bool:
-        for d, k, v in self.links:
-            if d.get(k) is not v:
-                return False
-        return [p.data_ptr() for p in self.params] == self.ptrs
+        if self.native is not None:
+            return self.native.current()
+        return (all(d.get(k) is v for d, k, v in self.links)
+                and [p.data_ptr() for p in self.params if p is not None] == self.ptrs)
 
     def _child(self, module, *names):
         for n in names:
@@ -215,7 +218,7 @@ class _Plan:
         m.layer = ctypes.cast(arr, ctypes.POINTER(_lib.CfhModelLayer))
         for T, (mod, W, b, relu) in zip(m.head, self.head):
             T.W, T.b, T.K, T.O, T.relu = W.data_ptr(), b.data_ptr(), mod.in_features, mod.out_features, relu
-        return m, arr, K.NOISE_SEED_DEVICE, list(self.gauss)
+        return m, arr, (K.NOISE_SEED_DEVICE, list(self.gauss)), ctypes.addressof(m)
 
 
 def _switches_default() -> bool:
@@ -227,91 +230,23 @@ def _switches_default() -> bool:
             and K.DETERMINISTIC_WEIGHT_GRADIENTS and not K.GRAD_COEF_QUIRK and K.EVENT_LOG is None)
 
 
-def _arena(nbytes: int, dev) -> torch.Tensor:
-    """Memory of a pass.  Sizes are rounded up to an eighth of their power of two: the batches of an epoch differ a little from each
-    other, and the framework's allocator then finds a block to use again."""
-    step = max(1 << 9, 1 << max(nbytes.bit_length() - 4, 0))
-    return torch.empty((nbytes + step - 1) // step * step, dtype=torch.uint8, device=dev)
-
-
-def _sizes(m, b):
-    out = (ctypes.c_size_t * 4)()
-    n = _lib.load().cfh_model_sizes(m, b, out)
-    if n < 0:
-        _lib.check(int(n), "cfh_model_sizes")
-    return n, out
-
-
-def _forward(plan, data, keep: bool):
-    """(out, what the backward pass needs)."""
+def _forward(plan, args, keep: bool):
     from .cuda_funcs import KernelManager as K, LinearHIP
-    lib = _lib.load()
-    m, arr, seed_dev, gauss = plan.table()
+    table = plan.table()
+    m, arr = table[0], table[1]
     dev = plan.device
-    x, pos, batch, trans, sizes, E = data
-    N, B = x.shape[0], trans.shape[0]
-    b = _lib.CfhModelBatch(x.data_ptr(), pos.data_ptr(), batch.data_ptr(), trans.data_ptr(), sizes.data_ptr(), N, B, E)
-    b.keep = 1 if keep else 0
-    first = None
-    if keep and N > LinearHIP.SMALL_ROWS:
+    x = args[0]
+    first = ()
+    if keep and x.shape[0] > LinearHIP.SMALL_ROWS:
         # the embedding and the first projection of a long batch as the modules' path makes them, by the framework's
         # GEMM: a training step is then the same to the last bit whichever path makes it
-        x0 = torch.nn.functional.linear(x, plan.embedding)
-        first = (x0, torch.nn.functional.linear(x0, plan.in_proj, plan.in_proj_bias))
-        b.x0, b.qkv0 = first[0].data_ptr(), first[1].data_ptr()
-    seeds = None
+        with torch.no_grad():
+            x0 = torch.nn.functional.linear(x, plan.embedding)
+            first = (x0, torch.nn.functional.linear(x0, plan.in_proj, plan.in_proj_bias))
+    seeds = ()
     if K.NOISE_SEED is None and K.SYMM_BREAK_NOISE > 0:
-        seeds = (ctypes.c_uint64 * len(arr))(*[int(torch.randint(0, 2 ** 62, (1,)).item()) for _ in arr])
-        b.noise_seeds = seeds
-    total, nbytes = _sizes(m, b)
-    arena = _arena(nbytes[0], dev)
-    ws = _lib.workspace(dev, nbytes[1])
-    out = torch.empty((B, plan.out_features), dtype=torch.float32, device=dev)
-    b.arena, b.arena_bytes = arena.data_ptr(), arena.numel()
-    b.workspace, b.workspace_bytes = ws.data_ptr(), ws.numel()
-    b.stream = _lib.raw_stream(dev)
-    rc = lib.cfh_model_forward(m, b, out.data_ptr())
-    if rc:
-        _lib.check(rc, "cfh_model_forward")
-    return out, (m, arr, seed_dev, gauss, b, seeds, total, tuple(nbytes), arena, first)
-
-
-class ModelPassHIP(torch.autograd.Function):
-    """The model's forward pass as one node; see the module's docstring.  ``params``: the plan's parameters."""
-
-    @staticmethod
-    def forward(ctx, plan, data, *params):
-        out, kept = _forward(plan, data, True)
-        ctx.plan, ctx.kept, ctx.device = plan, kept[:-2], plan.device
-        ctx.versions = [p._version for p in params] + [g._version for g in plan.gauss]
-        ctx.save_for_backward(kept[-2], *data[:5], *(kept[-1] or ()))
-        ctx.set_materialize_grads(False)
-        return out
-
-    @staticmethod
-    def backward(ctx, gout):
-        plan = ctx.plan
-        arena, *_ = ctx.saved_tensors
-        if gout is None:
-            return (None,) * (2 + len(plan.params))
-        if [p._version for p in plan.params] + [g._version for g in plan.gauss] != ctx.versions:
-            raise RuntimeError("one of the variables needed for gradient computation has been modified by an inplace operation: "
-                               "a parameter of the model changed between its forward and its backward pass")
-        m, arr, seed_dev, gauss, b, seeds, total, nbytes = ctx.kept
-        dev = ctx.device
-        lib = _lib.load()
-        gout = gout.detach().to(torch.float32).contiguous()
-        grads = torch.empty(total, dtype=torch.float32, device=dev)
-        scratch = _arena(nbytes[2], dev)
-        with torch.cuda.device(dev):
-            ws = _lib.workspace(dev, nbytes[3])
-            q = _lib.CfhModelBatch.from_buffer_copy(b)
-            q.workspace, q.workspace_bytes, q.stream = ws.data_ptr(), ws.numel(), _lib.raw_stream(dev)
-            rc = lib.cfh_model_backward(m, q, gout.data_ptr(), scratch.data_ptr(), scratch.numel(), grads.data_ptr())
-        _lib.check(rc, "cfh_model_backward")
-        views = torch._C._nn.unflatten_dense_tensors(grads, plan.params)
-        del grads            # autograd adopts a view as .grad only if nobody else holds it
-        return (None, None, *views)
+        seeds = [int(torch.randint(0, 2 ** 62, (1,)).item()) for _ in arr]
+    return plan.native.forward(table[3], table, *args, keep, lambda n: _lib.workspace(dev, n), seeds, first)
 
 
 def run(model, data):
@@ -324,15 +259,7 @@ def run(model, data):
     if not plan.ok:
         return None
     x, pos, batch, trans, sizes = data.x, data.pos, data.batch, data.trans_vec, data.sizes
-    if sizes is None or torch.is_autocast_enabled():
-        return None
-    dev = plan.device
-    f32, i64 = torch.float32, torch.int64
-    if not (x.dtype is f32 and pos.dtype is f32 and trans.dtype is f32 and batch.dtype is i64 and sizes.dtype is i64
-            and x.dim() == 2 and x.shape[1] == plan.feat and x.shape[0] > 0
-            and x.device == dev and pos.device == dev and trans.device == dev and batch.device == dev and sizes.device == dev
-            and x.is_contiguous() and pos.is_contiguous() and trans.is_contiguous() and batch.is_contiguous()
-            and sizes.is_contiguous()):
+    if sizes is None or torch.is_autocast_enabled() or not plan.native.accepts(x, pos, batch, trans, sizes):
         return None
     for at in plan.attn:
         if at.frame_sink is not None or at.grad_sink is not None:
@@ -352,19 +279,16 @@ def run(model, data):
     lim = 1 << 30
     if x.shape[0] * plan.D >= lim or E * max(plan.H, 3) >= lim:
         return None
-    args = (x, pos, batch, trans, sizes, int(E))
+    keep = False
     if torch.is_grad_enabled():
         if x.requires_grad or pos.requires_grad or trans.requires_grad:
             return None
-        wants = [p.requires_grad for p in plan.params]
-        if all(wants):
-            if torch.cuda.current_device() != dev.index:
-                with torch.cuda.device(dev):
-                    return ModelPassHIP.apply(plan, args, *plan.params)
-            return ModelPassHIP.apply(plan, args, *plan.params)
-        if any(wants):
+        wanted = plan.native.wanted()
+        if wanted == 1:
             return None
-    if torch.cuda.current_device() != dev.index:
-        with torch.cuda.device(dev):
-            return _forward(plan, args, False)[0]
-    return _forward(plan, args, False)[0]
+        keep = wanted == 2
+    args = (x, pos, batch, trans, sizes, int(E))
+    if torch.cuda.current_device() != plan.device.index:
+        with torch.cuda.device(plan.device):
+            return _forward(plan, args, keep)
+    return _forward(plan, args, keep)

@@ -80,33 +80,11 @@ class AdamW(torch.optim.Optimizer):
             if st is None:
                 continue
             plan = self._plan(group, st)
-            jobs, offs = plan["jobs"], plan["offs"]
+            jobs = plan["jobs"]
             m0, v0 = st["exp_avg"].data_ptr(), st["exp_avg_sq"].data_ptr()
-            n, keep = 0, None
-            for p, off in zip(plan["params"], offs):
-                g = p.grad
-                if g is None:
-                    continue
-                if off is None:
-                    raise RuntimeError("a parameter that did not require a gradient at the first step has one now")
-                if g.is_sparse:
-                    raise RuntimeError("sparse gradients are not supported")
-                if not p.is_contiguous():
-                    raise RuntimeError("AdamW of crystalframer_amd needs contiguous parameters")
-                if not g.is_contiguous():
-                    g = g.contiguous()
-                    keep = (keep, g)
-                # a slot of the job table holds a parameter's addresses from the step before as long as the same
-                # parameters have gradients; only what differs is written (a ctypes field costs as much as a launch
-                # argument check, and there are five per parameter)
-                a = jobs[n]
-                known = plan["slot"][n]
-                pp = p.data_ptr()
-                if known[0] != off or known[1] != pp:
-                    a.param, a.exp_avg, a.exp_avg_sq, a.n = pp, m0 + 4 * off, v0 + 4 * off, p.numel()
-                    plan["slot"][n] = (off, pp)
-                a.grad = g.data_ptr()
-                n += 1
+            n, keep = plan["native"].fill(ctypes.addressof(jobs), m0, v0), None
+            if n < 0:
+                n, keep = self._fill(plan, m0, v0)      # a gradient that has to be looked at
             if n == 0:
                 continue
             dev = plan["device"]
@@ -121,6 +99,40 @@ class AdamW(torch.optim.Optimizer):
         return loss
 
     @staticmethod
+    def _fill(plan, m0, v0):
+        """The job table parameter by parameter: (jobs, gradients made contiguous here)."""
+        n, keep = 0, None
+        for p, off in zip(plan["params"], plan["offs"]):
+            g = p.grad
+            if g is None:
+                continue
+            if off is None:
+                raise RuntimeError("a parameter that did not require a gradient at the first step has one now")
+            if g.is_sparse:
+                raise RuntimeError("sparse gradients are not supported")
+            if not p.is_contiguous():
+                raise RuntimeError("AdamW of crystalframer_amd needs contiguous parameters")
+            if not g.is_contiguous():
+                g = g.contiguous()
+                keep = (keep, g)
+            a = plan["jobs"][n]
+            a.param, a.exp_avg, a.exp_avg_sq, a.n = p.data_ptr(), m0 + 4 * off, v0 + 4 * off, p.numel()
+            a.grad = g.data_ptr()
+            n += 1
+        return n, keep
+
+    def zero_grad(self, set_to_none: bool = True):
+        if not set_to_none or not self._flat:
+            return super().zero_grad(set_to_none=set_to_none)
+        for group in self.param_groups:
+            st = self._flat.get(id(group))
+            if st:
+                self._plan(group, st)["native"].drop()
+            else:
+                for p in group["params"]:
+                    p.grad = None
+
+    @staticmethod
     def _launch(lib, jobs, n, group, b1, b2, st, dev):
         return lib.cfh_adamw_step_batch(jobs, n, float(group["lr"]), float(b1), float(b2), float(group["eps"]),
                                         float(group["weight_decay"]), st["step"].data_ptr(), _lib.raw_stream(dev))
@@ -130,7 +142,8 @@ class AdamW(torch.optim.Optimizer):
         plan = st.get("plan")
         if plan is None or plan["count"] != len(group["params"]) or plan["moments"] != st["exp_avg"].data_ptr():
             ps = list(group["params"])
-            plan = st["plan"] = dict(params=ps, offs=[st["offset"].get(id(p)) for p in ps], count=len(group["params"]),
-                                     moments=st["exp_avg"].data_ptr(), jobs=(_lib.CfhAdamWJob * max(len(ps), 1))(),
-                                     slot=[(None, None)] * max(len(ps), 1), device=st["exp_avg"].device)
+            offs = [st["offset"].get(id(p)) for p in ps]
+            plan = st["plan"] = dict(params=ps, offs=offs, count=len(ps), moments=st["exp_avg"].data_ptr(),
+                                     jobs=(_lib.CfhAdamWJob * max(len(ps), 1))(), device=st["exp_avg"].device,
+                                     native=_lib.load_host().Updates(ps, [-1 if o is None else o for o in offs]))
         return plan

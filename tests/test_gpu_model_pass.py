@@ -31,7 +31,7 @@ def _both(mp, cb, seed=1):
                 ev = model(cb)
         finally:
             model_pass.ENABLED = True
-        assert (type(out.grad_fn).__name__ == "ModelPassHIPBackward") == on
+        assert (out.grad_fn.name() == "ModelPassHIPBackward") == on
         results.append((out.detach(), ev, {n: p.grad.clone() for n, p in model.named_parameters() if p.grad is not None}))
     return model, cb, results
 
