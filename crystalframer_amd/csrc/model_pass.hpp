@@ -81,7 +81,7 @@ void model_buffers(const cfh_model* m, const cfh_model_batch* b, ModelBuffers& M
     Carver c{reinterpret_cast<char*>(b->arena)};
     const size_t N = b->N, E = b->E, B = b->B, D = m->D, F = m->F, H = m->heads;
     const int ang = m->layer[0].core.angle_bins;
-    const size_t hw = cfh::core_hist_words(ang, !b->keep);
+    const size_t hw = cfh::core_hist_words(ang);
     M.edges = c.take<int64_t>(2 * E);
     M.e_start = c.take<int64_t>(N + 1);
     M.atom_start = c.take<int64_t>(B + 1);
