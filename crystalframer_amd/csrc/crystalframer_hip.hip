@@ -1245,6 +1245,9 @@ struct StreamList {
     }
     void flush() {
         if (T.n) hipLaunchKernelGGL(cfh::bridge_stream_kernel, dim3((unsigned)blocks), dim3(256), 0, st, T);
+        clear();
+    }
+    void clear() {
         T.n = 0;
         blocks = 0;
     }
@@ -1543,13 +1546,17 @@ struct CoreBuffers {
     bool wcat_ready;
     bool records_ready;
 };
+// Half-width of the usual box, whose shifts are sorted by length once per crystal (0: no tables for these parameters).
+int usual_half_width(const cfh_params* p, bool has_rvlen) {
+    const int R0 = has_rvlen && p->cutoff_radius != 0.0f ? p->minimum_range : p->lattice_range;
+    return R0 >= 1 && (2 * R0 + 1) * (2 * R0 + 1) * (2 * R0 + 1) <= cfh::FC_TCAP ? R0 : 0;
+}
 CoreBuffers fill_core(cfh::CoreArgs& C, const cfh_params* p, const CoreLayout& L, const float* qs, const float* k,
                       const float* v, bool has_rvlen, const cfh_core_cache* cache, void* workspace) {
     char* ws = reinterpret_cast<char*>(workspace);
     C.qs = qs; C.k = k; C.v = v;
-    const bool adaptive = has_rvlen && p->cutoff_radius != 0.0f;
-    const int R0 = adaptive ? p->minimum_range : p->lattice_range;
-    const bool tables = R0 >= 1 && (2 * R0 + 1) * (2 * R0 + 1) * (2 * R0 + 1) <= cfh::FC_TCAP;
+    const int R0 = usual_half_width(p, has_rvlen);
+    const bool tables = R0 > 0;
     CoreBuffers b;
     b.table = nullptr; b.near = nullptr; b.table_ready = false;
     if (tables) {
@@ -1619,7 +1626,7 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
                            const float* W_axis1, const float* W_axis2, const float* W_axis3, int64_t N, int64_t E,
                            int64_t B, float* frames, int32_t search_frames, float* z, float* prob, float* hist,
                            float* out, const cfh_core_cache* cache, void* workspace, size_t workspace_bytes,
-                           void* stream, bool lean) {
+                           void* stream, bool lean, bool wcat_made) {
     int rc = check_core_params(p);
     if (rc) return rc;
     if ((rc = check_geometry(a_ih, rpos, tvecs, batch, edges, e_start, N, E, B))) return rc;
@@ -1656,7 +1663,7 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
     const cfh::WcatArgs WA{W_dist, W_axis1, W_axis2, W_axis3, hw, p->dist_coef, p->angle_coef,
                            p->angle_wscale, wcat};
     {
-        const int prep_blocks = L.prep_blocks;
+        const int prep_blocks = L.prep_blocks, wcat_blocks = wcat_made ? 0 : p->num_heads * cfh::DH;
         // records whose box is not the table's are listed by the launch that makes them and taken first by the main kernel
         if (buf.table) {
             C.K.slow_count = reinterpret_cast<int32_t*>(ws + L.slow);
@@ -1673,7 +1680,7 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
             F.K.frames_to_records = 1;
             {
                 TimedScope timed("core_prepare", st);
-                hipLaunchKernelGGL(cfh::core_prepare_wcat_kernel, dim3(prep_blocks + p->num_heads * cfh::DH), dim3(256), 0, st,
+                hipLaunchKernelGGL(cfh::core_prepare_wcat_kernel, dim3(prep_blocks + wcat_blocks), dim3(256), 0, st,
                                    F.K, 1, prep_blocks, WA);
             }
             if (F.sorted_tab) {
@@ -1699,7 +1706,7 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
         } else {
             C.K.frames = has_ang ? frames : nullptr;
             TimedScope timed("core_prepare", st);
-            hipLaunchKernelGGL(cfh::core_prepare_wcat_kernel, dim3(prep_blocks + p->num_heads * cfh::DH), dim3(256), 0, st,
+            hipLaunchKernelGGL(cfh::core_prepare_wcat_kernel, dim3(prep_blocks + wcat_blocks), dim3(256), 0, st,
                                C.K, 0, prep_blocks, WA);
         }
     }
@@ -1748,7 +1755,7 @@ int cfh_fused_core_forward(const cfh_params* p, const float* qs, const float* k,
                            void* stream) {
     return fused_core_forward_impl(p, qs, k, v, a_ih, rpos, tvecs, rvlen, batch, edges, e_start, order, W_dist, W_axis1, W_axis2,
                                    W_axis3, N, E, B, frames, search_frames, z, prob, hist, out, cache, workspace,
-                                   workspace_bytes, stream, false);
+                                   workspace_bytes, stream, false, false);
 }
 
 int cfh_fused_core_backward(const cfh_params* p, const float* qs, const float* k, const float* v, const float* a_ih,
@@ -1972,4 +1979,5 @@ int cfh_fused_core_weight_gradients(const cfh_params* p, const cfh_core_wgrad_jo
 
 }  // extern "C"
 
+#include "model_start.hpp"
 #include "model_pass.hpp"

@@ -166,9 +166,8 @@ __device__ __forceinline__ int rint_i(float x) {
 // box: length +inf.  The low 7 bits of the length hold the translation's index in the reference's loop order (the
 // frame search breaks ties by it): the length is rounded down by at most 2^-16 of itself, which the margins of every
 // reach test cover.
-__global__ __launch_bounds__(FC_TCAP) void sorted_shifts_kernel(const float* __restrict__ tvecs, int R0, float4* __restrict__ out) {
-    __shared__ float key[FC_TCAP];
-    const int b = blockIdx.x, t = threadIdx.x;
+__device__ __forceinline__ void sorted_shifts_block(const float* __restrict__ tvecs, int R0, float4* __restrict__ out, int b, int t,
+                                                    float* key) {
     const int s = 2 * R0 + 1, T0 = s * s * s;
     float4 v = make_float4(0.f, 0.f, 0.f, __builtin_inff());
     if (t < T0) {
@@ -189,6 +188,10 @@ __global__ __launch_bounds__(FC_TCAP) void sorted_shifts_kernel(const float* __r
     if (t < T0) v.w = __uint_as_float((__float_as_uint(v.w) & ~(uint32_t)(FC_TCAP - 1)) | (uint32_t)t);
     out[(size_t)b * FC_TCAP + rank] = v;
 }
+__global__ __launch_bounds__(FC_TCAP) void sorted_shifts_kernel(const float* __restrict__ tvecs, int R0, float4* __restrict__ out) {
+    __shared__ float key[FC_TCAP];
+    sorted_shifts_block(tvecs, R0, out, (int)blockIdx.x, (int)threadIdx.x, key);
+}
 
 // Per pair, over the usual box of its crystal: the smallest squared distance of all images and of the images with
 // d^2 > 1e-5, the latter with the position of that image in the sorted table in its low 7 bits.  Both depend on the geometry alone, not on the head or the layer, so they are made once per batch:
@@ -198,15 +201,7 @@ __global__ __launch_bounds__(FC_TCAP) void sorted_shifts_kernel(const float* __r
 // two minima (an entry behind that point cannot lower either minimum, so taking the rest of its group of eight
 // along changes nothing).  Same arithmetic for d^2 as the sweeps.  A thread per pair walking the table alone took
 // 16 us for its chain of dependent steps; this takes 7.
-__global__ __launch_bounds__(256) void pair_nearest_kernel(const float* __restrict__ rpos, const int64_t* __restrict__ edges,
-                                                           const int64_t* __restrict__ batch,
-                                                           const float4* __restrict__ sorted_tab, int T0, int E,
-                                                           float2* __restrict__ out) {
-    const int g = blockIdx.x * blockDim.x + threadIdx.x;
-    const int e = min(g >> 3, E - 1), sub = g & 7;       // (the lanes of a group past the end redo the last pair)
-    const int b = (int)batch[edges[e]];
-    const float4* tab = sorted_tab + (size_t)b * FC_TCAP;
-    const float rx = rpos[(size_t)e * 3 + 0], ry = rpos[(size_t)e * 3 + 1], rz = rpos[(size_t)e * 3 + 2];
+__device__ __forceinline__ float2 pair_nearest(float rx, float ry, float rz, const float4* tab, int T0, int sub) {
     const float r = sqrtf(fmaf(rx, rx, fmaf(ry, ry, rz * rz)));
     // (dval carries the table position of its image in its low 7 bits -- it is rounded down by at most 2^-16 of itself,
     // which the margins of every test that uses it cover -- so that the minimum over the lanes brings the position along)
@@ -225,11 +220,21 @@ __global__ __launch_bounds__(256) void pair_nearest_kernel(const float* __restri
         dall = half_min(dall);
         dval = half_min(dval);
     }
-    if (sub == 0 && (g >> 3) < E) out[e] = make_float2(dall, dval);
+    return make_float2(dall, dval);
+}
+__global__ __launch_bounds__(256) void pair_nearest_kernel(const float* __restrict__ rpos, const int64_t* __restrict__ edges,
+                                                           const int64_t* __restrict__ batch,
+                                                           const float4* __restrict__ sorted_tab, int T0, int E,
+                                                           float2* __restrict__ out) {
+    const int g = blockIdx.x * blockDim.x + threadIdx.x;
+    const int e = min(g >> 3, E - 1), sub = g & 7;       // (the lanes of a group past the end redo the last pair)
+    const float2 near = pair_nearest(rpos[(size_t)e * 3 + 0], rpos[(size_t)e * 3 + 1], rpos[(size_t)e * 3 + 2],
+                                     sorted_tab + (size_t)batch[edges[e]] * FC_TCAP, T0, sub);
+    if (sub == 0 && (g >> 3) < E) out[e] = near;
 }
 
 // ---- projection weights with the moment matrices folded in ---------------------------------------------------
-// Table in LDS, made by the 256 threads of a block: dtab[o * NODE_TAB + 3 m - NODE_STEP n + NODE_OFF] = coefficient of
+// Table in LDS, made by the threads of a block: dtab[o * NODE_TAB + 3 m - NODE_STEP n + NODE_OFF] = coefficient of
 // eps^o around node n of the basis function of bin m.  The terms of order NORD and more of the Taylor series are folded into the
 // lower ones modulo the Chebyshev polynomial T_NORD (x^5 = (20 x^3 - 5 x) / 16, ...), which is what interpolating at its
 // zeros comes to.
@@ -237,7 +242,7 @@ constexpr int NODE_OFF = NODE_STEP * (NODES - 1), NODE_TAB = NODE_OFF + 3 * NBIN
 __device__ __forceinline__ void build_node_table(float* dtab, float ws) {
     static_assert(NORD == 5, "the coefficients below are those of T_5");
     const float r = NODE_STEP / 6.0f / ws, inv_ws = 1.0f / ws;
-    for (int u = threadIdx.x; u < NODE_TAB; u += 256) {
+    for (int u = threadIdx.x; u < NODE_TAB; u += blockDim.x) {
         // D_o = exp(-y^2/2) He_o(y) r^o / o!, by the recurrence of the Hermite polynomials
         const float y = ((float)(u - NODE_OFF) * (1.0f / 3.0f) - NODE_FIRST) * inv_ws;
         float D[9];
@@ -254,7 +259,7 @@ __device__ __forceinline__ void build_node_table(float* dtab, float ws) {
     __syncthreads();
 }
 // wcat (H,16,hw): [0,64) dist_coef W_dist;  64 + (ax NORD + o) NODES + n: angle_coef sum_m W_ax[c,m] D_o(m - t_n).
-// grid: H*16 blocks (h, c), 256 threads over the words.
+// grid: H*16 blocks (h, c), the threads over the words.
 struct WcatArgs {
     const float* Wd; const float* W1; const float* W2; const float* W3;      // (H,16,64) and (H,16,A) x 3
     int hw;
@@ -271,7 +276,7 @@ __device__ __forceinline__ void core_wcat_block(const WcatArgs& A, int hc) {
     __shared__ float dtab[NORD * NODE_TAB];
     if (hw == HW_ANG16) {
         // 16-bin basis: the weights themselves behind the distance block, zeros in the padding
-        for (int w = threadIdx.x; w < hw; w += 256) {
+        for (int w = threadIdx.x; w < hw; w += blockDim.x) {
             float val = 0.0f;
             if (w < HW_DIST) val = dist_coef * Wd[(size_t)hc * NBINS + w];
             else if (w < HW_DIST + 3 * SMALL_A) {
@@ -284,13 +289,13 @@ __device__ __forceinline__ void core_wcat_block(const WcatArgs& A, int hc) {
         return;
     }
     if (hw > HW_DIST) {
-        for (int u = threadIdx.x; u < 3 * NBINS; u += 256) {
+        for (int u = threadIdx.x; u < 3 * NBINS; u += blockDim.x) {
             const float* W = u < NBINS ? W1 : (u < 2 * NBINS ? W2 : W3);
             row[u / NBINS][u % NBINS] = W[(size_t)hc * NBINS + (u % NBINS)];
         }
         build_node_table(dtab, ws);
     }
-    for (int w = threadIdx.x; w < hw; w += 256) {
+    for (int w = threadIdx.x; w < hw; w += blockDim.x) {
         float val;
         if (w < HW_DIST) val = dist_coef * Wd[(size_t)hc * NBINS + w];
         else {

@@ -34,13 +34,13 @@ constexpr int GEO_KEYS = 2048;      // crystals of GEO_KEYS - 1 atoms or more sh
 // crystals and where each crystal's atoms go in the work order (descending size; equal sizes in crystal
 // order when B <= its size, in the order their atomics happen to arrive otherwise).
 #pragma clang fp contract(off)      // the framework expressions this replaces round every product and sum
-__global__ __launch_bounds__(GEO_THREADS) void geometry_crystals_kernel(const GeometryArgs P) {
+__device__ __forceinline__ void geometry_crystals_block(const GeometryArgs& P, int which) {
     __shared__ long long scan_a[GEO_THREADS], scan_p[GEO_THREADS];
     __shared__ long long carry_a, carry_p;
     __shared__ int hist[GEO_KEYS];
     const int t = threadIdx.x;
     const int T = blockDim.x;              // GEO_THREADS
-    if (blockIdx.x == 1) {
+    if (which == 1) {
         // reciprocal lattice (same operation order as the framework expressions it replaces)
         for (int b = t; b < P.B; b += T) {
             const float* m = P.tvecs + (size_t)b * 9;
@@ -157,9 +157,12 @@ __global__ __launch_bounds__(GEO_THREADS) void geometry_crystals_kernel(const Ge
     }
 }
 
+__global__ __launch_bounds__(GEO_THREADS) void geometry_crystals_kernel(const GeometryArgs P) {
+    geometry_crystals_block(P, (int)blockIdx.x);
+}
+
 // One thread per atom: first pair of its row and its place in the work order.
-__global__ __launch_bounds__(256) void geometry_atoms_kernel(const GeometryArgs P) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void geometry_atom(const GeometryArgs& P, int i) {
     if (i == 0) P.e_start[P.N] = P.pair_start[P.B];
     if (i >= P.N) return;
     const int b = (int)P.batch[i];
@@ -169,26 +172,43 @@ __global__ __launch_bounds__(256) void geometry_atoms_kernel(const GeometryArgs 
     P.order[P.order_start[b] + local] = i;
 }
 
-// One thread per pair: its crystal by bisection of the pairs' prefix sums, then (i, j) and the pair vector.
-__global__ __launch_bounds__(256) void geometry_pairs_kernel(const GeometryArgs P) {
-    const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= P.E || e >= P.pair_start[P.B]) return;      // never beyond the pairs that exist
+__global__ __launch_bounds__(256) void geometry_atoms_kernel(const GeometryArgs P) {
+    geometry_atom(P, (int)(blockIdx.x * blockDim.x + threadIdx.x));
+}
+
+// A pair: its crystal by bisection of the pairs' prefix sums, then (i, j) and the pair vector.  false: no such pair.
+struct PairGeometry { int crystal; long long i, j; float x, y, z; };
+__device__ __forceinline__ bool geometry_pair(const GeometryArgs& P, long long e, PairGeometry& g) {
+    if (e >= P.E || e >= P.pair_start[P.B]) return false;      // never beyond the pairs that exist
     int lo = 0, hi = P.B;                       // pair_start[lo] <= e < pair_start[hi]
     while (hi - lo > 1) {
         const int mid = (lo + hi) >> 1;
         if (P.pair_start[mid] <= e) lo = mid; else hi = mid;
     }
     const long long n = (long long)P.sizes[lo];
-    if (n <= 0) return;
+    if (n <= 0) return false;
     const long long local = e - P.pair_start[lo];
     const long long il = local / n, jl = local - il * n;
     const long long a0 = P.atom_start[lo];
-    const long long i = a0 + il, j = a0 + jl;
-    P.edges[e] = i;
-    P.edges[P.E + e] = j;
-    P.rpos[e * 3 + 0] = P.pos[j * 3 + 0] - P.pos[i * 3 + 0];
-    P.rpos[e * 3 + 1] = P.pos[j * 3 + 1] - P.pos[i * 3 + 1];
-    P.rpos[e * 3 + 2] = P.pos[j * 3 + 2] - P.pos[i * 3 + 2];
+    g.crystal = lo;
+    g.i = a0 + il;
+    g.j = a0 + jl;
+    g.x = P.pos[g.j * 3 + 0] - P.pos[g.i * 3 + 0];
+    g.y = P.pos[g.j * 3 + 1] - P.pos[g.i * 3 + 1];
+    g.z = P.pos[g.j * 3 + 2] - P.pos[g.i * 3 + 2];
+    return true;
+}
+__device__ __forceinline__ void geometry_store_pair(const GeometryArgs& P, long long e, const PairGeometry& g) {
+    P.edges[e] = g.i;
+    P.edges[P.E + e] = g.j;
+    P.rpos[e * 3 + 0] = g.x;
+    P.rpos[e * 3 + 1] = g.y;
+    P.rpos[e * 3 + 2] = g.z;
+}
+__global__ __launch_bounds__(256) void geometry_pairs_kernel(const GeometryArgs P) {
+    const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    PairGeometry g;
+    if (geometry_pair(P, e, g)) geometry_store_pair(P, e, g);
 }
 
 }  // namespace cfh

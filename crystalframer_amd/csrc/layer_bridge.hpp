@@ -58,13 +58,13 @@ struct BridgeStream {
 };
 constexpr int BR_MAX_STREAMS = 24;
 struct BridgeStreams { BridgeStream s[BR_MAX_STREAMS]; int n, D, F, feat; };
-// grid: blocks of all streams, 256 threads; a thread per float4.
-__global__ __launch_bounds__(256) void bridge_stream_kernel(const BridgeStreams T) {
+// A thread per float4 of the streams: thread `thread` of the block-th 256.
+__device__ __forceinline__ void bridge_stream_element(const BridgeStreams& T, int block, int thread) {
     int si = 0;
-    while (si + 1 < T.n && (int)blockIdx.x >= T.s[si + 1].block0) si++;
+    while (si + 1 < T.n && block >= T.s[si + 1].block0) si++;
     const BridgeStream& S = T.s[si];
     const int D = T.D, F = T.F, CT = D / 128, du = D / 16;
-    const int e = ((int)blockIdx.x - S.block0) * 256 + (int)threadIdx.x;
+    const int e = (block - S.block0) * 256 + thread;
     if (e >= BR_WAVES * S.steps * 64) return;
     const int lane = e & 63, step = (e >> 6) % S.steps, w = (e >> 6) / S.steps;
     const int col = lane & 15, kk = lane >> 4;
@@ -112,6 +112,11 @@ __global__ __launch_bounds__(256) void bridge_stream_kernel(const BridgeStreams 
         v = *reinterpret_cast<const float4*>(W + (size_t)n * ld + k);
     }
     reinterpret_cast<float4*>(S.dst)[e] = v;
+}
+
+// grid: blocks of all streams, 256 threads.
+__global__ __launch_bounds__(256) void bridge_stream_kernel(const BridgeStreams T) {
+    bridge_stream_element(T, (int)blockIdx.x, (int)threadIdx.x);
 }
 
 // A wavefront's stream, eight steps (a group) at a time: the group being used is in registers.

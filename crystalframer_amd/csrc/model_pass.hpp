@@ -104,6 +104,7 @@ void model_buffers(const cfh_model* m, const cfh_model_batch* b, ModelBuffers& M
         const bool next = l + 1 < m->layers;
         float* const stream = c.take<float>(bridge_stream_floats(cfh::BS_FORWARD, m->D, m->F, next));
         float* const stream_bwd = b->keep ? c.take<float>(bridge_stream_floats(cfh::BS_BACKWARD, m->D, m->F, next)) : nullptr;
+        float* const wcat = c.take<float>(D * hw);
         if (b->keep || l < 2) {
             L.qs = c.take<float>(N * D); L.k = c.take<float>(N * D); L.v = c.take<float>(N * D); L.a = c.take<float>(N * H);
             L.x2 = c.take<float>(N * D);
@@ -116,7 +117,6 @@ void model_buffers(const cfh_model* m, const cfh_model_batch* b, ModelBuffers& M
                 if (b->keep) { L.z = c.take<float>(E * H); L.prob = c.take<float>(E * H); }
                 L.hist = c.take<float>(H * N * hw);
                 L.out = c.take<float>(N * D);
-                L.wcat = c.take<float>(D * hw);
                 L.records = c.take<uint32_t>(N * H * cfh::REC_WORDS);
             }
             if (l < 2) set[l] = L;
@@ -127,6 +127,7 @@ void model_buffers(const cfh_model* m, const cfh_model_batch* b, ModelBuffers& M
         }
         L.stream = stream;
         L.stream_bwd = stream_bwd;
+        L.wcat = wcat;
     }
     M.total = c.off;
     if (b->x0 && b->qkv0 && b->keep) {        // (only read)
@@ -309,20 +310,53 @@ int cfh_model_forward(const cfh_model* m, const cfh_model_batch* b, float* out) 
     hipStream_t st = (hipStream_t)b->stream;
     const int64_t N = b->N, E = b->E, B = b->B;
     const int D = m->D, F = m->F, H = m->heads;
-    if ((rc = cfh_crystal_geometry(b->pos, b->batch, b->tvecs, b->sizes, N, B, E, M.edges, M.rpos, M.recip, M.rvlen, M.vcell,
-                                   M.e_start, M.atom_start, M.order, M.geo_ws, (2 * (size_t)B + 1) * sizeof(int64_t), b->stream)))
-        return rc;
-    {   // the weights of the bridges in the order of their use
+    // the weights of the bridges in the order of their use, the cores' concatenated weights, the geometry
+    {
+        cfh::StartArgs A{};
+        cfh::GeometryArgs& g = A.geo;
+        g.pos = b->pos; g.batch = b->batch; g.tvecs = b->tvecs; g.sizes = b->sizes;
+        g.edges = M.edges; g.rpos = M.rpos; g.recip = M.recip; g.rvlen = M.rvlen; g.vcell = M.vcell;
+        g.e_start = M.e_start; g.order = M.order; g.atom_start = M.atom_start;
+        g.pair_start = reinterpret_cast<int64_t*>(M.geo_ws);
+        g.order_start = g.pair_start + (B + 1);
+        g.N = (int32_t)N; g.B = (int32_t)B; g.E = E;
+        A.geo_blocks = 2;
+        A.table_R = usual_half_width(&m->layer[0].core, m->layer[0].adaptive != 0);
+        if (A.table_R > 0) {
+            constexpr int per = cfh::START_THREADS / cfh::FC_TCAP;
+            A.table = M.table;
+            A.near = reinterpret_cast<float2*>(M.near_);
+            A.table_blocks = (int)((B + per - 1) / per);
+        }
+        A.hc = H * cfh::DH;
         StreamList S(D, F, st, m->feat);
         S.add(cfh::BS_INPUTS, m->We, nullptr, nullptr, m->layer[0].Wqkv, M.front_stream);
         if (b->keep) S.add(cfh::BS_INPUTS_BACKWARD, nullptr, nullptr, nullptr, m->layer[0].Wqkv, M.front_stream_bwd);
+        int nw = 0;
+        auto launch = [&]() {      // (also when a table of the arguments is full)
+            A.streams = S.T;
+            A.stream_blocks = (S.blocks + cfh::START_THREADS / 256 - 1) / (cfh::START_THREADS / 256);
+            hipLaunchKernelGGL(cfh::model_start_kernel, dim3((unsigned)(A.geo_blocks + A.table_blocks + A.stream_blocks + nw * A.hc)),
+                               dim3(cfh::START_THREADS), 0, st, A);
+            S.clear();
+            A.geo_blocks = A.table_blocks = nw = 0;
+        };
         for (int l = 0; l < m->layers; l++) {
             const cfh_model_layer& L = m->layer[l];
+            const cfh_params& p = L.core;
             const float* const Wq = l + 1 < m->layers ? m->layer[l + 1].Wqkv : nullptr;
+            if (nw == cfh::START_MAX_WCAT || S.T.n + 2 > cfh::BR_MAX_STREAMS) launch();
             S.add(cfh::BS_FORWARD, L.Wo, L.W1, L.W2, Wq, M.layer[l].stream);
             if (b->keep) S.add(cfh::BS_BACKWARD, L.Wo, L.W1, L.W2, Wq, M.layer[l].stream_bwd);
+            const bool ang = p.angle_bins > 0;
+            A.wcat[nw++] = cfh::WcatArgs{L.W_dist, ang ? L.W_axis1 : nullptr, ang ? L.W_axis2 : nullptr, ang ? L.W_axis3 : nullptr,
+                                         cfh::core_hist_words(p.angle_bins), p.dist_coef, p.angle_coef, p.angle_wscale,
+                                         M.layer[l].wcat};
         }
-        S.flush();
+        launch();
+        const int atom_blocks = (int)((N + 256) / 256);
+        hipLaunchKernelGGL(cfh::model_pairs_kernel, dim3((unsigned)(atom_blocks + (E + 31) / 32)), dim3(256), 0, st, A, atom_blocks);
+        if ((rc = finish_launch("model_start"))) return rc;
     }
     {   // embedding and the inputs of the first layer
         const cfh_model_layer& L = m->layer[0];
@@ -348,14 +382,14 @@ int cfh_model_forward(const cfh_model* m, const cfh_model_batch* b, float* out) 
         const ModelLayerBuffers& Y = M.layer[l];
         cfh_params p = L.core;
         if (b->noise_seeds) p.noise_seed = b->noise_seeds[l];
-        const bool ready = l > 0 && same_tables(m->layer[l - 1], L);
+        const bool ready = l == 0 || same_tables(m->layer[l - 1], L);
         const cfh_core_cache cache{reinterpret_cast<float*>(M.table), M.near_, Y.wcat, Y.records, ready ? 1 : 0, 0, 0, 0};
         const bool ang = p.angle_bins > 0;
         if ((rc = fused_core_forward_impl(&p, Y.qs, Y.k, Y.v, Y.a, M.rpos, b->tvecs, L.adaptive ? M.rvlen : nullptr, b->batch,
                                          M.edges, M.e_start, M.order, L.W_dist, ang ? L.W_axis1 : nullptr,
                                          ang ? L.W_axis2 : nullptr, ang ? L.W_axis3 : nullptr, N, E, B,
                                          ang ? Y.frames : nullptr, ang ? 1 : 0, Y.z, Y.prob, Y.hist, Y.out, &cache,
-                                         b->workspace, b->workspace_bytes, b->stream, !b->keep)))
+                                         b->workspace, b->workspace_bytes, b->stream, !b->keep, true)))
             return rc;
         const bool next = l + 1 < m->layers;
         const cfh_model_layer& Ln = m->layer[next ? l + 1 : l];
