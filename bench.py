@@ -241,10 +241,10 @@ def lattice_roofline(kern_ms, kern_launches, stats, angle: bool, items_per_launc
         flop_frames = frame_terms * F_FRAME
         n = max(1.0, kern_launches[main])
         # projections: the reference's formulation makes one per (pair, head) and encoding; the fused core makes one
-        # per (atom, head) over its histogram of hw words (64 distance bins + 3 axes x 5 moments x 38 nodes, padded)
+        # per (atom, head) over its histogram of hw words (64 distance bins + 3 axes x 5 moments x 64 bins)
         flop_epi_reference = stats[pairs] * epi * passes
         if fused:
-            hw = {64: 640, 16: 128}.get(angle_bins, 64)
+            hw = {64: 1024, 16: 128}.get(angle_bins, 64)
             flop_epi = items_per_launch * n * 2 * 16 * hw * passes
         else:
             flop_epi = flop_epi_reference
@@ -443,7 +443,7 @@ def main():
                         "them, against the published 157.3 TFLOP/s (packed FP32, which this build does not use: 78.6 "
                         "unpacked).  Algorithmic = 488 (forward) / 709 (backward) flop per lattice term evaluated (the "
                         "reference's windowed formulation), 87 per candidate of the frame search, and the projections as "
-                        "made here, once per (atom, head) over 640 histogram words (the reference's one-per-pair "
+                        "made here, once per (atom, head) over 1024 histogram words (the reference's one-per-pair "
                         "projections are NOT counted; with them: reference_equivalent_tflops).  The lattice kernels "
                         "execute fewer flop per term than that (5 local moments per axis instead of a 33-bin window); "
                         "what they executed is under `executed`, from rocprofv3 counters of the same workload",

@@ -1576,12 +1576,6 @@ CoreBuffers fill_core(cfh::CoreArgs& C, const cfh_params* p, const CoreLayout& L
     C.skip_log2 = p->prune_log2 > 0.0f ? (p->prune_log2 + 8.0f > 32.0f ? p->prune_log2 + 8.0f : 32.0f) : 0.0f;
     return b;
 }
-// 64 angle bins: the main kernels measure the cosine in units of the nodes' distance, from the first node
-void core_node_units(cfh::BasisConsts& bc, const cfh_params* p) {
-    if (p->angle_bins != cfh::NBINS) return;
-    bc.ang_mu0 += cfh::NODE_FIRST * bc.ang_interval;
-    bc.ang_inv_interval *= 3.0f / cfh::NODE_STEP;
-}
 // Leading wavefronts of a main kernel, one per listed slow record (the host does not know how many are listed): a
 // sixteenth of the records, at least 256.  Listed records beyond that are taken in place like the unlisted.
 int slow_wave_count(int64_t N, int H) {
@@ -1599,13 +1593,14 @@ int launch_core(Kern kern, const cfh::CoreArgs& C, hipStream_t st, const char* w
     }
     return finish_launch(what);
 }
-// The slices of the sum over the words: 128 words per wavefront with the moments, 64 else.
+// The slices of the sum over the words: 256 words per wavefront with all moments, 128 with the nodes of inference.
 void project_launch(int hw, const float* hist, const float* wcat, float* out, int64_t N, int H, hipStream_t st) {
     const dim3 grid((unsigned)((N + 15) / 16), (unsigned)H);
     auto launch = [&](auto kern, int waves) {
         hipLaunchKernelGGL(kern, grid, dim3(cfh::WAVE * waves), 0, st, hist, wcat, out, (int)N, H);
     };
-    if (hw == cfh::HW_ANG) launch(cfh::core_project_kernel<5, 2>, 5);
+    if (hw == cfh::HW_ANG) launch(cfh::core_project_kernel<4, 4>, 4);
+    else if (hw == cfh::HW_LEAN) launch(cfh::core_project_kernel<5, 2>, 5);
     else if (hw == cfh::HW_ANG16) launch(cfh::core_project_kernel<2, 1>, 2);
     else launch(cfh::core_project_kernel<1, 1>, 1);
 }
@@ -1659,7 +1654,7 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
     }
     C.pair_near = buf.near;
     float* wcat = buf.wcat;
-    const int hw = L.hw;
+    const int hw = cfh::core_hist_words(p->angle_bins, lean);
     const cfh::WcatArgs WA{W_dist, W_axis1, W_axis2, W_axis3, hw, p->dist_coef, p->angle_coef,
                            p->angle_wscale, wcat};
     {
@@ -1718,8 +1713,11 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
     }
     C.slow_flag = cfh::REC_BOX_LISTED;
     const char* what = "fused_core_forward";
-    core_node_units(C.K.bc, p);
     if (lean) {
+        if (p->angle_bins == cfh::NBINS) {      // moments around the nodes of inference, every LEAN_STEP / 3 bins
+            C.K.bc.ang_mu0 += cfh::LEAN_FIRST * C.K.bc.ang_interval;
+            C.K.bc.ang_inv_interval *= 3.0f / cfh::LEAN_STEP;
+        }
         CFH_CORE_DISPATCH(CFH_CORE_FWD_LEAN);
     } else {
         CFH_CORE_DISPATCH(CFH_CORE_FWD);
@@ -1827,10 +1825,9 @@ int cfh_fused_core_backward(const cfh_params* p, const float* qs, const float* k
         int per_slice = (int)((N + nslices - 1) / nslices);
         per_slice = (per_slice + 15) & ~15;
         nslices = (int)((N + per_slice - 1) / per_slice);
-        const int gw_waves = cfh::core_gw_waves(L.hw);
         TimedScope timed("core_weight_gradients", st_w);
-        hipLaunchKernelGGL(cfh::core_gwcat_kernel, dim3((L.hw / 64 + gw_waves - 1) / gw_waves, p->num_heads, nslices),
-                           dim3(cfh::WAVE * gw_waves), 0, st_w, gout,
+        hipLaunchKernelGGL(cfh::core_gwcat_kernel, dim3((L.hw / 64 + cfh::GW_WPB - 1) / cfh::GW_WPB, p->num_heads, nslices),
+                           dim3(cfh::WAVE * cfh::GW_WPB), 0, st_w, gout,
                            hist, gwcat, (int)N, p->num_heads, L.hw, per_slice);
         hipLaunchKernelGGL(cfh::core_gw_finish_kernel, dim3(p->num_heads * cfh::DH), dim3(256), 0, st_w, gwcat, nslices,
                            p->num_heads, L.hw, p->dist_coef, p->angle_coef, p->angle_wscale, gW_dist, gW_axis1, gW_axis2,
@@ -1877,7 +1874,8 @@ int cfh_fused_core_backward(const cfh_params* p, const float* qs, const float* k
     if (buf.table && !buf.table_ready)
         hipLaunchKernelGGL(cfh::sorted_shifts_kernel, dim3((unsigned)B), dim3(cfh::FC_TCAP), 0, st, tvecs, C.table_R,
                            buf.table);
-    core_node_units(C.K.bc, p);
+    const bool wide = p->window_mode == CFH_WINDOW_WIDE;
+    const bool dyn = dist_window_dynamic(p);      // a distance window whose width is not one of the compiled ones
     const char* what = "fused_core_backward";
     CFH_CORE_DISPATCH(CFH_CORE_BWD);
 #undef CFH_CORE_DISPATCH
@@ -1935,7 +1933,6 @@ static int core_weight_gradients_impl(const cfh_params* p, const cfh_core_wgrad_
     int cus = device_cus();
     if (cus <= 0) cus = 256;
     const int blocks_per_slice = (hw / 64) * p->num_heads;
-    const int gw_waves = cfh::core_gw_waves(hw);
     TimedScope timed("core_weight_gradients", st);
     for (int32_t first = 0; first < njobs; first += cfh::CORE_WG_MAX_JOBS) {
         const int32_t last = njobs < first + cfh::CORE_WG_MAX_JOBS ? njobs : first + cfh::CORE_WG_MAX_JOBS;
@@ -1965,8 +1962,8 @@ static int core_weight_gradients_impl(const cfh_params* p, const cfh_core_wgrad_
             slices += nslices;
         }
         if (slices > 0)
-            hipLaunchKernelGGL(cfh::core_gwcat_multi_kernel, dim3((hw / 64 + gw_waves - 1) / gw_waves, p->num_heads, slices),
-                               dim3(cfh::WAVE * gw_waves), 0, st, T);
+            hipLaunchKernelGGL(cfh::core_gwcat_multi_kernel, dim3((hw / 64 + cfh::GW_WPB - 1) / cfh::GW_WPB, p->num_heads, slices),
+                               dim3(cfh::WAVE * cfh::GW_WPB), 0, st, T);
         hipLaunchKernelGGL(cfh::core_gw_finish_multi_kernel, dim3(p->num_heads * cfh::DH, T.njobs), dim3(256), 0, st, T);
     }
     return finish_launch("fused_core_weight_gradients");

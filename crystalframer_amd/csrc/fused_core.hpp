@@ -19,19 +19,18 @@
 //     weight can reach 2^-skip of the heaviest one in the prefix |s| <= |r| + sqrt(d2min + skip/(-a log2 e)):
 //     the two light sweeps read a fraction of the box instead of all of it twice.
 //   * angle encoding by local moments.  The Gaussian basis of the cosine has sigma = wscale bins (4), so around
-//     the node n* nearest to x (nodes t_n every 5/3 bins, half-width of their intervals g = 5/6 bin) the value of every
-//     basis function is a short power series in the offset eps = (u - t_n*) / g in [-1,1] (u = x in bin units):
-//         exp(-((m - u)/ws)^2 / 2) = sum_o eps^o D_o(m - t_n*),  D_o(d) = exp(-(d/ws)^2/2) He_o(d/ws) (g/ws)^o / o!
-//     (generating function of the Hermite polynomials), interpolated at the Chebyshev points of the interval by
-//     NORD = 5 terms: the error is below 2e-6 of the peak.  A term therefore adds NORD moments w eps^o at ONE node per axis
-//     instead of a 33-bin window, and
+//     the bin m* nearest to x the value of every basis function is a short power series in the offset
+//     eps = 2 (u - m*) in [-1,1] (u = x in bin units):
+//         exp(-((m - u)/ws)^2 / 2) = sum_o eps^o D_o(m - m*),  D_o(d) = exp(-(d/ws)^2/2) He_o(d/ws) / (o! (2 ws)^o)
+//     (generating function of the Hermite polynomials; truncated after NORD = 5 terms the error is below 2e-6 of
+//     the peak, 6 terms: 1e-7).  A term therefore adds NORD moments w eps^o at ONE bin per axis instead of a 33-bin window, and
 //     the constant matrices D_o are folded into the projection weights (core_wcat_kernel).  This is the FULL
 //     basis (no +-4 sigma truncation), i.e. the pure-PyTorch formulation of the reference
 //     (models/indexed_lattice_multi_head_attention.py:580-588) rather than the windowed one of its CUDA kernels.
 //     The distance basis (sigma = 1 bin) keeps its truncated window.
 //
-// Histogram of an item ("hist", HW words): [0,64) distance bins, then for axis ax and order o the moments of the nodes
-// at 64 + (ax NORD + o) NODES (zeros behind the last, up to whole 64-word blocks).  It is accumulated in LDS as signed 32-bit fixed point (round to nearest) in units of
+// Histogram of an item ("hist", HW words): [0,64) distance bins, then for axis ax and order o the 64 moment bins
+// at 64 + (ax NORD + o) 64.  It is accumulated in LDS as signed 32-bit fixed point (round to nearest) in units of
 // 2^30 / npairs relative to the heaviest pair of the row so far, and written out normalised as float32.
 #pragma once
 #include <type_traits>
@@ -56,17 +55,7 @@ constexpr int CORE_WPB = 1;                     // wavefronts per workgroup of t
                                                 // the two separate launches
 constexpr int FC_LOGCAP = 64;                   // logits of a row kept in LDS until the row is complete
 constexpr int HW_DIST = NBINS;
-// Nodes of the moments with the 64-bin angle encoding: one every NODE_STEP / 3 bins, and the series around a node is the
-// interpolation at the Chebyshev points of its interval instead of the Taylor polynomial of the same degree, which takes
-// 2^(1-NORD) of its error: with 5/3 bins and 5 terms 0.8 of the error of the Taylor series around every bin, with 640 words
-// per (atom, head) instead of 1024.  Every histogram, and in
-// training its gradient, passes through memory: at 2372 atoms the projection went from 22 to 14 us, the gradient's from 22
-// to 15, the weight gradients of four layers from 74 to 46, the training step from 1426 to 1310.
-constexpr int NODE_STEP = 5;
-constexpr int NODES = 38;
-constexpr float NODE_FIRST = 0.5f;              // centre of node 0 in bin units: the nodes' intervals cover [-1/3, 63]
-constexpr int HW_ANG = 640;
-static_assert(HW_ANG >= HW_DIST + 3 * NORD * NODES && HW_ANG % 64 == 0, "");
+constexpr int HW_ANG = NBINS * (1 + 3 * NORD);  // 1024 words per (atom, head) with the 64-bin angle encoding
 constexpr int SMALL_A = 16;                     // the 16-bin angle basis (the reference's lightweight setting): sigma is
                                                 // one bin or more, far too wide a step for the moment series, and the
                                                 // basis is small: every image adds its 16 basis values per axis directly
@@ -82,8 +71,20 @@ __host__ __device__ constexpr int core_hist_lds_words(int ang) {
     return ang == SMALL_A ? HW_DIST + A16_COPIES * A16_STRIDE : (ang == NBINS ? HW_ANG : HW_DIST);
 }
 // words of an item's histogram for `ang` angle bins (0: distance encoding alone)
-__host__ __device__ constexpr int core_hist_words(int ang) {
-    return ang == NBINS ? HW_ANG : (ang == SMALL_A ? HW_ANG16 : HW_DIST);
+__host__ __device__ constexpr int core_hist_words(int ang, bool lean = false);
+// Inference, where the histogram serves the projection alone, uses FEWER nodes for the moments of the angle encoding:
+// every LEAN_STEP / 3 bins instead of every bin, and the series around a node is the interpolation at the Chebyshev points
+// of its interval instead of the Taylor polynomial of the same degree, which takes 2^(1-NORD) of its error: with 5/3 bins
+// and 5 terms 0.8 of the error of the one-bin Taylor series, with 640 words instead of 1024.  At 22 528 atoms: projection
+// 204 -> 119 us, main kernel 404 -> 393 (its vector instructions, not its stores, bound it; making the projection in it,
+// four items of a head per workgroup behind a barrier, took 529 us for both).
+constexpr int LEAN_STEP = 5;
+constexpr int LEAN_NODES = 38;
+constexpr float LEAN_FIRST = 0.5f;              // centre of node 0 in bin units: the nodes' intervals cover [-1/3, 63]
+constexpr int HW_LEAN = 640;
+static_assert(HW_LEAN >= HW_DIST + 3 * NORD * LEAN_NODES && HW_LEAN % 64 == 0, "");
+__host__ __device__ constexpr int core_hist_words(int ang, bool lean) {
+    return ang == NBINS ? (lean ? HW_LEAN : HW_ANG) : (ang == SMALL_A ? HW_ANG16 : HW_DIST);
 }
 constexpr int REC_J0 = 30;                      // item record: first neighbour atom (pairs of an atom are j0, j0+1, ...)
 constexpr int REC_CRYSTAL = 31;                 // item record: crystal of the atom
@@ -234,31 +235,49 @@ __global__ __launch_bounds__(256) void pair_nearest_kernel(const float* __restri
 }
 
 // ---- projection weights with the moment matrices folded in ---------------------------------------------------
-// Table in LDS, made by the threads of a block: dtab[o * NODE_TAB + 3 m - NODE_STEP n + NODE_OFF] = coefficient of
-// eps^o around node n of the basis function of bin m.  The terms of order NORD and more of the Taylor series are folded into the
+// D_o(d) = exp(-(d/ws)^2/2) He_o(d/ws) / (o! (2 ws)^o)
+__device__ __forceinline__ float moment_matrix(int o, float d, float ws) {
+    const float y = d / ws;
+    float h0 = 1.0f, h1 = y;           // probabilists' Hermite polynomials
+    float he = o == 0 ? h0 : h1;
+    for (int n = 1; n < o; n++) { const float h2 = y * h1 - (float)n * h0; h0 = h1; h1 = h2; he = h2; }
+    float coef = 1.0f;
+    for (int n = 1; n <= o; n++) coef /= (float)n * (2.0f * ws);
+    return __expf(-0.5f * y * y) * he * coef;
+}
+// table of D_o(d) for d = -63 .. 63 in LDS, made by the threads of a block: dtab[o * 128 + d + 63]
+__device__ __forceinline__ void build_moment_table(float* dtab, float ws) {
+    for (int u = threadIdx.x; u < NORD * 128; u += blockDim.x) {
+        const int o = u >> 7, d = (u & 127) - 63;
+        dtab[u] = (u & 127) < 127 ? moment_matrix(o, (float)d, ws) : 0.0f;
+    }
+    __syncthreads();
+}
+// The same for the nodes of inference: dtab[o * LEAN_TAB + 3 m - LEAN_STEP n + LEAN_OFF] = coefficient of eps^o
+// around node n of the basis function of bin m.  The terms of order NORD and more of the Taylor series are folded into the
 // lower ones modulo the Chebyshev polynomial T_NORD (x^5 = (20 x^3 - 5 x) / 16, ...), which is what interpolating at its
 // zeros comes to.
-constexpr int NODE_OFF = NODE_STEP * (NODES - 1), NODE_TAB = NODE_OFF + 3 * NBINS;
+constexpr int LEAN_OFF = LEAN_STEP * (LEAN_NODES - 1), LEAN_TAB = LEAN_OFF + 3 * NBINS;
 __device__ __forceinline__ void build_node_table(float* dtab, float ws) {
     static_assert(NORD == 5, "the coefficients below are those of T_5");
-    const float r = NODE_STEP / 6.0f / ws, inv_ws = 1.0f / ws;
-    for (int u = threadIdx.x; u < NODE_TAB; u += blockDim.x) {
-        // D_o = exp(-y^2/2) He_o(y) r^o / o!, by the recurrence of the Hermite polynomials
-        const float y = ((float)(u - NODE_OFF) * (1.0f / 3.0f) - NODE_FIRST) * inv_ws;
+    const float r = LEAN_STEP / 6.0f / ws, inv_ws = 1.0f / ws;
+    for (int u = threadIdx.x; u < LEAN_TAB; u += blockDim.x) {
+        // exp(-y^2/2) He_o(y) r^o / o! by the recurrence of the Hermite polynomials
+        const float y = ((float)(u - LEAN_OFF) * (1.0f / 3.0f) - LEAN_FIRST) * inv_ws;
         float D[9];
         D[0] = __expf(-0.5f * y * y);
         D[1] = y * r * D[0];
 #pragma unroll
         for (int o = 2; o < 9; o++) D[o] = (y * D[o - 1] - r * D[o - 2]) * (r * (1.0f / (float)o));
         dtab[u] = D[0];
-        dtab[NODE_TAB + u] = D[1] - 0.3125f * D[5] - 0.390625f * D[7];
-        dtab[2 * NODE_TAB + u] = D[2] - 0.3125f * D[6] - 0.390625f * D[8];
-        dtab[3 * NODE_TAB + u] = D[3] + 1.25f * (D[5] + D[7]);
-        dtab[4 * NODE_TAB + u] = D[4] + 1.25f * (D[6] + D[8]);
+        dtab[LEAN_TAB + u] = D[1] - 0.3125f * D[5] - 0.390625f * D[7];
+        dtab[2 * LEAN_TAB + u] = D[2] - 0.3125f * D[6] - 0.390625f * D[8];
+        dtab[3 * LEAN_TAB + u] = D[3] + 1.25f * (D[5] + D[7]);
+        dtab[4 * LEAN_TAB + u] = D[4] + 1.25f * (D[6] + D[8]);
     }
     __syncthreads();
 }
-// wcat (H,16,hw): [0,64) dist_coef W_dist;  64 + (ax NORD + o) NODES + n: angle_coef sum_m W_ax[c,m] D_o(m - t_n).
+// wcat (H,16,hw): [0,64) dist_coef W_dist;  64 + (ax NORD + o) 64 + m': angle_coef sum_m W_ax[c,m] D_o(m - m').
 // grid: H*16 blocks (h, c), the threads over the words.
 struct WcatArgs {
     const float* Wd; const float* W1; const float* W2; const float* W3;      // (H,16,64) and (H,16,A) x 3
@@ -273,7 +292,7 @@ __device__ __forceinline__ void core_wcat_block(const WcatArgs& A, int hc) {
     const float dist_coef = A.dist_coef, angle_coef = A.angle_coef, ws = A.ws;
     float* __restrict__ wcat = A.wcat;
     __shared__ float row[3][NBINS];
-    __shared__ float dtab[NORD * NODE_TAB];
+    __shared__ float dtab[NORD * LEAN_TAB];
     if (hw == HW_ANG16) {
         // 16-bin basis: the weights themselves behind the distance block, zeros in the padding
         for (int w = threadIdx.x; w < hw; w += blockDim.x) {
@@ -293,19 +312,27 @@ __device__ __forceinline__ void core_wcat_block(const WcatArgs& A, int hc) {
             const float* W = u < NBINS ? W1 : (u < 2 * NBINS ? W2 : W3);
             row[u / NBINS][u % NBINS] = W[(size_t)hc * NBINS + (u % NBINS)];
         }
-        build_node_table(dtab, ws);
+        if (hw == HW_LEAN) build_node_table(dtab, ws);
+        else build_moment_table(dtab, ws);
     }
     for (int w = threadIdx.x; w < hw; w += blockDim.x) {
         float val;
         if (w < HW_DIST) val = dist_coef * Wd[(size_t)hc * NBINS + w];
-        else {
-            const int u = w - HW_DIST, ax = u / (NORD * NODES), o = (u / NODES) % NORD, n = u % NODES;
-            const float* dt = dtab + o * NODE_TAB + NODE_OFF - NODE_STEP * n;
+        else if (hw == HW_LEAN) {
+            const int u = w - HW_DIST, ax = u / (NORD * LEAN_NODES), o = (u / LEAN_NODES) % NORD, n = u % LEAN_NODES;
+            const float* dt = dtab + o * LEAN_TAB + LEAN_OFF - LEAN_STEP * n;
             float acc = 0.0f;
             if (ax < 3) {                  // (words past the last node: zero)
 #pragma unroll 8
                 for (int m = 0; m < NBINS; m++) acc = fmaf(row[ax][m], dt[3 * m], acc);
             }
+            val = angle_coef * acc;
+        } else {
+            const int u = w - HW_DIST, ax = u / (NORD * NBINS), o = (u / NBINS) % NORD, mp = u % NBINS;
+            const float* dt = dtab + o * 128 + 63 - mp;
+            float acc = 0.0f;
+#pragma unroll 8
+            for (int m = 0; m < NBINS; m++) acc = fmaf(row[ax][m], dt[m], acc);
             val = angle_coef * acc;
         }
         wcat[(size_t)hc * hw + w] = val;
@@ -330,14 +357,14 @@ __device__ __forceinline__ float core_slice_sum(const float* __restrict__ g, int
     for (int sl = 0; sl < CORE_GW_SLICES; sl++) sum += sl < nslices ? v[sl] : 0.0f;
     return sum;
 }
-// The way back: gW_dist = dist_coef gwcat[.., 0:64];  gW_ax[c,m] = angle_coef sum_{o,n} gwcat[.., ax,o,n] D_o(m - t_n).
+// The way back: gW_dist = dist_coef gwcat[.., 0:64];  gW_ax[c,m] = angle_coef sum_{o,m'} gwcat[.., ax,o,m'] D_o(m - m').
 // Block hc = (head, channel), 256 threads = (enc 0..3, bin m).  acc_dst: added to what the destinations hold.
 __device__ __forceinline__ void core_gw_finish_block(const float* __restrict__ gwcat, int nslices, size_t slice_stride,
                                                      int hw, float dist_coef, float angle_coef, float ws,
                                                      float* __restrict__ gWd, float* __restrict__ gW1,
                                                      float* __restrict__ gW2, float* __restrict__ gW3, int hc, bool acc_dst) {
-    __shared__ float dtab[NORD * NODE_TAB];
-    __shared__ float grow[3 * NORD * NODES];
+    __shared__ float dtab[NORD * 128];
+    __shared__ float grow[3 * NORD * NBINS];
     const int enc = threadIdx.x >> 6, m = threadIdx.x & 63;
     const float* g = gwcat + (size_t)hc * hw;
     if (hw == HW_ANG16) {
@@ -352,10 +379,10 @@ __device__ __forceinline__ void core_gw_finish_block(const float* __restrict__ g
         return;
     }
     if (hw > HW_DIST) {
-        for (int u = threadIdx.x; u < 3 * NORD * NODES; u += 256) {
+        for (int u = threadIdx.x; u < 3 * NORD * NBINS; u += 256) {
             grow[u] = core_slice_sum(g + HW_DIST + u, nslices, slice_stride);
         }
-        build_node_table(dtab, ws);
+        build_moment_table(dtab, ws);
     }
     if (enc == 0) {
         if (gWd) {
@@ -370,10 +397,10 @@ __device__ __forceinline__ void core_gw_finish_block(const float* __restrict__ g
     if (!dst) return;
     float acc = 0.0f;
     for (int o = 0; o < NORD; o++) {
-        const float* gr = grow + ((enc - 1) * NORD + o) * NODES;
-        const float* dt = dtab + o * NODE_TAB + NODE_OFF + 3 * m;
-#pragma unroll
-        for (int n = 0; n < NODES; n++) acc = fmaf(gr[n], dt[-NODE_STEP * n], acc);
+        const float* gr = grow + ((enc - 1) * NORD + o) * NBINS;
+        const float* dt = dtab + o * 128 + 63 + m;
+#pragma unroll 8
+        for (int mp = 0; mp < NBINS; mp++) acc = fmaf(gr[mp], dt[-mp], acc);
     }
     float* d = dst + (size_t)hc * NBINS + m;
     *d = (acc_dst ? *d : 0.0f) + angle_coef * acc;
@@ -570,7 +597,7 @@ struct CoreFwdShared {
     float pairC[FC_GROUP];       // exp(logit - running max) / S in fixed-point units
     float logit_s[NLOGIT];       // logits of the row (rows of more pairs park them in the probability array)
 };
-// LEAN: inference, nothing is kept for a backward pass: z and the probabilities are not written.
+// LEAN: inference, nothing is kept for a backward pass: fewer nodes for the moments; z and the probabilities are not written.
 template <int WL, int ANG, bool COS_ABS, bool LEAN = false>
 // ANG: angle bins, 0 (distance encoding alone), 64 (moment series) or 16 (basis values added directly)
 // (distance encoding alone: 4.8 KB of LDS per item allow eight wavefronts per SIMD; seven, with 72 registers and
@@ -578,8 +605,9 @@ template <int WL, int ANG, bool COS_ABS, bool LEAN = false>
 __global__ __launch_bounds__(WAVE * CORE_WPB) __attribute__((amdgpu_waves_per_eu(ANG > 0 ? 1 : 7)))
 void fused_core_fwd_kernel(const CoreArgs C) {
     constexpr bool HAS_ANG = ANG > 0;
-    constexpr int HWK = core_hist_words(ANG);                // words per item in memory
-    constexpr int HWL = core_hist_lds_words(ANG);            // ... and in LDS
+    constexpr int HWK = core_hist_words(ANG, LEAN);          // words per item in memory
+    constexpr int HWL = LEAN && ANG == NBINS ? HWK : core_hist_lds_words(ANG);      // ... and in LDS
+    constexpr int NODES = LEAN ? LEAN_NODES : NBINS;
     constexpr bool VEC = HWL == HWK && HWK >= 4 * WAVE;      // clear, rescale and store four words per lane at a time
     constexpr int NW = VEC ? (HWK / 4 + WAVE - 1) / WAVE : 1;
     constexpr bool FULL = HWK % (4 * WAVE) == 0;
@@ -749,7 +777,7 @@ void fused_core_fwd_kernel(const CoreArgs C) {
                             for (int ax = 0; ax < 3; ax++) {
                                 float cs = (dx * f[ax][0] + dy * f[ax][1] + dz * f[ax][2]) * rinv;
                                 if (COS_ABS) cs = fabsf(cs);
-                                const float uu = (cs - bc.ang_mu0) * bc.ang_inv_interval;      // in bin units (64 bins: in units of the nodes' distance)
+                                const float uu = (cs - bc.ang_mu0) * bc.ang_inv_interval;      // in bin (LEAN: node) units
                                 if (ANG == SMALL_A) {
                                     // all 16 basis values, outwards from bin 8 by the two-sided recurrence (sigma >= 1
                                     // bin: the value at bin 8 is at least e^-32 of the peak, no underflow)
@@ -763,7 +791,7 @@ void fused_core_fwd_kernel(const CoreArgs C) {
 #ifndef CFH_EXP_NOCONFLICT
                                 int32_t* hb = hist + HW_DIST + ax * NORD * NODES + (int)mf;
 #else
-                                int32_t* hb = hist + HW_DIST + ax * NORD * NODES + ((int)mf & 0) + lane;
+                                int32_t* hb = hist + HW_DIST + ax * NORD * NBINS + ((int)mf & 0) + lane;
 #endif
                                 float val = w;
                                 atomicAdd(hb, rint_i(val));
@@ -1094,12 +1122,12 @@ __global__ __launch_bounds__(WAVE) void core_gbuild_kernel(const float* __restri
 }
 
 // gwcat (slice,H,16,hw) = sum over a slice of the atoms of go (.,h,16) (x) hist (h,.,hw): wavefront per (head, 64-word
-// block, slice); four MFMA tiles with interleaved columns as above.  grid (ceil(hw/64 / waves), H, nslices), at most
+// block, slice); four MFMA tiles with interleaved columns as above.  grid (ceil(hw/64 / GW_WPB), H, nslices), at most
 // CORE_GW_SLICES slices.
 __device__ __forceinline__ void core_gwcat_block(const float* __restrict__ go, const float* __restrict__ hist,
                                                  float* __restrict__ gwcat, int N, int H, int hw, int per_slice, int slice) {
-    // the wavefronts of a workgroup take neighbouring pieces of the same rows at the same time: each 256
-    // contiguous bytes behind the one before, instead of 256 bytes every 4 KB (82 -> 70 us for the four layers of the benchmark)
+    // the GW_WPB wavefronts of a workgroup take neighbouring pieces of the same rows at the same time: GW_WPB x 256
+    // contiguous bytes of a row instead of 256 bytes every 4 KB (82 -> 70 us for the four layers of the benchmark)
     const int lane = threadIdx.x & (WAVE - 1), col = lane & 15, kk = lane >> 4;
     const int w0 = ((int)blockIdx.x * (int)(blockDim.x >> 6) + (int)(threadIdx.x >> 6)) * 64, h = blockIdx.y;
     if (w0 >= hw) return;
@@ -1146,14 +1174,12 @@ __device__ __forceinline__ void core_gwcat_block(const float* __restrict__ go, c
         *reinterpret_cast<float4*>(part + ((size_t)h * DH + 4 * kk + r) * hw + w0 + 4 * col) =
             make_float4(acc[0][r], acc[1][r], acc[2][r], acc[3][r]);
 }
-// wavefronts per workgroup of the two kernels below: the blocks of 64 words of a row, shared evenly (640 words: 2 x 5)
-constexpr int GW_WPB = 5;
-__host__ __device__ constexpr int core_gw_waves(int hw) { return hw / 64 <= GW_WPB ? hw / 64 : GW_WPB; }
+constexpr int GW_WPB = 4;          // wavefronts per workgroup of the two kernels below (8: the same; 16: far slower)
 __global__ __launch_bounds__(WAVE * GW_WPB) void core_gwcat_kernel(const float* __restrict__ go, const float* __restrict__ hist,
                                                           float* __restrict__ gwcat, int N, int H, int hw, int per_slice) {
     core_gwcat_block(go, hist, gwcat, N, H, hw, per_slice, (int)blockIdx.z);
 }
-// several jobs: grid (ceil(hw/64 / waves), H, slices of all jobs); the job of a slice by a scan of the (few) jobs
+// several jobs: grid (ceil(hw/64 / GW_WPB), H, slices of all jobs); the job of a slice by a scan of the (few) jobs
 __global__ __launch_bounds__(WAVE * GW_WPB) void core_gwcat_multi_kernel(const CoreWgradJobs T) {
     int j = 0;
     while (j + 1 < T.njobs && (int)blockIdx.z >= T.job[j + 1].slice0) j++;
@@ -1239,16 +1265,13 @@ __global__ __launch_bounds__(WAVE * CORE_WPB) void fused_core_bwd_kernel(const C
         {
             const float* src = C.G + ((size_t)h * P.N + i) * HWK;
             if (HWK >= 4 * WAVE) {
-                constexpr int NW = (HWK / 4 + WAVE - 1) / WAVE;
-                constexpr bool FULL = HWK % (4 * WAVE) == 0;
+                constexpr int NW = HWK >= 4 * WAVE ? HWK / (4 * WAVE) : 1;
                 float4 g4[NW];
 #pragma unroll
-                for (int u = 0; u < NW; u++)
-                    g4[u] = FULL || lane + WAVE * u < HWK / 4 ? reinterpret_cast<const float4*>(src)[lane + WAVE * u]
-                                                              : make_float4(0.f, 0.f, 0.f, 0.f);
+                for (int u = 0; u < NW; u++) g4[u] = reinterpret_cast<const float4*>(src)[lane + WAVE * u];
 #pragma unroll
                 for (int u = 0; u < NW; u++) {
-                    if (FULL || lane + WAVE * u < HWK / 4) reinterpret_cast<float4*>(Gs)[lane + WAVE * u] = g4[u];
+                    reinterpret_cast<float4*>(Gs)[lane + WAVE * u] = g4[u];
                     gabs += (fabsf(g4[u].x) + fabsf(g4[u].y)) + (fabsf(g4[u].z) + fabsf(g4[u].w));
                 }
             } else {
@@ -1329,18 +1352,18 @@ __global__ __launch_bounds__(WAVE * CORE_WPB) void fused_core_bwd_kernel(const C
                             for (int ax = 0; ax < 3; ax++) {
                                 float cs = (dx * f[ax][0] + dy * f[ax][1] + dz * f[ax][2]) * rinv;
                                 if (COS_ABS) cs = fabsf(cs);
-                                const float uu = (cs - bc.ang_mu0) * bc.ang_inv_interval;      // (as in the forward)
+                                const float uu = (cs - bc.ang_mu0) * bc.ang_inv_interval;
                                 if (ANG == SMALL_A) {
                                     const WindowSeed sa = window_seed(((float)(SMALL_A / 2) - uu) * bc.ang_step, bc.ang_step, 1.0f);
                                     bg += window_gather<SMALL_A>(Gs + HW_DIST + ax * SMALL_A, sa, bc.ang_cc);
                                     continue;
                                 }
-                                const float mf = clampf(__builtin_rintf(uu), 0.0f, (float)(NODES - 1));
+                                const float mf = clampf(__builtin_rintf(uu), 0.0f, (float)(NBINS - 1));
                                 const float eps = 2.0f * (uu - mf);
-                                const float* gb = Gs + HW_DIST + ax * NORD * NODES + (int)mf;
+                                const float* gb = Gs + HW_DIST + ax * NORD * NBINS + (int)mf;
                                 float pw = eps, part = gb[0];
 #pragma unroll
-                                for (int o = 1; o < NORD; o++) { part = fmaf(pw, gb[o * NODES], part); pw *= eps; }
+                                for (int o = 1; o < NORD; o++) { part = fmaf(pw, gb[o * NBINS], part); pw *= eps; }
                                 bg += part;
                             }
                         }

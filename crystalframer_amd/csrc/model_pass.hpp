@@ -81,7 +81,7 @@ void model_buffers(const cfh_model* m, const cfh_model_batch* b, ModelBuffers& M
     Carver c{reinterpret_cast<char*>(b->arena)};
     const size_t N = b->N, E = b->E, B = b->B, D = m->D, F = m->F, H = m->heads;
     const int ang = m->layer[0].core.angle_bins;
-    const size_t hw = cfh::core_hist_words(ang);
+    const size_t hw = cfh::core_hist_words(ang, !b->keep);
     M.edges = c.take<int64_t>(2 * E);
     M.e_start = c.take<int64_t>(N + 1);
     M.atom_start = c.take<int64_t>(B + 1);
@@ -350,7 +350,7 @@ int cfh_model_forward(const cfh_model* m, const cfh_model_batch* b, float* out) 
             if (b->keep) S.add(cfh::BS_BACKWARD, L.Wo, L.W1, L.W2, Wq, M.layer[l].stream_bwd);
             const bool ang = p.angle_bins > 0;
             A.wcat[nw++] = cfh::WcatArgs{L.W_dist, ang ? L.W_axis1 : nullptr, ang ? L.W_axis2 : nullptr, ang ? L.W_axis3 : nullptr,
-                                         cfh::core_hist_words(p.angle_bins), p.dist_coef, p.angle_coef, p.angle_wscale,
+                                         cfh::core_hist_words(p.angle_bins, !b->keep), p.dist_coef, p.angle_coef, p.angle_wscale,
                                          M.layer[l].wcat};
         }
         launch();

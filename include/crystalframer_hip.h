@@ -319,7 +319,7 @@ int cfh_framed_pe_backward_pairwise(const cfh_params* p, const float* a_ih, cons
  * qs = query / sqrt(Dh).
  * Results kept for the backward: z (E,H), prob (E,H) = P, hist (H,N,words) the normalised histograms
  * (head-major: the kernels that contract them with the weights read the rows of a head one after the other)
- * (words = cfh_fused_core_hist_words: 64 distance bins, then per axis and order 38 moment nodes, padded to 640; with 16
+ * (words = cfh_fused_core_hist_words: 64 distance bins, then per axis and order 64 moment bins = 1024; with 16
  * angle bins 64 + 3 x 16 padded to 128), out (N,H,Dh).
  * workspace: cfh_fused_core_workspace_bytes(p, N, E, B, 0).
  *
