@@ -1604,6 +1604,21 @@ void project_launch(int hw, const float* hist, const float* wcat, float* out, in
     else if (hw == cfh::HW_ANG16) launch(cfh::core_project_kernel<2, 1>, 2);
     else launch(cfh::core_project_kernel<1, 1>, 1);
 }
+// Up to this many (atom, head) items the forward pass of a layer is one wavefront per item from the record to the sums: about
+// as many as are resident at once (19 to 23 per compute unit).  Measured with and without, whole calls: 976 items 274 and 256
+// us, 4592 items 412 and 380, 7712 items 446 and 415, 10 696 items 398 and 441; cells of 40 to 200 atoms lose from 5760 items
+// on (386 and 397), where the frame search of four heads per wavefront counts for more than the launch it takes.
+constexpr int64_t ITEM_PASS_MAX = 5120;
+template <typename Kern>
+int launch_item_pass(Kern kern, const cfh::CoreArgs& C, bool search, hipStream_t st, const char* what) {
+    {
+        TimedScope timed(what, st);
+        hipLaunchKernelGGL(kern, dim3((unsigned)C.K.N * (unsigned)C.K.H), dim3(cfh::WAVE), 0, st, C, search ? 1 : 0);
+    }
+    return finish_launch(what);
+}
+#define CFH_ITEM_PASS(...) launch_item_pass(cfh::item_pass_kernel<__VA_ARGS__>, C, search, st, what)
+#define CFH_ITEM_PASS_LEAN(...) launch_item_pass(cfh::item_pass_kernel<__VA_ARGS__, true>, C, search, st, what)
 #define CFH_CORE_FWD(...) launch_core(cfh::fused_core_fwd_kernel<__VA_ARGS__>, C, st, what)
 #define CFH_CORE_FWD_LEAN(...) launch_core(cfh::fused_core_fwd_kernel<__VA_ARGS__, true>, C, st, what)
 #define CFH_CORE_BWD(...) launch_core(cfh::fused_core_bwd_kernel<__VA_ARGS__>, C, st, what)
@@ -1657,7 +1672,16 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
     const int hw = cfh::core_hist_words(p->angle_bins, lean);
     const cfh::WcatArgs WA{W_dist, W_axis1, W_axis2, W_axis3, hw, p->dist_coef, p->angle_coef,
                            p->angle_wscale, wcat};
-    {
+    // (the word of the noise's seed is copied and advanced by the launch that makes the records)
+    const bool one_launch = N * p->num_heads <= ITEM_PASS_MAX && !(search && p->symm_break_noise > 0.0f && C.K.seed_dev);
+    if (one_launch) {
+        if (!wcat_made) {
+            TimedScope timed("core_prepare", st);
+            hipLaunchKernelGGL(cfh::core_wcat_kernel, dim3(p->num_heads * cfh::DH), dim3(256), 0, st, WA);
+        }
+        if (search) { C.K.q = qs; C.K.k = k; C.K.out_frame = frames; C.K.frames_to_records = 1; }
+        else C.K.frames = has_ang ? frames : nullptr;
+    } else {
         const int prep_blocks = L.prep_blocks, wcat_blocks = wcat_made ? 0 : p->num_heads * cfh::DH;
         // records whose box is not the table's are listed by the launch that makes them and taken first by the main kernel
         if (buf.table) {
@@ -1718,9 +1742,11 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
             C.K.bc.ang_mu0 += cfh::LEAN_FIRST * C.K.bc.ang_interval;
             C.K.bc.ang_inv_interval *= 3.0f / cfh::LEAN_STEP;
         }
-        CFH_CORE_DISPATCH(CFH_CORE_FWD_LEAN);
+        if (one_launch) { CFH_CORE_DISPATCH(CFH_ITEM_PASS_LEAN); }
+        else { CFH_CORE_DISPATCH(CFH_CORE_FWD_LEAN); }
     } else {
-        CFH_CORE_DISPATCH(CFH_CORE_FWD);
+        if (one_launch) { CFH_CORE_DISPATCH(CFH_ITEM_PASS); }
+        else { CFH_CORE_DISPATCH(CFH_CORE_FWD); }
     }
     if (rc) return rc;
     {

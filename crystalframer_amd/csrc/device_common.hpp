@@ -487,6 +487,53 @@ __device__ __forceinline__ uint32_t load_record(const KernelArgs& P, int it, int
     return (it >= 0 && threadIdx.x < REC_WORDS) ? P.items[((size_t)it * P.H + h) * REC_WORDS + threadIdx.x] : 0u;
 }
 
+// What an item's record says besides its lattice rows and its query or frames.
+struct RecordHead {
+    int i, b, e0, npairs, j0;
+    float a;
+    Box bx;
+    uint32_t boxw;
+};
+__device__ __forceinline__ RecordHead record_head(const KernelArgs& P, int it, int h) {
+    RecordHead R;
+    R.i = P.order ? P.order[it] : it;
+    R.b = (int)P.batch[R.i];
+    R.a = P.a_ih[(size_t)R.i * P.H + h];
+    float rvl1 = 0.f, rvl2 = 0.f, rvl3 = 0.f;
+    if (P.rvlen) { rvl1 = P.rvlen[(size_t)R.b * 3 + 0]; rvl2 = P.rvlen[(size_t)R.b * 3 + 1]; rvl3 = P.rvlen[(size_t)R.b * 3 + 2]; }
+    R.bx = translation_box(R.a, rvl1, rvl2, rvl3, P.cutoff_radius, P.lattice_range, P.minimum_range);
+    if (R.bx.over && P.status) atomicOr(P.status, 1);
+    R.boxw = (uint32_t)(R.bx.R1 | (R.bx.R2 << 8) | (R.bx.R3 << 16));
+    R.e0 = (int)P.e_start[R.i];
+    R.npairs = (int)P.e_start[R.i + 1] - R.e0;
+    R.j0 = R.npairs > 0 ? (int)P.edges[(size_t)P.E + R.e0] : R.i;      // first neighbour atom
+    if (P.contiguous_neighbours) {
+        // a layout other than whole n x n blocks would make the kernels read other atoms than the pairs name, or
+        // past the last atom: say so in the status word and keep every read inside the arrays
+        const int np = R.npairs;
+        const bool bad = R.j0 < 0 || R.j0 + np > P.N || (np > 0 && (int)P.edges[(size_t)P.E + R.e0 + np - 1] != R.j0 + np - 1);
+        if (bad) {
+            if (P.status) atomicOr(P.status, 2);
+            R.j0 = max(0, min(R.j0, P.N - np));
+        }
+    }
+    return R;
+}
+// The record of an item made by the wavefront that needs it: the word of this lane.
+__device__ __forceinline__ uint32_t make_record_lane(const KernelArgs& P, int it, int h, int lane, bool with_query) {
+    const RecordHead R = record_head(P, it, h);
+    if (lane >= REC_LATTICE && lane < REC_LATTICE + 9) return __float_as_uint(P.tvecs[(size_t)R.b * 9 + (lane - REC_LATTICE)]);
+    if (with_query && lane >= REC_QUERY && lane < REC_QUERY + DH)
+        return __float_as_uint(P.q[((size_t)R.i * P.H + h) * DH + (lane - REC_QUERY)]);
+    if (!with_query && P.frames && lane >= REC_FRAMES && lane < REC_FRAMES + 9) {
+        const int c = lane - REC_FRAMES, ax = c / 3, d = c - 3 * ax;
+        return __float_as_uint(P.frames[(((size_t)ax * P.N + R.i) * P.H + h) * 3 + d]);
+    }
+    return lane == REC_ATOM ? (uint32_t)R.i : lane == REC_E0 ? (uint32_t)R.e0 : lane == REC_NPAIRS ? (uint32_t)R.npairs
+         : lane == REC_BOX ? R.boxw : lane == REC_A ? __float_as_uint(R.a) : lane == 30 ? (uint32_t)R.j0
+         : lane == 31 ? (uint32_t)R.b : 0u;
+}
+
 // One thread per (item, head): builds the records, clears the work queues of the launch and (backward)
 // the weight-gradient outputs that the reduction after the main kernel adds into.
 __device__ __forceinline__ void prepare_items_block(const KernelArgs& P, int with_query, int block) {
@@ -507,45 +554,34 @@ __device__ __forceinline__ void prepare_items_block(const KernelArgs& P, int wit
     }
     const bool valid = idx < P.N * P.H;
     bool slow = false;
-    uint32_t* rec = P.items + (size_t)(valid ? idx : 0) * REC_WORDS;
-    uint32_t boxw = 0;
+    RecordHead R{};
+    float4 tail[7];               // words 4 .. 31
     if (valid) {
         const int it = idx / P.H, h = idx - it * P.H;
-        const int i = P.order ? P.order[it] : it;
-        const int b = (int)P.batch[i];
-        const float a = P.a_ih[(size_t)i * P.H + h];
-        float rvl1 = 0.f, rvl2 = 0.f, rvl3 = 0.f;
-        if (P.rvlen) { rvl1 = P.rvlen[(size_t)b * 3 + 0]; rvl2 = P.rvlen[(size_t)b * 3 + 1]; rvl3 = P.rvlen[(size_t)b * 3 + 2]; }
-        const Box bx = translation_box(a, rvl1, rvl2, rvl3, P.cutoff_radius, P.lattice_range, P.minimum_range);
-        if (bx.over && P.status) atomicOr(P.status, 1);
-        const int e0 = (int)P.e_start[i];
-        rec[REC_ATOM] = (uint32_t)i;
-        rec[REC_E0] = (uint32_t)e0;
-        rec[REC_NPAIRS] = (uint32_t)((int)P.e_start[i + 1] - e0);
-        boxw = (uint32_t)(bx.R1 | (bx.R2 << 8) | (bx.R3 << 16));
-        slow = P.slow_count != nullptr && !(bx.R1 == P.slow_R && bx.R2 == P.slow_R && bx.R3 == P.slow_R);
-        rec[REC_A] = __float_as_uint(a);
-        for (int d = 0; d < 9; d++) rec[REC_LATTICE + d] = __float_as_uint(P.tvecs[(size_t)b * 9 + d]);
-        int j0 = P.e_start[i + 1] > e0 ? (int)P.edges[(size_t)P.E + e0] : i;      // first neighbour atom
-        if (P.contiguous_neighbours) {
-            // a layout other than whole n x n blocks would make the kernels read other atoms than the pairs name, or
-            // past the last atom: say so in the status word and keep every read inside the arrays
-            const int np = (int)P.e_start[i + 1] - e0;
-            const bool bad = j0 < 0 || j0 + np > P.N || (np > 0 && (int)P.edges[(size_t)P.E + e0 + np - 1] != j0 + np - 1);
-            if (bad) {
-                if (P.status) atomicOr(P.status, 2);
-                j0 = max(0, min(j0, P.N - np));
-            }
-        }
-        rec[30] = (uint32_t)j0;
-        rec[31] = (uint32_t)b;                                                                  // crystal
+        R = record_head(P, it, h);
+        slow = P.slow_count != nullptr && !(R.bx.R1 == P.slow_R && R.bx.R2 == P.slow_R && R.bx.R3 == P.slow_R);
+        const float* L = P.tvecs + (size_t)R.b * 9;
+        float q[DH] = {};
         if (with_query) {
-            for (int c = 0; c < DH; c++) rec[REC_QUERY + c] = __float_as_uint(P.q[((size_t)i * P.H + h) * DH + c]);
+            const float4* src = reinterpret_cast<const float4*>(P.q + ((size_t)R.i * P.H + h) * DH);
+#pragma unroll
+            for (int c = 0; c < DH / 4; c++) {
+                const float4 v = src[c];
+                q[4 * c] = v.x; q[4 * c + 1] = v.y; q[4 * c + 2] = v.z; q[4 * c + 3] = v.w;
+            }
         } else if (P.frames) {
+#pragma unroll
             for (int ax = 0; ax < 3; ax++)
-                for (int d = 0; d < 3; d++)
-                    rec[REC_FRAMES + ax * 3 + d] = __float_as_uint(P.frames[(((size_t)ax * P.N + i) * P.H + h) * 3 + d]);
+#pragma unroll
+                for (int d = 0; d < 3; d++) q[ax * 3 + d] = P.frames[(((size_t)ax * P.N + R.i) * P.H + h) * 3 + d];
         }
+        tail[0] = make_float4(R.a, L[0], L[1], L[2]);
+        tail[1] = make_float4(L[3], L[4], L[5], L[6]);
+        tail[2] = make_float4(L[7], L[8], q[0], q[1]);
+        tail[3] = make_float4(q[2], q[3], q[4], q[5]);
+        tail[4] = make_float4(q[6], q[7], q[8], q[9]);
+        tail[5] = make_float4(q[10], q[11], q[12], q[13]);
+        tail[6] = make_float4(q[14], q[15], __int_as_float(R.j0), __int_as_float(R.b));
     }
     // The records whose box is not the usual one take several times as long as the others in the kernels that
     // follow, and most of them are atoms of small crystals at the END of the work order, where they alone make the
@@ -562,11 +598,17 @@ __device__ __forceinline__ void prepare_items_block(const KernelArgs& P, int wit
         for (int w = 0; w < 4; w++) { rank += w < wv ? slow_in_wave[w] : 0; total += slow_in_wave[w]; }
         if (slow) {
             P.slow_list[block * SLOW_PREP_SLOTS + rank] = idx;
-            boxw |= REC_BOX_LISTED;
+            R.boxw |= REC_BOX_LISTED;
         }
         if (threadIdx.x == 0) P.slow_count[block] = total;
     }
-    if (valid) rec[REC_BOX] = boxw;
+    if (valid) {
+        // (16 bytes at a time: a record is a cache line of its own)
+        uint32_t* rec = P.items + (size_t)idx * REC_WORDS;
+        *reinterpret_cast<uint4*>(rec) = make_uint4((uint32_t)R.i, (uint32_t)R.e0, (uint32_t)R.npairs, R.boxw);
+#pragma unroll
+        for (int u = 0; u < 7; u++) reinterpret_cast<float4*>(rec)[1 + u] = tail[u];
+    }
 }
 __global__ __launch_bounds__(256) void prepare_items_kernel(const KernelArgs P, int with_query) {
     prepare_items_block(P, with_query, (int)blockIdx.x);

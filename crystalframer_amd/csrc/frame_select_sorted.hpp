@@ -696,4 +696,25 @@ __global__ __launch_bounds__(WAVE * CORE_WPB) void frame_axes_kernel(const CoreA
     frame_item_body(C, shared[wv].item, wid, lane, !listed, !listed && slow_blocks > 0);
 }
 
+// Everything of an item in one wavefront, for few items: its record, the search for its frame, the lattice sums.  In
+// launches of their own each of the three is a chain of dependent steps behind a launch that fills a fraction of the chip.
+// One crystal of 8 atoms: 22 us in three launches, 17 in one; a whole call of four layers 185 -> 173.
+template <int WL, int ANG, bool COS_ABS, bool LEAN = false>
+__global__ __launch_bounds__(WAVE) void item_pass_kernel(const CoreArgs C, int search) {
+    __shared__ union { FrameShared frame; CoreFwdLds<ANG, LEAN> core; } sh;
+    const KernelArgs& P = C.K;
+    const int wid = (int)blockIdx.x, lane = (int)threadIdx.x;
+    const int it = div_heads(P, wid), h = wid - it * P.H;
+    if (it >= P.N) return;
+    // (the record goes to memory: the searches and sums read it there, and so does a backward pass)
+    const uint32_t rec = make_record_lane(P, it, h, lane, search != 0);
+    if (lane < REC_WORDS) P.items[((size_t)it * P.H + h) * REC_WORDS + lane] = rec;
+    __threadfence_block();
+    if (ANG > 0 && search) {
+        frame_item_body(C, sh.frame, wid, lane, false, false);
+        __threadfence_block();
+    }
+    fused_core_fwd_body<WL, ANG, COS_ABS, LEAN>(C, sh.core, wid);
+}
+
 }  // namespace cfh

@@ -598,12 +598,12 @@ struct CoreFwdShared {
     float logit_s[NLOGIT];       // logits of the row (rows of more pairs park them in the probability array)
 };
 // LEAN: inference, nothing is kept for a backward pass: fewer nodes for the moments; z and the probabilities are not written.
-template <int WL, int ANG, bool COS_ABS, bool LEAN = false>
+template <int ANG, bool LEAN>
+using CoreFwdLds = CoreFwdShared<LEAN && ANG == NBINS ? core_hist_words(ANG, LEAN) : core_hist_lds_words(ANG), LEAN ? 4 : FC_LOGCAP>;
 // ANG: angle bins, 0 (distance encoding alone), 64 (moment series) or 16 (basis values added directly)
-// (distance encoding alone: 4.8 KB of LDS per item allow eight wavefronts per SIMD; seven, with 72 registers and
-// nothing spilled, ran faster than eight with 64 and nine spilled)
-__global__ __launch_bounds__(WAVE * CORE_WPB) __attribute__((amdgpu_waves_per_eu(ANG > 0 ? 1 : 7)))
-void fused_core_fwd_kernel(const CoreArgs C) {
+// wid: this wavefront's (item, head)
+template <int WL, int ANG, bool COS_ABS, bool LEAN>
+__device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLds<ANG, LEAN>& sh, int wid) {
     constexpr bool HAS_ANG = ANG > 0;
     constexpr int HWK = core_hist_words(ANG, LEAN);          // words per item in memory
     constexpr int HWL = LEAN && ANG == NBINS ? HWK : core_hist_lds_words(ANG);      // ... and in LDS
@@ -611,9 +611,6 @@ void fused_core_fwd_kernel(const CoreArgs C) {
     constexpr bool VEC = HWL == HWK && HWK >= 4 * WAVE;      // clear, rescale and store four words per lane at a time
     constexpr int NW = VEC ? (HWK / 4 + WAVE - 1) / WAVE : 1;
     constexpr bool FULL = HWK % (4 * WAVE) == 0;
-    using Shared = CoreFwdShared<HWL, LEAN ? 4 : FC_LOGCAP>;
-    __shared__ Shared shared[CORE_WPB];
-    Shared& sh = shared[threadIdx.x >> 6];
     float4* const tab = sh.tab;
     uint16_t* const list = sh.list;
     int32_t* const hist = sh.hist;
@@ -624,8 +621,6 @@ void fused_core_fwd_kernel(const CoreArgs C) {
     const KernelArgs& P = C.K;
     const int lane = threadIdx.x & (WAVE - 1);
     const int H = P.H;
-    const int wid = core_wave_record(C, (int)blockIdx.x * CORE_WPB + (int)(threadIdx.x >> 6), lane);      // this wavefront's (item, head)
-    if (wid < 0) return;
     const int it_cur = div_heads(P, wid);      // items in descending order of their pair count: the long ones start first
     const int h = wid - it_cur * H;
     const int pr = lane >> 3;          // pair of the group served by this 8-lane row
@@ -996,6 +991,16 @@ void fused_core_fwd_kernel(const CoreArgs C) {
             atomicAdd(P.stats + STAT_FWD_SEEN, n_seen);
         }
     }
+}
+
+// (distance encoding alone: 4.8 KB of LDS per item allow eight wavefronts per SIMD; seven, with 72 registers and
+// nothing spilled, ran faster than eight with 64 and nine spilled)
+template <int WL, int ANG, bool COS_ABS, bool LEAN = false>
+__global__ __launch_bounds__(WAVE * CORE_WPB) __attribute__((amdgpu_waves_per_eu(ANG > 0 ? 1 : 7)))
+void fused_core_fwd_kernel(const CoreArgs C) {
+    __shared__ CoreFwdLds<ANG, LEAN> shared[CORE_WPB];
+    const int wid = core_wave_record(C, (int)blockIdx.x * CORE_WPB + (int)(threadIdx.x >> 6), (int)threadIdx.x & (WAVE - 1));
+    if (wid >= 0) fused_core_fwd_body<WL, ANG, COS_ABS, LEAN>(C, shared[threadIdx.x >> 6], wid);
 }
 
 // out (N,H,16) += Wcat_h (16, hw) . hist (H,N,hw): one workgroup of WAVES wavefronts per (16 atoms, head); each

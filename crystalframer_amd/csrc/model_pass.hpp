@@ -325,37 +325,39 @@ int cfh_model_forward(const cfh_model* m, const cfh_model_batch* b, float* out) 
         if (A.table_R > 0) {
             constexpr int per = cfh::START_THREADS / cfh::FC_TCAP;
             A.table = M.table;
-            A.near = reinterpret_cast<float2*>(M.near_);
             A.table_blocks = (int)((B + per - 1) / per);
         }
-        A.hc = H * cfh::DH;
         StreamList S(D, F, st, m->feat);
         S.add(cfh::BS_INPUTS, m->We, nullptr, nullptr, m->layer[0].Wqkv, M.front_stream);
         if (b->keep) S.add(cfh::BS_INPUTS_BACKWARD, nullptr, nullptr, nullptr, m->layer[0].Wqkv, M.front_stream_bwd);
-        int nw = 0;
-        auto launch = [&]() {      // (also when a table of the arguments is full)
+        cfh::StartWcat W{};
+        W.hc = H * cfh::DH;
+        auto launch = [&]() {      // (also when the list of the streams is full)
             A.streams = S.T;
-            A.stream_blocks = (S.blocks + cfh::START_THREADS / 256 - 1) / (cfh::START_THREADS / 256);
-            hipLaunchKernelGGL(cfh::model_start_kernel, dim3((unsigned)(A.geo_blocks + A.table_blocks + A.stream_blocks + nw * A.hc)),
+            const int stream_blocks = (S.blocks + cfh::START_THREADS / 256 - 1) / (cfh::START_THREADS / 256);
+            hipLaunchKernelGGL(cfh::model_start_kernel, dim3((unsigned)(A.geo_blocks + A.table_blocks + stream_blocks)),
                                dim3(cfh::START_THREADS), 0, st, A);
             S.clear();
-            A.geo_blocks = A.table_blocks = nw = 0;
+            A.geo_blocks = A.table_blocks = 0;
         };
         for (int l = 0; l < m->layers; l++) {
             const cfh_model_layer& L = m->layer[l];
             const cfh_params& p = L.core;
             const float* const Wq = l + 1 < m->layers ? m->layer[l + 1].Wqkv : nullptr;
-            if (nw == cfh::START_MAX_WCAT || S.T.n + 2 > cfh::BR_MAX_STREAMS) launch();
+            if (S.T.n + 2 > cfh::BR_MAX_STREAMS) launch();
             S.add(cfh::BS_FORWARD, L.Wo, L.W1, L.W2, Wq, M.layer[l].stream);
             if (b->keep) S.add(cfh::BS_BACKWARD, L.Wo, L.W1, L.W2, Wq, M.layer[l].stream_bwd);
             const bool ang = p.angle_bins > 0;
-            A.wcat[nw++] = cfh::WcatArgs{L.W_dist, ang ? L.W_axis1 : nullptr, ang ? L.W_axis2 : nullptr, ang ? L.W_axis3 : nullptr,
-                                         cfh::core_hist_words(p.angle_bins, !b->keep), p.dist_coef, p.angle_coef, p.angle_wscale,
-                                         M.layer[l].wcat};
+            const cfh::WcatArgs w{L.W_dist, ang ? L.W_axis1 : nullptr, ang ? L.W_axis2 : nullptr, ang ? L.W_axis3 : nullptr,
+                                  cfh::core_hist_words(p.angle_bins, !b->keep), p.dist_coef, p.angle_coef, p.angle_wscale,
+                                  M.layer[l].wcat};
+            if (W.n < cfh::START_MAX_WCAT) W.w[W.n++] = w;
+            else hipLaunchKernelGGL(cfh::core_wcat_kernel, dim3((unsigned)W.hc), dim3(256), 0, st, w);
         }
         launch();
         const int atom_blocks = (int)((N + 256) / 256);
-        hipLaunchKernelGGL(cfh::model_pairs_kernel, dim3((unsigned)(atom_blocks + (E + 31) / 32)), dim3(256), 0, st, A, atom_blocks);
+        const cfh::PairsArgs P{g, A.table, reinterpret_cast<float2*>(M.near_), A.table_R, atom_blocks};
+        hipLaunchKernelGGL(cfh::model_pairs_kernel, dim3((unsigned)(W.n * W.hc + atom_blocks + (E + 31) / 32)), dim3(256), 0, st, P, W);
         if ((rc = finish_launch("model_start"))) return rc;
     }
     {   // embedding and the inputs of the first layer

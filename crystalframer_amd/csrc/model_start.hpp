@@ -1,7 +1,7 @@
 // What a pass over a batch starts with, in two launches: everything that depends on nothing but the caller's tensors, then
 // what is made of it per atom and pair.  The parts are those of geometry.hpp, fused_core.hpp and layer_bridge.hpp; each is
-// a few microseconds of work that fills a fraction of the chip, and one by one -- five launches, and a part of every layer's
-// launch that makes the item records -- they took @@.
+// a few microseconds of work that fills a fraction of the chip.  One by one -- six launches, and a part of every layer's
+// launch that makes the item records -- they made up 35 of the 196 us of a call for one crystal; together 20.
 #pragma once
 #include "fused_core.hpp"
 #include "geometry.hpp"
@@ -10,19 +10,23 @@
 namespace cfh {
 
 constexpr int START_THREADS = GEO_THREADS;
-constexpr int START_MAX_WCAT = 8;
+constexpr int START_MAX_WCAT = 24;
 struct StartArgs {
     GeometryArgs geo;
     float4* table;                // sorted shifts of every crystal, or null
-    float2* near;                 // nearest images of every pair over that table
     int table_R;
-    int geo_blocks, table_blocks, stream_blocks;      // workgroups of the parts, in this order; then heads x 16 per layer
-    int hc;                       // heads x 16
+    int geo_blocks, table_blocks;      // workgroups of the parts, in this order; behind them the streams
     BridgeStreams streams;
-    WcatArgs wcat[START_MAX_WCAT];
+};
+// What the second launch makes besides: the cores' concatenated weights, heads x 16 workgroups per layer (the first launch
+// has the longer chain without them).
+struct StartWcat {
+    WcatArgs w[START_MAX_WCAT];
+    int n, hc;                    // layers, heads x 16
 };
 // The prefix sums over the crystals (one workgroup, the longest part) come first.
-__global__ __launch_bounds__(START_THREADS) void model_start_kernel(const StartArgs A) {
+// (two workgroups per compute unit)
+__global__ __launch_bounds__(START_THREADS) __attribute__((amdgpu_waves_per_eu(8))) void model_start_kernel(const StartArgs A) {
     int block = (int)blockIdx.x;
     if (block < A.geo_blocks) { geometry_crystals_block(A.geo, block); return; }
     block -= A.geo_blocks;
@@ -35,16 +39,20 @@ __global__ __launch_bounds__(START_THREADS) void model_start_kernel(const StartA
         return;
     }
     block -= A.table_blocks;
-    if (block < A.stream_blocks) {
-        bridge_stream_element(A.streams, block * (START_THREADS / 256) + (int)threadIdx.x / 256, (int)threadIdx.x % 256);
-        return;
-    }
-    block -= A.stream_blocks;
-    core_wcat_block(A.wcat[block / A.hc], block % A.hc);
+    bridge_stream_element(A.streams, block * (START_THREADS / 256) + (int)threadIdx.x / 256, (int)threadIdx.x % 256);
 }
-// Workgroups of 256: a thread per atom (and one more), then eight lanes per pair.
-__global__ __launch_bounds__(256) void model_pairs_kernel(const StartArgs A, int atom_blocks) {
-    const int block = (int)blockIdx.x;
+// Workgroups of 256: the concatenated weights, a thread per atom (and one more), eight lanes per pair.
+struct PairsArgs {
+    GeometryArgs geo;
+    float4* table;
+    float2* near;
+    int table_R, atom_blocks;
+};
+__global__ __launch_bounds__(256) void model_pairs_kernel(const PairsArgs A, const StartWcat W) {
+    int block = (int)blockIdx.x;
+    if (block < W.n * W.hc) { core_wcat_block(W.w[block / W.hc], block % W.hc); return; }
+    block -= W.n * W.hc;
+    const int atom_blocks = A.atom_blocks;
     if (block < atom_blocks) { geometry_atom(A.geo, block * 256 + (int)threadIdx.x); return; }
     const long long e = (long long)(block - atom_blocks) * 32 + (threadIdx.x >> 3);
     const int sub = threadIdx.x & 7;
