@@ -1593,16 +1593,16 @@ int launch_core(Kern kern, const cfh::CoreArgs& C, hipStream_t st, const char* w
     }
     return finish_launch(what);
 }
-// The slices of the sum over the words: 256 words per wavefront with all moments, 128 with the nodes of inference.
+// The slices of the sum over the words: 256 words per wavefront with all moments, 176 with the nodes of inference.
 void project_launch(int hw, const float* hist, const float* wcat, float* out, int64_t N, int H, hipStream_t st) {
     const dim3 grid((unsigned)((N + 15) / 16), (unsigned)H);
     auto launch = [&](auto kern, int waves) {
         hipLaunchKernelGGL(kern, grid, dim3(cfh::WAVE * waves), 0, st, hist, wcat, out, (int)N, H);
     };
-    if (hw == cfh::HW_ANG) launch(cfh::core_project_kernel<4, 4>, 4);
-    else if (hw == cfh::HW_LEAN) launch(cfh::core_project_kernel<5, 2>, 5);
-    else if (hw == cfh::HW_ANG16) launch(cfh::core_project_kernel<2, 1>, 2);
-    else launch(cfh::core_project_kernel<1, 1>, 1);
+    if (hw == cfh::HW_ANG) launch(cfh::core_project_kernel<4, 16>, 4);
+    else if (hw == cfh::HW_LEAN) launch(cfh::core_project_kernel<4, 11>, 4);
+    else if (hw == cfh::HW_ANG16) launch(cfh::core_project_kernel<2, 4>, 2);
+    else launch(cfh::core_project_kernel<1, 4>, 1);
 }
 // Up to this many (atom, head) items the forward pass of a layer is one wavefront per item from the record to the sums: about
 // as many as are resident at once (19 to 23 per compute unit).  Measured with and without, whole calls: 976 items 274 and 256
@@ -1738,9 +1738,9 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
     C.slow_flag = cfh::REC_BOX_LISTED;
     const char* what = "fused_core_forward";
     if (lean) {
-        if (p->angle_bins == cfh::NBINS) {      // moments around the nodes of inference, every LEAN_STEP / 3 bins
+        if (p->angle_bins == cfh::NBINS) {      // moments around the nodes of inference
             C.K.bc.ang_mu0 += cfh::LEAN_FIRST * C.K.bc.ang_interval;
-            C.K.bc.ang_inv_interval *= 3.0f / cfh::LEAN_STEP;
+            C.K.bc.ang_inv_interval *= (float)cfh::LEAN_DEN / cfh::LEAN_NUM;
         }
         if (one_launch) { CFH_CORE_DISPATCH(CFH_ITEM_PASS_LEAN); }
         else { CFH_CORE_DISPATCH(CFH_CORE_FWD_LEAN); }

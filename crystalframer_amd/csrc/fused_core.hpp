@@ -35,6 +35,7 @@
 #pragma once
 #include <type_traits>
 #include "device_common.hpp"
+#include "moment_series.hpp"
 
 namespace cfh {
 
@@ -44,10 +45,6 @@ constexpr int FC_LISTCAP = FC_GROUP * FC_TCAP;  // a group's survivors always fi
 constexpr int FC_SHIFT = 7;                     // list entry = pair-in-group << 7 | table index
 constexpr int FC_BIGSHIFT = 13;                 // ... of an item of several chunks: pair-in-group << 13 | index in its box
 constexpr int FC_BIGT = 1 << FC_BIGSHIFT;       // (boxes of up to 8192 translations)
-#ifndef CFH_NORD
-#define CFH_NORD 5
-#endif
-constexpr int NORD = CFH_NORD;                  // moments per axis
 constexpr int CORE_WPB = 1;                     // wavefronts per workgroup of the main kernels: each takes an item of its
                                                 // own (no barriers).  Workgroups of 4 or 8 items of one head that make the
                                                 // products with the head's weights themselves (projection, G) were slower:
@@ -72,16 +69,11 @@ __host__ __device__ constexpr int core_hist_lds_words(int ang) {
 }
 // words of an item's histogram for `ang` angle bins (0: distance encoding alone)
 __host__ __device__ constexpr int core_hist_words(int ang, bool lean = false);
-// Inference, where the histogram serves the projection alone, uses FEWER nodes for the moments of the angle encoding:
-// every LEAN_STEP / 3 bins instead of every bin, and the series around a node is the interpolation at the Chebyshev points
-// of its interval instead of the Taylor polynomial of the same degree, which takes 2^(1-NORD) of its error: with 5/3 bins
-// and 5 terms 0.8 of the error of the one-bin Taylor series, with 640 words instead of 1024.  At 22 528 atoms: projection
-// 204 -> 119 us, main kernel 404 -> 393 (its vector instructions, not its stores, bound it; making the projection in it,
-// four items of a head per workgroup behind a barrier, took 529 us for both).
-constexpr int LEAN_STEP = 5;
-constexpr int LEAN_NODES = 38;
-constexpr float LEAN_FIRST = 0.5f;              // centre of node 0 in bin units: the nodes' intervals cover [-1/3, 63]
-constexpr int HW_LEAN = 640;
+// Inference, where the histogram serves the projection alone, uses FEWER nodes for the moments of the angle encoding than
+// one per bin (moment_series.hpp): 704 words instead of 1024, with an error of the series that is no larger.  At 22 528 atoms:
+// projection 204 -> 131 us, main kernel 404 -> 387 (its vector instructions, not its stores, bound it; making the projection
+// in it, four items of a head per workgroup behind a barrier, took 529 us for both at 640 words).
+constexpr int HW_LEAN = 704;
 static_assert(HW_LEAN >= HW_DIST + 3 * NORD * LEAN_NODES && HW_LEAN % 64 == 0, "");
 __host__ __device__ constexpr int core_hist_words(int ang, bool lean) {
     return ang == NBINS ? (lean ? HW_LEAN : HW_ANG) : (ang == SMALL_A ? HW_ANG16 : HW_DIST);
@@ -235,45 +227,24 @@ __global__ __launch_bounds__(256) void pair_nearest_kernel(const float* __restri
 }
 
 // ---- projection weights with the moment matrices folded in ---------------------------------------------------
-// D_o(d) = exp(-(d/ws)^2/2) He_o(d/ws) / (o! (2 ws)^o)
-__device__ __forceinline__ float moment_matrix(int o, float d, float ws) {
-    const float y = d / ws;
-    float h0 = 1.0f, h1 = y;           // probabilists' Hermite polynomials
-    float he = o == 0 ? h0 : h1;
-    for (int n = 1; n < o; n++) { const float h2 = y * h1 - (float)n * h0; h0 = h1; h1 = h2; he = h2; }
-    float coef = 1.0f;
-    for (int n = 1; n <= o; n++) coef /= (float)n * (2.0f * ws);
-    return __expf(-0.5f * y * y) * he * coef;
-}
 // table of D_o(d) for d = -63 .. 63 in LDS, made by the threads of a block: dtab[o * 128 + d + 63]
 __device__ __forceinline__ void build_moment_table(float* dtab, float ws) {
     for (int u = threadIdx.x; u < NORD * 128; u += blockDim.x) {
         const int o = u >> 7, d = (u & 127) - 63;
-        dtab[u] = (u & 127) < 127 ? moment_matrix(o, (float)d, ws) : 0.0f;
+        dtab[u] = (u & 127) < 127 ? moment_matrix<float>(o, (float)d, ws) : 0.0f;
     }
     __syncthreads();
 }
-// The same for the nodes of inference: dtab[o * LEAN_TAB + 3 m - LEAN_STEP n + LEAN_OFF] = coefficient of eps^o
-// around node n of the basis function of bin m.  The terms of order NORD and more of the Taylor series are folded into the
-// lower ones modulo the Chebyshev polynomial T_NORD (x^5 = (20 x^3 - 5 x) / 16, ...), which is what interpolating at its
-// zeros comes to.
-constexpr int LEAN_OFF = LEAN_STEP * (LEAN_NODES - 1), LEAN_TAB = LEAN_OFF + 3 * NBINS;
+// The same for the nodes of inference: dtab[o * LEAN_TAB + LEAN_DEN m - LEAN_NUM n + LEAN_OFF] = coefficient of eps^o
+// around node n of the basis function of bin m.
+constexpr int LEAN_OFF = LEAN_NUM * (LEAN_NODES - 1), LEAN_TAB = LEAN_OFF + LEAN_DEN * NBINS;
 __device__ __forceinline__ void build_node_table(float* dtab, float ws) {
-    static_assert(NORD == 5, "the coefficients below are those of T_5");
-    const float r = LEAN_STEP / 6.0f / ws, inv_ws = 1.0f / ws;
+    const float r = 0.5f * LEAN_NUM / LEAN_DEN / ws, inv_ws = 1.0f / ws;
     for (int u = threadIdx.x; u < LEAN_TAB; u += blockDim.x) {
-        // exp(-y^2/2) He_o(y) r^o / o! by the recurrence of the Hermite polynomials
-        const float y = ((float)(u - LEAN_OFF) * (1.0f / 3.0f) - LEAN_FIRST) * inv_ws;
-        float D[9];
-        D[0] = __expf(-0.5f * y * y);
-        D[1] = y * r * D[0];
+        float c[NORD];
+        node_coefficients(((float)(u - LEAN_OFF) * (1.0f / LEAN_DEN) - LEAN_FIRST) * inv_ws, r, c);
 #pragma unroll
-        for (int o = 2; o < 9; o++) D[o] = (y * D[o - 1] - r * D[o - 2]) * (r * (1.0f / (float)o));
-        dtab[u] = D[0];
-        dtab[LEAN_TAB + u] = D[1] - 0.3125f * D[5] - 0.390625f * D[7];
-        dtab[2 * LEAN_TAB + u] = D[2] - 0.3125f * D[6] - 0.390625f * D[8];
-        dtab[3 * LEAN_TAB + u] = D[3] + 1.25f * (D[5] + D[7]);
-        dtab[4 * LEAN_TAB + u] = D[4] + 1.25f * (D[6] + D[8]);
+        for (int o = 0; o < NORD; o++) dtab[o * LEAN_TAB + u] = c[o];
     }
     __syncthreads();
 }
@@ -320,11 +291,11 @@ __device__ __forceinline__ void core_wcat_block(const WcatArgs& A, int hc) {
         if (w < HW_DIST) val = dist_coef * Wd[(size_t)hc * NBINS + w];
         else if (hw == HW_LEAN) {
             const int u = w - HW_DIST, ax = u / (NORD * LEAN_NODES), o = (u / LEAN_NODES) % NORD, n = u % LEAN_NODES;
-            const float* dt = dtab + o * LEAN_TAB + LEAN_OFF - LEAN_STEP * n;
+            const float* dt = dtab + o * LEAN_TAB + LEAN_OFF - LEAN_NUM * n;
             float acc = 0.0f;
             if (ax < 3) {                  // (words past the last node: zero)
 #pragma unroll 8
-                for (int m = 0; m < NBINS; m++) acc = fmaf(row[ax][m], dt[3 * m], acc);
+                for (int m = 0; m < NBINS; m++) acc = fmaf(row[ax][m], dt[LEAN_DEN * m], acc);
             }
             val = angle_coef * acc;
         } else {
@@ -1004,30 +975,30 @@ void fused_core_fwd_kernel(const CoreArgs C) {
 }
 
 // out (N,H,16) += Wcat_h (16, hw) . hist (H,N,hw): one workgroup of WAVES wavefronts per (16 atoms, head); each
-// wavefront takes STEPS x 64 words of the reduction index through MFMA 16x16x4 (the four lanes of a row read 64
+// wavefront takes UNITS x 16 words of the reduction index through MFMA 16x16x4 (the four lanes of a row read 64
 // consecutive bytes of it per load), the slices meet in LDS and are added in a fixed order by the first
 // wavefront (no atomics: the result does not depend on timing).  grid (ceil(N/16), H), block 64 * WAVES.
-// Bound by reading the histograms: 461 MB (22 528 atoms, 640 words) in 119 us (3.9 TB/s), 129 us with 10 steps dealt to
-// four wavefronts and half of the loads ahead of the products; four tiles per workgroup with the weights in registers: 115.
-template <int WAVES, int STEPS>
+// Bound by reading the histograms: 508 MB (22 528 atoms, 704 words) in 131 us (3.9 TB/s).  Measured at 640 words, 119 us: 129
+// with half of the loads ahead of the products; 115 with four tiles per workgroup and the weights in registers.
+template <int WAVES, int UNITS>
 __global__ __launch_bounds__(WAVE * WAVES) void core_project_kernel(const float* __restrict__ hist, const float* __restrict__ wcat,
                                                                     float* __restrict__ out, int N, int H) {
-    constexpr int hw = WAVES * STEPS * 64;
+    constexpr int hw = WAVES * UNITS * 16;
     __shared__ float part[WAVES][4][WAVE];
     const int lane = threadIdx.x & (WAVE - 1), wv = threadIdx.x >> 6, col = lane & 15, kk = lane >> 4;
     const int h = blockIdx.y, i0 = blockIdx.x * 16;
     const int row = min(i0 + col, N - 1);
     // the four lanes (kk) of a row read 64 consecutive bytes per load; which word of the reduction index a lane
     // holds does not matter as long as both operands agree
-    const float4* ap = reinterpret_cast<const float4*>(hist + ((size_t)h * N + row) * hw + wv * STEPS * 64) + kk;
-    const float4* bp = reinterpret_cast<const float4*>(wcat + ((size_t)h * DH + col) * hw + wv * STEPS * 64) + kk;
+    const float4* ap = reinterpret_cast<const float4*>(hist + ((size_t)h * N + row) * hw + wv * UNITS * 16) + kk;
+    const float4* bp = reinterpret_cast<const float4*>(wcat + ((size_t)h * DH + col) * hw + wv * UNITS * 16) + kk;
     v4f_c acc = {0.f, 0.f, 0.f, 0.f};
-    float4 a4[STEPS * 4], b4[STEPS * 4];
+    float4 a4[UNITS], b4[UNITS];
 #pragma unroll
-    for (int u = 0; u < STEPS * 4; u++) { a4[u] = ap[4 * u]; b4[u] = bp[4 * u]; }
+    for (int u = 0; u < UNITS; u++) { a4[u] = ap[4 * u]; b4[u] = bp[4 * u]; }
     __builtin_amdgcn_sched_barrier(0);         // (all loads in flight before the first product)
 #pragma unroll
-    for (int u = 0; u < STEPS * 4; u++) {
+    for (int u = 0; u < UNITS; u++) {
         acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[u].x, b4[u].x, acc, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[u].y, b4[u].y, acc, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[u].z, b4[u].z, acc, 0, 0, 0);
