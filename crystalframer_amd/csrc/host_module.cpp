@@ -138,13 +138,19 @@ struct Plan {
     // collector cannot see).
     struct Link { PyObject *dict, *key, *value; };
     std::vector<Link> links;
+    struct Walked { PyObject* dict; Py_ssize_t entries; };
+    std::vector<Walked> walked;
     std::vector<void*> ptrs;
 
-    Plan(py::list links_, std::vector<at::Tensor> params, std::vector<at::Tensor> gauss, int64_t feat, int64_t D, int64_t H,
-         int64_t out_features) {
+    Plan(py::list links_, py::list walked_, std::vector<at::Tensor> params, std::vector<at::Tensor> gauss, int64_t feat, int64_t D,
+         int64_t H, int64_t out_features) {
         for (auto l : links_) {
             auto t = py::reinterpret_borrow<py::tuple>(l);
             links.push_back({PyTuple_GET_ITEM(t.ptr(), 0), PyTuple_GET_ITEM(t.ptr(), 1), PyTuple_GET_ITEM(t.ptr(), 2)});
+        }
+        for (auto w : walked_) {
+            auto t = py::reinterpret_borrow<py::tuple>(w);
+            walked.push_back({PyTuple_GET_ITEM(t.ptr(), 0), PyLong_AsSsize_t(PyTuple_GET_ITEM(t.ptr(), 1))});
         }
         S->params = std::move(params);
         S->gauss = std::move(gauss);
@@ -157,8 +163,10 @@ struct Plan {
         S->device = S->params[0].device();
         S->feat = feat; S->D = D; S->H = H; S->out_features = out_features;
     }
-    // Whether the modules and parameters are still those the plan was made from, in the same storages.
+    // Whether the modules and parameters are still those the plan was made from, no more and no fewer, in the same storages.
     bool current() const {
+        for (auto& w : walked)
+            if (PyDict_GET_SIZE(w.dict) != w.entries) return false;
         for (auto& l : links) {
             PyObject* v = PyDict_GetItemWithError(l.dict, l.key);
             if (v != l.value) {
@@ -273,7 +281,7 @@ PYBIND11_MODULE(_host, mod) {
     });
     mod.attr("abi") = CFH_ABI_VERSION;
     py::class_<Plan>(mod, "Plan")
-        .def(py::init<py::list, std::vector<at::Tensor>, std::vector<at::Tensor>, int64_t, int64_t, int64_t, int64_t>())
+        .def(py::init<py::list, py::list, std::vector<at::Tensor>, std::vector<at::Tensor>, int64_t, int64_t, int64_t, int64_t>())
         .def("current", &Plan::current)
         .def("accepts", &Plan::accepts)
         .def("wanted", &Plan::wanted)

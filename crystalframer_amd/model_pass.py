@@ -23,27 +23,36 @@ from . import _lib
 ENABLED = True
 
 
+def _on_device(weight) -> bool:
+    return weight.is_cuda
+
+
 def _no_plan():
     return None
 
 
 class _Plan:
     """What a model's passes share: its parameters in the library's order, the structures that hold their addresses, and
-    the objects all of it was derived from.  ``current()`` is False as soon as a module or parameter was exchanged or a
-    parameter got another storage; the plan is then made again.  The plan keeps the storages it points at alive."""
+    the objects all of it was derived from.  ``current()`` is False as soon as a module or parameter was added, removed or
+    exchanged or a parameter got another storage; the plan is then made again.  The plan keeps the storages it points at
+    alive."""
 
     def __init__(self, model):
         self.links = []          # (dict, key, value): the plan holds while dict[key] is value
+        self.walked = []         # (dict, entries): ... and while the dicts whose entries were walked have as many of them
+        self.seen = set()
         self.params = []         # in the order of the library's gradients
         self.ok = False
         self.tables = {}         # kernel constants -> (layer structures, objects kept alive)
         self.hooked = []         # modules whose hooks the library call would pass over
         self.attn = []
         self._collect(model)
+        del self.seen
         self.native = None
         if self.ok:
             self.alive = [p.detach() for p in self.params]
-            self.native = _lib.load_host().Plan(self.links, self.params, self.gauss, self.feat, self.D, self.H, self.out_features)
+            self.native = _lib.load_host().Plan(self.links, self.walked, self.params, self.gauss, self.feat, self.D, self.H,
+                                                  self.out_features)
         else:
             self.ptrs = [p.data_ptr() for p in self.params if p is not None]
 
@@ -53,21 +62,33 @@ class _Plan:
     def current(self) -> bool:
         if self.native is not None:
             return self.native.current()
-        return (all(d.get(k) is v for d, k, v in self.links)
+        return (all(d.get(k) is v for d, k, v in self.links) and all(len(d) == n for d, n in self.walked)
                 and [p.data_ptr() for p in self.params if p is not None] == self.ptrs)
 
-    def _child(self, module, *names):
-        for n in names:
-            child = module._modules.get(n)
-            self.links.append((module._modules, n, child))
-            module = child
-            if module is None:
-                return None
-        return module
+    def _dict(self, module, name):
+        """A module's ``_modules`` or ``_parameters``: taking an entry out of a ModuleList puts another dict in its place."""
+        d = module.__dict__[name]
+        if (id(module), name) not in self.seen:
+            self.seen.add((id(module), name))
+            self.links.append((module.__dict__, name, d))
+        return d
+
+    def _child(self, module, name):
+        d = self._dict(module, "_modules")
+        child = d.get(name)
+        self.links.append((d, name, child))
+        return child
+
+    def _children(self, module):
+        """The names of all children, in the order in which a forward pass goes through them."""
+        d = self._dict(module, "_modules")
+        self.walked.append((d, len(d)))
+        return list(d)
 
     def _param(self, module, name):
-        p = module._parameters.get(name)
-        self.links.append((module._parameters, name, p))
+        d = self._dict(module, "_parameters")
+        p = d.get(name)
+        self.links.append((d, name, p))
         return p
 
     def _collect(self, model):
@@ -81,7 +102,7 @@ class _Plan:
         if not (isinstance(emb, nn.Linear) and isinstance(mlp, nn.Sequential) and isinstance(pre, nn.Identity)
                 and model.__dict__.get("pooling_layer") is avr_pool and enc is not None and enc._modules.get("norm") is None):
             return
-        self.links.append((enc._modules, "norm", enc._modules.get("norm")))
+        self._child(enc, "norm")
         self.hooked.append(enc)
         layers = self._child(enc, "layers")
         We = self._param(emb, "weight")
@@ -89,7 +110,7 @@ class _Plan:
             return
         self.params.append(We)
         self.layers = []
-        for name in layers._modules:
+        for name in self._children(layers):
             layer = self._child(layers, name)
             at = self._child(layer, "self_attn")
             out_proj = self._child(at, "out_proj")
@@ -123,7 +144,7 @@ class _Plan:
             self.layers.append((at, ps, gauss, A))
         self.head = []
         mods = []
-        for name in mlp._modules:
+        for name in self._children(mlp):
             m = self._child(mlp, name)
             if isinstance(m, nn.Linear):
                 W, b = self._param(m, "weight"), self._param(m, "bias")
@@ -146,7 +167,7 @@ class _Plan:
         self.head, self.out_features = mods, width
         self.D, self.F, self.H, self.feat = D, self.layers[0][1][-4].shape[0], self.attn[0].num_heads, We.shape[1]
         dev = We.device
-        if not We.is_cuda or not 1 <= self.feat <= 512 or We.shape[0] != D:
+        if not _on_device(We) or not 1 <= self.feat <= 512 or We.shape[0] != D:
             return
         for p in self.params:
             if p.dtype != torch.float32 or p.device != dev or not p.is_contiguous():
