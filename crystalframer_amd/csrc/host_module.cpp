@@ -140,7 +140,8 @@ struct Plan {
     std::vector<Link> links;
     struct Walked { PyObject* dict; Py_ssize_t entries; };
     std::vector<Walked> walked;
-    std::vector<void*> ptrs;
+    struct Layout { void* ptr; std::vector<int64_t> sizes; };
+    std::vector<Layout> layout;                // of params, then gauss; all of them contiguous float32
 
     Plan(py::list links_, py::list walked_, std::vector<at::Tensor> params, std::vector<at::Tensor> gauss, int64_t feat, int64_t D,
          int64_t H, int64_t out_features) {
@@ -158,12 +159,14 @@ struct Plan {
         for (auto& p : S->params) {
             S->offset.push_back(off);
             off += p.numel();
-            ptrs.push_back(p.data_ptr());
         }
+        for (auto* list : {&S->params, &S->gauss})
+            for (auto& p : *list) layout.push_back({p.data_ptr(), p.sizes().vec()});
         S->device = S->params[0].device();
         S->feat = feat; S->D = D; S->H = H; S->out_features = out_features;
     }
-    // Whether the modules and parameters are still those the plan was made from, no more and no fewer, in the same storages.
+    // Whether the modules and parameters are still those the plan was made from, no more and no fewer, in the same storages
+    // and with the same layout.
     bool current() const {
         for (auto& w : walked)
             if (PyDict_GET_SIZE(w.dict) != w.entries) return false;
@@ -174,8 +177,13 @@ struct Plan {
                 if (v || l.value != Py_None) return false;
             }
         }
-        for (size_t i = 0; i < ptrs.size(); i++)
-            if (S->params[i].data_ptr() != ptrs[i]) return false;
+        const Layout* l = layout.data();
+        for (auto* list : {&S->params, &S->gauss})
+            for (auto& p : *list) {
+                if (p.data_ptr() != l->ptr || p.scalar_type() != at::kFloat || !p.is_contiguous() || p.sizes() != l->sizes)
+                    return false;
+                l++;
+            }
         return true;
     }
     // The batch is one that the library call takes.

@@ -22,6 +22,11 @@ from . import _lib
 
 ENABLED = True
 
+# what a layer's pass takes from its attention's hyper-parameters
+_SETTINGS = ("value_pe_dist_real", "value_pe_dist_max", "value_pe_dist_wscale", "value_pe_dist_coef", "value_pe_angle_real",
+             "value_pe_angle_wscale", "value_pe_angle_coef", "cos_abs", "scale_real", "adaptive_cutoff_sigma", "gauss_lb_real",
+             "positive_func_beta", "normalize_gauss", "frame_method")
+
 
 def _on_device(weight) -> bool:
     return weight.is_cuda
@@ -34,8 +39,8 @@ def _no_plan():
 class _Plan:
     """What a model's passes share: its parameters in the library's order, the structures that hold their addresses, and
     the objects all of it was derived from.  ``current()`` is False as soon as a module or parameter was added, removed or
-    exchanged or a parameter got another storage; the plan is then made again.  The plan keeps the storages it points at
-    alive."""
+    exchanged, a parameter got another storage or layout, or a layer another setting; the plan is then made again.  The plan
+    keeps the storages it points at alive."""
 
     def __init__(self, model):
         self.links = []          # (dict, key, value): the plan holds while dict[key] is value
@@ -91,6 +96,11 @@ class _Plan:
         self.links.append((d, name, p))
         return p
 
+    def _setting(self, owner, name):
+        v = owner.__dict__.get(name)
+        self.links.append((owner.__dict__, name, v))
+        return v
+
     def _collect(self, model):
         from . import cuda_funcs
         from .latticeformer import avr_pool
@@ -105,6 +115,7 @@ class _Plan:
         self._child(enc, "norm")
         self.hooked.append(enc)
         layers = self._child(enc, "layers")
+        self._setting(enc, "d_model")
         We = self._param(emb, "weight")
         if self._param(emb, "bias") is not None or len(layers) < 1:
             return
@@ -119,7 +130,12 @@ class _Plan:
                 if not isinstance(self._child(layer, n), nn.Identity):
                     return
             self.links.append((layer.__dict__, "activation", layer.activation))
-            P = at.params
+            P = self._setting(at, "params")
+            for n in ("num_heads", "head_dim", "kdim", "vdim"):
+                self._setting(at, n)
+            # (compared by identity from call to call: a value that can change in place is left to the modules)
+            if not all([isinstance(self._setting(P, n), (bool, int, float, str)) for n in _SETTINGS]):
+                return
             A = P.value_pe_angle_real
             if not (layer.activation is torch.nn.functional.relu and P.frame_method == "max" and at.kdim == at.vdim == enc.d_model
                     and P.value_pe_dist_real > 0 and at.head_dim == 16
@@ -134,7 +150,7 @@ class _Plan:
             gauss = self._param(at, "gauss_scale")
             if any(p is None for p in ps):
                 return
-            if not (cuda_funcs.LayerBridgeHIP.supported(enc.d_model, l1.out_features, at.num_heads)
+            if not (cuda_funcs.LayerBridgeHIP.supported(enc.d_model, ps[-4].shape[0], at.num_heads)
                     and cuda_funcs.PeriodicAttentionCoreHIP.supported(
                         P.value_pe_dist_real, A, P.value_pe_dist_wscale, P.value_pe_angle_wscale, at.pe_dist_proj,
                         at.proj_angle1 if A > 0 else None)):
@@ -150,19 +166,20 @@ class _Plan:
                 W, b = self._param(m, "weight"), self._param(m, "bias")
                 if b is None:
                     return
-                mods.append([m, W, b, 0])
-            elif isinstance(m, nn.ReLU) and mods and not mods[-1][3]:
-                mods[-1][3] = 1
+                mods.append([W, b, 0])
+            elif isinstance(m, nn.ReLU) and mods and not mods[-1][2]:
+                mods[-1][2] = 1
             elif not isinstance(m, nn.Identity):
                 return
         D = enc.d_model
-        if not 1 <= len(mods) <= _lib.MODEL_MAX_LINEARS or mods[-1][3] or D > _lib.MODEL_MAX_WIDTH or len(self.attn) > 64:
+        if not 1 <= len(mods) <= _lib.MODEL_MAX_LINEARS or mods[-1][2] or D > _lib.MODEL_MAX_WIDTH or len(self.attn) > 64:
             return
         width = D
-        for m, W, b, relu in mods:
-            if m.in_features != width or width % 16 or m.out_features > _lib.MODEL_MAX_WIDTH:
+        for m in mods:
+            W, b, relu = m
+            if W.dim() != 2 or W.shape[1] != width or width % 16 or b.shape != W.shape[:1] or W.shape[0] > _lib.MODEL_MAX_WIDTH:
                 return
-            width = m.out_features
+            width = W.shape[0]
             self.params += [W, b]
         self.head, self.out_features = mods, width
         self.D, self.F, self.H, self.feat = D, self.layers[0][1][-4].shape[0], self.attn[0].num_heads, We.shape[1]
@@ -173,9 +190,13 @@ class _Plan:
             if p.dtype != torch.float32 or p.device != dev or not p.is_contiguous():
                 return
         for at, ps, gauss, A in self.layers:
-            if (ps[-4].shape[0] != self.F or at.num_heads != self.H or A != self.layers[0][3]
-                    or gauss.device != dev or gauss.dtype != torch.float32
-                    or any(w.dim() == 4 and w.shape[0] != 1 for w in ps)):
+            F, H = self.F, self.H
+            shapes = [(D, D)] * 3 + [(3 * D,), (D, D), (D,), (D,), (1, H, 16, 64)] + [(1, H, 16, A)] * (3 if A > 0 else 0)
+            shapes += [(F, D), (F,), (D, F), (D,)]
+            # (the value encodings with or without their leading dimension)
+            if (at.num_heads != H or A != self.layers[0][3]
+                    or any(tuple(w.shape) != s and (1,) + tuple(w.shape) != s for w, s in zip(ps, shapes))
+                    or gauss.device != dev or gauss.dtype != torch.float32 or gauss.numel() != 2 or not gauss.is_contiguous()):
                 return
             stack = at._stacked_in_proj()    # query, key and value weights as adjacent rows of one storage
             if at is self.attn[0]:
@@ -194,7 +215,7 @@ class _Plan:
         from .cuda_funcs import KernelManager as K
         sd = K.NOISE_SEED_DEVICE
         return (K.LATTICE_RANGE, K.MINIMUM_RANGE, K.CORE_WINDOW_MODE, K.PRUNE_LOG2, K.SYMM_BREAK_NOISE, K.NOISE_SEED,
-                None if sd is None else sd.data_ptr(), bool(K.COLLECT_STATS), tuple([g.data_ptr() for g in self.gauss]))
+                None if sd is None else sd.data_ptr(), bool(K.COLLECT_STATS))
 
     def table(self):
         key = self.constants()
@@ -237,8 +258,8 @@ class _Plan:
         m.layers, m.heads, m.D, m.F, m.feat, m.linears = len(self.layers), self.H, self.D, self.F, self.feat, len(self.head)
         m.We = self.params[0].data_ptr()
         m.layer = ctypes.cast(arr, ctypes.POINTER(_lib.CfhModelLayer))
-        for T, (mod, W, b, relu) in zip(m.head, self.head):
-            T.W, T.b, T.K, T.O, T.relu = W.data_ptr(), b.data_ptr(), mod.in_features, mod.out_features, relu
+        for T, (W, b, relu) in zip(m.head, self.head):
+            T.W, T.b, T.K, T.O, T.relu = W.data_ptr(), b.data_ptr(), W.shape[1], W.shape[0], relu
         return m, arr, (K.NOISE_SEED_DEVICE, list(self.gauss)), ctypes.addressof(m)
 
 

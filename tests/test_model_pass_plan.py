@@ -37,3 +37,54 @@ def test_an_added_or_removed_module_makes_the_plan_anew(planned):
     assert plan.ok
     model.mlp.insert(1, nn.ReLU())
     assert not plan.current()
+
+
+def test_another_layout_at_the_same_address_makes_the_plan_anew(planned):
+    model, plan = planned
+    at, head = model.encoder.layers[1].self_attn, model.mlp[0]
+    for p in (at.out_proj.weight, head.weight):
+        p.data = p.data.t()                          # square: same address, same sizes
+        assert not plan.current() and not model_pass._Plan(model).ok
+        p.data = p.data.t()
+        assert plan.current()
+    lin = model.encoder.layers[0].linear1
+    lin.weight.data = lin.weight.data.view(128, 512)
+    assert not plan.current() and not model_pass._Plan(model).ok
+    lin.weight.data = lin.weight.data.view(512, 128)
+    at.gauss_scale.data = torch.zeros(4)[::2]
+    assert not plan.current() and not model_pass._Plan(model).ok
+
+
+@pytest.mark.parametrize("name,value", [
+    ("value_pe_dist_max", -8.0), ("value_pe_dist_wscale", 1.5), ("value_pe_dist_coef", 2.0), ("value_pe_angle_wscale", 5.0),
+    ("value_pe_angle_coef", 3.0), ("cos_abs", 1), ("scale_real", 1.3), ("adaptive_cutoff_sigma", 2.5), ("gauss_lb_real", 0.4),
+    ("positive_func_beta", 0.2), ("normalize_gauss", False), ("frame_method", "pca"), ("value_pe_angle_real", 0),
+    ("value_pe_dist_real", 0)])
+def test_another_setting_of_a_layer_makes_the_plan_anew(planned, name, value):
+    model, plan = planned
+    P = model.encoder.layers[1].self_attn.params
+    old = getattr(P, name)
+    setattr(P, name, value)
+    assert not plan.current()
+    model_pass._Plan(model)                          # (covered or not, it can be asked)
+    setattr(P, name, old)
+    assert plan.current()
+    setattr(P, name, torch.tensor(1.0))              # may change in place: not covered
+    assert not plan.current() and not model_pass._Plan(model).ok
+
+
+def test_weights_of_another_shape_are_not_covered(planned):
+    """The library reads as many words as the widths say."""
+    model, plan = planned
+    lin = model.mlp[3]                               # 128 -> 1
+    lin.out_features = 4
+    assert model_pass._Plan(model).out_features == 1
+    lin.bias = nn.Parameter(torch.zeros(2))
+    assert not plan.current() and not model_pass._Plan(model).ok
+    lin.bias = nn.Parameter(torch.zeros(1))
+    assert model_pass._Plan(model).ok
+    at = model.encoder.layers[0].self_attn
+    at.proj_angle2 = nn.Parameter(torch.zeros(1, 8, 16, 32))
+    assert not model_pass._Plan(model).ok
+    at.proj_angle2 = nn.Parameter(torch.zeros(8, 16, 64))
+    assert model_pass._Plan(model).ok
