@@ -198,9 +198,12 @@ class _Plan:
                     or any(tuple(w.shape) != s and (1,) + tuple(w.shape) != s for w, s in zip(ps, shapes))
                     or gauss.device != dev or gauss.dtype != torch.float32 or gauss.numel() != 2 or not gauss.is_contiguous()):
                 return
-            stack = at._stacked_in_proj()    # query, key and value weights as adjacent rows of one storage
-            if at is self.attn[0]:
-                self.in_proj = stack.detach()
+            at._stacked_in_proj()            # query, key and value weights as adjacent rows of one storage
+        for at, ps, gauss, A in self.layers:
+            q, k, v = ps[:3]                 # (they cannot be where a weight is shared, in a layer or between layers)
+            if not (k.data_ptr() == q.data_ptr() + 4 * D * D and v.data_ptr() == k.data_ptr() + 4 * D * D):
+                return
+        self.in_proj = self.attn[0]._in_proj_stack.detach()
         # the gradients lie one behind the other: every one but the last starts on 16 bytes
         if any(p.numel() % 4 for p in self.params[:-1]):
             return

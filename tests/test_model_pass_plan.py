@@ -88,3 +88,16 @@ def test_weights_of_another_shape_are_not_covered(planned):
     assert not model_pass._Plan(model).ok
     at.proj_angle2 = nn.Parameter(torch.zeros(8, 16, 64))
     assert model_pass._Plan(model).ok
+
+
+def test_shared_projection_weights_are_not_covered(planned):
+    """The library reads the query, key and value weights as one matrix, from the address of the first."""
+    model, plan = planned
+    first, second = (layer.self_attn for layer in model.encoder.layers)
+    own = first.k_proj_weight
+    first.k_proj_weight = first.q_proj_weight
+    assert not plan.current() and not model_pass._Plan(model).ok
+    first.k_proj_weight = own
+    assert model_pass._Plan(model).ok
+    second.q_proj_weight = first.q_proj_weight
+    assert not model_pass._Plan(model).ok
