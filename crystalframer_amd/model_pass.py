@@ -117,7 +117,8 @@ class _Plan:
         layers = self._child(enc, "layers")
         self._setting(enc, "d_model")
         We = self._param(emb, "weight")
-        if self._param(emb, "bias") is not None or len(layers) < 1:
+        # (a weight that a parametrization or a pruning mask makes is no parameter of its module)
+        if We is None or self._param(emb, "bias") is not None or emb.bias is not None or len(layers) < 1:
             return
         self.params.append(We)
         self.layers = []
@@ -164,7 +165,7 @@ class _Plan:
             m = self._child(mlp, name)
             if isinstance(m, nn.Linear):
                 W, b = self._param(m, "weight"), self._param(m, "bias")
-                if b is None:
+                if W is None or b is None:
                     return
                 mods.append([W, b, 0])
             elif isinstance(m, nn.ReLU) and mods and not mods[-1][2]:

@@ -3,6 +3,7 @@ when what it was derived from changes, and a pass it does not cover is left to t
 import pytest
 import torch
 from torch import nn
+import torch.nn.utils.prune  # noqa: F401
 
 from crystalframer_amd import encoder, latticeformer, model_pass, params
 
@@ -101,3 +102,24 @@ def test_shared_projection_weights_are_not_covered(planned):
     assert model_pass._Plan(model).ok
     second.q_proj_weight = first.q_proj_weight
     assert not model_pass._Plan(model).ok
+
+
+@pytest.mark.parametrize("where", ["input_embeddings", "mlp.0", "mlp.3", "encoder.layers.1.linear2",
+                                   "encoder.layers.0.self_attn.out_proj"])
+def test_reparametrised_weights_are_not_covered(planned, where):
+    model, plan = planned
+    module = model.get_submodule(where)
+    nn.utils.parametrizations.weight_norm(module)
+    assert not plan.current() and not model_pass._Plan(model).ok
+    nn.utils.parametrize.remove_parametrizations(module, "weight")
+    assert model_pass._Plan(model).ok
+    nn.utils.prune.l1_unstructured(module, "weight", amount=0.5)
+    assert not model_pass._Plan(model).ok
+
+
+def test_an_embedding_with_a_bias_is_not_covered(planned):
+    model, plan = planned
+    model.input_embeddings.bias = nn.Parameter(torch.ones(128))
+    assert not plan.current() and not model_pass._Plan(model).ok
+    nn.utils.parametrize.register_parametrization(model.input_embeddings, "bias", nn.Identity())
+    assert model.input_embeddings.bias is not None and not model_pass._Plan(model).ok
