@@ -12,8 +12,12 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/utils/pybind.h>
+#include <torch/csrc/jit/frontend/tracer.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/SavedTensorHooks.h>
 
 #include "../../include/crystalframer_hip.h"
 
@@ -247,6 +251,18 @@ struct Plan {
     }
 };
 
+// Who would see the framework's operations in this thread beside autograd's backward pass.
+enum : int { WATCHED = 1, FUNCTION_MODE = 2, SAVED_TENSOR_HOOKS = 4 };
+int watchers() {
+    int seen = 0;
+    if (torch::jit::tracer::isTracing() || c10::impl::TorchDispatchModeTLS::stack_len() > 0 ||
+        c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode))
+        seen |= WATCHED;
+    if (at::impl::PythonTorchFunctionTLS::stack_len() > 0) seen |= FUNCTION_MODE;
+    if (at::SavedTensorDefaultHooks::get_hooks().has_value()) seen |= SAVED_TENSOR_HOOKS;
+    return seen;
+}
+
 // Addresses of an optimizer's launch: fills the jobs of the parameters that have a gradient.  Returns how many, or -1 when a
 // gradient is one that the Python side has to look at (not contiguous, sparse, another type).
 struct Updates {
@@ -288,6 +304,10 @@ PYBIND11_MODULE(_host, mod) {
         g_lib.last_error = reinterpret_cast<decltype(g_lib.last_error)>(last_error);
     });
     mod.attr("abi") = CFH_ABI_VERSION;
+    mod.attr("WATCHED") = (int)WATCHED;
+    mod.attr("FUNCTION_MODE") = (int)FUNCTION_MODE;
+    mod.attr("SAVED_TENSOR_HOOKS") = (int)SAVED_TENSOR_HOOKS;
+    mod.def("watchers", &watchers);
     py::class_<Plan>(mod, "Plan")
         .def(py::init<py::list, py::list, std::vector<at::Tensor>, std::vector<at::Tensor>, int64_t, int64_t, int64_t, int64_t>())
         .def("current", &Plan::current)

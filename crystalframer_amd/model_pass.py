@@ -16,7 +16,10 @@ import ctypes
 import math
 
 import torch
+import torch.autograd.forward_ad as fwAD
 from torch import nn
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from . import _lib
 
@@ -295,9 +298,25 @@ def _forward(plan, args, keep: bool):
     return plan.native.forward(table[3], table, *args, keep, lambda n: _lib.workspace(dev, n), seeds, first)
 
 
-def run(model, data):
-    """The model's output for ``data``, or None when the pass is not one this path covers."""
-    if not _switches_default():
+def _eager(host, keep: bool) -> bool:
+    """Whether what the pass does to tensors is seen by nobody but autograd's backward pass: one native call has no forward-mode
+    derivative, no batching rule and nothing that a tracer or a mode could record."""
+    seen = host.watchers()
+    if seen == 0 and fwAD._current_level < 0:
+        return True
+    if fwAD._current_level >= 0 or seen & host.WATCHED or (keep and seen & host.SAVED_TENSOR_HOOKS):
+        return False
+    # a function mode that only chooses the device of new tensors (torch.set_default_device) changes nothing here
+    return not seen & host.FUNCTION_MODE or all(type(m) is DeviceContext for m in _get_current_function_mode_stack())
+
+
+def covered(model, data):
+    """(plan, arguments, keep) of the native call for ``data``, or None when the pass is not one this path covers."""
+    if torch.compiler.is_compiling() or not _switches_default():
+        return None
+    host = _lib.load_host()
+    keep = torch.is_grad_enabled()
+    if not _eager(host, keep):
         return None
     plan = model.__dict__.get("_pass_plan")
     if plan is None or not plan.current():
@@ -325,15 +344,22 @@ def run(model, data):
     lim = 1 << 30
     if x.shape[0] * plan.D >= lim or E * max(plan.H, 3) >= lim:
         return None
-    keep = False
-    if torch.is_grad_enabled():
+    if keep:
         if x.requires_grad or pos.requires_grad or trans.requires_grad:
             return None
         wanted = plan.native.wanted()
         if wanted == 1:
             return None
         keep = wanted == 2
-    args = (x, pos, batch, trans, sizes, int(E))
+    return plan, (x, pos, batch, trans, sizes, int(E)), keep
+
+
+def run(model, data):
+    """The model's output for ``data``, or None when the pass is not one this path covers."""
+    found = covered(model, data)
+    if found is None:
+        return None
+    plan, args, keep = found
     if torch.cuda.current_device() != plan.device.index:
         with torch.cuda.device(plan.device):
             return _forward(plan, args, keep)

@@ -2,10 +2,15 @@
 when what it was derived from changes, and a pass it does not cover is left to the modules."""
 import pytest
 import torch
-from torch import nn
+import torch.autograd.forward_ad as fwAD
 import torch.nn.utils.prune  # noqa: F401
+from torch import nn
+from torch._subclasses.fake_tensor import FakeTensorMode
+from torch.fx.experimental.proxy_tensor import make_fx
+from torch.overrides import TorchFunctionMode
+from torch.utils._python_dispatch import TorchDispatchMode
 
-from crystalframer_amd import encoder, latticeformer, model_pass, params
+from crystalframer_amd import encoder, latticeformer, model_pass, params, synthetic
 
 
 @pytest.fixture
@@ -14,6 +19,8 @@ def planned(monkeypatch):
     monkeypatch.setattr(model_pass, "_on_device", lambda weight: True)
     torch.manual_seed(0)
     model = latticeformer.Latticeformer(params.ModelParams(num_layers=2))
+    for layer in model.encoder.layers:
+        layer.self_attn.gauss_scale.data.fill_(0.5)
     plan = model_pass._Plan(model)
     assert plan.ok and plan.current()
     return model, plan
@@ -123,3 +130,54 @@ def test_an_embedding_with_a_bias_is_not_covered(planned):
     assert not plan.current() and not model_pass._Plan(model).ok
     nn.utils.parametrize.register_parametrization(model.input_embeddings, "bias", nn.Identity())
     assert model.input_embeddings.bias is not None and not model_pass._Plan(model).ok
+
+
+def _batch():
+    return synthetic.make_config("C1", seed=5, num_crystals=3)
+
+
+def test_forward_derivatives_tracers_and_modes_are_left_to_the_modules(planned):
+    model, plan = planned
+    cb = _batch()
+    covered = lambda data=cb: model_pass.covered(model, data) is not None  # noqa: E731
+    assert covered()
+    with fwAD.dual_level():
+        assert not covered()
+    seen = []
+    look = lambda t: (seen.append(covered()), t.sum())[1]  # noqa: E731
+    torch.func.grad(look)(torch.ones(3))
+    torch.func.vmap(look)(torch.ones(3, 2))
+    torch.func.jvp(look, (torch.ones(3),), (torch.ones(3),))
+    torch.jit.trace(look, (torch.ones(3),), check_trace=False)
+    make_fx(look)(torch.ones(3))
+    assert len(seen) >= 5 and not any(seen)
+    with FakeTensorMode():
+        assert not covered()
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    for mode in (Dispatch(), Function()):
+        with mode:
+            assert not covered()
+    with torch.device("cpu"):                        # only chooses the device of new tensors
+        assert covered()
+        with Function():
+            assert not covered()
+    assert covered()
+
+
+def test_hooks_on_saved_tensors_are_left_to_the_modules(planned):
+    model, plan = planned
+    cb = _batch()
+    with torch.autograd.graph.save_on_cpu():         # (activation checkpointing is one of these as well)
+        assert model_pass.covered(model, cb) is None
+        with torch.no_grad():                        # nothing is saved
+            assert model_pass.covered(model, cb) is not None
+    with torch.autograd.graph.disable_saved_tensors_hooks("none"):
+        assert model_pass.covered(model, cb) is not None
