@@ -25,6 +25,10 @@ from . import _lib
 
 ENABLED = True
 
+# hooks of all modules of the program
+_GLOBAL_HOOKS = [getattr(torch.nn.modules.module, n) for n in (
+    "_global_forward_hooks", "_global_forward_pre_hooks", "_global_backward_hooks", "_global_backward_pre_hooks")]
+
 # what a layer's pass takes from its attention's hyper-parameters
 _SETTINGS = ("value_pe_dist_real", "value_pe_dist_max", "value_pe_dist_wscale", "value_pe_dist_coef", "value_pe_angle_real",
              "value_pe_angle_wscale", "value_pe_angle_coef", "cos_abs", "scale_real", "adaptive_cutoff_sigma", "gauss_lb_real",
@@ -52,7 +56,7 @@ class _Plan:
         self.params = []         # in the order of the library's gradients
         self.ok = False
         self.tables = {}         # kernel constants -> (layer structures, objects kept alive)
-        self.hooked = []         # modules whose hooks the library call would pass over
+        self.hooks = []          # hooks of the modules that a pass calls as modules: dicts that have to be empty
         self.attn = []
         self._collect(model)
         del self.seen
@@ -104,19 +108,28 @@ class _Plan:
         self.links.append((owner.__dict__, name, v))
         return v
 
+    def _called(self, module, kind) -> bool:
+        """A module that the modules' path calls, so that hooks, a forward of its own and compilation count."""
+        if type(module) is not kind:
+            return False
+        for n in ("_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks"):
+            self.hooks.append(self._setting(module, n))
+        own = [self._setting(module, n) for n in ("forward", "_compiled_call_impl")]
+        return own == [None, None]
+
     def _collect(self, model):
         from . import cuda_funcs
+        from .attention import CrystalformerMultiheadAttentionCUDA
+        from .encoder import CrystalformerEncoderCUDA
         from .latticeformer import avr_pool
         enc = self._child(model, "encoder")
         emb = self._child(model, "input_embeddings")
         mlp = self._child(model, "mlp")
         pre = self._child(model, "proj_before_pooling")
         self.links.append((model.__dict__, "pooling_layer", model.__dict__.get("pooling_layer")))
-        if not (isinstance(emb, nn.Linear) and isinstance(mlp, nn.Sequential) and isinstance(pre, nn.Identity)
-                and model.__dict__.get("pooling_layer") is avr_pool and enc is not None and enc._modules.get("norm") is None):
+        if not (isinstance(emb, nn.Linear) and isinstance(mlp, nn.Sequential) and self._called(pre, nn.Identity)
+                and self._called(enc, CrystalformerEncoderCUDA) and model.__dict__.get("pooling_layer") is avr_pool and self._child(enc, "norm") is None):
             return
-        self._child(enc, "norm")
-        self.hooked.append(enc)
         layers = self._child(enc, "layers")
         self._setting(enc, "d_model")
         We = self._param(emb, "weight")
@@ -138,6 +151,9 @@ class _Plan:
             for n in ("num_heads", "head_dim", "kdim", "vdim"):
                 self._setting(at, n)
             # (compared by identity from call to call: a value that can change in place is left to the modules)
+            if type(at) is not CrystalformerMultiheadAttentionCUDA or [
+                    n for n in ("attention_core", "project_inputs") if self._setting(at, n) is not None]:
+                return
             if not all([isinstance(self._setting(P, n), (bool, int, float, str)) for n in _SETTINGS]):
                 return
             A = P.value_pe_angle_real
@@ -331,9 +347,8 @@ def covered(model, data):
             return None
         if at.params.normalize_gauss and not at._gauss_scale_ready():
             return None
-    for mod in plan.hooked:
-        if mod._forward_hooks or mod._forward_pre_hooks or mod._backward_hooks or mod._backward_pre_hooks:
-            return None
+    if any(plan.hooks) or any(_GLOBAL_HOOKS):
+        return None
     if not getattr(data, "zero_based", False):       # the reference subtracts batch[0]
         batch = batch - batch[0]
     E = getattr(data, "num_pairs", -1)

@@ -181,3 +181,51 @@ def test_hooks_on_saved_tensors_are_left_to_the_modules(planned):
             assert model_pass.covered(model, cb) is not None
     with torch.autograd.graph.disable_saved_tensors_hooks("none"):
         assert model_pass.covered(model, cb) is not None
+
+
+@pytest.mark.parametrize("where", ["encoder", "proj_before_pooling"])
+def test_hooks_and_own_forwards_of_the_called_modules_are_left_to_the_modules(planned, where):
+    model, plan = planned
+    cb = _batch()
+    module = model.get_submodule(where)
+    covered = lambda: model_pass.covered(model, cb) is not None  # noqa: E731
+    for register in (module.register_forward_hook, module.register_forward_pre_hook, module.register_full_backward_hook,
+                     module.register_full_backward_pre_hook):
+        handle = register(lambda *a: None)
+        assert not covered()
+        handle.remove()
+        assert covered()
+    module.forward = module.forward
+    assert not covered()
+    del module.forward
+    assert covered()
+    module.compile()
+    assert not covered()
+
+    class Other(type(module)):
+        pass
+
+    if where == "proj_before_pooling":
+        model.proj_before_pooling = Other()
+        assert not covered()
+
+
+def test_hooks_of_all_modules_are_left_to_the_modules(planned):
+    model, plan = planned
+    cb = _batch()
+    for register in (nn.modules.module.register_module_forward_hook, nn.modules.module.register_module_forward_pre_hook,
+                     nn.modules.module.register_module_full_backward_hook,
+                     nn.modules.module.register_module_full_backward_pre_hook):
+        handle = register(lambda *a: None)
+        assert model_pass.covered(model, cb) is None
+        handle.remove()
+        assert model_pass.covered(model, cb) is not None
+
+
+def test_an_attention_with_methods_of_its_own_is_left_to_the_modules(planned):
+    model, plan = planned
+    at = model.encoder.layers[1].self_attn
+    at.attention_core = at.attention_core
+    assert not plan.current() and not model_pass._Plan(model).ok
+    del at.attention_core
+    assert plan.current()
