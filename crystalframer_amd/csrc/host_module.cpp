@@ -190,14 +190,16 @@ struct Plan {
             }
         return true;
     }
-    // The batch is one that the library call takes.
+    // The batch is one that the library call takes: it reads as many words of each tensor as x and trans have rows.
     bool accepts(const at::Tensor& x, const at::Tensor& pos, const at::Tensor& batch, const at::Tensor& trans,
                  const at::Tensor& sizes) const {
         auto good = [&](const at::Tensor& t, at::ScalarType ty) {
             return t.scalar_type() == ty && t.device() == S->device && t.is_contiguous();
         };
         return good(x, at::kFloat) && good(pos, at::kFloat) && good(trans, at::kFloat) && good(batch, at::kLong) &&
-               good(sizes, at::kLong) && x.dim() == 2 && x.size(1) == S->feat && x.size(0) > 0 && trans.dim() > 0;
+               good(sizes, at::kLong) && x.dim() == 2 && x.size(1) == S->feat && x.size(0) > 0 &&
+               pos.dim() == 2 && pos.size(0) == x.size(0) && pos.size(1) == 3 && batch.dim() == 1 && batch.size(0) == x.size(0) &&
+               trans.dim() == 3 && trans.size(1) == 3 && trans.size(2) == 3 && sizes.dim() == 1 && sizes.size(0) == trans.size(0);
     }
     // How many of the parameters want a gradient: 0 none, 1 some, 2 all.
     int wanted() const {

@@ -229,3 +229,15 @@ def test_an_attention_with_methods_of_its_own_is_left_to_the_modules(planned):
     assert not plan.current() and not model_pass._Plan(model).ok
     del at.attention_core
     assert plan.current()
+
+
+@pytest.mark.parametrize("name,change", [
+    ("pos", lambda t: t[:-1]), ("pos", lambda t: t[:, :2].contiguous()), ("batch", lambda t: t[:-1]), ("sizes", lambda t: t[:-1]),
+    ("sizes", lambda t: t[None]), ("trans_vec", lambda t: t.reshape(-1, 9)), ("trans_vec", lambda t: t.flatten()),
+    ("pos", lambda t: t.t().contiguous().t()), ("x", lambda t: t[:-1])])
+def test_batches_of_other_shapes_are_left_to_the_modules(planned, name, change):
+    model, plan = planned
+    cb = _batch()
+    assert model_pass.covered(model, cb) is not None
+    setattr(cb, name, change(getattr(cb, name)))
+    assert model_pass.covered(model, cb) is None
