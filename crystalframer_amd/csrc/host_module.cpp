@@ -53,6 +53,7 @@ at::Tensor arena(size_t n, const c10::Device& dev) {
 struct Shared {
     std::vector<at::Tensor> params;            // in the order of the library's gradients
     std::vector<at::Tensor> gauss;
+    std::vector<at::Tensor> alive;             // params and gauss as the plan was made: the library has their addresses
     std::vector<int64_t> offset;               // of a parameter's gradient, in floats
     c10::Device device{c10::kCPU};
     int64_t feat = 0, D = 0, H = 0, out_features = 0;
@@ -104,6 +105,8 @@ struct ModelPassBackward : public torch::autograd::Node {
                     "have already been freed). Saved intermediate values of the graph are freed when you call .backward() or "
                     "autograd.grad(). Specify retain_graph=True if you need to backward through the graph a second time or if "
                     "you need to access saved tensors after calling backward.");
+        // A parameter whose .data was exchanged since the forward pass: the addresses are those of the storages before, which
+        // plan->alive keeps, and the gradients those of what the forward pass computed.
         const size_t n = plan->params.size();
         torch::autograd::variable_list out(n);
         if (!grads[0].defined()) return out;
@@ -129,7 +132,7 @@ struct ModelPassBackward : public torch::autograd::Node {
             auto t = at::detail::make_tensor<c10::TensorImpl>(c10::Storage(storage), flat.key_set(), flat.dtype());
             c10::TensorImpl* impl = t.unsafeGetTensorImpl();
             impl->set_storage_offset(plan->offset[i]);
-            impl->set_sizes_contiguous(plan->params[i].sizes());
+            impl->set_sizes_contiguous(plan->alive[i].sizes());
             out[i] = std::move(t);
         }
         return out;
@@ -165,7 +168,10 @@ struct Plan {
             off += p.numel();
         }
         for (auto* list : {&S->params, &S->gauss})
-            for (auto& p : *list) layout.push_back({p.data_ptr(), p.sizes().vec()});
+            for (auto& p : *list) {
+                layout.push_back({p.data_ptr(), p.sizes().vec()});
+                S->alive.push_back(p.detach());
+            }
         S->device = S->params[0].device();
         S->feat = feat; S->D = D; S->H = H; S->out_features = out_features;
     }

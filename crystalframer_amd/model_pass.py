@@ -46,8 +46,8 @@ def _no_plan():
 class _Plan:
     """What a model's passes share: its parameters in the library's order, the structures that hold their addresses, and
     the objects all of it was derived from.  ``current()`` is False as soon as a module or parameter was added, removed or
-    exchanged, a parameter got another storage or layout, or a layer another setting; the plan is then made again.  The plan
-    keeps the storages it points at alive."""
+    exchanged, a parameter got another storage or layout, or a layer another setting; the plan is then made again.  The native
+    part keeps the storages whose addresses the library has, and a backward pass keeps the native part's."""
 
     def __init__(self, model):
         self.links = []          # (dict, key, value): the plan holds while dict[key] is value
@@ -62,7 +62,6 @@ class _Plan:
         del self.seen
         self.native = None
         if self.ok:
-            self.alive = [p.detach() for p in self.params]
             self.native = _lib.load_host().Plan(self.links, self.walked, self.params, self.gauss, self.feat, self.D, self.H,
                                                   self.out_features)
         else:

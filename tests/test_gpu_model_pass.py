@@ -92,6 +92,28 @@ def test_copies_exchanged_weights_and_changes_before_the_backward_pass():
         out.sum().backward()
 
 
+def test_backward_pass_after_the_storages_of_the_weights_were_exchanged():
+    """The gradients are those of what the forward pass computed, whatever the parameters hold by then."""
+    from crystalframer_amd import params, synthetic
+    mp = params.ModelParams(num_layers=2, symm_break_noise=0.0)
+    cb = synthetic.make_batch(5, atoms="uniform", atoms_lo=1, atoms_hi=5, len_lo=3.0, len_hi=9.0, ang_lo=65.0, ang_hi=115.0,
+                              seed=6)
+    model, cb, ((_, _, want), _) = _both(mp, cb)
+    target = torch.linspace(-1, 1, 5, device="cuda").view(5, 1)
+    model.zero_grad(set_to_none=True)
+    loss = torch.nn.functional.mse_loss(model(cb), target)
+    with torch.no_grad():
+        for p in model.parameters():
+            p.data = p.data * 3.0 + 1.0
+        model(cb)                                    # (the plan is made again)
+        fill = [torch.full_like(p, 7.0) for p in model.parameters() for _ in range(3)]      # takes the memory given back
+    loss.backward()
+    for n, p in model.named_parameters():
+        if n in want:
+            assert torch.equal(p.grad, want[n]), n
+    assert len(fill) > 0
+
+
 # a tile of 16 rows and its edges; either side of the row counts at which the bridge takes one launch instead of two and 32
 # rows per workgroup instead of 16; both widths; one and several chunks of the feed-forward block's inside
 @pytest.mark.parametrize("D,F,N", [(128, 128, 17), (128, 384, 1), (128, 384, 1361), (128, 384, 1393), (128, 256, 16351),
