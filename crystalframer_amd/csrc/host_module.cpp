@@ -277,6 +277,17 @@ struct Updates {
     std::vector<at::Tensor> params;
     std::vector<int64_t> offset;               // of a parameter's moments, in floats (-1: none)
     Updates(std::vector<at::Tensor> p, std::vector<int64_t> o) : params(std::move(p)), offset(std::move(o)) {}
+    // Whether these are the tensors of the list, in its order.
+    bool of(py::object list) const {
+        py::object seq = py::reinterpret_steal<py::object>(PySequence_Fast(list.ptr(), "the parameters of a group"));
+        if (!seq) throw py::error_already_set();
+        if (PySequence_Fast_GET_SIZE(seq.ptr()) != (Py_ssize_t)params.size()) return false;
+        PyObject** const items = PySequence_Fast_ITEMS(seq.ptr());
+        for (size_t i = 0; i < params.size(); i++)
+            if (!THPVariable_Check(items[i]) || THPVariable_Unpack(items[i]).unsafeGetTensorImpl() != params[i].unsafeGetTensorImpl())
+                return false;
+        return true;
+    }
     int64_t fill(uintptr_t jobs, uintptr_t m, uintptr_t v) const {
         cfh_adamw_job* const J = reinterpret_cast<cfh_adamw_job*>(jobs);
         int64_t n = 0;
@@ -324,6 +335,7 @@ PYBIND11_MODULE(_host, mod) {
         .def("forward", &Plan::forward);
     py::class_<Updates>(mod, "Updates")
         .def(py::init<std::vector<at::Tensor>, std::vector<int64_t>>())
+        .def("of", &Updates::of)
         .def("fill", &Updates::fill)
         .def("drop", &Updates::drop);
 }

@@ -107,7 +107,8 @@ class AdamW(torch.optim.Optimizer):
             if g is None:
                 continue
             if off is None:
-                raise RuntimeError("a parameter that did not require a gradient at the first step has one now")
+                raise RuntimeError("a parameter that was not in the group, or did not require a gradient, at the first step "
+                                   "has a gradient now")
             if g.is_sparse:
                 raise RuntimeError("sparse gradients are not supported")
             if not p.is_contiguous():
@@ -138,12 +139,12 @@ class AdamW(torch.optim.Optimizer):
                                         float(group["weight_decay"]), st["step"].data_ptr(), _lib.raw_stream(dev))
 
     def _plan(self, group, st):
-        """Job table of the group's launch, kept from step to step (made again when the group's parameters changed)."""
+        """Job table of the group's launch, kept from step to step (made again when the group holds other parameters)."""
         plan = st.get("plan")
-        if plan is None or plan["count"] != len(group["params"]) or plan["moments"] != st["exp_avg"].data_ptr():
+        if plan is None or not plan["native"].of(group["params"]) or plan["moments"] != st["exp_avg"].data_ptr():
             ps = list(group["params"])
             offs = [st["offset"].get(id(p)) for p in ps]
-            plan = st["plan"] = dict(params=ps, offs=offs, count=len(ps), moments=st["exp_avg"].data_ptr(),
+            plan = st["plan"] = dict(params=ps, offs=offs, moments=st["exp_avg"].data_ptr(),
                                      jobs=(_lib.CfhAdamWJob * max(len(ps), 1))(), device=st["exp_avg"].device,
                                      native=_lib.load_host().Updates(ps, [-1 if o is None else o for o in offs]))
         return plan
