@@ -272,11 +272,15 @@ int watchers() {
 }
 
 // Addresses of an optimizer's launch: fills the jobs of the parameters that have a gradient.  Returns how many, or -1 when a
-// gradient is one that the Python side has to look at (not contiguous, sparse, another type).
+// gradient is one that the Python side has to look at (not contiguous, sparse, another type) or does not fit the moments:
+// the kernel goes over as many words of parameter, gradient and moments as the parameter had when these were made.
 struct Updates {
     std::vector<at::Tensor> params;
     std::vector<int64_t> offset;               // of a parameter's moments, in floats (-1: none)
-    Updates(std::vector<at::Tensor> p, std::vector<int64_t> o) : params(std::move(p)), offset(std::move(o)) {}
+    std::vector<int64_t> numel;                // of a parameter's moments
+    c10::Device device;                        // of the moments
+    Updates(std::vector<at::Tensor> p, std::vector<int64_t> o, std::vector<int64_t> n, const at::Tensor& moments)
+        : params(std::move(p)), offset(std::move(o)), numel(std::move(n)), device(moments.device()) {}
     // Whether these are the tensors of the list, in its order.
     bool of(py::object list) const {
         py::object seq = py::reinterpret_steal<py::object>(PySequence_Fast(list.ptr(), "the parameters of a group"));
@@ -296,7 +300,8 @@ struct Updates {
             const at::Tensor& g = p.grad();
             if (!g.defined()) continue;
             if (offset[i] < 0 || g.layout() != at::kStrided || g.scalar_type() != at::kFloat || !g.is_contiguous() ||
-                !p.is_contiguous() || g.device() != p.device())
+                !p.is_contiguous() || p.scalar_type() != at::kFloat || p.numel() != numel[i] || g.numel() != numel[i] ||
+                p.device() != device || g.device() != device)
                 return -1;
             cfh_adamw_job& j = J[n++];
             j.param = reinterpret_cast<float*>(p.data_ptr());
@@ -334,7 +339,7 @@ PYBIND11_MODULE(_host, mod) {
         .def("wanted", &Plan::wanted)
         .def("forward", &Plan::forward);
     py::class_<Updates>(mod, "Updates")
-        .def(py::init<std::vector<at::Tensor>, std::vector<int64_t>>())
+        .def(py::init<std::vector<at::Tensor>, std::vector<int64_t>, std::vector<int64_t>, const at::Tensor&>())
         .def("of", &Updates::of)
         .def("fill", &Updates::fill)
         .def("drop", &Updates::drop);

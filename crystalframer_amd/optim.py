@@ -46,6 +46,7 @@ class AdamW(torch.optim.Optimizer):
             st["exp_avg_sq"] = torch.zeros(total, dtype=torch.float32, device=dev)
             st["step"] = torch.zeros(1, dtype=torch.int64, device=dev)
             st["offset"] = {id(p): o for p, o in zip(ps, offs)}
+            st["numel"] = {id(p): p.numel() for p in ps}
             for p, o in zip(ps, offs):
                 self.state[p] = dict(step=st["step"], exp_avg=st["exp_avg"][o:o + p.numel()].view_as(p),
                                      exp_avg_sq=st["exp_avg_sq"][o:o + p.numel()].view_as(p))
@@ -102,7 +103,7 @@ class AdamW(torch.optim.Optimizer):
     def _fill(plan, m0, v0):
         """The job table parameter by parameter: (jobs, gradients made contiguous here)."""
         n, keep = 0, None
-        for p, off in zip(plan["params"], plan["offs"]):
+        for p, off, count in zip(plan["params"], plan["offs"], plan["counts"]):
             g = p.grad
             if g is None:
                 continue
@@ -113,6 +114,10 @@ class AdamW(torch.optim.Optimizer):
                 raise RuntimeError("sparse gradients are not supported")
             if not p.is_contiguous():
                 raise RuntimeError("AdamW of crystalframer_amd needs contiguous parameters")
+            if p.numel() != count or g.numel() != count or p.device != plan["device"] or g.device != plan["device"]:
+                raise RuntimeError("a parameter or its gradient has another size or device than at the first step")
+            if p.dtype != torch.float32 or g.dtype != torch.float32:
+                raise RuntimeError("AdamW of crystalframer_amd needs float32 parameters and gradients")
             if not g.is_contiguous():
                 g = g.contiguous()
                 keep = (keep, g)
@@ -144,7 +149,9 @@ class AdamW(torch.optim.Optimizer):
         if plan is None or not plan["native"].of(group["params"]) or plan["moments"] != st["exp_avg"].data_ptr():
             ps = list(group["params"])
             offs = [st["offset"].get(id(p)) for p in ps]
-            plan = st["plan"] = dict(params=ps, offs=offs, moments=st["exp_avg"].data_ptr(),
+            counts = [st["numel"].get(id(p), 0) for p in ps]
+            plan = st["plan"] = dict(params=ps, offs=offs, counts=counts, moments=st["exp_avg"].data_ptr(),
                                      jobs=(_lib.CfhAdamWJob * max(len(ps), 1))(), device=st["exp_avg"].device,
-                                     native=_lib.load_host().Updates(ps, [-1 if o is None else o for o in offs]))
+                                     native=_lib.load_host().Updates(ps, [-1 if o is None else o for o in offs], counts,
+                                                                     st["exp_avg"]))
         return plan
