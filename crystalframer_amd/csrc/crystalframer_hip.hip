@@ -1252,16 +1252,17 @@ struct StreamList {
         blocks = 0;
     }
 };
-// Dynamic LDS of more than 64 KB has to be asked for, once per kernel and device.
-template <typename Kern>
-int allow_lds(Kern kern, size_t lds) {
+// More than 64 KB of LDS have to be asked for, once per kernel and device (here from 48 KB of dynamic LDS on: the kernel's own
+// arrays come on top).
+template <auto KERN>
+int allow_lds(size_t lds) {
     static int lds_set[64] = {0};
-    if (lds <= 64 * 1024) return CFH_OK;
+    if (lds <= 48 * 1024) return CFH_OK;
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return fail(CFH_ELAUNCH, "layer bridge: no current device");
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return fail(CFH_ELAUNCH, "no current device");
     if (lds_set[dev] < (int)lds) {
-        if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
-            return fail(CFH_ELAUNCH, "layer bridge: %zu bytes of LDS refused", lds);
+        if (hipFuncSetAttribute((const void*)KERN, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+            return fail(CFH_ELAUNCH, "%zu bytes of LDS refused", lds);
         lds_set[dev] = (int)lds;
     }
     return CFH_OK;
@@ -1274,11 +1275,11 @@ int bridge_forward(const cfh::BridgeArgs& A, int D, hipStream_t st) {
         const dim3 g1(tiles, (unsigned)(A.F / 128)), g2(tiles, A.qs ? 3u : 1u);
         const size_t lds = 16 * (size_t)(A.F + cfh::BR_PAD) * sizeof(float);
         if (D == 128) {
-            if (int rc = allow_lds(cfh::layer_bridge_fwd_split2_kernel<1>, lds)) return rc;
+            if (int rc = allow_lds<cfh::layer_bridge_fwd_split2_kernel<1>>(lds)) return rc;
             hipLaunchKernelGGL(cfh::layer_bridge_fwd_split1_kernel<1>, g1, block, 0, st, A);
             hipLaunchKernelGGL(cfh::layer_bridge_fwd_split2_kernel<1>, g2, block, lds, st, A);
         } else {
-            if (int rc = allow_lds(cfh::layer_bridge_fwd_split2_kernel<2>, lds)) return rc;
+            if (int rc = allow_lds<cfh::layer_bridge_fwd_split2_kernel<2>>(lds)) return rc;
             hipLaunchKernelGGL(cfh::layer_bridge_fwd_split1_kernel<2>, g1, block, 0, st, A);
             hipLaunchKernelGGL(cfh::layer_bridge_fwd_split2_kernel<2>, g2, block, lds, st, A);
         }
@@ -1307,11 +1308,11 @@ int bridge_backward(cfh::BridgeBwdArgs A, int D, hipStream_t st) {
         const dim3 g1(tiles, (unsigned)(A.F / 128));
         const size_t lds = 16 * (size_t)(A.F + cfh::BR_PAD) * sizeof(float);
         if (D == 128) {
-            if (int rc = allow_lds(cfh::layer_bridge_bwd_split2_kernel<1>, lds)) return rc;
+            if (int rc = allow_lds<cfh::layer_bridge_bwd_split2_kernel<1>>(lds)) return rc;
             hipLaunchKernelGGL(cfh::layer_bridge_bwd_split1_kernel<1>, g1, block, 0, st, A);
             hipLaunchKernelGGL(cfh::layer_bridge_bwd_split2_kernel<1>, dim3(tiles), block, lds, st, A);
         } else {
-            if (int rc = allow_lds(cfh::layer_bridge_bwd_split2_kernel<2>, lds)) return rc;
+            if (int rc = allow_lds<cfh::layer_bridge_bwd_split2_kernel<2>>(lds)) return rc;
             hipLaunchKernelGGL(cfh::layer_bridge_bwd_split1_kernel<2>, g1, block, 0, st, A);
             hipLaunchKernelGGL(cfh::layer_bridge_bwd_split2_kernel<2>, dim3(tiles), block, lds, st, A);
         }

@@ -269,6 +269,7 @@ void tail_args(const cfh_model* m, const cfh_model_batch* b, const ModelBuffers&
 int tail_launch(const cfh::TailArgs& T, const float* gout, hipStream_t st) {
     const dim3 grid((unsigned)((T.B + T.per_wg - 1) / T.per_wg)), block(64 * cfh::TAIL_WAVES);
     const size_t lds = 2 * (size_t)cfh::TAIL_ROWS * T.ld * sizeof(float);
+    if (int rc = gout ? allow_lds<cfh::model_tail_bwd_kernel>(lds) : allow_lds<cfh::model_tail_fwd_kernel>(lds)) return rc;
     if (gout) hipLaunchKernelGGL(cfh::model_tail_bwd_kernel, grid, block, lds, st, T, gout);
     else hipLaunchKernelGGL(cfh::model_tail_fwd_kernel, grid, block, lds, st, T);
     return finish_launch("model_tail");

@@ -57,9 +57,11 @@ def test_one_call_equals_the_modules_path(B, hi, bins, layers):
         assert Hh.rel_err(g1[n], g2[n].double()) < (1e-5 if B <= 512 else 2e-3), n
 
 
-def test_head_of_several_layers_and_targets():
+# (from 445 features on, a workgroup of the tail takes more than 64 KB of LDS; 480 is the widest head it takes)
+@pytest.mark.parametrize("widths", [[64, 208], [448], [464], [480, 16, 480]])
+def test_head_of_several_layers_and_targets(widths):
     from crystalframer_amd import params, synthetic
-    mp = params.ModelParams(num_layers=1, symm_break_noise=0.0, embedding_dim=[64, 208], targets=["a", "b", "c"])
+    mp = params.ModelParams(num_layers=1, symm_break_noise=0.0, embedding_dim=widths, targets=["a", "b", "c"])
     cb = synthetic.make_batch(21, atoms="uniform", atoms_lo=1, atoms_hi=5, len_lo=3.0, len_hi=9.0, ang_lo=65.0, ang_hi=115.0,
                               seed=4)
     model, cb, ((o1, e1, g1), (o2, e2, g2)) = _both(mp, cb)
