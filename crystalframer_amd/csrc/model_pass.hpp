@@ -67,12 +67,19 @@ int check_model(const cfh_model* m, const cfh_model_batch* b) {
     return check_core_sizes(&m->layer[0].core, b->N, b->E);
 }
 
-// The tables of the geometry (sorted shifts, nearest images) are shared by the layers whose box rule agrees.
-bool same_tables(const cfh_model_layer& a, const cfh_model_layer& b) {
-    auto R0 = [](const cfh_model_layer& L) {
-        return L.adaptive && L.core.cutoff_radius != 0.0f ? L.core.minimum_range : L.core.lattice_range;
-    };
-    return R0(a) == R0(b);
+// The tables of the geometry (sorted shifts, nearest images) are those of one half-width at a time: a layer that needs another
+// one than the arena holds makes them again.
+int layer_half_width(const cfh_model_layer& L) { return usual_half_width(&L.core, L.adaptive != 0); }
+// What the arena holds before a backward pass: the half-width that all layers with tables share; -1 when they differ (the
+// layers of the forward pass and of an earlier backward pass have then left one or the other).
+int shared_half_width(const cfh_model* m) {
+    int R = 0;
+    for (int l = 0; l < m->layers; l++) {
+        const int r = layer_half_width(m->layer[l]);
+        if (r > 0 && R > 0 && r != R) return -1;
+        if (r > 0) R = r;
+    }
+    return R;
 }
 
 // Layout of the arena.  keep: every layer its own buffers, for the backward pass; else the layers share one set (a layer
@@ -322,7 +329,7 @@ int cfh_model_forward(const cfh_model* m, const cfh_model_batch* b, float* out) 
         g.order_start = g.pair_start + (B + 1);
         g.N = (int32_t)N; g.B = (int32_t)B; g.E = E;
         A.geo_blocks = 2;
-        A.table_R = usual_half_width(&m->layer[0].core, m->layer[0].adaptive != 0);
+        A.table_R = layer_half_width(m->layer[0]);
         if (A.table_R > 0) {
             constexpr int per = cfh::START_THREADS / cfh::FC_TCAP;
             A.table = M.table;
@@ -380,12 +387,15 @@ int cfh_model_forward(const cfh_model* m, const cfh_model_batch* b, float* out) 
             if ((rc = bridge_front(A, D, st))) return rc;
         }
     }
+    int held = layer_half_width(m->layer[0]);
     for (int l = 0; l < m->layers; l++) {
         const cfh_model_layer& L = m->layer[l];
         const ModelLayerBuffers& Y = M.layer[l];
         cfh_params p = L.core;
         if (b->noise_seeds) p.noise_seed = b->noise_seeds[l];
-        const bool ready = l == 0 || same_tables(m->layer[l - 1], L);
+        const int R = layer_half_width(L);
+        const bool ready = R == held;
+        if (R > 0) held = R;
         const cfh_core_cache cache{reinterpret_cast<float*>(M.table), M.near_, Y.wcat, Y.records, ready ? 1 : 0, 0, 0, 0};
         const bool ang = p.angle_bins > 0;
         if ((rc = fused_core_forward_impl(&p, Y.qs, Y.k, Y.v, Y.a, M.rpos, b->tvecs, L.adaptive ? M.rvlen : nullptr, b->batch,
@@ -441,6 +451,7 @@ int cfh_model_backward(const cfh_model* m, const cfh_model_batch* b, const float
     T.gx = G.layer[m->layers - 1].g2;
     if ((rc = tail_launch(T, gout, st))) return rc;
 
+    int held = shared_half_width(m);
     for (int l = m->layers - 1; l >= 0; l--) {
         // the projections between the core of layer l and the inputs of layer l + 1
         const cfh_model_layer& L = m->layer[l];
@@ -463,9 +474,9 @@ int cfh_model_backward(const cfh_model* m, const cfh_model_batch* b, const float
         if ((rc = bridge_backward(A, D, st))) return rc;
         cfh_params p = L.core;
         p.flags |= CFH_FLAG_NO_WEIGHT_GRADS;
-        // (the table in the arena is that of the last layer whose box rule differs from its predecessor's)
-        bool table_ready = true;
-        for (int u = l + 1; u < m->layers; u++) table_ready = table_ready && same_tables(L, m->layer[u]);
+        const int R = layer_half_width(L);
+        const bool table_ready = R == held;
+        if (R > 0) held = R;
         const cfh_core_cache cache{reinterpret_cast<float*>(M.table), nullptr, Y.wcat, Y.records, table_ready ? 1 : 0, 1, 1, 0};
         const bool ang = p.angle_bins > 0;
         if ((rc = cfh_fused_core_backward(&p, Y.qs, Y.k, Y.v, Y.a, M.rpos, b->tvecs, L.adaptive ? M.rvlen : nullptr, b->batch,

@@ -11,22 +11,36 @@ import helpers as Hh
 pytestmark = pytest.mark.gpu
 
 
-def _both(mp, cb, seed=1):
-    from crystalframer_amd import latticeformer, model_pass
+def _model(mp, cb, seed=1, change=None):
+    from crystalframer_amd import latticeformer
     dev = torch.device("cuda:0")
     torch.manual_seed(seed)
     model = latticeformer.Latticeformer(mp).to(dev)
+    if change is not None:
+        change(model)
     cb = cb.to(dev)
     model.train()
     model(cb)                                   # stores the normalisation of alpha (modules' path)
+    return model, cb
+
+
+def _both(mp, cb, seed=1, change=None, before=None):
+    """Outputs and gradients of the native call and of the modules.  change: of the model; before: each of the passes."""
+    from crystalframer_amd import model_pass
+    dev = torch.device("cuda:0")
+    model, cb = _model(mp, cb, seed, change)
     target = torch.linspace(-1, 1, cb.num_crystals * model.mlp[-1].out_features, device=dev).view(cb.num_crystals, -1)
     results = []
     for on in (True, False):
         model_pass.ENABLED = on
         try:
             model.zero_grad(set_to_none=True)
+            if before is not None:
+                before()
             out = model(cb)
             torch.nn.functional.mse_loss(out, target).backward()
+            if before is not None:
+                before()
             with torch.no_grad():
                 ev = model(cb)
         finally:
@@ -114,6 +128,43 @@ def test_backward_pass_after_the_storages_of_the_weights_were_exchanged():
         if n in want:
             assert torch.equal(p.grad, want[n]), n
     assert len(fill) > 0
+
+
+@pytest.fixture
+def kernel_constants():
+    """The constants of the kernels, put back after a test."""
+    from crystalframer_amd.cuda_funcs import KernelManager as K
+    names = ("NOISE_SEED", "NOISE_SEED_DEVICE", "SYMM_BREAK_NOISE", "LATTICE_RANGE", "MINIMUM_RANGE")
+    saved = {n: getattr(K, n) for n in names}
+    yield K
+    for n, v in saved.items():
+        setattr(K, n, v)
+
+
+# (half-width of the layers' usual box without and with the adaptive cutoff): the tables of one serve some layers only
+@pytest.mark.parametrize("fixed,adaptive", [(2, 1), (2, 0), (1, 2)])
+@pytest.mark.parametrize("rules", ["fa", "af", "faf", "afa", "aaf"])
+def test_layers_with_different_box_rules(kernel_constants, fixed, adaptive, rules):
+    from crystalframer_amd import params, synthetic
+    mp = params.ModelParams(num_layers=len(rules), symm_break_noise=0.0)
+    cb = synthetic.make_batch(9, atoms="uniform", atoms_lo=1, atoms_hi=6, len_lo=3.0, len_hi=9.0, ang_lo=65.0, ang_hi=115.0,
+                              seed=4)
+
+    def change(model):
+        kernel_constants.LATTICE_RANGE, kernel_constants.MINIMUM_RANGE = fixed, adaptive
+        for layer, rule in zip(model.encoder.layers, rules):
+            if rule == "f":
+                layer.self_attn.params.adaptive_cutoff_sigma = 0.0
+
+    model, cb, ((o1, e1, g1), (o2, e2, g2)) = _both(mp, cb, change=change)
+    assert torch.equal(o1, o2) and Hh.rel_err(e1, e2.double()) < 1e-6
+    for n in g1:
+        assert torch.equal(g1[n], g2[n]), n
+    out = model(cb)
+    g = torch.ones_like(out)
+    first = torch.autograd.grad(out, [model.mlp[0].weight, model.input_embeddings.weight], g, retain_graph=True)
+    second = torch.autograd.grad(out, [model.mlp[0].weight, model.input_embeddings.weight], g)
+    assert torch.equal(first[0], second[0]) and torch.equal(first[1], second[1])
 
 
 # a tile of 16 rows and its edges; either side of the row counts at which the bridge takes one launch instead of two and 32
