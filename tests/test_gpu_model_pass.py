@@ -141,6 +141,50 @@ def kernel_constants():
         setattr(K, n, v)
 
 
+# few items, of which a wavefront takes each from its record to the sums, and more (5120 items and 8 heads: 640 atoms)
+@pytest.mark.parametrize("B,hi", [(7, 6), (97, 16)])
+@pytest.mark.parametrize("seeds", ["fixed", "drawn", "on the device"])
+def test_noise_of_the_frame_search(kernel_constants, B, hi, seeds):
+    """The same seeds for the same layers as in the modules' path: fixed, drawn per layer and pass, or mixed with a word on the
+    device that every search advances."""
+    from crystalframer_amd import params, synthetic
+    K = kernel_constants
+    mp = params.ModelParams(num_layers=3, symm_break_noise=1e-2)      # (large: another seed is another frame)
+    cb = synthetic.make_batch(B, atoms="uniform", atoms_lo=1, atoms_hi=hi, len_lo=3.0, len_hi=9.0, ang_lo=65.0, ang_hi=115.0,
+                              seed=B)
+    word = torch.zeros(1, dtype=torch.int64, device="cuda")
+    K.NOISE_SEED = None if seeds == "drawn" else 77
+
+    def before(start=5):
+        torch.manual_seed(start)
+        K.NOISE_SEED_DEVICE = word if seeds == "on the device" else None
+        word.fill_(start)
+
+    model, cb, ((o1, e1, g1), (o2, e2, g2)) = _both(mp, cb, before=before)
+    assert torch.equal(o1, o2)
+    for n in g1:
+        # (with seeds of their own the modules' path sums the layers' core weights in separate launches, the atoms in other
+        # slices: a rounding of 6e-8 per atom at worst)
+        sliced = seeds == "drawn" and ("proj_angle" in n or "pe_dist" in n)
+        err = Hh.rel_err(g1[n], g2[n].double())
+        assert err < 6e-8 * cb.pos.shape[0] if sliced else torch.equal(g1[n], g2[n]), (n, err)
+    assert Hh.rel_err(e1, e2.double()) < 1e-4
+    if seeds != "fixed":
+        before(6)
+        assert not torch.equal(model(cb), o1)
+
+
+def test_wide_model():
+    from crystalframer_amd import params, synthetic
+    mp = params.ModelParams(num_layers=2, symm_break_noise=0.0, model_dim=256, ff_dim=384, head_num=16, embedding_dim=[256])
+    cb = synthetic.make_batch(19, atoms="uniform", atoms_lo=1, atoms_hi=7, len_lo=3.0, len_hi=9.0, ang_lo=65.0, ang_hi=115.0,
+                              seed=4)
+    model, cb, ((o1, e1, g1), (o2, e2, g2)) = _both(mp, cb)
+    assert torch.equal(o1, o2) and Hh.rel_err(e1, e2.double()) < 1e-6
+    for n in g1:
+        assert torch.equal(g1[n], g2[n]), n
+
+
 # (half-width of the layers' usual box without and with the adaptive cutoff): the tables of one serve some layers only
 @pytest.mark.parametrize("fixed,adaptive", [(2, 1), (2, 0), (1, 2)])
 @pytest.mark.parametrize("rules", ["fa", "af", "faf", "afa", "aaf"])
@@ -165,6 +209,94 @@ def test_layers_with_different_box_rules(kernel_constants, fixed, adaptive, rule
     first = torch.autograd.grad(out, [model.mlp[0].weight, model.input_embeddings.weight], g, retain_graph=True)
     second = torch.autograd.grad(out, [model.mlp[0].weight, model.input_embeddings.weight], g)
     assert torch.equal(first[0], second[0]) and torch.equal(first[1], second[1])
+
+
+# few atoms and more than the slow lists' leading wavefronts serve
+@pytest.mark.parametrize("B,hi,bins", [(7, 6, 64), (150, 20, 64), (150, 20, 0), (60, 12, 16)])
+def test_backward_passes_as_autograd_makes_them(B, hi, bins):
+    """A second pass over a kept graph, gradients of some parameters only, accumulation, another stream, and a graph that is
+    used up."""
+    from crystalframer_amd import params, synthetic
+    kw = dict(value_pe_angle_wscale=1.0, value_pe_dist_coef=1.5, value_pe_angle_coef=6.0) if bins == 16 else {}
+    mp = params.ModelParams(num_layers=2, value_pe_angle_real=bins, symm_break_noise=0.0, **kw)
+    cb = synthetic.make_batch(B, atoms="uniform", atoms_lo=1, atoms_hi=hi, len_lo=3.0, len_hi=9.0, ang_lo=65.0, ang_hi=115.0,
+                              seed=B)
+    model, cb = _model(mp, cb)
+    named = {n: p for n, p in model.named_parameters() if p.requires_grad}
+    gout = torch.linspace(-1, 1, B, device="cuda").view(B, 1)
+    out = model(cb)
+    assert out.grad_fn.name() == "ModelPassHIPBackward"
+    want = dict(zip(named, torch.autograd.grad(out, list(named.values()), gout, retain_graph=True)))
+    some = [n for n in named if n.endswith("linear1.weight") or n == "input_embeddings.weight"]
+    for n, g in zip(some, torch.autograd.grad(out, [named[n] for n in some], gout, retain_graph=True)):
+        assert torch.equal(g, want[n]), n
+    out.backward(gout)                               # .grad made
+    for n, p in named.items():
+        assert torch.equal(p.grad, want[n]), n
+    with pytest.raises(RuntimeError, match="second time"):
+        out.backward(gout)
+    model(cb).backward(gout)                         # added to .grad
+    for n, p in named.items():
+        assert torch.equal(p.grad, 2.0 * want[n]), n
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        model.zero_grad(set_to_none=True)
+        here = model(cb)
+        assert torch.equal(here, out)
+        here.backward(gout)
+    torch.cuda.current_stream().wait_stream(side)
+    for n, p in named.items():
+        assert torch.equal(p.grad, want[n]), n
+    # two passes over other batches between a forward pass and its backward pass
+    model.zero_grad(set_to_none=True)
+    out = model(cb)
+    other = synthetic.make_batch(3, atoms="uniform", atoms_lo=1, atoms_hi=4, len_lo=3.0, len_hi=9.0, ang_lo=65.0, ang_hi=115.0,
+                                 seed=1).to("cuda")
+    model(other)
+    torch.autograd.grad(model(other).sum(), list(named.values()))
+    out.backward(gout)
+    for n, p in named.items():
+        assert torch.equal(p.grad, want[n]), n
+
+
+@pytest.mark.parametrize("bins", [64, 16, 0])
+def test_items_in_one_launch_and_in_several(bins):
+    """Up to 5120 (atom, head) items a wavefront takes an item through a layer, above the items go through three launches: the
+    crystals of the smaller batch are answered alike in the larger one."""
+    from crystalframer_amd import params, synthetic
+    kw = dict(value_pe_angle_wscale=1.0, value_pe_dist_coef=1.5, value_pe_angle_coef=6.0) if bins == 16 else {}
+    mp = params.ModelParams(num_layers=2, value_pe_angle_real=bins, symm_break_noise=0.0, **kw)
+    B = 80
+    cb = synthetic.make_batch(B + 1, atoms="uniform", atoms_lo=8, atoms_hi=8, len_lo=3.0, len_hi=9.0, ang_lo=65.0, ang_hi=115.0,
+                              seed=3)
+    less = synthetic.CrystalBatch(cb.x[:8 * B], cb.pos[:8 * B], cb.batch[:8 * B], cb.trans_vec[:B], cb.sizes[:B], zero_based=True)
+    model, less = _model(mp, less)
+    more = cb.to("cuda")
+    assert less.x.shape[0] * 8 == 5120 and more.x.shape[0] * 8 == 5184
+    gout = torch.linspace(-1, 1, B, device="cuda").view(B, 1)
+    named = [p for p in model.parameters() if p.requires_grad]
+    a, b = model(less), model(more)
+    assert Hh.rel_err(b[:B], a.double()) < 1e-6
+    with torch.no_grad():
+        assert Hh.rel_err(model(more)[:B], model(less).double()) < 1e-6
+    ga = torch.autograd.grad(a, named, gout)
+    gb = torch.autograd.grad(b, named, torch.cat([gout, torch.zeros(1, 1, device="cuda")]))
+    for p, q in zip(ga, gb):
+        assert Hh.rel_err(q, p.double()) < 2e-5      # (sums over the atoms in other slices)
+
+
+def test_forward_derivatives_are_refused():
+    import torch.autograd.forward_ad as fwAD
+    from crystalframer_amd import params, synthetic
+    cb = synthetic.make_batch(3, atoms="uniform", atoms_lo=1, atoms_hi=4, len_lo=3.0, len_hi=9.0, ang_lo=65.0, ang_hi=115.0,
+                              seed=1)
+    model, cb = _model(params.ModelParams(num_layers=1, symm_break_noise=0.0), cb)
+    with fwAD.dual_level():
+        cb.pos = fwAD.make_dual(cb.pos, torch.ones_like(cb.pos))
+        cb.x = fwAD.make_dual(cb.x, torch.ones_like(cb.x))
+        with pytest.raises((NotImplementedError, RuntimeError)):
+            model(cb)
 
 
 # a tile of 16 rows and its edges; either side of the row counts at which the bridge takes one launch instead of two and 32
