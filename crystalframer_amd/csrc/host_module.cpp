@@ -101,18 +101,15 @@ struct ModelPassBackward : public torch::autograd::Node {
         return v;
     }
     torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
-        TORCH_CHECK(!released, "Trying to backward through the graph a second time (or directly access saved tensors after they "
-                    "have already been freed). Saved intermediate values of the graph are freed when you call .backward() or "
-                    "autograd.grad(). Specify retain_graph=True if you need to backward through the graph a second time or if "
-                    "you need to access saved tensors after calling backward.");
+        TORCH_CHECK(!released, "the backward pass of this model output has been made and what its forward pass kept is given back; to "
+                    "make it a second time, make the first one with retain_graph=True");
         // A parameter whose .data was exchanged since the forward pass: the addresses are those of the storages before, which
         // plan->alive keeps, and the gradients those of what the forward pass computed.
         const size_t n = plan->params.size();
         torch::autograd::variable_list out(n);
         if (!grads[0].defined()) return out;
         TORCH_CHECK(current_versions(*plan) == versions,
-                    "one of the variables needed for gradient computation has been modified by an inplace operation: a parameter "
-                    "of the model changed between its forward and its backward pass");
+                    "a parameter of the model was modified by an inplace operation between its forward and its backward pass");
         for (auto& s : data) s.unpack(shared_from_this());       // (says so if an input was changed in place)
         const at::Tensor gout = grads[0].detach().to(at::kFloat).contiguous();
         c10::DeviceGuard guard(plan->device);
