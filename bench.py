@@ -50,7 +50,7 @@ COUNTER_SOURCE = "profiles/fused_core_valu_lds_counters_C3.md"
 # (cfh_timing_enable): the algorithmic flop of a path are divided by the SUM of their durations.
 PATHS = {
     "forward": {
-        "fused": ("core_tables", "core_prepare", "frame_axes", "fused_core_forward", "core_project"),
+        "fused": ("core_tables", "model_start", "core_prepare", "frame_axes", "item_pass", "fused_core_forward", "core_project"),
         "two_step": ("frame_axes", "framed_pe_forward"),
     },
     "backward": {
@@ -60,7 +60,9 @@ PATHS = {
 }
 KERNEL_NAMES = {
     "core_tables": "sorted_shifts_kernel + pair_nearest_kernel (once per batch)",
+    "model_start": "model_start_kernel + model_pairs_kernel (once per pass: geometry, tables, weights in the order of their use)",
     "core_prepare": "core_prepare_wcat_kernel", "frame_axes": "frame_axes_kernel",
+    "item_pass": "item_pass_kernel (few items: record, frame search and lattice sums of an item in one wavefront)",
     "fused_core_forward": "fused_core_fwd_kernel", "core_project": "core_project_kernel",
     "core_prepare_bwd": "core_wcat_kernel / prepare_items_kernel (only when the forward's are not kept)",
     "core_gbuild": "core_gbuild_kernel", "fused_core_backward": "fused_core_bwd_kernel",
@@ -172,29 +174,43 @@ def timed(run, steps: int) -> float:
 
 
 KERNELS = tuple(KERNEL_NAMES)
+# whole passes and the kernels between the cores, as the library times them
+CALLS = ("model_forward", "model_backward")
+BETWEEN = ("layer_front", "layer_bridge_forward", "layer_bridge_backward", "model_tail", "linear_weight_gradients")
 
 
 def instrumented(fn, nprof: int, dev, count_terms: bool = True):
-    """Run ``fn`` eagerly ``nprof`` times with the library's own HIP events around its lattice kernels and around
-    every library call, then ``nprof`` times with the term counters.  Kept out of every timed region."""
+    """Run ``fn`` eagerly ``nprof`` times, as in the timed region, with the library's own HIP events around its kernels and
+    around every whole pass, then ``nprof`` times with the term counters.  Kept out of every timed region."""
     import crystalframer_amd as cf
     from crystalframer_amd import _lib
     KM = cf.KernelManager
-    for what in KERNELS:                    # drop what earlier runs recorded
+    for what in KERNELS + CALLS + BETWEEN:      # drop what earlier runs recorded
         _lib.read_kernel_timing(what)
-    KM.EVENT_LOG = []
     _lib.kernel_timing(True)
     for _ in range(nprof):
         fn()
     torch.cuda.synchronize()
     _lib.kernel_timing(False)
-    log, KM.EVENT_LOG = KM.EVENT_LOG, None
-    kern_ms, kern_launches = {}, {}
-    for what in KERNELS:
+    kern_ms, kern_launches, calls = {}, {}, {}
+    for what in KERNELS + BETWEEN:
         total, count = _lib.read_kernel_timing(what)
         if count:
             kern_ms[what] = total / count
             kern_launches[what] = count / nprof
+    for what in CALLS:
+        total, count = _lib.read_kernel_timing(what)
+        if count:
+            calls[what] = [total / count] * count
+    if not calls:
+        # the sequence of operators: every library call bracketed by the Python side
+        KM.EVENT_LOG = []
+        for _ in range(nprof):
+            fn()
+        torch.cuda.synchronize()
+        log, KM.EVENT_LOG = KM.EVENT_LOG, None
+        for name, s, e in log:
+            calls.setdefault(name, []).append(s.elapsed_time(e))
     stats = None
     if count_terms:
         KM.COLLECT_STATS = True
@@ -204,13 +220,11 @@ def instrumented(fn, nprof: int, dev, count_terms: bool = True):
         torch.cuda.synchronize()
         KM.COLLECT_STATS = False
         stats = {k: v / nprof for k, v in _lib.read_stats(dev, reset=True).items() if not isinstance(v, list)}
-    calls = {}
-    for name, s, e in log:
-        calls.setdefault(name, []).append(s.elapsed_time(e))
     return kern_ms, kern_launches, stats, calls
 
 
-def lattice_roofline(kern_ms, kern_launches, stats, angle: bool, items_per_launch: int, angle_bins: int = 64):
+def lattice_roofline(kern_ms, kern_launches, stats, angle: bool, items_per_launch: int, angle_bins: int = 64,
+                     inference: bool = False):
     """Per pass (all layers of one step), forward and backward: algorithmic flop over the SUM of the durations of
     every kernel that executes part of that work, each measured by the library with HIP events on its launch stream.
     Algorithmic flop = the per-term counts above x the terms actually evaluated, 87 flop per candidate the frame
@@ -218,7 +232,7 @@ def lattice_roofline(kern_ms, kern_launches, stats, angle: bool, items_per_launc
     ``items_per_launch`` per layer for the fused core; one per (pair, head) and encoding for the two-step operators).
     The projections of the reference's formulation (per pair) are reported beside it, not counted: the fused core does
     not execute them."""
-    fused = "fused_core_forward" in kern_ms
+    fused = "fused_core_forward" in kern_ms or "item_pass" in kern_ms
     kind = "fused" if fused else "two_step"
     f_fwd, f_bwd, epi = (F_FWD, F_BWD, EPI_FWD) if angle else (F_FWD_DIST, F_BWD_DIST, EPI_FWD_DIST)
     if angle and angle_bins == 16:      # the whole 16-bin basis per axis instead of a 33-bin window
@@ -229,6 +243,8 @@ def lattice_roofline(kern_ms, kern_launches, stats, angle: bool, items_per_launc
     for path, (ev, pairs) in (("forward", ("fwd_evaluated", "fwd_pairs")), ("backward", ("bwd_evaluated", "bwd_pairs"))):
         names = [k for k in PATHS[path][kind] if k in kern_ms]
         main = ("fused_core_" if fused else "framed_pe_") + path
+        if path == "forward" and "item_pass" in kern_ms:
+            main = "item_pass"
         if main not in kern_ms:
             continue
         per_kernel = {k: {"kernel": KERNEL_NAMES[k], "avg_launch_ms": kern_ms[k], "launches_per_step": kern_launches[k],
@@ -244,7 +260,7 @@ def lattice_roofline(kern_ms, kern_launches, stats, angle: bool, items_per_launc
         # per (atom, head) over its histogram of hw words (64 distance bins + 3 axes x 5 moments x 64 bins)
         flop_epi_reference = stats[pairs] * epi * passes
         if fused:
-            hw = {64: 1024, 16: 128}.get(angle_bins, 64)
+            hw = {64: 704 if inference else 1024, 16: 128}.get(angle_bins, 64)
             flop_epi = items_per_launch * n * 2 * 16 * hw * passes
         else:
             flop_epi = flop_epi_reference
@@ -254,7 +270,7 @@ def lattice_roofline(kern_ms, kern_launches, stats, angle: bool, items_per_launc
                                         "projections_of_the_reference_formulation": flop_epi_reference},
                      "achieved": flop / t / 1e12, "frac": flop / t / 1e12 / PEAK_FP32_TFLOPS,
                      "reference_equivalent_tflops": (flop_terms + flop_frames + flop_epi_reference) / t / 1e12,
-                     "main_kernel": KERNEL_NAMES[main], "main_kernel_avg_launch_ms": kern_ms[main],
+                     "main_kernel": KERNEL_NAMES[main], "main_launches_per_step": kern_launches[main], "main_kernel_avg_launch_ms": kern_ms[main],
                      "terms_evaluated_per_launch": stats[ev] / n,
                      "terms_in_box_per_launch": stats["fwd_in_box" if path == "forward" else "bwd_in_box"] / n,
                      "frame_candidates_per_launch": frame_terms / n,
@@ -292,7 +308,8 @@ def other_config(name: str, dev, *, layers: int, backward: bool, angle_bins: int
     run = graphed(fn, 2)
     sec = timed(run, steps)
     kern_ms, kern_launches, stats, _ = instrumented(fn, 2, dev)
-    roof = lattice_roofline(kern_ms, kern_launches, stats, angle_bins > 0, int(cb_cpu.pos.shape[0]) * mp.head_num, angle_bins)
+    roof = lattice_roofline(kern_ms, kern_launches, stats, angle_bins > 0, int(cb_cpu.pos.shape[0]) * mp.head_num, angle_bins,
+                            inference=not backward)
     return {"workload": f"{name}: {B} crystals, {int(cb_cpu.pos.shape[0])} atoms, {int((cb_cpu.sizes ** 2).sum())} atom pairs; "
                         f"{layers}-layer max-frame model ({'64 + %d bins' % angle_bins if angle_bins else '64 distance bins, no angle encoding'}), "
                         f"{'forward + backward' if backward else 'forward only'}, one HIP graph per pass",
@@ -401,7 +418,7 @@ def main():
         return
     roof = lattice_roofline(kern_ms, kern_launches, stats, True, int(cb.pos.shape[0]) * mp.head_num)
     dom_name, dom = max(roof.items(), key=lambda kv: kv[1]["ms_per_step"])
-    fused = "fused_core_forward" in kern_ms
+    fused = attention.FUSED_CORE
     wide = KM.CORE_WINDOW_MODE == _lib.CFH_WINDOW_WIDE
     headline_setting = args.batch == 256 and fused and wide
     # counters of the committed profiles (headline workload and setting only)
@@ -468,7 +485,7 @@ def main():
         terms[k + "_terms_in_box_per_s"] = r["terms_in_box_per_launch"] / t
         terms[k + "_terms_evaluated_per_s"] = r["terms_evaluated_per_launch"] / t
         terms[k + "_terms_evaluated_per_s_over_the_path"] = (r["terms_evaluated_per_launch"] *
-                                                            r["kernels"][[n for n in r["kernels"] if n.endswith(k)][0]]["launches_per_step"]
+                                                            r["main_launches_per_step"]
                                                             / (r["ms_per_step"] * 1e-3))
     if "forward" in roof:
         terms["evaluated_fraction"] = roof["forward"]["terms_evaluated_per_launch"] / max(1.0, roof["forward"]["terms_in_box_per_launch"])

@@ -1271,6 +1271,7 @@ int allow_lds(size_t lds) {
 int bridge_forward(const cfh::BridgeArgs& A, int D, hipStream_t st) {
     const unsigned tiles = (unsigned)((A.N + 15) / 16);
     const dim3 block(64 * cfh::BR_WAVES);
+    TimedScope timed("layer_bridge_forward", st);
     if (bridge_split(A.N, A.F) && A.x1 && A.h) {
         const dim3 g1(tiles, (unsigned)(A.F / 128)), g2(tiles, A.qs ? 3u : 1u);
         const size_t lds = 16 * (size_t)(A.F + cfh::BR_PAD) * sizeof(float);
@@ -1296,6 +1297,7 @@ int bridge_front(const cfh::BridgeArgs& A, int D, hipStream_t st) {
     const unsigned tiles = (unsigned)((A.N + 15) / 16), parts = bridge_split(A.N, A.F) ? 3u : 1u;
     const dim3 block(64 * cfh::BR_WAVES);
     const size_t lds = 16 * (size_t)(16 * cfh::bridge_feat_steps(A.feat) + cfh::BR_PAD) * sizeof(float);
+    TimedScope timed("layer_front", st);
     if (D == 256) hipLaunchKernelGGL(cfh::layer_front_fwd_kernel<2>, dim3(tiles, parts), block, lds, st, A);
     else hipLaunchKernelGGL(cfh::layer_front_fwd_kernel<1>, dim3(tiles, parts), block, lds, st, A);
     return finish_launch("layer_front_forward");
@@ -1304,6 +1306,7 @@ int bridge_backward(cfh::BridgeBwdArgs A, int D, hipStream_t st) {
     A.klen_h = bridge_klen(D, A.F); A.klen_1 = bridge_klen(A.F, D); A.klen_o = bridge_klen(D, D);
     const unsigned tiles = (unsigned)((A.N + 15) / 16);
     const dim3 block(64 * cfh::BR_WAVES);
+    TimedScope timed("layer_bridge_backward", st);
     if (bridge_split(A.N, A.F) && !A.inputs_only) {
         const dim3 g1(tiles, (unsigned)(A.F / 128));
         const size_t lds = 16 * (size_t)(A.F + cfh::BR_PAD) * sizeof(float);
@@ -1737,7 +1740,7 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
         C.slow_wgs = slow_wave_count(N, p->num_heads);
     }
     C.slow_flag = cfh::REC_BOX_LISTED;
-    const char* what = "fused_core_forward";
+    const char* what = one_launch ? "item_pass" : "fused_core_forward";
     if (lean) {
         if (p->angle_bins == cfh::NBINS) {      // moments around the nodes of inference
             C.K.bc.ang_mu0 += cfh::LEAN_FIRST * C.K.bc.ang_interval;

@@ -1,5 +1,5 @@
 // The projections between the attention cores of two consecutive encoder layers, which act on every atom (row)
-// separately, in one launch each way:
+// separately, in one launch each way (two for few rows):
 //     x1  = x_res + attn Wo^T + bo              (output projection of the attention + residual)
 //     h   = relu(x1 W1^T + b1)                  (feed-forward, first half)
 //     x2  = x1 + h W2^T + b2                    (second half + residual: the layer's output)

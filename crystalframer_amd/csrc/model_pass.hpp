@@ -276,6 +276,7 @@ void tail_args(const cfh_model* m, const cfh_model_batch* b, const ModelBuffers&
 int tail_launch(const cfh::TailArgs& T, const float* gout, hipStream_t st) {
     const dim3 grid((unsigned)((T.B + T.per_wg - 1) / T.per_wg)), block(64 * cfh::TAIL_WAVES);
     const size_t lds = 2 * (size_t)cfh::TAIL_ROWS * T.ld * sizeof(float);
+    TimedScope timed("model_tail", st);
     if (int rc = gout ? allow_lds<cfh::model_tail_bwd_kernel>(lds) : allow_lds<cfh::model_tail_fwd_kernel>(lds)) return rc;
     if (gout) hipLaunchKernelGGL(cfh::model_tail_bwd_kernel, grid, block, lds, st, T, gout);
     else hipLaunchKernelGGL(cfh::model_tail_fwd_kernel, grid, block, lds, st, T);
@@ -318,8 +319,10 @@ int cfh_model_forward(const cfh_model* m, const cfh_model_batch* b, float* out) 
     hipStream_t st = (hipStream_t)b->stream;
     const int64_t N = b->N, E = b->E, B = b->B;
     const int D = m->D, F = m->F, H = m->heads;
+    TimedScope whole("model_forward", st);
     // the weights of the bridges in the order of their use, the cores' concatenated weights, the geometry
     {
+        TimedScope timed("model_start", st);
         cfh::StartArgs A{};
         cfh::GeometryArgs& g = A.geo;
         g.pos = b->pos; g.batch = b->batch; g.tvecs = b->tvecs; g.sizes = b->sizes;
@@ -445,6 +448,7 @@ int cfh_model_backward(const cfh_model* m, const cfh_model_batch* b, const float
     hipStream_t st = (hipStream_t)b->stream;
     const int64_t N = b->N, E = b->E, B = b->B;
     const int D = m->D, F = m->F, H = m->heads;
+    TimedScope whole("model_backward", st);
     cfh::TailArgs T;
     tail_args(m, b, M, T);
     for (int i = 0; i < m->linears; i++) T.lin[i].gy = G.gy[i];
@@ -506,9 +510,12 @@ int cfh_model_backward(const cfh_model* m, const cfh_model_batch* b, const float
     std::vector<float*> core_grads(4 * (size_t)m->layers, nullptr);
     const std::vector<cfh_linear_grad_job> jobs = model_wgrad_jobs(m, b, M, G, grads, core_grads.data());
     const std::vector<int32_t> group = model_wgrad_groups(m);
-    if ((rc = linear_wgrad_batch_impl(jobs.data(), (int32_t)jobs.size(), G.wgrad_ws, G.wgrad_bytes, b->stream, true,
-                                      group.empty() ? nullptr : group.data())))
-        return rc;
+    {
+        TimedScope timed("linear_weight_gradients", st);
+        if ((rc = linear_wgrad_batch_impl(jobs.data(), (int32_t)jobs.size(), G.wgrad_ws, G.wgrad_bytes, b->stream, true,
+                                          group.empty() ? nullptr : group.data())))
+            return rc;
+    }
     std::vector<cfh_core_wgrad_job> cj;
     for (int l = 0; l < m->layers; l++) {
         cj.push_back(cfh_core_wgrad_job{G.layer[l].g_attn, M.layer[l].hist, N, core_grads[4 * l], core_grads[4 * l + 1],

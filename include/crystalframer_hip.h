@@ -123,12 +123,14 @@ int cfh_abi_version(void);
 const char* cfh_last_error(void);
 
 /*
- * Diagnostics with no counterpart in the reference.  After cfh_timing_enable(1) every call of the
- * frame-search and value-encoding entry points brackets its lattice-sum kernel (that kernel alone,
- * not the small kernels around it) with HIP events on the stream of the call; cfh_timing_read waits
- * for the launches recorded under `what` ("frame_axis1", "frame_axis2", "frame_axes",
- * "framed_pe_forward", "framed_pe_backward"), returns their summed duration and count, and forgets
- * them.  Not to be enabled while the stream is being captured into a graph.
+ * Diagnostics with no counterpart in the reference.  After cfh_timing_enable(1) the entry points bracket their kernels with
+ * HIP events on the stream of the call; cfh_timing_read waits for the launches recorded under `what`, returns their summed
+ * duration and count, and forgets them.  Names: "frame_axis1", "frame_axis2", "framed_pe_forward", "framed_pe_backward" (the
+ * lattice-sum kernel alone, not the small kernels around it); "core_tables", "core_prepare", "frame_axes", "item_pass" (few
+ * items: record, frame and sums in one launch), "fused_core_forward", "core_project", "core_prepare_bwd", "core_gbuild",
+ * "fused_core_backward", "core_bwd_col", "core_weight_gradients"; "layer_front", "layer_bridge_forward",
+ * "layer_bridge_backward"; "model_start", "model_tail", "linear_weight_gradients", and "model_forward", "model_backward"
+ * around a whole pass.  Not to be enabled while the stream is being captured into a graph.
  */
 int cfh_timing_enable(int on);
 int cfh_timing_read(const char* what, double* total_ms, int64_t* launches);
@@ -528,8 +530,8 @@ int cfh_small_linear_dx(const float* dy, const float* W, int64_t M, int64_t N, i
  *   them from qkv (Wqkv NULL: the chain ends with x2 and the last eight outputs are not touched).
  * Weights as torch.nn.Linear stores them, biases may be NULL; D = 16 H, 128 or 256, and F a multiple of 128.  Every
  * intermediate is an output because the backward pass needs it.  workspace:
- * cfh_layer_bridge_workspace_bytes(D, F), for the weights in the order in which the launch reads them; laid out anew by every
- * call.  Replaces, for a layer without layer norm and dropout and with the ReLU activation, the out_proj of
+ * cfh_layer_bridge_workspace_bytes(D, F), for the weights in the order in which the launches read them; laid out anew by every
+ * call (one launch), then the chain in one launch, or in two for few rows (several workgroups per 16 of them).  Replaces, for a layer without layer norm and dropout and with the ReLU activation, the out_proj of
  * the attention and the residual (models/indexed_lattice_multi_head_attention_cuda.py:734,
  * models/indexed_latticeformer_encoder.py:639-648), the feed-forward block (:606, :644-648) and the
  * input projection, query scaling and Gaussian coefficient of the next layer

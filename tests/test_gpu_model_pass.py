@@ -286,6 +286,29 @@ def test_items_in_one_launch_and_in_several(bins):
         assert Hh.rel_err(q, p.double()) < 2e-5      # (sums over the atoms in other slices)
 
 
+def test_the_library_times_the_kernels_of_the_model_pass():
+    """What bench.py reports per kernel comes from the pass it times."""
+    from crystalframer_amd import _lib, params, synthetic
+    cb = synthetic.make_batch(7, atoms="uniform", atoms_lo=1, atoms_hi=4, len_lo=3.0, len_hi=9.0, ang_lo=65.0, ang_hi=115.0,
+                              seed=1)
+    model, cb = _model(params.ModelParams(num_layers=3, symm_break_noise=0.0), cb)
+    names = dict(model_forward=1, model_backward=1, model_start=1, layer_front=1, item_pass=3, core_project=3,
+                 layer_bridge_forward=3, model_tail=2, layer_bridge_backward=4, core_gbuild=3, fused_core_backward=3,
+                 core_bwd_col=3, linear_weight_gradients=1, core_weight_gradients=1, fused_core_forward=0, core_prepare=0)
+    for n in names:
+        _lib.read_kernel_timing(n)
+    _lib.kernel_timing(True)
+    try:
+        out = model(cb)
+        assert out.grad_fn.name() == "ModelPassHIPBackward"
+        out.sum().backward()
+    finally:
+        _lib.kernel_timing(False)
+    read = {n: _lib.read_kernel_timing(n) for n in names}
+    assert {n: c for n, (ms, c) in read.items()} == names
+    assert all(ms > 0.0 for ms, c in read.values() if c)
+
+
 def test_forward_derivatives_are_refused():
     import torch.autograd.forward_ad as fwAD
     from crystalframer_amd import params, synthetic
