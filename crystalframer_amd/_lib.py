@@ -322,8 +322,9 @@ def workspace(device: torch.device, nbytes: int) -> torch.Tensor:
             # a HIP graph captured on this stream holds the address of the buffer it was given: a superseded
             # buffer stays allocated, so that replays keep writing into memory that is still theirs
             _superseded.append(buf)
-        buf = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
-        buf[:512].zero_()          # work-queue heads and the statistics block
+        with torch.inference_mode(False):      # (kept for later calls, whatever mode this one is made in)
+            buf = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
+            buf[:512].zero_()          # work-queue heads and the statistics block
         _workspaces[key] = buf
     return buf
 
@@ -339,7 +340,8 @@ def wgrad_scratch(device: torch.device, stream_ptr, nbytes: int) -> torch.Tensor
     if buf is None or buf.numel() < nbytes:
         if buf is not None:
             _superseded.append(buf)      # a captured graph may still hold its address
-        buf = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
+        with torch.inference_mode(False):
+            buf = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
         _wgrad_scratch[key] = buf
     return buf
 

@@ -208,7 +208,7 @@ class CrystalformerMultiheadAttentionCUDA(nn.Module):
                     and v.data_ptr() == k.data_ptr() + k.numel() * es
                     and q.is_contiguous() and k.is_contiguous() and v.is_contiguous())
         if not adjacent:
-            with torch.no_grad():
+            with torch.inference_mode(False), torch.no_grad():      # (the parameters outlive a pass in inference mode)
                 st = torch.cat([q.data, k.data, v.data], dim=0)
                 q.data = st[:q.shape[0]]
                 k.data = st[q.shape[0]:q.shape[0] + k.shape[0]]

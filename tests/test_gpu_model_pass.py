@@ -309,6 +309,22 @@ def test_the_library_times_the_kernels_of_the_model_pass():
     assert all(ms > 0.0 for ms, c in read.values() if c)
 
 
+def test_training_after_a_first_pass_in_inference_mode():
+    from crystalframer_amd import params, synthetic
+    cb = synthetic.make_batch(3, atoms="uniform", atoms_lo=1, atoms_hi=4, len_lo=3.0, len_hi=9.0, ang_lo=65.0, ang_hi=115.0,
+                              seed=1)
+    model, cb = _model(params.ModelParams(num_layers=2, symm_break_noise=0.0), cb)
+    for layer in model.encoder.layers:               # storages of their own, as after loading: stacked again by the next pass
+        for p in (layer.self_attn.q_proj_weight, layer.self_attn.k_proj_weight, layer.self_attn.v_proj_weight):
+            p.data = p.data.clone()
+    with torch.inference_mode():
+        first = model(cb)
+    out = model(cb)
+    assert out.grad_fn.name() == "ModelPassHIPBackward" and Hh.rel_err(out, first.double()) < 1e-6
+    out.sum().backward()
+    assert all(p.grad is not None for p in model.parameters() if p.requires_grad)
+
+
 def test_forward_derivatives_are_refused():
     import torch.autograd.forward_ad as fwAD
     from crystalframer_amd import params, synthetic

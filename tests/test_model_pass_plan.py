@@ -241,3 +241,14 @@ def test_batches_of_other_shapes_are_left_to_the_modules(planned, name, change):
     assert model_pass.covered(model, cb) is not None
     setattr(cb, name, change(getattr(cb, name)))
     assert model_pass.covered(model, cb) is None
+
+
+def test_a_plan_made_in_inference_mode_leaves_the_parameters_trainable(monkeypatch):
+    monkeypatch.setattr(model_pass, "_on_device", lambda weight: True)
+    model = latticeformer.Latticeformer(params.ModelParams(num_layers=2))
+    with torch.inference_mode():
+        assert model_pass._Plan(model).ok
+    for n, p in model.named_parameters():
+        assert not p.is_inference() and not p.data.is_inference(), n
+        assert p.requires_grad == (not n.endswith("_scale")), n
+    assert model_pass._Plan(model).native.wanted() == 2
