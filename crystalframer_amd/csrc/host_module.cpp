@@ -49,11 +49,20 @@ at::Tensor arena(size_t n, const c10::Device& dev) {
     return bytes((n + step - 1) / step * step, dev);
 }
 
+// Memory whose address the library was given: kept, and still where it was.
+struct Held {
+    c10::Storage storage;
+    const void* base;
+    explicit Held(const at::Tensor& t) : storage(t.storage()), base(storage.data()) {}
+    bool there() const { return storage.data() == base; }
+};
+
 // What a plan's passes share (see model_pass._Plan).
 struct Shared {
     std::vector<at::Tensor> params;            // in the order of the library's gradients
     std::vector<at::Tensor> gauss;
-    std::vector<at::Tensor> alive;             // params and gauss as the plan was made: the library has their addresses
+    std::vector<Held> held;                    // of params and gauss as the plan was made
+    std::vector<std::vector<int64_t>> sizes;   // of params
     std::vector<int64_t> offset;               // of a parameter's gradient, in floats
     c10::Device device{c10::kCPU};
     int64_t feat = 0, D = 0, H = 0, out_features = 0;
@@ -81,6 +90,7 @@ struct ModelPassBackward : public torch::autograd::Node {
     std::vector<uint64_t> seeds;
     at::Tensor arena_, workspace_;
     std::vector<torch::autograd::SavedVariable> data;
+    std::vector<Held> held;                    // of the batch
     std::vector<at::Tensor> first;
     std::vector<int64_t> versions;
     bool released = false;
@@ -91,6 +101,7 @@ struct ModelPassBackward : public torch::autograd::Node {
         arena_.reset();
         workspace_.reset();
         data.clear();
+        held.clear();
         first.clear();
     }
     static std::vector<int64_t> current_versions(const Shared& P) {
@@ -103,14 +114,18 @@ struct ModelPassBackward : public torch::autograd::Node {
     torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
         TORCH_CHECK(!released, "the backward pass of this model output has been made and what its forward pass kept is given back; to "
                     "make it a second time, make the first one with retain_graph=True");
-        // A parameter whose .data was exchanged since the forward pass: the addresses are those of the storages before, which
-        // plan->alive keeps, and the gradients those of what the forward pass computed.
+        // The .data of a parameter or of the batch was exchanged since the forward pass: the addresses are those of the storages
+        // before, which are held, and the gradients those of what the forward pass computed.
         const size_t n = plan->params.size();
         torch::autograd::variable_list out(n);
         if (!grads[0].defined()) return out;
         TORCH_CHECK(current_versions(*plan) == versions,
                     "a parameter of the model was modified by an inplace operation between its forward and its backward pass");
         for (auto& s : data) s.unpack(shared_from_this());       // (says so if an input was changed in place)
+        for (auto* list : {&plan->held, &held})
+            for (auto& h : *list)
+                TORCH_CHECK(h.there(), "the memory of a parameter of the model or of the batch was resized or given back between the "
+                            "forward and the backward pass");
         const at::Tensor gout = grads[0].detach().to(at::kFloat).contiguous();
         c10::DeviceGuard guard(plan->device);
         const at::Tensor flat = at::empty({total}, at::TensorOptions().dtype(at::kFloat).device(plan->device));
@@ -129,7 +144,7 @@ struct ModelPassBackward : public torch::autograd::Node {
             auto t = at::detail::make_tensor<c10::TensorImpl>(c10::Storage(storage), flat.key_set(), flat.dtype());
             c10::TensorImpl* impl = t.unsafeGetTensorImpl();
             impl->set_storage_offset(plan->offset[i]);
-            impl->set_sizes_contiguous(plan->alive[i].sizes());
+            impl->set_sizes_contiguous(plan->sizes[i]);
             out[i] = std::move(t);
         }
         return out;
@@ -167,8 +182,9 @@ struct Plan {
         for (auto* list : {&S->params, &S->gauss})
             for (auto& p : *list) {
                 layout.push_back({p.data_ptr(), p.sizes().vec()});
-                S->alive.push_back(p.detach());
+                S->held.emplace_back(p);
             }
+        for (auto& p : S->params) S->sizes.push_back(p.sizes().vec());
         S->device = S->params[0].device();
         S->feat = feat; S->D = D; S->H = H; S->out_features = out_features;
     }
@@ -246,7 +262,10 @@ struct Plan {
         node->workspace_ = std::move(ws);
         node->first = std::move(first);
         node->versions = ModelPassBackward::current_versions(*S);
-        for (const at::Tensor* t : {&x, &pos, &batch, &trans, &sizes}) node->data.emplace_back(*t, false);
+        for (const at::Tensor* t : {&x, &pos, &batch, &trans, &sizes}) {
+            node->data.emplace_back(*t, false);
+            node->held.emplace_back(*t);
+        }
         torch::autograd::edge_list edges;
         edges.reserve(S->params.size());
         for (auto& p : S->params) edges.push_back(torch::autograd::impl::gradient_edge(p));

@@ -122,12 +122,25 @@ def test_backward_pass_after_the_storages_of_the_weights_were_exchanged():
         for p in model.parameters():
             p.data = p.data * 3.0 + 1.0
         model(cb)                                    # (the plan is made again)
-        fill = [torch.full_like(p, 7.0) for p in model.parameters() for _ in range(3)]      # takes the memory given back
+        for n in ("x", "pos", "trans_vec", "sizes", "batch"):
+            t = getattr(cb, n)
+            t.data = t.clone()
+        # takes the memory given back
+        fill = [torch.full_like(p, 7.0) for p in model.parameters() for _ in range(3)]
+        fill += [torch.full_like(getattr(cb, n), 7) for n in ("x", "pos", "trans_vec", "sizes", "batch") for _ in range(3)]
     loss.backward()
     for n, p in model.named_parameters():
         if n in want:
             assert torch.equal(p.grad, want[n]), n
     assert len(fill) > 0
+    # memory that is no longer there is not read
+    for t in (cb.pos, model.mlp[0].weight):
+        out, copy_of_t, size = model(cb), t.detach().clone(), t.untyped_storage().nbytes()
+        t.untyped_storage().resize_(0)
+        with pytest.raises(RuntimeError, match="resized or given back"):
+            out.sum().backward()
+        t.untyped_storage().resize_(size)
+        t.detach().copy_(copy_of_t)
 
 
 @pytest.fixture
