@@ -19,6 +19,8 @@
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/SavedTensorHooks.h>
 
+#include <mutex>
+
 #include "../../include/crystalframer_hip.h"
 
 namespace py = pybind11;
@@ -35,6 +37,11 @@ struct Library {
 void check(int rc, const char* what) {
     TORCH_CHECK(rc == 0, what, " failed (", rc, "): ", g_lib.last_error ? g_lib.last_error() : "");
 }
+
+// The launches of a pass share the scratch of their stream, and a backward pass is enqueued by a thread of the autograd engine
+// without the interpreter's lock: no other thread's launches come between those of a pass.  (Nothing that is done with this
+// held waits for the interpreter.)
+std::mutex g_enqueue;
 
 at::Tensor bytes(size_t n, const c10::Device& dev) {
     return at::empty({(int64_t)n}, at::TensorOptions().dtype(at::kByte).device(dev));
@@ -134,9 +141,13 @@ struct ModelPassBackward : public torch::autograd::Node {
         q.workspace = workspace_.data_ptr();
         q.workspace_bytes = (size_t)workspace_.numel();
         q.stream = (void*)c10::hip::getCurrentHIPStream(plan->device.index()).stream();
-        check(g_lib.backward(model.m, &q, gout.data_ptr<float>(), scratch.data_ptr(), (size_t)scratch.numel(),
-                             flat.data_ptr<float>()),
-              "cfh_model_backward");
+        int rc;
+        {
+            std::lock_guard<std::mutex> lock(g_enqueue);
+            rc = g_lib.backward(model.m, &q, gout.data_ptr<float>(), scratch.data_ptr(), (size_t)scratch.numel(),
+                                flat.data_ptr<float>());
+        }
+        check(rc, "cfh_model_backward");
         // a tensor of its own per parameter over the common storage (autograd adopts it as .grad: nobody else holds it)
         const c10::Storage& storage = flat.storage();
         for (size_t i = 0; i < n; i++) {
@@ -249,7 +260,12 @@ struct Plan {
         b.arena = arena_.data_ptr(); b.arena_bytes = (size_t)arena_.numel();
         b.workspace = ws.data_ptr(); b.workspace_bytes = (size_t)ws.numel();
         b.stream = (void*)c10::hip::getCurrentHIPStream(S->device.index()).stream();
-        check(g_lib.forward(m, &b, out.data_ptr<float>()), "cfh_model_forward");
+        int rc;
+        {
+            std::lock_guard<std::mutex> lock(g_enqueue);
+            rc = g_lib.forward(m, &b, out.data_ptr<float>());
+        }
+        check(rc, "cfh_model_forward");
         if (!keep) return out;
         auto node = std::shared_ptr<ModelPassBackward>(new ModelPassBackward(), torch::autograd::deleteNode);
         node->plan = S;

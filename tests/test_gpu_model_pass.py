@@ -322,6 +322,36 @@ def test_the_library_times_the_kernels_of_the_model_pass():
     assert all(ms > 0.0 for ms, c in read.values() if c)
 
 
+def test_passes_of_several_threads_on_one_stream():
+    """A thread trains, another predicts, both on the default stream, whose scratch they share."""
+    import threading
+    from crystalframer_amd import params, synthetic
+    kw = dict(atoms="uniform", atoms_lo=1, atoms_hi=12, len_lo=3.0, len_hi=9.0, ang_lo=65.0, ang_hi=115.0)
+    mp = params.ModelParams(num_layers=2, symm_break_noise=0.0)
+    train, cb = _model(mp, synthetic.make_batch(110, seed=1, **kw), seed=1)
+    serve, other = _model(mp, synthetic.make_batch(90, seed=2, **kw), seed=2)
+    named = [p for p in train.parameters() if p.requires_grad]
+    step = lambda: torch.autograd.grad(train(cb).sum(), named)  # noqa: E731
+    want = step()
+    with torch.no_grad():
+        expected = serve(other)
+    seen, stop = [], threading.Event()
+
+    def serving():
+        with torch.no_grad():
+            while not stop.is_set() and len(seen) < 400:
+                seen.append(serve(other))
+
+    thread = threading.Thread(target=serving)
+    thread.start()
+    got = [step() for _ in range(40)]
+    stop.set()
+    thread.join()
+    assert len(seen) > 0 and all(torch.equal(o, expected) for o in seen)
+    for g in got:
+        assert all(torch.equal(a, b) for a, b in zip(g, want))
+
+
 def test_training_after_a_first_pass_in_inference_mode():
     from crystalframer_amd import params, synthetic
     cb = synthetic.make_batch(3, atoms="uniform", atoms_lo=1, atoms_hi=4, len_lo=3.0, len_hi=9.0, ang_lo=65.0, ang_hi=115.0,
