@@ -50,6 +50,7 @@ class _Plan:
     part keeps the storages whose addresses the library has, and a backward pass keeps the native part's."""
 
     def __init__(self, model):
+        self.owner = model.__dict__
         self.links = []          # (dict, key, value): the plan holds while dict[key] is value
         self.walked = []         # (dict, entries): ... and while the dicts whose entries were walked have as many of them
         self.seen = set()
@@ -334,7 +335,7 @@ def covered(model, data):
     if not _eager(host, keep):
         return None
     plan = model.__dict__.get("_pass_plan")
-    if plan is None or not plan.current():
+    if plan is None or plan.owner is not model.__dict__ or not plan.current():      # (a shallow copy has its original's plan)
         plan = model.__dict__["_pass_plan"] = _Plan(model)
     if not plan.ok:
         return None

@@ -1,5 +1,7 @@
 """What the whole-model pass keeps between calls (model_pass._Plan), looked at on the CPU: the plan of a model is made again
 when what it was derived from changes, and a pass it does not cover is left to the modules."""
+import copy
+
 import pytest
 import torch
 import torch.autograd.forward_ad as fwAD
@@ -252,3 +254,14 @@ def test_a_plan_made_in_inference_mode_leaves_the_parameters_trainable(monkeypat
         assert not p.is_inference() and not p.data.is_inference(), n
         assert p.requires_grad == (not n.endswith("_scale")), n
     assert model_pass._Plan(model).native.wanted() == 2
+
+
+def test_a_shallow_copy_has_a_plan_of_its_own(planned):
+    model, plan = planned
+    cb = _batch()
+    assert model_pass.covered(model, cb) is not None
+    other = copy.copy(model)
+    assert model_pass.covered(other, cb)[0] is not model_pass.covered(model, cb)[0]
+    other = copy.copy(model)
+    other.pooling_layer = latticeformer.max_pool
+    assert model_pass.covered(other, cb) is None and model_pass.covered(model, cb) is not None
