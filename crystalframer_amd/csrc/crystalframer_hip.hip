@@ -317,7 +317,7 @@ struct TimedScope {
     ~TimedScope() {
         if (on && hipEventRecord(t.stop, st) == hipSuccess) {
             std::lock_guard<std::mutex> lock(g_timing_mutex);
-            g_timed.push_back(t);
+            try { g_timed.push_back(t); } catch (const std::exception&) {}      // (a record lost, no more)
         }
     }
     TimedScope(const TimedScope&) = delete;

@@ -286,7 +286,7 @@ int tail_launch(const cfh::TailArgs& T, const float* gout, hipStream_t st) {
 
 extern "C" {
 
-int64_t cfh_model_sizes(const cfh_model* m, const cfh_model_batch* b, size_t bytes[4]) {
+int64_t cfh_model_sizes(const cfh_model* m, const cfh_model_batch* b, size_t bytes[4]) try {
     if (int rc = check_model(m, b)) return rc;
     if (!bytes) return fail(CFH_EINVAL, "bytes must not be NULL");
     cfh_model_batch q = *b;
@@ -305,9 +305,11 @@ int64_t cfh_model_sizes(const cfh_model* m, const cfh_model_batch* b, size_t byt
         if (wg > bytes[3]) bytes[3] = wg;
     }
     return model_gradient_floats(m);
+} catch (const std::exception& e) {
+    return fail(CFH_ELAUNCH, "model: %s", e.what());      // (host memory: nothing is thrown through a C entry point)
 }
 
-int cfh_model_forward(const cfh_model* m, const cfh_model_batch* b, float* out) {
+int cfh_model_forward(const cfh_model* m, const cfh_model_batch* b, float* out) try {
     int rc = check_model(m, b);
     if (rc) return rc;
     if (!b->x || !b->pos || !b->batch || !b->tvecs || !b->sizes || !out)
@@ -428,10 +430,12 @@ int cfh_model_forward(const cfh_model* m, const cfh_model_batch* b, float* out) 
     T.x = M.layer[m->layers - 1].x2;
     T.lin[m->linears - 1].y = out;
     return tail_launch(T, nullptr, st);
+} catch (const std::exception& e) {
+    return fail(CFH_ELAUNCH, "model forward: %s", e.what());
 }
 
 int cfh_model_backward(const cfh_model* m, const cfh_model_batch* b, const float* gout, void* scratch,
-                       size_t scratch_bytes, float* grads) {
+                       size_t scratch_bytes, float* grads) try {
     int rc = check_model(m, b);
     if (rc) return rc;
     if (!b->x || !b->pos || !b->batch || !b->tvecs || !b->sizes || !gout || !grads || !b->keep)
@@ -531,6 +535,8 @@ int cfh_model_backward(const cfh_model* m, const cfh_model_batch* b, const float
         }
     }
     return CFH_OK;
+} catch (const std::exception& e) {
+    return fail(CFH_ELAUNCH, "model backward: %s", e.what());
 }
 
 }  // extern "C"
