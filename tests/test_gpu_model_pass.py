@@ -322,6 +322,20 @@ def test_the_library_times_the_kernels_of_the_model_pass():
     assert all(ms > 0.0 for ms, c in read.values() if c)
 
 
+# more layers than a launch's table holds: 32 weight gradients of linear layers, 8 of cores, 24 weight streams, 24 layers' weights
+@pytest.mark.parametrize("layers,bins", [(7, 16), (9, 64), (13, 0), (26, 64)])
+def test_deep_models(layers, bins):
+    from crystalframer_amd import params, synthetic
+    kw = dict(value_pe_angle_wscale=1.0, value_pe_dist_coef=1.5, value_pe_angle_coef=6.0) if bins == 16 else {}
+    mp = params.ModelParams(num_layers=layers, value_pe_angle_real=bins, symm_break_noise=0.0, **kw)
+    cb = synthetic.make_batch(5, atoms="uniform", atoms_lo=1, atoms_hi=5, len_lo=3.0, len_hi=9.0, ang_lo=65.0, ang_hi=115.0,
+                              seed=layers)
+    model, cb, ((o1, e1, g1), (o2, e2, g2)) = _both(mp, cb)
+    assert torch.equal(o1, o2) and Hh.rel_err(e1, e2.double()) < 1e-6 * layers
+    for n in g1:                                # (sums over the atoms in other slices: a rounding of 6e-8 per atom at worst)
+        assert Hh.rel_err(g1[n], g2[n].double()) < 6e-8 * cb.pos.shape[0], n
+
+
 def test_passes_of_several_threads_on_one_stream():
     """A thread trains, another predicts, both on the default stream, whose scratch they share."""
     import threading
