@@ -1,7 +1,7 @@
 // What a pass over a batch starts with, in two launches: everything that depends on nothing but the caller's tensors, then
 // what is made of it per atom and pair.  The parts are those of geometry.hpp, fused_core.hpp and layer_bridge.hpp; each is
 // a few microseconds of work that fills a fraction of the chip.  One by one -- six launches, and a part of every layer's
-// launch that makes the item records -- they made up 35 of the 196 us of a call for one crystal; together 20.
+// launch that makes the item records -- they made up 35 of the 196 us of a call for one crystal; together 15.
 #pragma once
 #include "fused_core.hpp"
 #include "geometry.hpp"
