@@ -260,7 +260,7 @@ def lattice_roofline(kern_ms, kern_launches, stats, angle: bool, items_per_launc
         # per (atom, head) over its histogram of hw words (64 distance bins + 3 axes x 5 moments x 64 bins)
         flop_epi_reference = stats[pairs] * epi * passes
         if fused:
-            hw = {64: 704 if inference else 1024, 16: 128}.get(angle_bins, 64)
+            hw = {64: 720 if inference else 1024, 16: 128}.get(angle_bins, 64)
             flop_epi = items_per_launch * n * 2 * 16 * hw * passes
         else:
             flop_epi = flop_epi_reference

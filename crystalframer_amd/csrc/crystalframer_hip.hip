@@ -1597,14 +1597,14 @@ int launch_core(Kern kern, const cfh::CoreArgs& C, hipStream_t st, const char* w
     }
     return finish_launch(what);
 }
-// The slices of the sum over the words: 256 words per wavefront with all moments, 176 with the nodes of inference.
+// The slices of the sum over the words: 256 words per wavefront with all moments, 144 with the nodes of inference.
 void project_launch(int hw, const float* hist, const float* wcat, float* out, int64_t N, int H, hipStream_t st) {
     const dim3 grid((unsigned)((N + 15) / 16), (unsigned)H);
     auto launch = [&](auto kern, int waves) {
         hipLaunchKernelGGL(kern, grid, dim3(cfh::WAVE * waves), 0, st, hist, wcat, out, (int)N, H);
     };
     if (hw == cfh::HW_ANG) launch(cfh::core_project_kernel<4, 16>, 4);
-    else if (hw == cfh::HW_LEAN) launch(cfh::core_project_kernel<4, 11>, 4);
+    else if (hw == cfh::HW_LEAN) launch(cfh::core_project_kernel<5, 9>, 5);
     else if (hw == cfh::HW_ANG16) launch(cfh::core_project_kernel<2, 4>, 2);
     else launch(cfh::core_project_kernel<1, 4>, 1);
 }
@@ -1742,10 +1742,8 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
     C.slow_flag = cfh::REC_BOX_LISTED;
     const char* what = one_launch ? "item_pass" : "fused_core_forward";
     if (lean) {
-        if (p->angle_bins == cfh::NBINS) {      // moments around the nodes of inference
-            C.K.bc.ang_mu0 += cfh::LEAN_FIRST * C.K.bc.ang_interval;
-            C.K.bc.ang_inv_interval *= (float)cfh::LEAN_DEN / cfh::LEAN_NUM;
-        }
+        if (p->angle_bins == cfh::NBINS)        // moments around the nodes of inference
+            C.K.bc.ang_inv_interval = (float)((double)C.K.bc.ang_inv_interval * cfh::LEAN_DEN / cfh::LEAN_NUM);
         if (one_launch) { CFH_CORE_DISPATCH(CFH_ITEM_PASS_LEAN); }
         else { CFH_CORE_DISPATCH(CFH_CORE_FWD_LEAN); }
     } else {

@@ -70,11 +70,11 @@ __host__ __device__ constexpr int core_hist_lds_words(int ang) {
 // words of an item's histogram for `ang` angle bins (0: distance encoding alone)
 __host__ __device__ constexpr int core_hist_words(int ang, bool lean = false);
 // Inference, where the histogram serves the projection alone, uses FEWER nodes for the moments of the angle encoding than
-// one per bin (moment_series.hpp): 704 words instead of 1024, with an error of the series that is no larger.  At 22 528 atoms:
-// projection 204 -> 131 us, main kernel 404 -> 387 (its vector instructions, not its stores, bound it; making the projection
+// one per bin (moment_series.hpp): 720 words instead of 1024, with an error of the series that is no larger.  At 22 528 atoms:
+// projection 204 -> 131 us, main kernel 404 -> 383 (its vector instructions, not its stores, bound it; making the projection
 // in it, four items of a head per workgroup behind a barrier, took 529 us for both at 640 words).
-constexpr int HW_LEAN = 704;
-static_assert(HW_LEAN >= HW_DIST + 3 * NORD * LEAN_NODES && HW_LEAN % 64 == 0, "");
+constexpr int HW_LEAN = 720;
+static_assert(HW_LEAN >= HW_DIST + 3 * NORD * LEAN_NODES && HW_LEAN % 16 == 0, "");
 __host__ __device__ constexpr int core_hist_words(int ang, bool lean) {
     return ang == NBINS ? (lean ? HW_LEAN : HW_ANG) : (ang == SMALL_A ? HW_ANG16 : HW_DIST);
 }
@@ -242,7 +242,7 @@ __device__ __forceinline__ void build_node_table(float* dtab, float ws) {
     const float r = 0.5f * LEAN_NUM / LEAN_DEN / ws, inv_ws = 1.0f / ws;
     for (int u = threadIdx.x; u < LEAN_TAB; u += blockDim.x) {
         float c[NORD];
-        node_coefficients(((float)(u - LEAN_OFF) * (1.0f / LEAN_DEN) - LEAN_FIRST) * inv_ws, r, c);
+        node_coefficients((float)(u - LEAN_OFF) * (1.0f / LEAN_DEN) * inv_ws, r, c);
 #pragma unroll
         for (int o = 0; o < NORD; o++) dtab[o * LEAN_TAB + u] = c[o];
     }
@@ -978,7 +978,7 @@ void fused_core_fwd_kernel(const CoreArgs C) {
 // wavefront takes UNITS x 16 words of the reduction index through MFMA 16x16x4 (the four lanes of a row read 64
 // consecutive bytes of it per load), the slices meet in LDS and are added in a fixed order by the first
 // wavefront (no atomics: the result does not depend on timing).  grid (ceil(N/16), H), block 64 * WAVES.
-// Bound by reading the histograms: 508 MB (22 528 atoms, 704 words) in 131 us (3.9 TB/s).  Measured at 640 words, 119 us: 129
+// Bound by reading the histograms: 519 MB (22 528 atoms, 720 words) in 131 us (4.0 TB/s).  Measured at 640 words, 119 us: 129
 // with half of the loads ahead of the products; 115 with four tiles per workgroup and the weights in registers.
 template <int WAVES, int UNITS>
 __global__ __launch_bounds__(WAVE * WAVES) void core_project_kernel(const float* __restrict__ hist, const float* __restrict__ wcat,

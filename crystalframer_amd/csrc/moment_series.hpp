@@ -8,12 +8,16 @@
 //
 // Two sets of nodes:
 //   every bin (training)    nodes at the 64 bins, half = 1/2, the series cut after NORD terms;
-//   42 nodes (inference)    3/2 bins apart, half = 3/4; the terms of order NORD and more are folded into the lower ones
+//   43 nodes (inference)    3/2 bins apart, half = 3/4; the terms of order NORD and more are folded into the lower ones
 //                           modulo a quintic between the Legendre polynomial, whose mean square on [-1, 1] is the smallest,
 //                           and the Chebyshev polynomial, whose maximum is: close to 1/8 of the cut series' error.
-// Error over all u and bins, against 64 bits (ws = 4): every bin 1.43e-6 at most, 1.35e-7 rms; 42 nodes 1.22e-6, 1.31e-7.
+// Error over all u and bins, against 64 bits (ws = 4): every bin 1.43e-6 at most, 1.35e-7 rms; 43 nodes 1.22e-6, 1.31e-7.
 // It is the mean square that a sum over many images shows: 38 nodes 5/3 bins apart, interpolated at the Chebyshev points, stay
-// below 1.17e-6 but have 2.52e-7 rms.  46 nodes 11/8 bins apart: 0.44e-6 and 0.95e-7, for 64 words more per item.
+// below 1.17e-6 but have 2.52e-7 rms.  And not all cosines are alike: the image that sets the first axis has the cosine 1 to
+// it and 0 to the others, its opposite -1 and 0.  There the nodes of inference are exact (u = 63, 31.5 and 0 are nodes; with 42
+// of them between the ends they were the ends of intervals), where the bins, for the cosine 0, are at their worst.  Output of
+// one layer with large angle weights against float64, relative rms: every bin 8.0e-7, 43 nodes 3.0e-7; 42 nodes 9.0e-7, the 38
+// nodes 8.1e-7.
 #pragma once
 #ifdef __HIPCC__
 #define CFH_SERIES_FN __host__ __device__ __forceinline__
@@ -29,8 +33,7 @@ namespace cfh {
 #endif
 constexpr int NORD = CFH_NORD;                  // moments per axis
 constexpr int LEAN_NUM = 3, LEAN_DEN = 2;       // distance of the nodes of inference in bins
-constexpr int LEAN_NODES = 42;
-constexpr float LEAN_FIRST = 0.75f;             // centre of node 0 in bin units: the nodes' intervals cover [0, 63]
+constexpr int LEAN_NODES = 43;                  // node 0 at bin 0, node 42 at bin 63
 constexpr double LEAN_FOLD_3 = 1.15, LEAN_FOLD_1 = 0.26;      // the quintic eps^5 - 1.15 eps^3 + 0.26 eps
 
 CFH_SERIES_FN float series_exp(float x) {

@@ -322,6 +322,49 @@ def test_the_library_times_the_kernels_of_the_model_pass():
     assert all(ms > 0.0 for ms, c in read.values() if c)
 
 
+# (with |cos| the cosines 0 and 1 are nodes of both series: what is left are errors of the same size, measured at some thousand
+# outputs)
+@pytest.mark.parametrize("cos_abs,slack", [(0, 1.0), (1, 1.15)])
+def test_inference_is_as_close_to_float64_as_training(cos_abs, slack):
+    """One layer with large angle weights, its atoms' outputs pooled and read through an identity head."""
+    from crystalframer_amd import params, synthetic
+    from oracle import cpu_model
+    wrong = {"inference": 0.0, "training": 0.0}
+    for seed in range(4):
+        mp = params.ModelParams(num_layers=1, symm_break_noise=0.0, cos_abs=cos_abs)
+        cb = synthetic.make_batch(24, atoms="uniform", atoms_lo=1, atoms_hi=6, len_lo=3.0, len_hi=9.0, ang_lo=65.0, ang_hi=115.0,
+                                  seed=seed + 50)
+        host = cb
+
+        def change(model):
+            at = model.encoder.layers[0].self_attn
+            model.mlp[3] = torch.nn.Linear(128, 128).cuda()
+            with torch.no_grad():
+                for n in (1, 2, 3):
+                    getattr(at, f"proj_angle{n}").mul_(8.0)
+                at.v_proj_weight.mul_(0.1)
+                at.pe_dist_proj.mul_(0.1)
+                for i in (0, 3):
+                    model.mlp[i].weight.copy_(torch.eye(128))
+                    model.mlp[i].bias.zero_()
+
+        model, cb = _model(mp, cb, seed, change)
+        at = model.encoder.layers[0].self_attn
+        at.frame_sink = []
+        with torch.no_grad():
+            model(cb)
+            frames = [[f.detach().cpu().double() for f in at.frame_sink[0]]]
+            at.frame_sink = None
+            out = {"inference": model(cb)}
+        out["training"] = model(cb).detach()
+        sd = {k: v.detach().cpu().double() for k, v in model.state_dict().items()}
+        ref = cpu_model.model_forward(sd, host, mp, dtype=torch.float64, frames_per_layer=frames, windows="full")
+        for k, o in out.items():
+            assert Hh.rel_err(o, ref) < 1e-5
+            wrong[k] += float(((o.cpu().double() - ref) ** 2).sum())
+    assert wrong["inference"] <= slack ** 2 * wrong["training"], {k: v ** 0.5 for k, v in wrong.items()}
+
+
 # more layers than a launch's table holds: 32 weight gradients of linear layers, 8 of cores, 24 weight streams, 24 layers' weights
 @pytest.mark.parametrize("layers,bins", [(7, 16), (9, 64), (13, 0), (26, 64)])
 def test_deep_models(layers, bins):

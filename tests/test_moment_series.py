@@ -13,8 +13,8 @@ SHIM = r"""
 #include "moment_series.hpp"
 using namespace cfh;
 template <typename T> static void node(double u, T ws, double* c, double* eps) {
-    const double step = (double)LEAN_NUM / LEAN_DEN, n = std::nearbyint((u - LEAN_FIRST) / step);
-    const double at = std::min(std::max(n, 0.0), LEAN_NODES - 1.0) * step + LEAN_FIRST;
+    const double step = (double)LEAN_NUM / LEAN_DEN, n = std::nearbyint(u / step);
+    const double at = std::min(std::max(n, 0.0), LEAN_NODES - 1.0) * step;
     for (int m = 0; m < 64; m++) {
         T out[NORD];
         node_coefficients((T)(m - at) / ws, (T)(0.5 * step) / ws, out);
@@ -65,7 +65,8 @@ def _errors(series, name, ws, points):
 @pytest.mark.parametrize("ws", [3.0, 4.0, 6.0, 8.0])      # (the core takes the series from 3 bins on)
 def test_inference_nodes_are_as_good_as_a_node_per_bin(series, ws):
     points = (np.arange(63 * 96) + 0.5) / 96
-    ends = np.concatenate([[0.0, 63.0]] + [np.arange(63) + 0.5 + s for s in (-1e-9, 1e-9)])      # (where two nodes of training meet)
+    # (the ends, and where two nodes meet)
+    ends = np.concatenate([[0.0, 63.0]] + [t + s for t in (np.arange(63) + 0.5, 1.5 * np.arange(42) + 0.75) for s in (-1e-9, 1e-9)])
     top, rms = _errors(series, "training", ws, points)
     top = max(top, _errors(series, "training", ws, ends)[0])
     top_i, rms_i = _errors(series, "inference", ws, points)
@@ -77,4 +78,7 @@ def test_inference_nodes_are_as_good_as_a_node_per_bin(series, ws):
     # the coefficients in 32 bits: each a sum of a few products below 1, a rounding of 6e-8 each
     top_f, rms_f = _errors(series, "inference32", ws, points)
     assert top_f <= top_i + 5e-7 and rms_f <= rms_i + 1e-7
-    assert series.words() <= 704
+    # the cosines that every frame has, 1, 0 and -1 (with |cos| 0 and 1): nodes, exact but for the rounding of a coefficient
+    for u in (63.0, 31.5, 0.0):
+        assert _errors(series, "inference", ws, [u])[0] < 1e-9 and _errors(series, "inference32", ws, [u])[0] < 2e-7
+    assert series.words() <= 720
