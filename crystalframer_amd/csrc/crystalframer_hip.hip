@@ -26,6 +26,7 @@
 #include "linear_grad.hpp"
 #include "small_gemm.hpp"
 #include "layer_bridge.hpp"
+#include "bridge_infer.hpp"
 #include "adamw.hpp"
 #include "model_tail.hpp"
 
@@ -1228,17 +1229,23 @@ int check_bridge(int64_t N, int32_t D, int32_t F) {
 size_t bridge_stream_floats(int kind, int D, int F, bool next, int feat = 0) {
     return (size_t)(cfh::BR_WAVES * cfh::bridge_stream_steps(kind, D, F, next, feat) + cfh::BR_RING) * 64 * 4;
 }
+size_t split_stream_floats(int kind, int D, int F, bool next, int feat = 0) {
+    return (size_t)(cfh::BR_WAVES * cfh::split_stream_steps(kind, D, F, next, feat) + cfh::BI_STEPS) * 192 * 4;
+}
 // Collects weight streams and makes them in as few launches as the argument table allows.
 struct StreamList {
     cfh::BridgeStreams T{};
     int blocks = 0;
     hipStream_t st;
-    StreamList(int D, int F, hipStream_t stream, int feat = 0) : st(stream) { T.D = D; T.F = F; T.feat = feat; }
+    StreamList(int D, int F, hipStream_t stream, int feat = 0, bool split = false) : st(stream) {
+        T.D = D; T.F = F; T.feat = feat; T.split = split ? 1 : 0;
+    }
     int add(int kind, const float* Wo, const float* W1, const float* W2, const float* Wq, float* dst) {
         if (T.n == cfh::BR_MAX_STREAMS) flush();
         cfh::BridgeStream& S = T.s[T.n++];
         S.Wo = Wo; S.W1 = W1; S.W2 = W2; S.Wq = Wq; S.dst = dst; S.kind = kind;
-        S.steps = cfh::bridge_stream_steps(kind, T.D, T.F, Wq != nullptr, T.feat);
+        S.steps = T.split ? cfh::split_stream_steps(kind, T.D, T.F, Wq != nullptr, T.feat)
+                          : cfh::bridge_stream_steps(kind, T.D, T.F, Wq != nullptr, T.feat);
         S.block0 = blocks;
         blocks += (cfh::BR_WAVES * S.steps * 64 + 255) / 256;
         return S.steps;
@@ -1301,6 +1308,53 @@ int bridge_front(const cfh::BridgeArgs& A, int D, hipStream_t st) {
     if (D == 256) hipLaunchKernelGGL(cfh::layer_front_fwd_kernel<2>, dim3(tiles, parts), block, lds, st, A);
     else hipLaunchKernelGGL(cfh::layer_front_fwd_kernel<1>, dim3(tiles, parts), block, lds, st, A);
     return finish_launch("layer_front_forward");
+}
+// The forms of the inference kernels (bridge_infer.hpp).  Two launches while there are at most two workgroups (16 rows, chunk) per
+// compute unit: 1024 rows 10.9 us against 15.5 in one, 2048 14.9 and 16.0, 2560 18.1 and 16.3.  32 rows per workgroup once 16
+// of them do not fit the compute units at one each: 4096 rows 17.0 us with 16 and 20.8 with 32, 5120 25.8 and 21.1, 22 528
+// 75.5 and 57.0.
+bool infer_split(int64_t N, int F) {
+    int cus = device_cus();
+    if (cus <= 0) cus = 256;
+    return ((N + 15) / 16) * (F / 128) <= 2 * (int64_t)cus;
+}
+bool infer_rows32(int64_t N) {
+    int cus = device_cus();
+    if (cus <= 0) cus = 256;
+    return (N + 15) / 16 > cus;
+}
+// The same where nothing is kept (A.stream a split one; A.h: (F / 128, N, D) floats of scratch for the form in two launches).
+template <int CT>
+int bridge_infer_launch(const cfh::BridgeArgs& A, hipStream_t st) {
+    const unsigned tiles = (unsigned)((A.N + 15) / 16);
+    const dim3 block(64 * cfh::BR_WAVES);
+    TimedScope timed("layer_bridge_forward", st);
+    if (infer_split(A.N, A.F)) {
+        hipLaunchKernelGGL(cfh::bridge_infer_split1_kernel<CT>, dim3(tiles, (unsigned)(A.F / 128)), block, 0, st, A);
+        hipLaunchKernelGGL(cfh::bridge_infer_split2_kernel<CT>, dim3(tiles, A.qs ? 3u : 1u), block, 0, st, A);
+    } else if (CT == 1 && infer_rows32(A.N)) {
+        hipLaunchKernelGGL((cfh::bridge_infer_kernel<CT == 1 ? 2 : 1, CT>), dim3((tiles + 1) / 2), block, 0, st, A);
+    } else {
+        hipLaunchKernelGGL((cfh::bridge_infer_kernel<1, CT>), dim3(tiles), block, 0, st, A);
+    }
+    return finish_launch("layer_bridge_forward");
+}
+int bridge_infer(const cfh::BridgeArgs& A, int D, hipStream_t st) {
+    return D == 128 ? bridge_infer_launch<1>(A, st) : bridge_infer_launch<2>(A, st);
+}
+template <int TR, int CT>
+int front_infer_launch(const cfh::BridgeArgs& A, unsigned parts, hipStream_t st) {
+    const size_t lds = 3 * 16 * TR * (size_t)(16 * cfh::bridge_feat_steps(A.feat) + cfh::BI_PAD) * sizeof(__bf16);
+    TimedScope timed("layer_front", st);
+    if (int rc = allow_lds<cfh::front_infer_kernel<TR, CT>>(lds)) return rc;
+    hipLaunchKernelGGL((cfh::front_infer_kernel<TR, CT>), dim3((unsigned)((A.N + 16 * TR - 1) / (16 * TR)), parts),
+                       dim3(64 * cfh::BR_WAVES), lds, st, A);
+    return finish_launch("layer_front_forward");
+}
+int front_infer(const cfh::BridgeArgs& A, int D, hipStream_t st) {
+    const unsigned parts = infer_split(A.N, A.F) ? 3u : 1u;
+    if (D == 256) return front_infer_launch<1, 2>(A, parts, st);
+    return infer_rows32(A.N) && A.feat <= 128 ? front_infer_launch<2, 1>(A, parts, st) : front_infer_launch<1, 1>(A, parts, st);
 }
 int bridge_backward(cfh::BridgeBwdArgs A, int D, hipStream_t st) {
     A.klen_h = bridge_klen(D, A.F); A.klen_1 = bridge_klen(A.F, D); A.klen_o = bridge_klen(D, D);

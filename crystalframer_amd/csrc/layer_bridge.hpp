@@ -57,7 +57,7 @@ struct BridgeStream {
     int kind, steps, block0;
 };
 constexpr int BR_MAX_STREAMS = 24;
-struct BridgeStreams { BridgeStream s[BR_MAX_STREAMS]; int n, D, F, feat; };
+struct BridgeStreams { BridgeStream s[BR_MAX_STREAMS]; int n, D, F, feat; int split; };      // split: see bridge_infer.hpp
 // A thread per float4 of the streams: thread `thread` of the block-th 256.
 __device__ __forceinline__ void bridge_stream_element(const BridgeStreams& T, int block, int thread) {
     int si = 0;

@@ -102,14 +102,17 @@ void model_buffers(const cfh_model* m, const cfh_model_batch* b, ModelBuffers& M
     M.near_ = c.take<float>(2 * E);
     M.x0 = c.take<float>(N * D);
     M.pooled = c.take<float>(B * D);
-    M.front_stream = c.take<float>(bridge_stream_floats(cfh::BS_INPUTS, m->D, m->F, true, m->feat));
+    // (a pass that keeps nothing has its own bridges, with streams of their own)
+    M.front_stream = c.take<float>(b->keep ? bridge_stream_floats(cfh::BS_INPUTS, m->D, m->F, true, m->feat)
+                                           : split_stream_floats(cfh::BS_INPUTS, m->D, m->F, true, m->feat));
     M.front_stream_bwd = b->keep ? c.take<float>(bridge_stream_floats(cfh::BS_INPUTS_BACKWARD, m->D, m->F, true)) : nullptr;
     for (int i = 0; i + 1 < m->linears; i++) M.y[i] = c.take<float>(B * (size_t)m->head[i].out);
     ModelLayerBuffers set[2];
     for (int l = 0; l < m->layers; l++) {
         ModelLayerBuffers& L = M.layer[l];
         const bool next = l + 1 < m->layers;
-        float* const stream = c.take<float>(bridge_stream_floats(cfh::BS_FORWARD, m->D, m->F, next));
+        float* const stream = c.take<float>(b->keep ? bridge_stream_floats(cfh::BS_FORWARD, m->D, m->F, next)
+                                                    : split_stream_floats(cfh::BS_FORWARD, m->D, m->F, next));
         float* const stream_bwd = b->keep ? c.take<float>(bridge_stream_floats(cfh::BS_BACKWARD, m->D, m->F, next)) : nullptr;
         float* const wcat = c.take<float>(D * hw);
         if (b->keep || l < 2) {
@@ -117,9 +120,9 @@ void model_buffers(const cfh_model* m, const cfh_model_batch* b, ModelBuffers& M
             L.x2 = c.take<float>(N * D);
             L.qkv = b->keep ? c.take<float>(N * 3 * D) : nullptr;
             if (b->keep || l == 0) {
-                const bool split = bridge_split(b->N, m->F);      // (the bridge in two launches passes them through memory)
-                L.x1 = b->keep || split ? c.take<float>(N * D) : nullptr;
-                L.h = b->keep || split ? c.take<float>(N * F) : nullptr;
+                const bool split = infer_split(b->N, m->F);      // (the bridge in two launches passes its parts through memory)
+                L.x1 = b->keep ? c.take<float>(N * D) : nullptr;
+                L.h = b->keep ? c.take<float>(N * F) : (split ? c.take<float>(F / 128 * N * D) : nullptr);
                 L.frames = c.take<float>(9 * N * H);
                 if (b->keep) { L.z = c.take<float>(E * H); L.prob = c.take<float>(E * H); }
                 L.hist = c.take<float>(H * N * hw);
@@ -340,7 +343,7 @@ int cfh_model_forward(const cfh_model* m, const cfh_model_batch* b, float* out) 
             A.table = M.table;
             A.table_blocks = (int)((B + per - 1) / per);
         }
-        StreamList S(D, F, st, m->feat);
+        StreamList S(D, F, st, m->feat, !b->keep);
         S.add(cfh::BS_INPUTS, m->We, nullptr, nullptr, m->layer[0].Wqkv, M.front_stream);
         if (b->keep) S.add(cfh::BS_INPUTS_BACKWARD, nullptr, nullptr, nullptr, m->layer[0].Wqkv, M.front_stream_bwd);
         cfh::StartWcat W{};
@@ -384,12 +387,14 @@ int cfh_model_forward(const cfh_model* m, const cfh_model_batch* b, float* out) 
         } else {
             cfh::BridgeArgs A{};
             A.attn = b->x; A.x2 = M.x0; A.feat = m->feat;
-            A.stream = M.front_stream; A.steps = cfh::bridge_stream_steps(cfh::BS_INPUTS, D, F, true, m->feat);
+            A.stream = M.front_stream;
+            A.steps = b->keep ? cfh::bridge_stream_steps(cfh::BS_INPUTS, D, F, true, m->feat)
+                              : cfh::split_stream_steps(cfh::BS_INPUTS, D, F, true, m->feat);
             A.bq = L.bqkv; A.lattice_w = L.lattice_w; A.gauss = L.gauss_scale_dev;
             A.qkv = Y.qkv; A.qs = Y.qs; A.k = Y.k; A.v = Y.v; A.a = Y.a;
             A.N = (int)N; A.D = D; A.F = F; A.H = H;
             A.c1 = L.c1; A.lb = L.lb; A.c2 = L.c2; A.q_scale = L.q_scale;
-            if ((rc = bridge_front(A, D, st))) return rc;
+            if ((rc = b->keep ? bridge_front(A, D, st) : front_infer(A, D, st))) return rc;
         }
     }
     int held = layer_half_width(m->layer[0]);
@@ -415,7 +420,8 @@ int cfh_model_forward(const cfh_model* m, const cfh_model_batch* b, float* out) 
         cfh::BridgeArgs A{};
         A.attn = Y.out; A.xres = l ? M.layer[l - 1].x2 : M.x0;
         A.bo = L.bo; A.b1 = L.b1; A.b2 = L.b2;
-        A.stream = Y.stream; A.steps = cfh::bridge_stream_steps(cfh::BS_FORWARD, D, F, next);
+        A.stream = Y.stream;
+        A.steps = b->keep ? cfh::bridge_stream_steps(cfh::BS_FORWARD, D, F, next) : cfh::split_stream_steps(cfh::BS_FORWARD, D, F, next);
         A.x1 = Y.x1; A.h = Y.h; A.x2 = Y.x2;
         A.N = (int)N; A.D = D; A.F = F; A.H = H;
         if (next) {
@@ -423,7 +429,7 @@ int cfh_model_forward(const cfh_model* m, const cfh_model_batch* b, float* out) 
             A.qkv = Yn.qkv; A.qs = Yn.qs; A.k = Yn.k; A.v = Yn.v; A.a = Yn.a;
             A.c1 = Ln.c1; A.lb = Ln.lb; A.c2 = Ln.c2; A.q_scale = Ln.q_scale;
         }
-        if ((rc = bridge_forward(A, D, st))) return rc;
+        if ((rc = b->keep ? bridge_forward(A, D, st) : bridge_infer(A, D, st))) return rc;
     }
     cfh::TailArgs T;
     tail_args(m, b, M, T);

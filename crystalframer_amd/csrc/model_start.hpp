@@ -5,7 +5,7 @@
 #pragma once
 #include "fused_core.hpp"
 #include "geometry.hpp"
-#include "layer_bridge.hpp"
+#include "bridge_infer.hpp"
 
 namespace cfh {
 
@@ -39,7 +39,9 @@ __global__ __launch_bounds__(START_THREADS) __attribute__((amdgpu_waves_per_eu(8
         return;
     }
     block -= A.table_blocks;
-    bridge_stream_element(A.streams, block * (START_THREADS / 256) + (int)threadIdx.x / 256, (int)threadIdx.x % 256);
+    const int block256 = block * (START_THREADS / 256) + (int)threadIdx.x / 256, thread = (int)threadIdx.x % 256;
+    if (A.streams.split) split_stream_element(A.streams, block256, thread);
+    else bridge_stream_element(A.streams, block256, thread);
 }
 // Workgroups of 256: the concatenated weights, a thread per atom (and one more), eight lanes per pair.
 struct PairsArgs {

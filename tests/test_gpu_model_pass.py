@@ -470,3 +470,51 @@ def test_bridge_launch_forms(D, F, N):
     torch.autograd.backward(out, [gi.float().cuda().view(o.shape) for o, gi in zip(out, g)])
     for n in t64:
         assert Hh.rel_err(p[n].grad, t64[n].grad) < 5e-6, n
+
+
+# The bridges of inference: a row, a tile of 16 rows and its edges; either side of the row counts where they take one launch
+# instead of two (2048 at F = 512, 4096 at F = 256) and 32 rows per workgroup instead of 16 (4096); both widths; one, an odd
+# number and more chunks of the feed-forward block's inside than are read at a time; more features than a group of 128.
+@pytest.mark.parametrize("D,F,N,feat", [(128, 512, 1, 98), (128, 128, 15, 98), (128, 384, 17, 130), (128, 640, 33, 98),
+                                        (128, 512, 2048, 98), (128, 512, 2049, 98), (128, 256, 4096, 98), (128, 512, 4097, 98),
+                                        (128, 512, 4129, 200), (256, 512, 31, 98), (256, 512, 2065, 140)])
+def test_bridges_of_inference(D, F, N, feat):
+    """Against the modules' path (float32 matrix instructions), and, on a part of the atoms, float64."""
+    from crystalframer_amd import latticeformer, model_pass, params, synthetic
+    from oracle import cpu_model
+    mp = params.ModelParams(num_layers=2, symm_break_noise=0.0, value_pe_angle_real=0, model_dim=D, ff_dim=F, head_num=D // 16)
+    torch.manual_seed(N)
+    sizes = torch.full((N,), 1)
+    cb = synthetic.make_batch(N, atoms="uniform", atoms_lo=1, atoms_hi=1, len_lo=3.0, len_hi=6.0, ang_lo=70.0, ang_hi=110.0, seed=N)
+    x = torch.zeros(N, feat)
+    x[torch.arange(N), torch.arange(N) % feat] = 1.0 + torch.rand(N)
+    host = synthetic.CrystalBatch(x, cb.pos, cb.batch, cb.trans_vec, sizes, zero_based=True)
+    model = latticeformer.Latticeformer(mp)
+    if feat != model.input_embeddings.in_features:
+        model.input_embeddings = torch.nn.Linear(feat, D, bias=False)
+    model.mlp[0], model.mlp[3] = torch.nn.Linear(D, D), torch.nn.Linear(D, D)
+    with torch.no_grad():
+        for i in (0, 3):                        # the atoms' outputs, those that the rectifier passes on
+            model.mlp[i].weight.copy_(torch.eye(D))
+            model.mlp[i].bias.zero_()
+    model, cb = model.cuda(), host.to("cuda")
+    model.train()
+    model(cb)
+    model.eval()
+    out = []
+    for on in (True, False):
+        model_pass.ENABLED = on
+        try:
+            with torch.no_grad():
+                out.append(model(cb))
+        finally:
+            model_pass.ENABLED = True
+    limit = 2e-6                                # (sums of up to 640 float32 numbers: 640 ** 0.5 * 2 ** -24)
+    assert model_pass.covered(model, cb) and not torch.equal(out[0], out[1])
+    assert Hh.rel_err(out[0], out[1].double()) < limit
+    some = slice(max(0, N - 40), N)
+    part = synthetic.CrystalBatch(host.x[some], host.pos[some], torch.arange(N)[some] - max(0, N - 40), host.trans_vec[some], sizes[some],
+                                  zero_based=True)
+    sd = {k: v.detach().cpu().double() for k, v in model.state_dict().items()}
+    ref = cpu_model.model_forward(sd, part, mp, dtype=torch.float64, windows="full")
+    assert Hh.rel_err(out[0][some], ref) < limit
