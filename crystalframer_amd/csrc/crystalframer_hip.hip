@@ -1667,16 +1667,26 @@ void project_launch(int hw, const float* hist, const float* wcat, float* out, in
 // us, 4592 items 412 and 380, 7712 items 446 and 415, 10 696 items 398 and 441; cells of 40 to 200 atoms lose from 5760 items
 // on (386 and 397), where the frame search of four heads per wavefront counts for more than the launch it takes.
 constexpr int64_t ITEM_PASS_MAX = 5120;
+// Inference, where the histogram serves the projection alone: the wavefront of such an item makes the product with the head's
+// weights itself, which saves a launch and a round trip of the histogram but reads the weights (46 KB at 64 bins) once per item
+// instead of once per 16.  Whole calls of four layers in us, with a launch for the products and without: 64 bins, 64 items 158
+// and 142, 600 items 207 and 189, 1208 items 191 and 173, 2416 items 210 and 187, 4872 items 320 and 250; so the one launch pays
+// for more items, 6488 items 347 (several launches) and 291, 7712 items 334 and 346.  Of fewer words the launch is short: 16 bins,
+// 576 items 173 and 154; distances alone, 1152 items 129 and 126, 4608 items 142 and 154.
+constexpr int64_t ITEM_PROJECT_FEW_WORDS = 1536, ITEM_PROJECT_MAX = 6656;
+bool item_project(const cfh_params* p, int64_t items) {
+    return items <= (p->angle_bins == cfh::NBINS ? ITEM_PROJECT_MAX : ITEM_PROJECT_FEW_WORDS);
+}
 template <typename Kern>
-int launch_item_pass(Kern kern, const cfh::CoreArgs& C, bool search, hipStream_t st, const char* what) {
+int launch_item_pass(Kern kern, const cfh::CoreArgs& C, bool search, const float* wcat, hipStream_t st, const char* what) {
     {
         TimedScope timed(what, st);
-        hipLaunchKernelGGL(kern, dim3((unsigned)C.K.N * (unsigned)C.K.H), dim3(cfh::WAVE), 0, st, C, search ? 1 : 0);
+        hipLaunchKernelGGL(kern, dim3((unsigned)C.K.N * (unsigned)C.K.H), dim3(cfh::WAVE), 0, st, C, search ? 1 : 0, wcat);
     }
     return finish_launch(what);
 }
-#define CFH_ITEM_PASS(...) launch_item_pass(cfh::item_pass_kernel<__VA_ARGS__>, C, search, st, what)
-#define CFH_ITEM_PASS_LEAN(...) launch_item_pass(cfh::item_pass_kernel<__VA_ARGS__, true>, C, search, st, what)
+#define CFH_ITEM_PASS(...) launch_item_pass(cfh::item_pass_kernel<__VA_ARGS__>, C, search, nullptr, st, what)
+#define CFH_ITEM_PASS_LEAN(...) launch_item_pass(cfh::item_pass_kernel<__VA_ARGS__, true>, C, search, project ? wcat : nullptr, st, what)
 #define CFH_CORE_FWD(...) launch_core(cfh::fused_core_fwd_kernel<__VA_ARGS__>, C, st, what)
 #define CFH_CORE_FWD_LEAN(...) launch_core(cfh::fused_core_fwd_kernel<__VA_ARGS__, true>, C, st, what)
 #define CFH_CORE_BWD(...) launch_core(cfh::fused_core_bwd_kernel<__VA_ARGS__>, C, st, what)
@@ -1731,7 +1741,8 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
     const cfh::WcatArgs WA{W_dist, W_axis1, W_axis2, W_axis3, hw, p->dist_coef, p->angle_coef,
                            p->angle_wscale, wcat};
     // (the word of the noise's seed is copied and advanced by the launch that makes the records)
-    const bool one_launch = N * p->num_heads <= ITEM_PASS_MAX && !(search && p->symm_break_noise > 0.0f && C.K.seed_dev);
+    const bool project_by_item = lean && item_project(p, N * p->num_heads);
+    const bool one_launch = (N * p->num_heads <= ITEM_PASS_MAX || project_by_item) && !(search && p->symm_break_noise > 0.0f && C.K.seed_dev);
     if (one_launch) {
         if (!wcat_made) {
             TimedScope timed("core_prepare", st);
@@ -1794,6 +1805,7 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
         C.slow_wgs = slow_wave_count(N, p->num_heads);
     }
     C.slow_flag = cfh::REC_BOX_LISTED;
+    const bool project = one_launch && project_by_item;
     const char* what = one_launch ? "item_pass" : "fused_core_forward";
     if (lean) {
         if (p->angle_bins == cfh::NBINS)        // moments around the nodes of inference
@@ -1804,7 +1816,7 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
         if (one_launch) { CFH_CORE_DISPATCH(CFH_ITEM_PASS); }
         else { CFH_CORE_DISPATCH(CFH_CORE_FWD); }
     }
-    if (rc) return rc;
+    if (rc || project) return rc;
     {
         TimedScope timed("core_project", st);
         project_launch(hw, hist, wcat, out, N, p->num_heads, st);

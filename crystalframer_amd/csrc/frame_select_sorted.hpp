@@ -87,8 +87,9 @@ struct FrameShared {
 // one wavefront, one item: wid = item * H + head.  `others_only`: only the items that the four-heads-per-wavefront
 // search leaves out (box not the table's, or more pairs than it takes).
 // `skip_listed`: the records listed for the first wavefronts of the launch are theirs.
+// `own`: not null: the item's record, in registers; the frames go into it instead of memory (`keep`: as well).
 __device__ __forceinline__ void frame_item_body(const CoreArgs& C, FrameShared& sh, int wid, int lane, bool others_only,
-                                                bool skip_listed) {
+                                                bool skip_listed, uint32_t* own = nullptr, bool keep = true) {
     float4* const tab = sh.tab;
     float4* const pq = sh.pq;
     uint32_t* const markw = sh.markw;
@@ -108,7 +109,7 @@ __device__ __forceinline__ void frame_item_body(const CoreArgs& C, FrameShared& 
 
     if (it_cur >= P.N) return;
     {
-        const uint32_t rec_cur = load_record_lane(P, it_cur, h, lane);
+        const uint32_t rec_cur = own ? *own : load_record_lane(P, it_cur, h, lane);
         if (skip_listed && ((uint32_t)__builtin_amdgcn_readlane((int)rec_cur, REC_BOX) & REC_BOX_LISTED) != 0u &&
             core_slow_rank(C, wid, lane) < C.slow_wgs)
             return;      // (a listed record of higher rank stays here)
@@ -351,15 +352,20 @@ __device__ __forceinline__ void frame_item_body(const CoreArgs& C, FrameShared& 
             else { f2x = vx; f2y = vy; f2z = vz; }
         }
 
-        if (lane == 0) {
-            float gx, gy, gz, hx, hy, hz;
-            orthonormal_axes(f1x, f1y, f1z, f2x, f2y, f2z, gx, gy, gz, hx, hy, hz);
+        float gx, gy, gz, hx, hy, hz;
+        orthonormal_axes(f1x, f1y, f1z, f2x, f2y, f2z, gx, gy, gz, hx, hy, hz);
+        if (own) {
+            const float f[9] = {f1x, f1y, f1z, gx, gy, gz, hx, hy, hz};
+#pragma unroll
+            for (int c = 0; c < 9; c++) *own = lane == REC_FRAMES + c ? __float_as_uint(f[c]) : *own;
+        }
+        if (lane == 0 && keep) {
             const size_t stride = (size_t)P.N * H * 3;
             float* o = P.out_frame + ((size_t)i * H + h) * 3;
             o[0] = f1x; o[1] = f1y; o[2] = f1z;
             o[stride + 0] = gx; o[stride + 1] = gy; o[stride + 2] = gz;
             o[2 * stride + 0] = hx; o[2 * stride + 1] = hy; o[2 * stride + 2] = hz;
-            if (P.frames_to_records) {
+            if (!own && P.frames_to_records) {
                 // the record of this item becomes that of the kernel that follows: the query makes room for the frames
                 float* r = reinterpret_cast<float*>(P.items + ((size_t)it_cur * H + h) * REC_WORDS + REC_FRAMES);
                 r[0] = f1x; r[1] = f1y; r[2] = f1z;
@@ -698,23 +704,26 @@ __global__ __launch_bounds__(WAVE * CORE_WPB) void frame_axes_kernel(const CoreA
 
 // Everything of an item in one wavefront, for few items: its record, the search for its frame, the lattice sums.  In
 // launches of their own each of the three is a chain of dependent steps behind a launch that fills a fraction of the chip.
-// One crystal of 8 atoms: 22 us in three launches, 17 in one; a whole call of four layers 185 -> 173.
+// One crystal of 8 atoms: 22 us in three launches, 17 in one; a whole call of four layers 185 -> 173.  The record in registers
+// and the sums' first operands asked for ahead of the search, instead of both through memory: 153 -> 149.
 template <int WL, int ANG, bool COS_ABS, bool LEAN = false>
-__global__ __launch_bounds__(WAVE) void item_pass_kernel(const CoreArgs C, int search) {
+__global__ __launch_bounds__(WAVE) void item_pass_kernel(const CoreArgs C, int search, const float* __restrict__ wcat) {
     __shared__ union { FrameShared frame; CoreFwdLds<ANG, LEAN> core; } sh;
     const KernelArgs& P = C.K;
     const int wid = (int)blockIdx.x, lane = (int)threadIdx.x;
     const int it = div_heads(P, wid), h = wid - it * P.H;
     if (it >= P.N) return;
-    // (the record goes to memory: the searches and sums read it there, and so does a backward pass)
-    const uint32_t rec = make_record_lane(P, it, h, lane, search != 0);
-    if (lane < REC_WORDS) P.items[((size_t)it * P.H + h) * REC_WORDS + lane] = rec;
-    __threadfence_block();
+    // (the record stays in registers, and what the sums need first is asked for ahead of the search; a backward pass reads the
+    // record from memory)
+    CoreOwn own;
+    own.rec = make_record_lane(P, it, h, lane, search != 0);
+    own.pf = core_prefetch(C, own.rec, it, h, lane);
     if (ANG > 0 && search) {
-        frame_item_body(C, sh.frame, wid, lane, false, false);
+        frame_item_body(C, sh.frame, wid, lane, false, false, &own.rec, !LEAN);
         __threadfence_block();
     }
-    fused_core_fwd_body<WL, ANG, COS_ABS, LEAN>(C, sh.core, wid);
+    if (!LEAN && lane < REC_WORDS) P.items[((size_t)it * P.H + h) * REC_WORDS + lane] = own.rec;
+    fused_core_fwd_body<WL, ANG, COS_ABS, LEAN>(C, sh.core, wid, wcat, &own);
 }
 
 }  // namespace cfh

@@ -571,10 +571,24 @@ struct CoreFwdShared {
 // LEAN: inference, nothing is kept for a backward pass: fewer nodes for the moments; z and the probabilities are not written.
 template <int ANG, bool LEAN>
 using CoreFwdLds = CoreFwdShared<LEAN && ANG == NBINS ? core_hist_words(ANG, LEAN) : core_hist_lds_words(ANG), LEAN ? 4 : FC_LOGCAP>;
+// Sums of 4 values over the lanes of a wavefront: lane l gets the sum of value l / 16.
+__device__ __forceinline__ float wave_sum4(const float (&v)[4], int lane) {
+    // each step halves the values a lane holds: it keeps one half and hands its partner the other
+    const bool b5 = (lane & 32) != 0, b4 = (lane & 16) != 0;
+    const float p = (b5 ? v[2] : v[0]) + __shfl_xor(b5 ? v[0] : v[2], 32), q = (b5 ? v[3] : v[1]) + __shfl_xor(b5 ? v[1] : v[3], 32);
+    float s = (b4 ? q : p) + __shfl_xor(b4 ? p : q, 16);
+    s += dpp_move<0xB1>(s); s += dpp_move<0x4E>(s); s += dpp_move<0x141>(s);
+    return s + dpp_move<0x128>(s);
+}
 // ANG: angle bins, 0 (distance encoding alone), 64 (moment series) or 16 (basis values added directly)
 // wid: this wavefront's (item, head)
+// wcat: not null: the wavefront makes the product of its histogram with the head's weights itself, the histogram stays in
+// LDS (LEAN only)
+// own: not null: the item's record and first operands, in registers
+struct CoreOwn { uint32_t rec; CorePrefetch pf; };
 template <int WL, int ANG, bool COS_ABS, bool LEAN>
-__device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLds<ANG, LEAN>& sh, int wid) {
+__device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLds<ANG, LEAN>& sh, int wid,
+                                                    const float* __restrict__ wcat = nullptr, const CoreOwn* own = nullptr) {
     constexpr bool HAS_ANG = ANG > 0;
     constexpr int HWK = core_hist_words(ANG, LEAN);          // words per item in memory
     constexpr int HWL = LEAN && ANG == NBINS ? HWK : core_hist_lds_words(ANG);      // ... and in LDS
@@ -613,9 +627,9 @@ __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLd
 
     CFH_PH_DECL
     {
-        const uint32_t rec_cur = load_record_lane(P, it_cur, h, lane);
-        if (core_record_taken_elsewhere(C, rec_cur, wid, lane)) return;
-        const CorePrefetch pf = core_prefetch(C, rec_cur, it_cur, h, lane);
+        const uint32_t rec_cur = own ? own->rec : load_record_lane(P, it_cur, h, lane);
+        if (!own && core_record_taken_elsewhere(C, rec_cur, wid, lane)) return;
+        const CorePrefetch pf = own ? own->pf : core_prefetch(C, rec_cur, it_cur, h, lane);
         CFH_PH(0);
         const CoreItem ci = core_unpack(C, rec_cur, true);
         const int i = ci.item.i;
@@ -909,14 +923,78 @@ __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLd
         CFH_PH(7);
         const float D = uniform_f(wave_sum(Dl));
         const float inv = D > 0.0f ? hw_rcp(D) : 0.0f;
-        {
+        const float sc = inv * hw_rcp(fixs);
+        if (LEAN && wcat) {
+            // Four words per lane at a time (fewer words: one).  A loop over the channels, four at a time with their loads in
+            // flight together: a wavefront runs through this once, and fetching the instructions of all sixteen took longer than
+            // the loop's waits for weights (a layer's launch of 64 items 20.0 us, in the loop 18.2; whole calls of 4872 items 272 and
+            // 250 us).  The loads of eight channels together: 136 registers, three wavefronts per SIMD.
+            constexpr int NV = VEC ? 4 * NW : HWK / WAVE;
+            float word[NV];
+            if (VEC) {
+#pragma unroll
+                for (int u = 0; u < NW; u++) {
+                    int4 hv = make_int4(0, 0, 0, 0);
+                    if (FULL || lane + WAVE * u < HWL / 4) hv = reinterpret_cast<const int4*>(hist)[lane + WAVE * u];
+                    word[4 * u] = (float)hv.x * sc; word[(4 * u + 1) % NV] = (float)hv.y * sc;
+                    word[(4 * u + 2) % NV] = (float)hv.z * sc; word[(4 * u + 3) % NV] = (float)hv.w * sc;
+                }
+            } else {
+#pragma unroll
+                for (int u = 0; u < NV; u++) {
+                    const int w = lane + WAVE * u;
+                    int32_t sum = 0;
+                    if (ANG != SMALL_A || w < HW_DIST) sum = hist[w];
+                    else if (w < HW_DIST + 3 * SMALL_A) {
+#pragma unroll
+                        for (int c = 0; c < A16_COPIES; c++) sum += hist[HW_DIST + c * A16_STRIDE + (w - HW_DIST)];
+                    }
+                    word[u] = (float)sum * sc;
+                }
+            }
+            const float ox = rows8_sum(accv.x) * inv, oy = rows8_sum(accv.y) * inv;      // (the same in every 8-lane row)
+            const float* Wh = wcat + (size_t)h * DH * HWK;
+            float* const dst = C.out + ih * DH;
+#pragma unroll 1
+            for (int c0 = 0; c0 < DH; c0 += 4, Wh += 4 * HWK) {
+                float v[4];
+#pragma unroll
+                for (int c = 0; c < 4; c++) v[c] = lane == ((c0 + c) >> 1) ? ((c & 1) ? oy : ox) : 0.0f;
+                if (VEC) {
+                    float4 wt[4][NW];
+#pragma unroll
+                    for (int c = 0; c < 4; c++)
+#pragma unroll
+                        for (int u = 0; u < NW; u++)      // (a lane past the end reads the last words; its own are zero)
+                            wt[c][u] = *reinterpret_cast<const float4*>(Wh + c * HWK + 4 * min(lane + WAVE * u, HWK / 4 - 1));
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int c = 0; c < 4; c++)
+#pragma unroll
+                        for (int u = 0; u < NW; u++)
+                            v[c] = fmaf(word[4 * u], wt[c][u].x, fmaf(word[(4 * u + 1) % NV], wt[c][u].y,
+                                   fmaf(word[(4 * u + 2) % NV], wt[c][u].z, fmaf(word[(4 * u + 3) % NV], wt[c][u].w, v[c]))));
+                } else {
+                    float wt[4][NV];
+#pragma unroll
+                    for (int c = 0; c < 4; c++)
+#pragma unroll
+                        for (int u = 0; u < NV; u++) wt[c][u] = Wh[c * HWK + lane + WAVE * u];
+#pragma unroll
+                    for (int c = 0; c < 4; c++)
+#pragma unroll
+                        for (int u = 0; u < NV; u++) v[c] = fmaf(word[u], wt[c][u], v[c]);
+                }
+                const float sum = wave_sum4(v, lane);
+                if ((lane & 15) == 0) dst[c0 + (lane >> 4)] = sum;
+            }
+        } else {
             const float ox = rows8_sum(accv.x) * inv, oy = rows8_sum(accv.y) * inv;
             if (lane < FC_GROUP) *reinterpret_cast<float2*>(C.out + ih * DH + 2 * sub) = make_float2(ox, oy);
         }
-        {
+        if (!(LEAN && wcat)) {
             // all reads first (one LDS round trip instead of one per word), then store; a lane takes four
             // consecutive words at a time
-            const float sc = inv * hw_rcp(fixs);
             float* dst = C.hist + ((size_t)h * P.N + i) * HWK;      // head-major: the rows of a head are contiguous
             if (ANG == SMALL_A) {
                 // distance bins as they are, every angle bin as the sum of its copies (integers: any order), zeros behind

@@ -518,3 +518,23 @@ def test_bridges_of_inference(D, F, N, feat):
     sd = {k: v.detach().cpu().double() for k, v in model.state_dict().items()}
     ref = cpu_model.model_forward(sd, part, mp, dtype=torch.float64, windows="full")
     assert Hh.rel_err(out[0][some], ref) < limit
+
+
+# Inference of few items: the product of an item's histogram with the weights by its own wavefront.  One atom, a few, either side
+# of the item counts where a launch of its own makes it (6656 with the 64-bin encoding, 1536 without).
+@pytest.mark.parametrize("bins,B,atoms", [(64, 1, 1), (64, 3, 7), (64, 64, 10), (64, 832, 1), (64, 833, 1), (16, 1, 1), (16, 24, 8),
+                                          (16, 193, 1), (0, 1, 1), (0, 24, 8), (0, 193, 1)])
+def test_products_of_few_items(bins, B, atoms):
+    """Against the same pass with everything kept, whose products have a launch of their own: two sums of 720 float32 products
+    (of a 64-bin pass: around other nodes, 1.4e-6 of the basis' peak, a few 1e-6 of a layer's output)."""
+    from crystalframer_amd import params, synthetic
+    kw = dict(value_pe_angle_wscale=1.0, value_pe_dist_coef=1.5, value_pe_angle_coef=6.0) if bins == 16 else {}
+    mp = params.ModelParams(num_layers=1, value_pe_angle_real=bins, symm_break_noise=0.0, **kw)
+    cb = synthetic.make_batch(B, atoms="uniform", atoms_lo=atoms, atoms_hi=atoms, len_lo=3.0, len_hi=9.0, ang_lo=65.0,
+                              ang_hi=115.0, seed=B)
+    model, cb = _model(mp, cb)
+    model.eval()
+    kept = model(cb).detach()
+    with torch.no_grad():
+        out = model(cb)
+    assert Hh.rel_err(out, kept.double()) < 5e-6
