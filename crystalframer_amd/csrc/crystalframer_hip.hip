@@ -1671,9 +1671,10 @@ constexpr int64_t ITEM_PASS_MAX = 5120;
 // weights itself, which saves a launch and a round trip of the histogram but reads the weights (46 KB at 64 bins) once per item
 // instead of once per 16.  Whole calls of four layers in us, with a launch for the products and without: 64 bins, 64 items 158
 // and 142, 600 items 207 and 189, 1208 items 191 and 173, 2416 items 210 and 187, 4872 items 320 and 250; so the one launch pays
-// for more items, 6488 items 347 (several launches) and 291, 7712 items 334 and 346.  Of fewer words the launch is short: 16 bins,
+// for more items: against several launches 6488 items 346 and 291, 7712 items 333 and 314, 9216 items 294 and 275, 10 696 items
+// 369 and 364, 11 440 items 359 and 373.  Of fewer words the launch is short: 16 bins,
 // 576 items 173 and 154; distances alone, 1152 items 129 and 126, 4608 items 142 and 154.
-constexpr int64_t ITEM_PROJECT_FEW_WORDS = 1536, ITEM_PROJECT_MAX = 6656;
+constexpr int64_t ITEM_PROJECT_FEW_WORDS = 1536, ITEM_PROJECT_MAX = 10240;
 bool item_project(const cfh_params* p, int64_t items) {
     return items <= (p->angle_bins == cfh::NBINS ? ITEM_PROJECT_MAX : ITEM_PROJECT_FEW_WORDS);
 }
