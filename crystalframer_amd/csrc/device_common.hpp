@@ -487,6 +487,14 @@ __device__ __forceinline__ uint32_t load_record(const KernelArgs& P, int it, int
     return (it >= 0 && threadIdx.x < REC_WORDS) ? P.items[((size_t)it * P.H + h) * REC_WORDS + threadIdx.x] : 0u;
 }
 
+// Consecutive workgroups go to the chip's eight dies in turn, each with an L2 of its own.  The place in the work order of
+// workgroup b of `total`: runs of 2^shift consecutive places on one die, the places of 8 runs dealt together (whatever is left
+// of the last 8 runs: in turn).
+__device__ __forceinline__ int die_order(int b, int total, int shift) {
+    const int span = 8 << shift;
+    if (b >= total - (total & (span - 1))) return b;
+    return (((((b >> (shift + 3)) << 3) | (b & 7)) << shift)) | ((b >> 3) & ((1 << shift) - 1));
+}
 // What an item's record says besides its lattice rows and its query or frames.
 struct RecordHead {
     int i, b, e0, npairs, j0;

@@ -50,6 +50,11 @@ constexpr int CORE_WPB = 1;                     // wavefronts per workgroup of t
                                                 // products with the head's weights themselves (projection, G) were slower:
                                                 // +25 us per kernel for the phases behind barriers, against 21 + 20 us for
                                                 // the two separate launches
+constexpr int CORE_DIE_SHIFT = 3;               // frame search and main kernels: runs of 8 items, an atom's with 8 heads, on one die
+                                                // (die_order): they share the pairs' geometry and the lines of k, v, z and P,
+                                                // where item by item every die had a head.  Whole passes: training step of
+                                                // 18 976 items 1279 -> 1265 us, with 16 angle bins 1260 -> 1237, cells of 40 to
+                                                // 200 atoms 1146 -> 1132, inference of 180 224 items 3033 -> 3026
 constexpr int FC_LOGCAP = 64;                   // logits of a row kept in LDS until the row is complete
 constexpr int HW_DIST = NBINS;
 constexpr int HW_ANG = NBINS * (1 + 3 * NORD);  // 1024 words per (atom, head) with the 64-bin angle encoding
@@ -536,7 +541,7 @@ __device__ __forceinline__ int core_slow_record(const CoreArgs& C, int r, int la
 // the others the records in work order.
 __device__ __forceinline__ int core_wave_record(const CoreArgs& C, int w, int lane) {
     // (the same in all lanes: said so, the index arithmetic that follows stays on the scalar unit)
-    return __builtin_amdgcn_readfirstlane(w < C.slow_wgs ? core_slow_record(C, w, lane) : w - C.slow_wgs);
+    return __builtin_amdgcn_readfirstlane(w < C.slow_wgs ? core_slow_record(C, w, lane) : die_order(w - C.slow_wgs, C.K.N * C.K.H, CORE_DIE_SHIFT));
 }
 // The rank over the slow lists of the listed record `wid`: the counts of the lists before its own, and its place in its
 // own list (records in ascending order: the entries below it).
