@@ -572,3 +572,15 @@ def test_layer_bridge_matches_framework_chain(N, has_next, normalised, with_bias
         KM.DEFER_WEIGHT_GRADS = True
     for n in used:
         assert Hh.rel_err(t32[n].grad, t64[n].grad) < 2e-5, n
+
+
+# The column sums four at a time: crystals of every remainder of four, around a step of 16 pairs, and more than one crystal of a
+# size; with fewer workgroups than the eight runs that are dealt to the dies together, and with a remainder of them.
+@pytest.mark.parametrize("atoms,crystals", [(1, 1), (2, 3), (3, 2), (4, 1), (5, 3), (15, 1), (16, 2), (17, 1), (18, 9), (35, 3), (8, 70)])
+def test_column_sums_by_groups_of_columns(atoms, crystals):
+    """Sums of up to 35 float32 products against float64: 35 * 2 ** -24, with the rounding of the probabilities."""
+    P = Hh.make_problem(num_crystals=crystals, atoms_lo=atoms, atoms_hi=atoms, seed=700 + atoms)
+    z, psi, gout = attention_case(P, atoms)
+    _, leaves64, _, leaves = run_both(P, z, psi, gout)
+    for l32, l64, name in zip(leaves[1:3], leaves64[1:3], "kv"):
+        assert Hh.rel_err(l32.grad.cpu().double(), l64.grad) < 5e-6, name
