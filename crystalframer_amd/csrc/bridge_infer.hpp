@@ -40,9 +40,7 @@ __device__ __forceinline__ void split_bf16(float v, __bf16& a, __bf16& b, __bf16
 }
 // Thread `thread` of the block-th 256: eight numbers of a step.
 __device__ __forceinline__ void split_stream_element(const BridgeStreams& T, int block, int thread) {
-    int si = 0;
-    while (si + 1 < T.n && block >= T.s[si + 1].block0) si++;
-    const BridgeStream& S = T.s[si];
+    const BridgeStream& S = T.s[bridge_stream_of(T, block)];
     const int D = T.D, F = T.F, CT = D / 128, du = D / 32;
     const int e = (block - S.block0) * 256 + thread;
     if (e >= BR_WAVES * S.steps * 64) return;

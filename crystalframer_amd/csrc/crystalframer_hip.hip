@@ -1246,7 +1246,7 @@ struct StreamList {
         S.Wo = Wo; S.W1 = W1; S.W2 = W2; S.Wq = Wq; S.dst = dst; S.kind = kind;
         S.steps = T.split ? cfh::split_stream_steps(kind, T.D, T.F, Wq != nullptr, T.feat)
                           : cfh::bridge_stream_steps(kind, T.D, T.F, Wq != nullptr, T.feat);
-        S.block0 = blocks;
+        S.block0 = T.first[T.n - 1] = blocks;
         blocks += (cfh::BR_WAVES * S.steps * 64 + 255) / 256;
         return S.steps;
     }

@@ -495,6 +495,20 @@ __device__ __forceinline__ int die_order(int b, int total, int shift) {
     if (b >= total - (total & (span - 1))) return b;
     return (((((b >> (shift + 3)) << 3) | (b & 7)) << shift)) | ((b >> 3) & ((1 << shift) - 1));
 }
+// Tables in the kernel arguments whose entries have ascending first numbers: the entry that number b (the same in all lanes)
+// belongs to, the last whose first(entry) is not above it.  Every lane looks at an entry of its own: one after the other, each
+// is a load that waits for the arguments' memory (25 entries: linear_wgrad_batch_kernel 69 -> 64 us, linear_wgrad_sum_kernel
+// 13 -> 6; a table behind a struct in the arguments went to scratch instead, see bridge_stream_of).
+template <typename First>
+__device__ __forceinline__ int table_entry(int entries, int b, First&& first) {
+    const int lane = (int)threadIdx.x & 63;
+    int below = 0;
+    for (int k0 = 0; k0 < entries; k0 += 64) {
+        const int k = min(k0 + lane, entries - 1);
+        below += __popcll(__ballot(k0 + lane < entries && first(k) <= b));
+    }
+    return __builtin_amdgcn_readfirstlane(max(below - 1, 0));
+}
 // What an item's record says besides its lattice rows and its query or frames.
 struct RecordHead {
     int i, b, e0, npairs, j0;

@@ -57,12 +57,24 @@ struct BridgeStream {
     int kind, steps, block0;
 };
 constexpr int BR_MAX_STREAMS = 24;
-struct BridgeStreams { BridgeStream s[BR_MAX_STREAMS]; int n, D, F, feat; int split; };      // split: see bridge_infer.hpp
+struct BridgeStreams {
+    BridgeStream s[BR_MAX_STREAMS];
+    int first[BR_MAX_STREAMS];    // their block0
+    int n, D, F, feat;
+    int split;                    // see bridge_infer.hpp
+};
+// The stream that a block (the same in all lanes) belongs to: the first blocks lie side by side and come with a load or two,
+// where a scan of the streams waited for the arguments' memory once per stream.
+__device__ __forceinline__ int bridge_stream_of(const BridgeStreams& T, int block) {
+    const int b = __builtin_amdgcn_readfirstlane(block);
+    int si = 0;
+#pragma unroll
+    for (int k = 1; k < BR_MAX_STREAMS; k++) si += k < T.n && b >= T.first[k] ? 1 : 0;
+    return si;
+}
 // A thread per float4 of the streams: thread `thread` of the block-th 256.
 __device__ __forceinline__ void bridge_stream_element(const BridgeStreams& T, int block, int thread) {
-    int si = 0;
-    while (si + 1 < T.n && block >= T.s[si + 1].block0) si++;
-    const BridgeStream& S = T.s[si];
+    const BridgeStream& S = T.s[bridge_stream_of(T, block)];
     const int D = T.D, F = T.F, CT = D / 128, du = D / 16;
     const int e = (block - S.block0) * 256 + thread;
     if (e >= BR_WAVES * S.steps * 64) return;

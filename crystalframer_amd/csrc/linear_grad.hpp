@@ -328,9 +328,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     const int per_die = (int)gridDim.x >> 3;
     const int block = ((int)blockIdx.x & 7) * per_die + ((int)blockIdx.x >> 3);
     if (block >= T.blocks) return;
-    int j = 0;
-    for (int t = 1; t < T.njobs; t++)
-        if (block >= T.job[t].block0) j = t;
+    const int j = table_entry(T.njobs, block, [&](int k) { return T.job[k].block0; });
     const WgradJob& J = T.job[j];
     const int b = block - J.block0;
     const int tiles = J.bx * J.by;
@@ -345,10 +343,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 __global__ __launch_bounds__(256) void linear_wgrad_sum_kernel(const WgradJobs T) {
     const int t = (int)blockIdx.x >> 2, quarter = (int)blockIdx.x & 3;
     if (t >= T.split_tiles) return;
-    int j = -1;
-    for (int n = 0; n < T.njobs; n++)
-        if (T.job[n].slices > 1 && t >= T.job[n].tile0) j = n;
-    if (j < 0) return;
+    // (jobs of one slice have no tiles here: the tile0 of the next that has)
+    const int lane = (int)threadIdx.x & 63, at = min(lane, T.njobs - 1);
+    static_assert(WGRAD_MAX_JOBS <= 64, "a job per lane");
+    const uint64_t begun = __ballot(lane < T.njobs && T.job[at].slices > 1 && t >= T.job[at].tile0);
+    if (begun == 0) return;
+    const int j = __builtin_amdgcn_readfirstlane(63 - __clzll((long long)begun));
     const WgradJob& J = T.job[j];
     const int tile = t - J.tile0, tiles = J.bx * J.by;
     if (tile >= tiles) return;

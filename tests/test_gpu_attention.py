@@ -584,3 +584,30 @@ def test_column_sums_by_groups_of_columns(atoms, crystals):
     _, leaves64, _, leaves = run_both(P, z, psi, gout)
     for l32, l64, name in zip(leaves[1:3], leaves64[1:3], "kv"):
         assert Hh.rel_err(l32.grad.cpu().double(), l64.grad) < 5e-6, name
+
+
+# One job, two, and a table that is full but for one, full, and one too many (two launches); every third job of one slice.
+@pytest.mark.parametrize("n_jobs", [1, 2, 31, 32, 33])
+def test_weight_gradient_tables(n_jobs):
+    """Every workgroup finds its job: sums of up to 700 float32 products against float64."""
+    from crystalframer_amd import _lib
+    lib = _lib.load()
+    gen = torch.Generator().manual_seed(n_jobs)
+    jobs, ops = (_lib.CfhLinearGradJob * n_jobs)(), []
+    for j, J in enumerate(jobs):
+        N, I, O = (20 if j % 3 == 1 else 500 + 20 * (j % 10)), (64, 40, 128)[j % 3], (64, 128, 72)[(j // 2) % 3]
+        x, dy = (f32(torch.randn(N, c, generator=gen, dtype=torch.float64)) for c in (I, O))
+        dW, db = torch.zeros(O, I, device=dev()), torch.zeros(O, device=dev())
+        J.x, J.dy, J.dW, J.db = (t.data_ptr() for t in (x, dy, dW, db))
+        J.N, J.I, J.O, J.ldx, J.ldy = N, I, O, I, O
+        ops.append((x, dy, dW, db))
+    ws = torch.empty(lib.cfh_linear_weight_bias_grad_batch_workspace_bytes(jobs, n_jobs), dtype=torch.uint8, device=dev())
+    for scratch in (ws, None):
+        for *_, dW, db in ops:
+            dW.zero_()
+            db.zero_()
+        _lib.check(lib.cfh_linear_weight_bias_grad_batch(jobs, n_jobs, _lib.ptr(scratch), scratch.numel() if scratch is not None else 0,
+                                                         _lib.current_stream_ptr(dev())), "batch")
+        for j, (x, dy, dW, db) in enumerate(ops):
+            assert Hh.rel_err(dW, dy.double().t() @ x.double()) < 5e-6, j
+            assert Hh.rel_err(db, dy.double().sum(0)) < 5e-6, j
