@@ -200,15 +200,19 @@ __global__ __launch_bounds__(FC_TCAP) void sorted_shifts_kernel(const float* __r
 // along changes nothing).  Same arithmetic for d^2 as the sweeps.  A thread per pair walking the table alone took
 // 16 us for its chain of dependent steps; this takes 7.
 __device__ __forceinline__ float2 pair_nearest(float rx, float ry, float rz, const float4* tab, int T0, int sub) {
-    const float r = sqrtf(fmaf(rx, rx, fmaf(ry, ry, rz * rz)));
+    const float r = hw_sqrt(fmaf(rx, rx, fmaf(ry, ry, rz * rz)));      // (here and below a bound with margins)
     // (dval carries the table position of its image in its low 7 bits -- it is rounded down by at most 2^-16 of itself,
     // which the margins of every test that uses it cover -- so that the minimum over the lanes brings the position along)
     float dall = 3.0e38f, dval = 3.0e38f;
+    float4 v = tab[sub];
+    float w = tab[0].w;
     for (int t0 = 0; t0 < T0; t0 += 8) {
         // the first entry of the group decides for all eight lanes whether the walk goes on
-        if (dval < 1.0e38f && tab[t0].w > fmaf(1.0001f, r + sqrtf(dval), 1e-3f)) break;
+        if (dval < 1.0e38f && w > fmaf(1.0001f, r + hw_sqrt(dval), 1e-3f)) break;
+        const int next = min(t0 + 8, FC_TCAP - 8);           // (the next group's entries, in flight meanwhile)
+        const float4 vn = tab[next + sub];
+        const float wn = tab[next].w;
         if (t0 + sub < T0) {
-            const float4 v = tab[t0 + sub];
             const float dx = rx + v.x, dy = ry + v.y, dz = rz + v.z;
             const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
             dall = fminf(dall, d2);
@@ -217,6 +221,7 @@ __device__ __forceinline__ float2 pair_nearest(float rx, float ry, float rz, con
         }
         dall = half_min(dall);
         dval = half_min(dval);
+        v = vn; w = wn;
     }
     return make_float2(dall, dval);
 }

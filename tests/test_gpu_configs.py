@@ -160,3 +160,21 @@ def test_geometry_launches_match_framework_expressions(num_crystals, atoms_hi):
     assert (n_of_atom[order][:-1] >= n_of_atom[order][1:]).all()
     if num_crystals <= 1024:
         assert torch.equal(got.order, ref.order)
+
+
+# The pairs' crystals from the wavefront's first pair on: 64 crystals of one pair to a wavefront, runs of crystals without atoms
+# within a wavefront, in front and at the end, and a crystal of many wavefronts.
+@pytest.mark.parametrize("sizes", [[1] * 200, [0, 0, 3, 0, 0, 0, 1, 0, 40, 1, 1, 0, 2, 0, 0], [1, 0] * 150 + [9], [33] + [0] * 70 + [2]])
+def test_pairs_of_ragged_batches(sizes):
+    from crystalframer_amd import geometry
+    gen = torch.Generator().manual_seed(len(sizes))
+    sizes = torch.tensor(sizes)
+    N, E = int(sizes.sum()), int((sizes ** 2).sum())
+    batch = torch.repeat_interleave(torch.arange(len(sizes)), sizes)
+    pos = torch.rand(N, 3, generator=gen)
+    trans = torch.eye(3).repeat(len(sizes), 1, 1) * 5.0
+    got = geometry.crystal_geometry(pos.to(dev()), batch.to(dev()), trans.to(dev()), sizes.to(dev()), E)
+    first = torch.cumsum(sizes, 0) - sizes
+    want = torch.tensor([(int(first[b]) + i, int(first[b]) + j) for b, n in enumerate(sizes.tolist()) for i in range(n) for j in range(n)]).t()
+    assert torch.equal(got.edges.cpu(), want)
+    assert torch.equal(got.rpos.cpu(), pos[want[1]] - pos[want[0]])
