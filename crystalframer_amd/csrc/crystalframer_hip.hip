@@ -1705,7 +1705,7 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
                            const float* W_axis1, const float* W_axis2, const float* W_axis3, int64_t N, int64_t E,
                            int64_t B, float* frames, int32_t search_frames, float* z, float* prob, float* hist,
                            float* out, const cfh_core_cache* cache, void* workspace, size_t workspace_bytes,
-                           void* stream, bool lean, bool wcat_made) {
+                           void* stream, bool lean, bool wcat_made, const int4* heads = nullptr) {
     int rc = check_core_params(p);
     if (rc) return rc;
     if ((rc = check_geometry(a_ih, rpos, tvecs, batch, edges, e_start, N, E, B))) return rc;
@@ -1723,6 +1723,7 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
     cfh::CoreArgs C;
     std::memset(&C, 0, sizeof(C));
     fill_common(C.K, p, a_ih, rpos, tvecs, rvlen, batch, edges, e_start, order, N, E, workspace);
+    C.K.heads = heads;
     C.K.contiguous_neighbours = 1;
     const CoreBuffers buf = fill_core(C, p, L, qs, k, v, rvlen != nullptr, cache, workspace);
     const bool search = has_ang && search_frames != 0;

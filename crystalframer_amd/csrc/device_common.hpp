@@ -348,6 +348,7 @@ struct KernelArgs {
     // geometry
     const float* a_ih; const float* rpos; const float* tvecs; const float* rvlen;
     const int64_t* batch; const int64_t* edges; const int64_t* e_start; const int32_t* order;
+    const int4* heads;            // optional: what the four say of an atom, in work order (GeometryArgs::heads)
     // attention operands for the frame search
     const float* q; const float* k; const float* frame1;
     // value-PE operands
@@ -518,14 +519,29 @@ struct RecordHead {
 };
 __device__ __forceinline__ RecordHead record_head(const KernelArgs& P, int it, int h) {
     RecordHead R;
-    R.i = P.order ? P.order[it] : it;
-    R.b = (int)P.batch[R.i];
+    if (P.heads) {      // (one load ahead of those that the atom and its crystal lead to; the arrays take two)
+        const int4 w = P.heads[2 * it];
+        R.i = w.x; R.b = w.y; R.e0 = w.z; R.npairs = w.w;
+        R.j0 = P.heads[2 * it + 1].x;
+    } else {
+        R.i = P.order ? P.order[it] : it;
+        R.b = (int)P.batch[R.i];
+    }
     R.a = P.a_ih[(size_t)R.i * P.H + h];
     float rvl1 = 0.f, rvl2 = 0.f, rvl3 = 0.f;
     if (P.rvlen) { rvl1 = P.rvlen[(size_t)R.b * 3 + 0]; rvl2 = P.rvlen[(size_t)R.b * 3 + 1]; rvl3 = P.rvlen[(size_t)R.b * 3 + 2]; }
     R.bx = translation_box(R.a, rvl1, rvl2, rvl3, P.cutoff_radius, P.lattice_range, P.minimum_range);
     if (R.bx.over && P.status) atomicOr(P.status, 1);
     R.boxw = (uint32_t)(R.bx.R1 | (R.bx.R2 << 8) | (R.bx.R3 << 16));
+    if (P.heads) {
+        // (sizes that do not add up to the atoms and pairs of the batch: no pairs, and the status word says so)
+        if (R.e0 < 0 || R.npairs < 0 || R.npairs > P.E - R.e0 || R.j0 < 0 || R.npairs > P.N - R.j0) {
+            if (P.status) atomicOr(P.status, 2);
+            R.e0 = R.npairs = 0;
+            R.j0 = R.i;
+        }
+        return R;
+    }
     R.e0 = (int)P.e_start[R.i];
     R.npairs = (int)P.e_start[R.i + 1] - R.e0;
     R.j0 = R.npairs > 0 ? (int)P.edges[(size_t)P.E + R.e0] : R.i;      // first neighbour atom
@@ -544,13 +560,16 @@ __device__ __forceinline__ RecordHead record_head(const KernelArgs& P, int it, i
 // The record of an item made by the wavefront that needs it: the word of this lane.
 __device__ __forceinline__ uint32_t make_record_lane(const KernelArgs& P, int it, int h, int lane, bool with_query) {
     const RecordHead R = record_head(P, it, h);
-    if (lane >= REC_LATTICE && lane < REC_LATTICE + 9) return __float_as_uint(P.tvecs[(size_t)R.b * 9 + (lane - REC_LATTICE)]);
-    if (with_query && lane >= REC_QUERY && lane < REC_QUERY + DH)
-        return __float_as_uint(P.q[((size_t)R.i * P.H + h) * DH + (lane - REC_QUERY)]);
-    if (!with_query && P.frames && lane >= REC_FRAMES && lane < REC_FRAMES + 9) {
-        const int c = lane - REC_FRAMES, ax = c / 3, d = c - 3 * ax;
-        return __float_as_uint(P.frames[(((size_t)ax * P.N + R.i) * P.H + h) * 3 + d]);
-    }
+    // (one load for the lattice rows and the query or frames, each lane its own: no load behind a branch)
+    const bool lattice = lane >= REC_LATTICE && lane < REC_LATTICE + 9;
+    const bool query = with_query && lane >= REC_QUERY && lane < REC_QUERY + DH;
+    const bool frame = !with_query && P.frames && lane >= REC_FRAMES && lane < REC_FRAMES + 9;
+    const int c = lane - REC_FRAMES, ax = c / 3, d = c - 3 * ax;
+    const float* src = P.tvecs + (size_t)R.b * 9 + (lattice ? lane - REC_LATTICE : 0);
+    if (query) src = P.q + ((size_t)R.i * P.H + h) * DH + (lane - REC_QUERY);
+    if (frame) src = P.frames + (((size_t)ax * P.N + R.i) * P.H + h) * 3 + d;
+    const uint32_t word = __float_as_uint(*src);
+    if (lattice || query || frame) return word;
     return lane == REC_ATOM ? (uint32_t)R.i : lane == REC_E0 ? (uint32_t)R.e0 : lane == REC_NPAIRS ? (uint32_t)R.npairs
          : lane == REC_BOX ? R.boxw : lane == REC_A ? __float_as_uint(R.a) : lane == 30 ? (uint32_t)R.j0
          : lane == 31 ? (uint32_t)R.b : 0u;

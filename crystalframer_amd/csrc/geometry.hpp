@@ -23,6 +23,7 @@ struct GeometryArgs {
     int64_t* atom_start;       // (B + 1) scratch / output: first atom of each crystal
     int64_t* pair_start;       // (B + 1) scratch: first pair of each crystal
     int64_t* order_start;      // (B) scratch: first position of each crystal's atoms in `order`
+    int4* heads;               // (N, 2) or null: in work order, atom, crystal, first pair, pairs, first neighbour
     int32_t N, B;
     int64_t E;
 };
@@ -168,8 +169,13 @@ __device__ __forceinline__ void geometry_atom(const GeometryArgs& P, int i) {
     const int b = (int)P.batch[i];
     const long long n = (long long)P.sizes[b];
     const long long local = (long long)i - P.atom_start[b];
-    P.e_start[i] = P.pair_start[b] + local * n;
-    P.order[P.order_start[b] + local] = i;
+    const long long e0 = P.pair_start[b] + local * n, at = P.order_start[b] + local;
+    P.e_start[i] = e0;
+    P.order[at] = i;
+    if (P.heads) {
+        P.heads[2 * at] = make_int4(i, b, (int)e0, (int)n);
+        P.heads[2 * at + 1] = make_int4((int)((long long)i - local), 0, 0, 0);
+    }
 }
 
 __global__ __launch_bounds__(256) void geometry_atoms_kernel(const GeometryArgs P) {

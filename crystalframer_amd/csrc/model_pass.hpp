@@ -17,6 +17,7 @@ constexpr int MODEL_MAX_LAYERS = 64;
 struct ModelBuffers {
     int64_t *edges, *e_start, *atom_start;
     int32_t* order;
+    int4* heads;
     float *rpos, *recip, *rvlen, *vcell, *near_, *x0, *pooled;
     float4* table;
     char* geo_ws;
@@ -93,6 +94,7 @@ void model_buffers(const cfh_model* m, const cfh_model_batch* b, ModelBuffers& M
     M.e_start = c.take<int64_t>(N + 1);
     M.atom_start = c.take<int64_t>(B + 1);
     M.order = c.take<int32_t>(N);
+    M.heads = c.take<int4>(2 * N);
     M.rpos = c.take<float>(3 * E);
     M.recip = c.take<float>(9 * B);
     M.rvlen = c.take<float>(3 * B);
@@ -332,7 +334,7 @@ int cfh_model_forward(const cfh_model* m, const cfh_model_batch* b, float* out) 
         cfh::GeometryArgs& g = A.geo;
         g.pos = b->pos; g.batch = b->batch; g.tvecs = b->tvecs; g.sizes = b->sizes;
         g.edges = M.edges; g.rpos = M.rpos; g.recip = M.recip; g.rvlen = M.rvlen; g.vcell = M.vcell;
-        g.e_start = M.e_start; g.order = M.order; g.atom_start = M.atom_start;
+        g.e_start = M.e_start; g.order = M.order; g.heads = M.heads; g.atom_start = M.atom_start;
         g.pair_start = reinterpret_cast<int64_t*>(M.geo_ws);
         g.order_start = g.pair_start + (B + 1);
         g.N = (int32_t)N; g.B = (int32_t)B; g.E = E;
@@ -412,7 +414,7 @@ int cfh_model_forward(const cfh_model* m, const cfh_model_batch* b, float* out) 
                                          M.edges, M.e_start, M.order, L.W_dist, ang ? L.W_axis1 : nullptr,
                                          ang ? L.W_axis2 : nullptr, ang ? L.W_axis3 : nullptr, N, E, B,
                                          ang ? Y.frames : nullptr, ang ? 1 : 0, Y.z, Y.prob, Y.hist, Y.out, &cache,
-                                         b->workspace, b->workspace_bytes, b->stream, !b->keep, true)))
+                                         b->workspace, b->workspace_bytes, b->stream, !b->keep, true, M.heads)))
             return rc;
         const bool next = l + 1 < m->layers;
         const cfh_model_layer& Ln = m->layer[next ? l + 1 : l];
