@@ -62,12 +62,21 @@ __device__ __forceinline__ void split_stream_element(const BridgeStreams& T, int
         } else { s -= head + chunks; W = S.Wq; t = 8 * (s / du) + w; u = s % du; }
     }
     const int n = 16 * t + col, k = 32 * u + 8 * kk;
+    // (rows of 16-byte aligned matrices four numbers at a time; the features' are seldom a multiple of four)
+    float v[8];
+    const float* const row = W + (size_t)n * ld + k;
+    if (valid == 0x7fffffff && (ld & 3) == 0 && ((uintptr_t)W & 15) == 0) {
+        const float4 v0 = *reinterpret_cast<const float4*>(row), v1 = *reinterpret_cast<const float4*>(row + 4);
+        v[0] = v0.x; v[1] = v0.y; v[2] = v0.z; v[3] = v0.w; v[4] = v1.x; v[5] = v1.y; v[6] = v1.z; v[7] = v1.w;
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] = k + i < valid ? row[i] : 0.0f;
+    }
     v8bf p[3];
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-        const float v = k + i < valid ? W[(size_t)n * ld + k + i] : 0.0f;
         __bf16 a, b, c;
-        split_bf16(v, a, b, c);
+        split_bf16(v[i], a, b, c);
         p[0][i] = a; p[1][i] = b; p[2][i] = c;
     }
     v8bf* const dst = reinterpret_cast<v8bf*>(S.dst) + (size_t)(w * S.steps + step) * 192 + lane;
