@@ -408,9 +408,24 @@ __global__ __launch_bounds__(64 * BR_WAVES) void front_infer_kernel(const Bridge
     const int parts = gridDim.y == 1 ? 3 : 1, part = blockIdx.y, g0 = CT * eg + part * CT * CT;
     SplitStream ws;
     ws.start(P.stream, P.steps, 0);
-    for (int idx = threadIdx.x; idx < R * pad; idx += 64 * BR_WAVES) {
-        const int m = idx / pad, c = idx - m * pad;
-        split_store(s_f + m * ldf + c, R * ldf, m < nrows && c < feat ? P.attn[(size_t)(r0 + m) * feat + c] : 0.0f);
+    // (a wavefront's rows of 128 features with all loads in flight: one by one 22 528 rows 34 us for the launch instead of 29, 8 rows 6.5 and 5.8)
+    constexpr int ROWS = R / BR_WAVES;
+    for (int c0 = 0; c0 < pad; c0 += 128) {
+        float v[ROWS][2];
+#pragma unroll
+        for (int r = 0; r < ROWS; r++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const int m = wave + BR_WAVES * r, c = c0 + 64 * j + lane;
+                v[r][j] = P.attn[(size_t)(r0 + min(m, nrows - 1)) * feat + min(c, feat - 1)];
+            }
+#pragma unroll
+        for (int r = 0; r < ROWS; r++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const int m = wave + BR_WAVES * r, c = c0 + 64 * j + lane;
+                split_store(s_f + m * ldf + c, R * ldf, m < nrows && c < feat ? v[r][j] : 0.0f);
+            }
     }
     __syncthreads();
 #pragma unroll
