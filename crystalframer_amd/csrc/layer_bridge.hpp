@@ -150,13 +150,22 @@ template <int TR, bool FOLD>
 __device__ __forceinline__ void bridge_steps(WeightStream& ws, int next, const float* arow, int lda, v4f_b2 (&acc)[TR],
                                              v4f_b2 (&sum)[TR], int klen, int& in_slice, bool& first) {
     const v4f_b2* const p = ws.group(next);
+    v4f_b2 an[TR];
+#pragma unroll
+    for (int tr = 0; tr < TR; tr++) an[tr] = *reinterpret_cast<const v4f_b2*>(arow + 16 * tr * lda);
 #pragma unroll
     for (int u = 0; u < BR_RING; u++) {
         const v4f_b2 w = ws.r[u];
         ws.r[u] = p[u * 64];
         v4f_b2 a[TR];
 #pragma unroll
-        for (int tr = 0; tr < TR; tr++) a[tr] = *reinterpret_cast<const v4f_b2*>(arow + 16 * tr * lda + 16 * u);
+        for (int tr = 0; tr < TR; tr++) {
+            a[tr] = an[tr];
+            if (u + 1 < BR_RING) an[tr] = *reinterpret_cast<const v4f_b2*>(arow + 16 * tr * lda + 16 * (u + 1));
+        }
+        // (said so, or the compiler puts the eight loads of the next group behind the products of this one, and every step's
+        // rows right in front of its products: 2372 rows 21.8 -> 20.4 us forward, 25.1 -> 24.6 backward)
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int j = 0; j < 4; j++)
 #pragma unroll
