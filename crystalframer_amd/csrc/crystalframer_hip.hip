@@ -1672,11 +1672,13 @@ constexpr int64_t ITEM_PASS_MAX = 5120;
 // instead of once per 16.  Whole calls of four layers in us, with a launch for the products and without: 64 bins, 64 items 158
 // and 142, 600 items 207 and 189, 1208 items 191 and 173, 2416 items 210 and 187, 4872 items 320 and 250; so the one launch pays
 // for more items: against several launches 6488 items 346 and 291, 7712 items 333 and 314, 9216 items 294 and 275, 10 696 items
-// 369 and 364, 11 440 items 359 and 373.  Of fewer words the launch is short: 16 bins,
-// 576 items 173 and 154; distances alone, 1152 items 129 and 126, 4608 items 142 and 154.
-constexpr int64_t ITEM_PROJECT_FEW_WORDS = 1536, ITEM_PROJECT_MAX = 10240;
+// 369 and 364, 11 440 items 359 and 373.  16 bins: 2304 items 171 and 160, 5056 items 199 and 192; 6496 items 257 (several
+// launches) and 231, 10 696 items 382 and 378, 12 256 items 317 and 324.  Distances alone, where the wavefronts are lighter: 1152
+// items 119 and 109, 4608 items 133 and 123; 9216 items 173 (several) and 159, 12 256 items 201 and 191, 18 432 items 237 and
+// 238, 36 864 items 400 and 434.
+constexpr int64_t ITEM_PROJECT_MAX = 10240, ITEM_PROJECT_MAX_DISTANCE = 16384;
 bool item_project(const cfh_params* p, int64_t items) {
-    return items <= (p->angle_bins == cfh::NBINS ? ITEM_PROJECT_MAX : ITEM_PROJECT_FEW_WORDS);
+    return items <= (p->angle_bins > 0 ? ITEM_PROJECT_MAX : ITEM_PROJECT_MAX_DISTANCE);
 }
 template <typename Kern>
 int launch_item_pass(Kern kern, const cfh::CoreArgs& C, bool search, const float* wcat, hipStream_t st, const char* what) {

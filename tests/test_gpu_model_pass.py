@@ -521,9 +521,9 @@ def test_bridges_of_inference(D, F, N, feat):
 
 
 # Inference of few items: the product of an item's histogram with the weights by its own wavefront.  One atom, a few, either side
-# of the item counts where a launch of its own makes it (10 240 with the 64-bin encoding, 1536 without).
+# of the item counts where a launch of its own makes it (10 240 with an angle encoding, 16 384 without).
 @pytest.mark.parametrize("bins,B,atoms", [(64, 1, 1), (64, 3, 7), (64, 64, 10), (64, 1280, 1), (64, 1281, 1), (16, 1, 1), (16, 24, 8),
-                                          (16, 193, 1), (0, 1, 1), (0, 24, 8), (0, 193, 1)])
+                                          (16, 1280, 1), (16, 1281, 1), (0, 1, 1), (0, 24, 8), (0, 2048, 1), (0, 2049, 1)])
 def test_products_of_few_items(bins, B, atoms):
     """Against the same pass with everything kept, whose products have a launch of their own: two sums of 720 float32 products
     (of a 64-bin pass: around other nodes, 1.4e-6 of the basis' peak, a few 1e-6 of a layer's output)."""
