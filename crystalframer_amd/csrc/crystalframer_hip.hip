@@ -1664,9 +1664,14 @@ void project_launch(int hw, const float* hist, const float* wcat, float* out, in
 }
 // Up to this many (atom, head) items the forward pass of a layer is one wavefront per item from the record to the sums: about
 // as many as are resident at once (19 to 23 per compute unit).  Measured with and without, whole calls: 976 items 274 and 256
-// us, 4592 items 412 and 380, 7712 items 446 and 415, 10 696 items 398 and 441; cells of 40 to 200 atoms lose from 5760 items
-// on (386 and 397), where the frame search of four heads per wavefront counts for more than the launch it takes.
-constexpr int64_t ITEM_PASS_MAX = 5120;
+// us, 4592 items 412 and 380, 7712 items 446 and 415, 10 696 items 398 and 441.  Short rows (a mean of at most 24 pairs) gain
+// beyond, where a wavefront that ends makes room soon: training steps of 5328 items 715 and 697 us, 6488 items 873 and 842, but
+// 7712 items 759 and 772; distances alone 6488 items 654 and 636, 9168 items 719 and 702.  Cells of 40 to 200 atoms lose from 5760
+// items on (384 and 392; 6720 items 404 and 418), distances alone too (8640 items 345 and 353).
+constexpr int64_t ITEM_PASS_MAX = 5120, ITEM_PASS_MAX_SHORT = 7168, ITEM_PASS_MAX_DISTANCE = 10240, SHORT_ROW = 24;
+int64_t item_pass_max(const cfh_params* p, int64_t N, int64_t E) {
+    return E > SHORT_ROW * N ? ITEM_PASS_MAX : (p->angle_bins > 0 ? ITEM_PASS_MAX_SHORT : ITEM_PASS_MAX_DISTANCE);
+}
 // Inference, where the histogram serves the projection alone: the wavefront of such an item makes the product with the head's
 // weights itself, which saves a launch and a round trip of the histogram but reads the weights (46 KB at 64 bins) once per item
 // instead of once per 16.  Whole calls of four layers in us, with a launch for the products and without: 64 bins, 64 items 158
@@ -1677,8 +1682,8 @@ constexpr int64_t ITEM_PASS_MAX = 5120;
 // items 119 and 109, 4608 items 133 and 123; 9216 items 173 (several) and 159, 12 256 items 201 and 191, 18 432 items 237 and
 // 238, 36 864 items 400 and 434.
 constexpr int64_t ITEM_PROJECT_MAX = 10240, ITEM_PROJECT_MAX_DISTANCE = 16384;
-bool item_project(const cfh_params* p, int64_t items) {
-    return items <= (p->angle_bins > 0 ? ITEM_PROJECT_MAX : ITEM_PROJECT_MAX_DISTANCE);
+bool item_project(const cfh_params* p, int64_t N, int64_t E) {
+    return N * p->num_heads <= (E > SHORT_ROW * N ? ITEM_PASS_MAX : (p->angle_bins > 0 ? ITEM_PROJECT_MAX : ITEM_PROJECT_MAX_DISTANCE));
 }
 template <typename Kern>
 int launch_item_pass(Kern kern, const cfh::CoreArgs& C, bool search, const float* wcat, hipStream_t st, const char* what) {
@@ -1745,8 +1750,8 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
     const cfh::WcatArgs WA{W_dist, W_axis1, W_axis2, W_axis3, hw, p->dist_coef, p->angle_coef,
                            p->angle_wscale, wcat};
     // (the word of the noise's seed is copied and advanced by the launch that makes the records)
-    const bool project_by_item = lean && item_project(p, N * p->num_heads);
-    const bool one_launch = (N * p->num_heads <= ITEM_PASS_MAX || project_by_item) && !(search && p->symm_break_noise > 0.0f && C.K.seed_dev);
+    const bool project_by_item = lean && item_project(p, N, E);
+    const bool one_launch = (N * p->num_heads <= item_pass_max(p, N, E) || project_by_item) && !(search && p->symm_break_noise > 0.0f && C.K.seed_dev);
     if (one_launch) {
         if (!wcat_made) {
             TimedScope timed("core_prepare", st);

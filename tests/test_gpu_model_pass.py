@@ -538,3 +538,25 @@ def test_products_of_few_items(bins, B, atoms):
     with torch.no_grad():
         out = model(cb)
     assert Hh.rel_err(out, kept.double()) < 5e-6
+
+
+# Either side of the item counts up to which a layer's items take one launch: 7168 with an angle encoding, 10 240 without (crystals
+# of 8 atoms), and 5120 for rows of more than 24 pairs on average (crystals of 25); inference, with the product: 10 240 and 16 384.
+@pytest.mark.parametrize("bins,atoms,B", [(64, 8, 112), (16, 8, 112), (0, 8, 160), (64, 25, 25), (0, 25, 25), (64, 24, 37), (64, 8, 160),
+                                          (0, 8, 256)])
+def test_item_counts_of_one_launch(bins, atoms, B):
+    """The crystals of a batch are answered alike in a batch of one more (no frame changes: the same operations per item, sums of
+    the layers' rows in other tiles)."""
+    from crystalframer_amd import params, synthetic
+    kw = dict(value_pe_angle_wscale=1.0, value_pe_dist_coef=1.5, value_pe_angle_coef=6.0) if bins == 16 else {}
+    mp = params.ModelParams(num_layers=1, value_pe_angle_real=bins, symm_break_noise=0.0, **kw)
+    cb = synthetic.make_batch(B + 1, atoms="uniform", atoms_lo=atoms, atoms_hi=atoms, len_lo=4.0, len_hi=9.0, ang_lo=65.0, ang_hi=115.0,
+                              seed=B)
+    n = atoms * B
+    less = synthetic.CrystalBatch(cb.x[:n], cb.pos[:n], cb.batch[:n], cb.trans_vec[:B], cb.sizes[:B], zero_based=True)
+    model, less = _model(mp, less)
+    more = cb.to("cuda")
+    a, b = model(less), model(more)
+    assert Hh.rel_err(b[:B], a.double()) < 1e-6
+    with torch.no_grad():
+        assert Hh.rel_err(model(more)[:B], model(less).double()) < 2e-6
