@@ -2,7 +2,8 @@
 // its products on the bfloat16 matrix instructions at float32 precision.
 //
 // A float32 number is the sum of three bfloat16 numbers to 2^-27 of itself (eight bits each, what is left rounded to
-// nearest again), so a product of two of them is nine bfloat16 products, of which the three smallest (a1 b2, a2 b1, a2 b2:
+// nearest again; from 2^-99 on, below which the third part is no normal number any more and 2^-126 takes the place of
+// 2^-27 of itself), so a product of two of them is nine bfloat16 products, of which the three smallest (a1 b2, a2 b1, a2 b2:
 // below 2^-25 of it) are left out.  The six others, exact in float32, go through v_mfma_f32_16x16x32_bf16 into ONE float32
 // accumulator, the small ones first: six roundings of the sum per 32 products where v_mfma_f32_16x16x4_f32 makes eight.
 // Error of the atoms' outputs against float64 (distance-only models, batches of 24 to 300 crystals, 2-norm): 1.3 to 1.4e-7
@@ -32,8 +33,11 @@ constexpr int BI_ROW = BR_CHUNK + BI_PAD;
 __host__ __device__ inline int split_stream_steps(int kind, int D, int F, bool next, int feat = 0) {
     return bridge_stream_steps(kind, D, F, next, feat) / 2;
 }
+// (the first part stays below the largest bfloat16 number, so that no finite number gets an infinite part; an infinity leaves
+// an infinite second and a NaN as the third, and every sum with it is a NaN)
+constexpr float BF16_LARGEST = 3.3895313892515355e38f;
 __device__ __forceinline__ void split_bf16(float v, __bf16& a, __bf16& b, __bf16& c) {
-    a = (__bf16)v;
+    a = (__bf16)__builtin_amdgcn_fmed3f(v, -BF16_LARGEST, BF16_LARGEST);
     const float r = v - (float)a;
     b = (__bf16)r;
     c = (__bf16)(r - (float)b);
@@ -205,7 +209,7 @@ __device__ __forceinline__ void split_hidden_chunk(const BridgeArgs& P, SplitStr
 #pragma unroll
     for (int tr = 0; tr < TR; tr++)
 #pragma unroll
-        for (int c = 0; c < 4; c++) fn(16 * tr + 4 * kk + c, 16 * wave + col, fmaxf(acc[tr][c] + bias, 0.0f));
+        for (int c = 0; c < 4; c++) fn(16 * tr + 4 * kk + c, 16 * wave + col, rectified(acc[tr][c] + bias));
 }
 // x2 = sums + bias + x1 into the planes s_x and, with `store`, memory.
 template <int TR, int CT>

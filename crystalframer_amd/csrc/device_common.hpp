@@ -118,6 +118,10 @@ __device__ __forceinline__ float rows_min(float x) {
 __device__ __forceinline__ float wave_sum(float v) { return rows_sum(row_sum(v)); }
 __device__ __forceinline__ float wave_min(float v) { return rows_min(row_min(v)); }
 
+// The rectifier of a projection's output.  A NaN stays one, as in torch's (fmaxf makes 0 of it, and what a weight gone wrong does
+// to the output would not show).
+__device__ __forceinline__ float rectified(float v) { return v < 0.0f ? 0.0f : v; }
+
 // Ordering point between the lanes of a ONE-wavefront workgroup that communicate through LDS.  The
 // LDS executes a wavefront's instructions in order, so no hardware barrier and no wait for
 // outstanding global stores is needed -- only the compiler must not move LDS accesses across.

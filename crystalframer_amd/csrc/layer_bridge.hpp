@@ -348,7 +348,7 @@ __device__ __forceinline__ void bridge_hidden_chunk(const BridgeArgs& P, WeightS
 #pragma unroll
         for (int c = 0; c < 4; c++) {
             const int m = 16 * tr + 4 * kk + c;
-            const float val = fmaxf(acc[tr][c] + bias, 0.0f);
+            const float val = rectified(acc[tr][c] + bias);
             if (hb) hb[m * ldh + 16 * wave + col] = val;
             if (P.h && m < nrows) P.h[(size_t)(r0 + m) * P.F + n] = val;
         }

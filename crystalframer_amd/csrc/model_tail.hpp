@@ -100,7 +100,7 @@ __global__ __launch_bounds__(64 * TAIL_WAVES) void model_tail_fwd_kernel(const T
             for (int c = 0; c < 4; c++) {
                 const int m = 4 * kk + c;
                 float val = acc[c] + bias;
-                if (T.relu) val = fmaxf(val, 0.0f);
+                if (T.relu) val = rectified(val);
                 if (n < O) {
                     outb[m * ld + n] = val;
                     if (m < nrows) T.y[(size_t)(b0 + m) * O + n] = val;

@@ -57,7 +57,7 @@ __global__ __launch_bounds__(256) void small_linear_fwd_kernel(const float* __re
     // accumulator component c of lane (kk, col): row 4 kk + c of the 16x16 block, column col
     const float ba = b ? b[ca] : 0.f, bb = b ? b[cb] : 0.f;
     auto put = [&](int r, int n, float v) {
-        if (r < M && n < N) y[(size_t)r * N + n] = relu ? fmaxf(v, 0.f) : v;
+        if (r < M && n < N) y[(size_t)r * N + n] = relu ? rectified(v) : v;
     };
 #pragma unroll
     for (int c = 0; c < 4; c++) {

@@ -520,6 +520,62 @@ def test_bridges_of_inference(D, F, N, feat):
     assert Hh.rel_err(out[0][some], ref) < limit
 
 
+def _one_layer_of_atoms(N, D=128, **kw):
+    """N crystals of one atom, one layer, distances alone (nothing that the weights behind the core hold reaches a lattice kernel),
+    and a head that passes on the atoms' outputs, those that the rectifier lets through."""
+    from crystalframer_amd import params, synthetic
+    mp = params.ModelParams(num_layers=1, symm_break_noise=0.0, value_pe_angle_real=0, model_dim=D, head_num=D // 16, **kw)
+    cb = synthetic.make_batch(N, atoms="uniform", atoms_lo=1, atoms_hi=1, len_lo=3.0, len_hi=6.0, ang_lo=70.0, ang_hi=110.0, seed=N)
+
+    def outputs_of_atoms(model):
+        for i in (0, 3):
+            model.mlp[i] = torch.nn.Linear(D, D).cuda()
+            with torch.no_grad():
+                model.mlp[i].weight.copy_(torch.eye(D))
+                model.mlp[i].bias.zero_()
+
+    return _model(mp, cb, change=outputs_of_atoms)
+
+
+# The bridges of inference and of training in their forms: two launches, one, 32 rows per workgroup
+@pytest.mark.parametrize("N", [33, 2065, 4129])
+@pytest.mark.parametrize("where,value", [("linear1", float("inf")), ("linear1", float("nan")), ("linear2", float("-inf")),
+                                         ("linear2", float("nan")), ("out_proj", float("inf"))])
+def test_weights_that_are_no_numbers_show(N, where, value):
+    """Where a pass that keeps everything gives no finite number, inference gives none either (an infinity may become a NaN there,
+    also one that the rectifier takes away in the other)."""
+    model, cb = _one_layer_of_atoms(N)
+    layer = model.encoder.layers[0]
+    with torch.no_grad():
+        (layer.self_attn if where == "out_proj" else layer).get_submodule(where).weight[3, 5] = value
+    kept = model(cb).detach()
+    model.eval()
+    with torch.no_grad():
+        out = model(cb)
+    lost = ~torch.isfinite(kept)
+    assert lost.any() and not torch.isfinite(out[lost]).any()
+    if value != value and where == "linear1":
+        assert lost.all()
+
+
+@pytest.mark.parametrize("N", [33, 2065, 4129])
+def test_largest_weights(N):
+    """A weight that rounds to an infinite bfloat16 number, times a feature that makes a product of ordinary size of it."""
+    model, cb = _one_layer_of_atoms(N)
+    layer = model.encoder.layers[0]
+    with torch.no_grad():
+        model.input_embeddings.weight[5] = 2.0 ** -126
+        layer.self_attn.out_proj.weight[5] = 0.0
+        layer.self_attn.out_proj.bias[5] = 0.0
+        layer.linear1.weight[:, 5] = 0.0
+        layer.linear1.weight[3, 5] = 3.402e38           # (4 of every atom's third inner feature)
+    kept = model(cb).detach()
+    model.eval()
+    with torch.no_grad():
+        out = model(cb)
+    assert torch.isfinite(kept).all() and Hh.rel_err(out, kept.double()) < 2e-6      # (sums of up to 512 products)
+
+
 # Inference of few items: the product of an item's histogram with the weights by its own wavefront.  One atom, a few, either side
 # of the item counts where a launch of its own makes it (10 240 with an angle encoding, 16 384 without).
 @pytest.mark.parametrize("bins,B,atoms", [(64, 1, 1), (64, 3, 7), (64, 64, 10), (64, 1280, 1), (64, 1281, 1), (16, 1, 1), (16, 24, 8),
