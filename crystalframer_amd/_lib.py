@@ -365,7 +365,7 @@ def read_stats(device: torch.device, reset: bool = False) -> dict:
 def read_status(device: torch.device, reset: bool = False) -> int:
     """Status word of this stream's workspace (synchronises): 1 when a launch had to cut a translation box
     back to the largest half-width the kernels sum (32), i.e. where the result differs from the reference's
-    box rule; 0 otherwise."""
+    box rule; 2 when the fused core found pairs that are not whole blocks (or fewer than the sizes say); 0 otherwise."""
     buf = workspace(device, 512)
     val = int(buf[16:20].view(torch.int32).cpu()[0])
     if reset:

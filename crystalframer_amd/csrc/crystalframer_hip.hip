@@ -1833,40 +1833,15 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
     return finish_launch("fused_core_project");
 }
 
-}  // namespace
-
-extern "C" {
-
-size_t cfh_fused_core_workspace_bytes(const cfh_params* p, int64_t N, int64_t E, int64_t B, int32_t backward) {
-    if (check_core_params(p) != CFH_OK) return 0;
-    return core_layout(p, N, E, B, backward != 0).total;
-}
-
-int32_t cfh_fused_core_hist_words(const cfh_params* p) {
-    if (check_core_params(p) != CFH_OK) return 0;
-    return cfh::core_hist_words(p->angle_bins);
-}
-
-int cfh_fused_core_forward(const cfh_params* p, const float* qs, const float* k, const float* v, const float* a_ih,
-                           const float* rpos, const float* tvecs, const float* rvlen, const int64_t* batch,
-                           const int64_t* edges, const int64_t* e_start, const int32_t* order, const float* W_dist,
-                           const float* W_axis1, const float* W_axis2, const float* W_axis3, int64_t N, int64_t E,
-                           int64_t B, float* frames, int32_t search_frames, float* z, float* prob, float* hist,
-                           float* out, const cfh_core_cache* cache, void* workspace, size_t workspace_bytes,
-                           void* stream) {
-    return fused_core_forward_impl(p, qs, k, v, a_ih, rpos, tvecs, rvlen, batch, edges, e_start, order, W_dist, W_axis1, W_axis2,
-                                   W_axis3, N, E, B, frames, search_frames, z, prob, hist, out, cache, workspace,
-                                   workspace_bytes, stream, false, false);
-}
-
-int cfh_fused_core_backward(const cfh_params* p, const float* qs, const float* k, const float* v, const float* a_ih,
-                            const float* rpos, const float* tvecs, const float* rvlen, const int64_t* batch,
-                            const int64_t* edges, const int64_t* e_start, const int32_t* order, const float* W_dist,
-                            const float* W_axis1, const float* W_axis2, const float* W_axis3, const float* frames,
-                            const float* z, const float* prob, const float* hist, const float* out, const float* gout,
-                            int64_t N, int64_t E, int64_t B, float* gq, float* gk, float* gv, float* ga, float* glogit,
-                            float* gW_dist, float* gW_axis1, float* gW_axis2, float* gW_axis3,
-                            const cfh_core_cache* cache, void* workspace, size_t workspace_bytes, void* stream) {
+// own_pairs: the pairs are those that the library made itself, whole blocks.
+int fused_core_backward_impl(const cfh_params* p, const float* qs, const float* k, const float* v, const float* a_ih,
+                             const float* rpos, const float* tvecs, const float* rvlen, const int64_t* batch,
+                             const int64_t* edges, const int64_t* e_start, const int32_t* order, const float* W_dist,
+                             const float* W_axis1, const float* W_axis2, const float* W_axis3, const float* frames,
+                             const float* z, const float* prob, const float* hist, const float* out, const float* gout,
+                             int64_t N, int64_t E, int64_t B, float* gq, float* gk, float* gv, float* ga, float* glogit,
+                             float* gW_dist, float* gW_axis1, float* gW_axis2, float* gW_axis3,
+                             const cfh_core_cache* cache, void* workspace, size_t workspace_bytes, void* stream, bool own_pairs) {
     int rc = check_core_params(p);
     if (rc) return rc;
     if ((rc = check_geometry(a_ih, rpos, tvecs, batch, edges, e_start, N, E, B))) return rc;
@@ -1990,6 +1965,8 @@ int cfh_fused_core_backward(const cfh_params* p, const float* qs, const float* k
         A.prob = const_cast<float*>(prob); A.go = gout; A.gk = gk; A.gv = gv; A.gaij = glogit;
         A.N = (int32_t)N; A.H = p->num_heads; A.E = (int32_t)E;
         A.items = C.K.items;
+        A.status = C.K.status;
+        if (own_pairs) A.e_start = nullptr;
         const int64_t items = N * p->num_heads;
         {
             TimedScope timed("core_bwd_col", st);
@@ -2007,6 +1984,45 @@ int cfh_fused_core_backward(const cfh_params* p, const float* qs, const float* k
     return rc ? rc : rc_w;
 }
 
+}  // namespace
+
+extern "C" {
+
+size_t cfh_fused_core_workspace_bytes(const cfh_params* p, int64_t N, int64_t E, int64_t B, int32_t backward) {
+    if (check_core_params(p) != CFH_OK) return 0;
+    return core_layout(p, N, E, B, backward != 0).total;
+}
+
+int32_t cfh_fused_core_hist_words(const cfh_params* p) {
+    if (check_core_params(p) != CFH_OK) return 0;
+    return cfh::core_hist_words(p->angle_bins);
+}
+
+int cfh_fused_core_forward(const cfh_params* p, const float* qs, const float* k, const float* v, const float* a_ih,
+                           const float* rpos, const float* tvecs, const float* rvlen, const int64_t* batch,
+                           const int64_t* edges, const int64_t* e_start, const int32_t* order, const float* W_dist,
+                           const float* W_axis1, const float* W_axis2, const float* W_axis3, int64_t N, int64_t E,
+                           int64_t B, float* frames, int32_t search_frames, float* z, float* prob, float* hist,
+                           float* out, const cfh_core_cache* cache, void* workspace, size_t workspace_bytes,
+                           void* stream) {
+    return fused_core_forward_impl(p, qs, k, v, a_ih, rpos, tvecs, rvlen, batch, edges, e_start, order, W_dist, W_axis1, W_axis2,
+                                   W_axis3, N, E, B, frames, search_frames, z, prob, hist, out, cache, workspace,
+                                   workspace_bytes, stream, false, false);
+}
+
+int cfh_fused_core_backward(const cfh_params* p, const float* qs, const float* k, const float* v, const float* a_ih,
+                            const float* rpos, const float* tvecs, const float* rvlen, const int64_t* batch,
+                            const int64_t* edges, const int64_t* e_start, const int32_t* order, const float* W_dist,
+                            const float* W_axis1, const float* W_axis2, const float* W_axis3, const float* frames,
+                            const float* z, const float* prob, const float* hist, const float* out, const float* gout,
+                            int64_t N, int64_t E, int64_t B, float* gq, float* gk, float* gv, float* ga, float* glogit,
+                            float* gW_dist, float* gW_axis1, float* gW_axis2, float* gW_axis3,
+                            const cfh_core_cache* cache, void* workspace, size_t workspace_bytes, void* stream) {
+    return fused_core_backward_impl(p, qs, k, v, a_ih, rpos, tvecs, rvlen, batch, edges, e_start, order, W_dist,
+                                    W_axis1, W_axis2, W_axis3, frames, z, prob, hist, out, gout, N, E, B, gq, gk,
+                                    gv, ga, glogit, gW_dist, gW_axis1, gW_axis2, gW_axis3, cache, workspace,
+                                    workspace_bytes, stream, false);
+}
 
 size_t cfh_fused_core_weight_gradients_workspace_bytes(const cfh_params* p, int32_t njobs) {
     if (check_core_params(p) != CFH_OK || njobs < 0) return 0;

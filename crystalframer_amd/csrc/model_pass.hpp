@@ -495,12 +495,12 @@ int cfh_model_backward(const cfh_model* m, const cfh_model_batch* b, const float
         if (R > 0) held = R;
         const cfh_core_cache cache{reinterpret_cast<float*>(M.table), nullptr, Y.wcat, Y.records, table_ready ? 1 : 0, 1, 1, 0};
         const bool ang = p.angle_bins > 0;
-        if ((rc = cfh_fused_core_backward(&p, Y.qs, Y.k, Y.v, Y.a, M.rpos, b->tvecs, L.adaptive ? M.rvlen : nullptr, b->batch,
+        if ((rc = fused_core_backward_impl(&p, Y.qs, Y.k, Y.v, Y.a, M.rpos, b->tvecs, L.adaptive ? M.rvlen : nullptr, b->batch,
                                           M.edges, M.e_start, M.order, L.W_dist, ang ? L.W_axis1 : nullptr,
                                           ang ? L.W_axis2 : nullptr, ang ? L.W_axis3 : nullptr, ang ? Y.frames : nullptr, Y.z,
                                           Y.prob, Y.hist, Y.out, G.layer[l].g_attn, N, E, B, G.gq, G.gk, G.gv, G.ga, G.glogit,
                                           nullptr, nullptr, nullptr, nullptr, &cache, b->workspace, b->workspace_bytes,
-                                          b->stream)))
+                                          b->stream, true)))
             return rc;
     }
     {   // the inputs of the first layer: gradient of its projection, of the embedded atoms (projection + residual)

@@ -586,6 +586,52 @@ def test_column_sums_by_groups_of_columns(atoms, crystals):
         assert Hh.rel_err(l32.grad.cpu().double(), l64.grad) < 5e-6, name
 
 
+# Pairs that are not the complete blocks, from the C ABI: a pair missing (the first of all: rows of the first crystal would begin
+# before the array; one of the second crystal), neighbours in descending order, rows of another length than the atoms of the
+# crystal.  And the last row cut off, as when fewer pairs are stated than there are.
+@pytest.mark.parametrize("bad", ["first pair", "a pair", "descending", "short rows", "last row"])
+def test_column_sums_of_other_layouts(bad):
+    """Every row of the gradients is written, and the crystals whose pairs are whole blocks have theirs."""
+    from crystalframer_amd import _lib
+    lib = _lib.load()
+    sizes = [5, 6, 9]
+    start = [0, 5, 11]
+    rows = [[(a + i, a + j) for j in range(n)] for a, n in zip(start, sizes) for i in range(n)]
+    spoilt = {"first pair": 0, "last row": 2}.get(bad, 1)
+    good = [r[:] for r in rows]
+    if bad == "first pair":
+        rows[0] = rows[0][1:]
+    elif bad == "a pair":
+        rows[7] = rows[7][:2] + rows[7][3:]
+    elif bad == "last row":
+        rows[-1] = []
+    else:
+        for i in range(5, 11):
+            rows[i] = rows[i][::-1] if bad == "descending" else rows[i][:3]
+    N, H, D = 20, Hh.H, Hh.DH
+    gen = torch.Generator().manual_seed(5)
+    q, k, v, go = (torch.randn(N, H, D, generator=gen).to(dev()) for _ in range(4))
+
+    def columns(rows):
+        edges = torch.tensor([p for r in rows for p in r]).t().contiguous().to(dev())
+        e_start = torch.tensor([0] + [len(r) for r in rows]).cumsum(0).to(dev())
+        E = edges.shape[1]
+        prob, out, gq, ga = (torch.empty(E, H, device=dev()), torch.empty_like(q), torch.empty_like(q), torch.empty(E, H, device=dev()))
+        gk, gv = torch.full_like(q, float("nan")), torch.full_like(q, float("nan"))
+        st, P = _lib.current_stream_ptr(dev()), _lib.ptr
+        _lib.check(lib.cfh_fused_dpa_forward(P(q), P(k), P(v), None, None, P(edges), P(e_start), N, H, D, E, P(prob), P(out), st), "fwd")
+        _lib.check(lib.cfh_fused_dpa_backward(P(q), P(k), P(v), None, None, P(edges), P(e_start), P(prob), P(out), P(go), N, H, D, E,
+                                              P(gq), P(gk), P(gv), P(ga), None, st), "bwd")
+        return gk, gv
+
+    for got, want in zip(columns(rows), columns(good)):
+        assert torch.isfinite(got).all()
+        for b in range(3):
+            if b != spoilt:
+                at = slice(start[b], start[b] + sizes[b])
+                assert torch.equal(got[at], want[at])
+
+
 # One job, two, and a table that is full but for one, full, and one too many (two launches); every third job of one slice.
 @pytest.mark.parametrize("n_jobs", [1, 2, 31, 32, 33])
 def test_weight_gradient_tables(n_jobs):

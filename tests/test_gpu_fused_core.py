@@ -429,3 +429,28 @@ def test_fused_core_reports_pairs_that_are_not_whole_blocks():
     torch.cuda.synchronize()
     assert _lib.read_status(dev(), reset=True) & 2 == 2
     assert torch.isfinite(out2).all()
+
+
+@pytest.mark.parametrize("bad", ["descending", "shorter rows"])
+def test_fused_core_backward_of_pairs_that_are_not_whole_blocks(bad):
+    """As above, with a backward pass: rows whose neighbours descend, and rows that leave out a crystal's last atom (each for
+    itself a run of atoms that the forward pass takes): bit 2 of the status word, and finite gradients."""
+    from crystalframer_amd import _lib, cuda_funcs as F
+    P = Hh.make_problem(num_crystals=6, atoms_lo=2, atoms_hi=7, seed=48)
+    j_last = torch.tensor([j == max(P.edges[1][P.edges[0] == i].tolist()) for i, j in P.edges.t().tolist()])
+    order = torch.arange(P.E)
+    if bad == "shorter rows":
+        order = order[~j_last]
+    else:
+        order = torch.cat([order[P.edges[0] == i].flip(0) for i in range(P.N)])
+    edges = P.edges[:, order].contiguous().to(dev())
+    leaves = [g(t).requires_grad_() for t in (P.q, P.k, P.v, P.a)]
+    _lib.read_status(dev(), reset=True)
+    F.declare_complete_blocks(edges)
+    out, _ = F.PeriodicAttentionCoreHIP.apply(
+        *leaves, g(P.rpos[order]), g(P.tvecs), P.batch.to(dev()), edges, 64, Hh.DIST_MAX, 1.0, g(P.W_k), g(P.W_ax[0]),
+        g(P.W_ax[1]), g(P.W_ax[2]), 64, 4.0, 0, 1.0, 1.0, g(P.rvlen), CUT, torch.stack([g(f) for f in P.frames], 0))
+    out.sum().backward()
+    torch.cuda.synchronize()
+    assert _lib.read_status(dev(), reset=True) & 2 == 2
+    assert torch.isfinite(out).all() and all(torch.isfinite(t.grad).all() for t in leaves)

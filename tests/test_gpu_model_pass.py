@@ -616,3 +616,37 @@ def test_item_counts_of_one_launch(bins, atoms, B):
     assert Hh.rel_err(b[:B], a.double()) < 1e-6
     with torch.no_grad():
         assert Hh.rel_err(model(more)[:B], model(less).double()) < 2e-6
+
+
+# One launch per layer (few items) and several; without and with an angle encoding.  The pairs stated end within the last
+# crystal's rows, at its first, and within a crystal before.
+@pytest.mark.parametrize("bins", [0, 64])
+@pytest.mark.parametrize("B,cut", [(5, 3), (5, 49), (5, 60), (260, 3), (260, 60)])
+def test_fewer_pairs_stated_than_there_are(bins, B, cut):
+    """The atoms whose pairs are not all there have none, the status word says so, every read stays inside the arrays, and the
+    crystals before are answered as with the right count."""
+    from crystalframer_amd import _lib, params, synthetic
+    mp = params.ModelParams(num_layers=2, value_pe_angle_real=bins, symm_break_noise=0.0)
+    cb = synthetic.make_batch(B, atoms="uniform", atoms_lo=7, atoms_hi=7, len_lo=4.0, len_hi=9.0, ang_lo=65.0, ang_hi=115.0, seed=B)
+    model, cb = _model(mp, cb)
+    dev = torch.device("cuda:0")
+
+    def passes():
+        _lib.read_status(dev, reset=True)
+        model.zero_grad(set_to_none=True)
+        out = model(cb)
+        assert out.grad_fn.name() == "ModelPassHIPBackward"
+        out.sum().backward()
+        with torch.no_grad():
+            served = model(cb)
+        grads = [p.grad for p in model.parameters() if p.grad is not None]
+        return out.detach(), served, grads, _lib.read_status(dev, reset=True)
+
+    want, want_served, _, status = passes()
+    assert status == 0
+    cb.num_pairs -= cut
+    out, served, grads, status = passes()
+    assert status & 2 == 2
+    whole = B - 1 - cut // 50
+    assert torch.equal(out[:whole], want[:whole]) and torch.equal(served[:whole], want_served[:whole])
+    assert torch.isfinite(out).all() and torch.isfinite(served).all() and all(torch.isfinite(t).all() for t in grads)
