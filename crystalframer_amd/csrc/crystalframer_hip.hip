@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -1259,19 +1260,23 @@ struct StreamList {
         blocks = 0;
     }
 };
-// More than 64 KB of LDS have to be asked for, once per kernel and device (here from 48 KB of dynamic LDS on: the kernel's own
-// arrays come on top).
+// More than 64 KB of LDS have to be asked for, once per kernel and device: the dynamic LDS and the kernel's own arrays together.
 template <auto KERN>
 int allow_lds(size_t lds) {
-    static int lds_set[64] = {0};
-    if (lds <= 48 * 1024) return CFH_OK;
+    static std::atomic<int> own_set[64], lds_set[64];      // the kernel's own arrays + 1 (0: not known yet), what is allowed
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return fail(CFH_ELAUNCH, "no current device");
-    if (lds_set[dev] < (int)lds) {
-        if (hipFuncSetAttribute((const void*)KERN, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
-            return fail(CFH_ELAUNCH, "%zu bytes of LDS refused", lds);
-        lds_set[dev] = (int)lds;
+    int own = own_set[dev].load(std::memory_order_relaxed) - 1;
+    if (own < 0) {
+        hipFuncAttributes attr;
+        if (hipFuncGetAttributes(&attr, (const void*)KERN) != hipSuccess) return fail(CFH_ELAUNCH, "no attributes of a kernel");
+        own = (int)attr.sharedSizeBytes;
+        own_set[dev].store(own + 1, std::memory_order_relaxed);
     }
+    if (lds + (size_t)own <= 64 * 1024 || lds_set[dev].load(std::memory_order_relaxed) >= (int)lds) return CFH_OK;
+    if (hipFuncSetAttribute((const void*)KERN, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+        return fail(CFH_ELAUNCH, "%zu bytes of LDS refused", lds);
+    lds_set[dev].store((int)lds, std::memory_order_relaxed);
     return CFH_OK;
 }
 // A.x1 and A.h: needed as memory between the two launches of the split form, else optional.
@@ -1305,6 +1310,7 @@ int bridge_front(const cfh::BridgeArgs& A, int D, hipStream_t st) {
     const dim3 block(64 * cfh::BR_WAVES);
     const size_t lds = 16 * (size_t)(16 * cfh::bridge_feat_steps(A.feat) + cfh::BR_PAD) * sizeof(float);
     TimedScope timed("layer_front", st);
+    if (int rc = D == 256 ? allow_lds<cfh::layer_front_fwd_kernel<2>>(lds) : allow_lds<cfh::layer_front_fwd_kernel<1>>(lds)) return rc;
     if (D == 256) hipLaunchKernelGGL(cfh::layer_front_fwd_kernel<2>, dim3(tiles, parts), block, lds, st, A);
     else hipLaunchKernelGGL(cfh::layer_front_fwd_kernel<1>, dim3(tiles, parts), block, lds, st, A);
     return finish_launch("layer_front_forward");

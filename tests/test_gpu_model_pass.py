@@ -650,3 +650,29 @@ def test_fewer_pairs_stated_than_there_are(bins, B, cut):
     whole = B - 1 - cut // 50
     assert torch.equal(out[:whole], want[:whole]) and torch.equal(served[:whole], want_served[:whole])
     assert torch.isfinite(out).all() and torch.isfinite(served).all() and all(torch.isfinite(t).all() for t in grads)
+
+
+# Kernels whose own arrays and dynamic LDS together pass 64 KB while the dynamic part alone does not reach 48: the embedding of
+# inference (257 to 384 features at a width of 256, and an edge), and the second launch of training's bridge (F = 512)
+@pytest.mark.parametrize("feat,F,N", [(256, 128, 5), (257, 128, 5), (384, 256, 40), (385, 128, 17), (98, 512, 33), (300, 512, 600)])
+def test_lds_of_a_kernel_and_of_its_launch_together(feat, F, N):
+    """Inference against the pass that keeps everything (float32 matrix instructions), sums of up to 512 products."""
+    from crystalframer_amd import params, synthetic
+    mp = params.ModelParams(num_layers=2, symm_break_noise=0.0, value_pe_angle_real=0, model_dim=256, head_num=16, ff_dim=F)
+    cb = synthetic.make_batch(N, atoms="uniform", atoms_lo=1, atoms_hi=1, len_lo=3.0, len_hi=6.0, ang_lo=70.0, ang_hi=110.0, seed=N)
+    x = torch.zeros(N, feat)
+    x[torch.arange(N), torch.arange(N) % feat] = 1.0
+    x[:, -1] = 0.5
+    cb = synthetic.CrystalBatch(x, cb.pos, cb.batch, cb.trans_vec, cb.sizes, zero_based=True)
+
+    def wide_input(model):
+        model.input_embeddings = torch.nn.Linear(feat, 256, bias=False).cuda()
+        for i in (0, 3):
+            model.mlp[i] = torch.nn.Linear(256, 256).cuda()
+
+    model, cb = _model(mp, cb, change=wide_input)
+    kept = model(cb)
+    assert kept.grad_fn.name() == "ModelPassHIPBackward"
+    with torch.no_grad():
+        served = model(cb)
+    assert Hh.rel_err(served, kept.detach().double()) < 2e-6
