@@ -867,6 +867,12 @@ int cfh_framed_pe_backward_pairwise(const cfh_params* p, const float* a_ih, cons
 }
 
 namespace {
+void column_launch(const cfh::DpaArgs& A, hipStream_t st) {
+    const int64_t items = (int64_t)A.N * A.H;
+    const dim3 grid((unsigned)((items + cfh::DPA_WAVES - 1) / cfh::DPA_WAVES)), block(cfh::WAVE * cfh::DPA_WAVES);
+    if (cfh::column_groups(A)) hipLaunchKernelGGL(cfh::dpa_bwd_col_kernel<cfh::COL_GROUP>, grid, block, 0, st, A);
+    else hipLaunchKernelGGL(cfh::dpa_bwd_col_kernel<1>, grid, block, 0, st, A);
+}
 int check_dpa(const void* q, const void* k, const void* v, const int64_t* edges, const int64_t* e_start,
               int64_t N, int64_t H, int64_t Dh, int64_t E) {
     if (N < 0 || E < 0) return fail(CFH_EINVAL, "negative size N=%lld E=%lld", (long long)N, (long long)E);
@@ -917,7 +923,7 @@ int cfh_fused_dpa_backward(const float* q, const float* k, const float* v, const
     const int64_t items = N * H;
     const dim3 grid((unsigned)((items + cfh::DPA_WAVES - 1) / cfh::DPA_WAVES)), block(cfh::WAVE * cfh::DPA_WAVES);
     hipLaunchKernelGGL(cfh::dpa_bwd_row_kernel, grid, block, 0, (hipStream_t)stream, A);
-    hipLaunchKernelGGL(cfh::dpa_bwd_col_kernel, grid, block, 0, (hipStream_t)stream, A);
+    column_launch(A, (hipStream_t)stream);
     return finish_launch("fused_dpa_backward");
 }
 
@@ -1973,11 +1979,9 @@ int fused_core_backward_impl(const cfh_params* p, const float* qs, const float* 
         A.items = C.K.items;
         A.status = C.K.status;
         if (own_pairs) A.e_start = nullptr;
-        const int64_t items = N * p->num_heads;
         {
             TimedScope timed("core_bwd_col", st);
-            hipLaunchKernelGGL(cfh::dpa_bwd_col_kernel, dim3((unsigned)((items + cfh::DPA_WAVES - 1) / cfh::DPA_WAVES)),
-                               dim3(cfh::WAVE * cfh::DPA_WAVES), 0, st, A);
+            column_launch(A, st);
         }
         rc = finish_launch("fused_core_backward");
     }

@@ -199,16 +199,28 @@ __global__ __launch_bounds__(WAVE * DPA_WAVES) void dpa_bwd_row_kernel(const Dpa
 
 // gk_j = sum_i gl_(i,j) q_i, gv_j = sum_i p_(i,j) go_i over the atoms i of the crystal of j; every
 // row of the crystal's block has n pairs, so pair (i, j) is at (first pair of the crystal) + r n + col.
-// A wavefront takes COL_GROUP consecutive columns of a head, those from a multiple of COL_GROUP on (the wavefronts of the
-// other atoms end): the rows of q and go are loaded once for all of them, and the four lanes of a slot load gl and p of
-// one column each, within one 128-byte line of 4 columns x 8 heads, and hand them round.  Every column's sum keeps its
-// order: slot by slot, then over the slots.
-// Bound by the lines its loads touch: one column per wavefront took 64 us for 32 cells of 40 to 200 atoms (31 now; 52 with
-// the order of the dies alone) and 10.7 us for 256 cells of 9 atoms on average (9.5).
+// A wavefront takes GROUP consecutive columns of a head, those from a multiple of GROUP on (the wavefronts of the other atoms
+// end).  Four: the rows of q and go are loaded once for all of them, and the four lanes of a slot load gl and p of one column
+// each, within one 128-byte line of 4 columns x 8 heads, and hand them round.  Every column's sum keeps its order: slot by
+// slot, then over the slots.  Bound by the lines its loads touch where there are many: 32 cells of 40 to 200 atoms 64 us with
+// one column per wavefront, 50 with the order of the dies, 32 with four columns; with few wavefronts by their chain of loads
+// and reductions, where four accumulators in turn on a quarter of the wavefronts take longer (column_groups).
 constexpr int COL_GROUP = 4;     // = the lanes of a slot
+// Four columns per wavefront, by what one and four measured (us a launch, 64 and no angle bins alike, the order of the dies in
+// both).  Rows of 137 pairs on average: 7680 items 14.0 and 15.0, 9600 18.9 and 25.0, 11 520 21.3 and 16.6, 30 720 50 and 32;
+// of 43: 7680 7.5 and 8.9, 10 240 9.9 and 9.4, 15 360 12.6 and 10.4; of 17: 16 384 8.8 and 9.1, 24 576 12.4 and 11.6; of 13.5:
+// 7432 5.0 and 6.2, 14 672 7.9 and 8.5, 17 112 9.4 and 9.4, 19 584 10.1 and 9.6, 39 216 17.4 and 15.9; of 7: 5632 4.9 and 5.5,
+// 22 528 9.6 and 10.1, 45 056 17.8 and 18.1.  Looking at the pairs first (those of a caller) takes 1.8 us more with four columns
+// and nothing with one: 19 584 items 11.4 and 10.1, so that rows of up to 24 pairs are left to one.
+inline bool column_groups(const DpaArgs& P) {
+    const int64_t N = P.N, E = P.E, items = N * P.H;
+    return E > 24 * N ? items >= 10240 : !P.e_start && E > 10 * N && items >= 18432;
+}
 template <int C>
 __device__ __forceinline__ float quad_lane(float x) { return dpp_move<C * 0x55>(x); }      // of the slot's lane C
+template <int GROUP>
 __global__ __launch_bounds__(WAVE * DPA_WAVES) void dpa_bwd_col_kernel(const DpaArgs P) {
+    static_assert(GROUP == 1 || GROUP == COL_GROUP, "a column per wavefront, or per lane of a slot");
     const int lane = threadIdx.x & (WAVE - 1);
     const int item = die_order((int)blockIdx.x, (int)gridDim.x, COL_DIE_SHIFT) * DPA_WAVES + (int)(threadIdx.x >> 6);
     if (item >= P.N * P.H) return;
@@ -236,9 +248,9 @@ __global__ __launch_bounds__(WAVE * DPA_WAVES) void dpa_bwd_col_kernel(const Dpa
     // Which rows of the group are of this block, as the pairs themselves have it (lane qd of a slot looks at row qd): the first
     // atom's wavefront writes those, the wavefronts of the others see the same and end.  It waits for the answer at its end only
     // (before its sums: 11.8 us for 256 cells of 9 atoms on average).
-    const int g0 = col & ~(COL_GROUP - 1);
-    bool same = whole && g0 + qd < n;
-    if (same && P.e_start) {
+    const int g0 = col & ~(GROUP - 1);
+    bool same = whole && qd < GROUP && g0 + qd < n;
+    if (GROUP > 1 && same && P.e_start) {
         const int c = g0 + qd, s = e0 + (c - col) * n;
         const int64_t s0 = P.e_start[first + c], s1 = P.e_start[first + c + 1], j0 = P.edges[(size_t)P.E + s];
         same = s0 == s && s1 == s + n && j0 == first;
@@ -249,12 +261,12 @@ __global__ __launch_bounds__(WAVE * DPA_WAVES) void dpa_bwd_col_kernel(const Dpa
         whole = false;
     }
     if (!whole) n = col = 0;
-    float4 gk[COL_GROUP], gv[COL_GROUP];
+    float4 gk[GROUP], gv[GROUP];
 #pragma unroll
-    for (int c = 0; c < COL_GROUP; c++) gk[c] = gv[c] = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int c = 0; c < GROUP; c++) gk[c] = gv[c] = make_float4(0.f, 0.f, 0.f, 0.f);
     if (n > 0) {
         const size_t eblock = (size_t)e0 - (size_t)col * n;    // first pair of the crystal
-        const int mine = min(col + qd, n - 1);                 // (past the last column: the last again, not written)
+        const int mine = GROUP == 1 ? col : min(col + qd, n - 1);                 // (past the last column: the last again, not written)
         for (int ib = 0; ib < n; ib += DPA_SLOTS) {
             const int r = ib + slot;
             if (r < n) {                                       // (the same in the lanes of a slot)
@@ -262,10 +274,15 @@ __global__ __launch_bounds__(WAVE * DPA_WAVES) void dpa_bwd_col_kernel(const Dpa
                 const size_t ih = (size_t)(first + r) * H + h;
                 const float gl = P.gaij[e * H + h], p = P.prob[e * H + h];
                 const float4 q4 = ld4(P.q, ih, qd), go4 = ld4(P.go, ih, qd);
-                const float gls[COL_GROUP] = {quad_lane<0>(gl), quad_lane<1>(gl), quad_lane<2>(gl), quad_lane<3>(gl)};
-                const float ps[COL_GROUP] = {quad_lane<0>(p), quad_lane<1>(p), quad_lane<2>(p), quad_lane<3>(p)};
+                float gls[GROUP], ps[GROUP];
+                if constexpr (GROUP == 1) {
+                    gls[0] = gl; ps[0] = p;
+                } else {
+                    gls[0] = quad_lane<0>(gl); gls[1] = quad_lane<1>(gl); gls[2] = quad_lane<2>(gl); gls[3] = quad_lane<3>(gl);
+                    ps[0] = quad_lane<0>(p); ps[1] = quad_lane<1>(p); ps[2] = quad_lane<2>(p); ps[3] = quad_lane<3>(p);
+                }
 #pragma unroll
-                for (int c = 0; c < COL_GROUP; c++) {
+                for (int c = 0; c < GROUP; c++) {
                     gk[c].x = fmaf(gls[c], q4.x, gk[c].x); gk[c].y = fmaf(gls[c], q4.y, gk[c].y);
                     gk[c].z = fmaf(gls[c], q4.z, gk[c].z); gk[c].w = fmaf(gls[c], q4.w, gk[c].w);
                     gv[c].x = fmaf(ps[c], go4.x, gv[c].x); gv[c].y = fmaf(ps[c], go4.y, gv[c].y);
@@ -274,14 +291,14 @@ __global__ __launch_bounds__(WAVE * DPA_WAVES) void dpa_bwd_col_kernel(const Dpa
             }
         }
     }
-    uint32_t rows = (uint32_t)ballot(same && whole) & ((1u << COL_GROUP) - 1);
+    uint32_t rows = (uint32_t)ballot(same && whole) & ((1u << GROUP) - 1);
     if ((rows & 1) == 0) {                                     // (this atom's zeros)
         if (pairs > 0 && P.status && lane == 0) atomicOr(P.status, 2);
         gk[0] = gv[0] = make_float4(0.f, 0.f, 0.f, 0.f);
         rows = 1;
     }
 #pragma unroll
-    for (int c = 0; c < COL_GROUP; c++) {
+    for (int c = 0; c < GROUP; c++) {
         if (((rows >> c) & 1) == 0) continue;
         const float4 k4 = slots_sum(gk[c]), v4 = slots_sum(gv[c]);
         if (slot == 0) {

@@ -586,18 +586,51 @@ def test_column_sums_by_groups_of_columns(atoms, crystals):
         assert Hh.rel_err(l32.grad.cpu().double(), l64.grad) < 5e-6, name
 
 
+# Four columns per wavefront: from 10 240 items on with rows of more than 24 pairs; either side of the line, crystals of every
+# remainder of four, around steps of 16 pairs, and one of a single atom last in the batch; one column for more items of short rows.
+@pytest.mark.parametrize("sizes", [[25, 31, 34, 36] * 10 + [33], [25, 31, 34, 36] * 10 + [18], [48, 49, 50, 51] * 7 + [1], [13] * 200])
+def test_column_sums_of_many_items(sizes):
+    """Sums of up to 51 float32 products against float64, as above."""
+    from crystalframer_amd import _lib
+    lib = _lib.load()
+    n = torch.tensor(sizes)
+    first, N, E = torch.cumsum(n, 0) - n, int(n.sum()), int((n * n).sum())
+    assert (E > 24 * N and N * Hh.H >= 10240) == (sizes[-1] in (1, 33))
+    atom = torch.arange(N)
+    i = torch.repeat_interleave(atom, torch.repeat_interleave(n, n))
+    crystal = torch.repeat_interleave(torch.arange(len(sizes)), n)
+    e_start = torch.cat([torch.zeros(1, dtype=torch.long), torch.cumsum(n[crystal], 0)])
+    j = first[crystal[i]] + torch.arange(E) - e_start[i]
+    gen = torch.Generator().manual_seed(N)
+    q, k, v, go = (torch.randn(N, Hh.H, Hh.DH, generator=gen) * 0.5 for _ in range(4))
+    edges = torch.stack([i, j]).contiguous()
+    q64, k64, v64 = (t.double().requires_grad_() for t in (q, k, v))
+    out64, _ = TO.softmax_attention(q64, k64, v64, None, None, crystal, edges)
+    (out64 * go.double()).sum().backward()
+    edges, e_start, q, k, v, go = (t.to(dev()) for t in (edges, e_start, q, k, v, go))
+    prob, ga = torch.empty(E, Hh.H, device=dev()), torch.empty(E, Hh.H, device=dev())
+    out, gq, gk, gv = (torch.full_like(q, float("nan")) for _ in range(4))
+    st, P = _lib.current_stream_ptr(dev()), _lib.ptr
+    _lib.check(lib.cfh_fused_dpa_forward(P(q), P(k), P(v), None, None, P(edges), P(e_start), N, Hh.H, Hh.DH, E, P(prob), P(out), st), "fwd")
+    _lib.check(lib.cfh_fused_dpa_backward(P(q), P(k), P(v), None, None, P(edges), P(e_start), P(prob), P(out), P(go), N, Hh.H, Hh.DH, E,
+                                          P(gq), P(gk), P(gv), P(ga), None, st), "bwd")
+    assert Hh.rel_err(gk, k64.grad) < 5e-6 and Hh.rel_err(gv, v64.grad) < 5e-6
+
+
 # Pairs that are not the complete blocks, from the C ABI: a pair missing (the first of all: rows of the first crystal would begin
 # before the array; one of the second crystal), neighbours in descending order, rows of another length than the atoms of the
 # crystal.  And the last row cut off, as when fewer pairs are stated than there are.
+# With crystals of 40 atoms behind the first three: four columns per wavefront.
+@pytest.mark.parametrize("more", [0, 33])
 @pytest.mark.parametrize("bad", ["first pair", "a pair", "descending", "short rows", "last row"])
-def test_column_sums_of_other_layouts(bad):
+def test_column_sums_of_other_layouts(bad, more):
     """Every row of the gradients is written, and the crystals whose pairs are whole blocks have theirs."""
     from crystalframer_amd import _lib
     lib = _lib.load()
-    sizes = [5, 6, 9]
-    start = [0, 5, 11]
+    sizes = [5, 6, 9] + [40] * more
+    start = [sum(sizes[:b]) for b in range(len(sizes))]
     rows = [[(a + i, a + j) for j in range(n)] for a, n in zip(start, sizes) for i in range(n)]
-    spoilt = {"first pair": 0, "last row": 2}.get(bad, 1)
+    spoilt = {"first pair": 0, "last row": len(sizes) - 1}.get(bad, 1)
     good = [r[:] for r in rows]
     if bad == "first pair":
         rows[0] = rows[0][1:]
@@ -608,7 +641,7 @@ def test_column_sums_of_other_layouts(bad):
     else:
         for i in range(5, 11):
             rows[i] = rows[i][::-1] if bad == "descending" else rows[i][:3]
-    N, H, D = 20, Hh.H, Hh.DH
+    N, H, D = sum(sizes), Hh.H, Hh.DH
     gen = torch.Generator().manual_seed(5)
     q, k, v, go = (torch.randn(N, H, D, generator=gen).to(dev()) for _ in range(4))
 
@@ -626,7 +659,7 @@ def test_column_sums_of_other_layouts(bad):
 
     for got, want in zip(columns(rows), columns(good)):
         assert torch.isfinite(got).all()
-        for b in range(3):
+        for b in range(len(sizes)):
             if b != spoilt:
                 at = slice(start[b], start[b] + sizes[b])
                 assert torch.equal(got[at], want[at])

@@ -71,6 +71,21 @@ def test_one_call_equals_the_modules_path(B, hi, bins, layers):
         assert Hh.rel_err(g1[n], g2[n].double()) < (1e-5 if B <= 512 else 2e-3), n
 
 
+# The sums over the pairs that point at an atom, four atoms per wavefront from 18 432 items on (here of 13 and 14 atoms each),
+# with rows of more than 24 pairs from 10 240 on; the modules' pairs are looked at first and rows of up to 24 take one.
+@pytest.mark.parametrize("B,lo,hi", [(177, 13, 14), (168, 13, 14), (46, 27, 31), (42, 27, 31)])
+def test_column_sums_of_a_batch(B, lo, hi):
+    from crystalframer_amd import params, synthetic
+    mp = params.ModelParams(num_layers=2, value_pe_angle_real=0, symm_break_noise=0.0)
+    cb = synthetic.make_batch(B, atoms="uniform", atoms_lo=lo, atoms_hi=hi, len_lo=4.0, len_hi=9.0, ang_lo=65.0, ang_hi=115.0, seed=B)
+    N = cb.pos.shape[0]
+    assert (8 * N >= (10240 if lo > 24 else 18432)) == (B in (177, 46))
+    _, _, ((o1, _, g1), (o2, _, g2)) = _both(mp, cb)
+    assert torch.equal(o1, o2)
+    for n in g1:
+        assert torch.equal(g1[n], g2[n]), n
+
+
 # (from 445 features on, a workgroup of the tail takes more than 64 KB of LDS; 480 is the widest head it takes)
 @pytest.mark.parametrize("widths", [[64, 208], [448], [464], [480, 16, 480]])
 def test_head_of_several_layers_and_targets(widths):
@@ -621,13 +636,13 @@ def test_item_counts_of_one_launch(bins, atoms, B):
 # One launch per layer (few items) and several; without and with an angle encoding.  The pairs stated end within the last
 # crystal's rows, at its first, and within a crystal before.
 @pytest.mark.parametrize("bins", [0, 64])
-@pytest.mark.parametrize("B,cut", [(5, 3), (5, 49), (5, 60), (260, 3), (260, 60)])
-def test_fewer_pairs_stated_than_there_are(bins, B, cut):
+@pytest.mark.parametrize("B,atoms,cut", [(5, 7, 3), (5, 7, 49), (5, 7, 60), (260, 7, 3), (260, 7, 60), (55, 25, 3), (55, 25, 650)])
+def test_fewer_pairs_stated_than_there_are(bins, B, atoms, cut):
     """The atoms whose pairs are not all there have none, the status word says so, every read stays inside the arrays, and the
     crystals before are answered as with the right count."""
     from crystalframer_amd import _lib, params, synthetic
     mp = params.ModelParams(num_layers=2, value_pe_angle_real=bins, symm_break_noise=0.0)
-    cb = synthetic.make_batch(B, atoms="uniform", atoms_lo=7, atoms_hi=7, len_lo=4.0, len_hi=9.0, ang_lo=65.0, ang_hi=115.0, seed=B)
+    cb = synthetic.make_batch(B, atoms="uniform", atoms_lo=atoms, atoms_hi=atoms, len_lo=4.0, len_hi=9.0, ang_lo=65.0, ang_hi=115.0, seed=B)
     model, cb = _model(mp, cb)
     dev = torch.device("cuda:0")
 
@@ -647,7 +662,7 @@ def test_fewer_pairs_stated_than_there_are(bins, B, cut):
     cb.num_pairs -= cut
     out, served, grads, status = passes()
     assert status & 2 == 2
-    whole = B - 1 - cut // 50
+    whole = B - -(-cut // atoms ** 2)
     assert torch.equal(out[:whole], want[:whole]) and torch.equal(served[:whole], want_served[:whole])
     assert torch.isfinite(out).all() and torch.isfinite(served).all() and all(torch.isfinite(t).all() for t in grads)
 
