@@ -1674,28 +1674,34 @@ void project_launch(int hw, const float* hist, const float* wcat, float* out, in
     else if (hw == cfh::HW_ANG16) launch(cfh::core_project_kernel<2, 4>, 2);
     else launch(cfh::core_project_kernel<1, 4>, 1);
 }
-// Up to this many (atom, head) items the forward pass of a layer is one wavefront per item from the record to the sums: about
-// as many as are resident at once (19 to 23 per compute unit).  Measured with and without, whole calls: 976 items 274 and 256
-// us, 4592 items 412 and 380, 7712 items 446 and 415, 10 696 items 398 and 441.  Short rows (a mean of at most 24 pairs) gain
-// beyond, where a wavefront that ends makes room soon: training steps of 5328 items 715 and 697 us, 6488 items 873 and 842, but
-// 7712 items 759 and 772; distances alone 6488 items 654 and 636, 9168 items 719 and 702.  Cells of 40 to 200 atoms lose from 5760
-// items on (384 and 392; 6720 items 404 and 418), distances alone too (8640 items 345 and 353).
-constexpr int64_t ITEM_PASS_MAX = 5120, ITEM_PASS_MAX_SHORT = 7168, ITEM_PASS_MAX_DISTANCE = 10240, SHORT_ROW = 24;
-int64_t item_pass_max(const cfh_params* p, int64_t N, int64_t E) {
-    return E > SHORT_ROW * N ? ITEM_PASS_MAX : (p->angle_bins > 0 ? ITEM_PASS_MAX_SHORT : ITEM_PASS_MAX_DISTANCE);
-}
-// Inference, where the histogram serves the projection alone: the wavefront of such an item makes the product with the head's
-// weights itself, which saves a launch and a round trip of the histogram but reads the weights (46 KB at 64 bins) once per item
-// instead of once per 16.  Whole calls of four layers in us, with a launch for the products and without: 64 bins, 64 items 158
-// and 142, 600 items 207 and 189, 1208 items 191 and 173, 2416 items 210 and 187, 4872 items 320 and 250; so the one launch pays
-// for more items: against several launches 6488 items 346 and 291, 7712 items 333 and 314, 9216 items 294 and 275, 10 696 items
-// 369 and 364, 11 440 items 359 and 373.  16 bins: 2304 items 171 and 160, 5056 items 199 and 192; 6496 items 257 (several
-// launches) and 231, 10 696 items 382 and 378, 12 256 items 317 and 324.  Distances alone, where the wavefronts are lighter: 1152
-// items 119 and 109, 4608 items 133 and 123; 9216 items 173 (several) and 159, 12 256 items 201 and 191, 18 432 items 237 and
-// 238, 36 864 items 400 and 434.
-constexpr int64_t ITEM_PROJECT_MAX = 10240, ITEM_PROJECT_MAX_DISTANCE = 16384;
-bool item_project(const cfh_params* p, int64_t N, int64_t E) {
-    return N * p->num_heads <= (E > SHORT_ROW * N ? ITEM_PASS_MAX : (p->angle_bins > 0 ? ITEM_PROJECT_MAX : ITEM_PROJECT_MAX_DISTANCE));
+// Up to this many (atom, head) items the forward pass of a layer is one launch, one wavefront per item from the record to the
+// sums, instead of records, frame search and main kernel: about as many as are resident at once (19 to 23 per compute unit) and,
+// where a wavefront that ends makes room soon, up to twice that.  The several launches take the items with a box of their own
+// first and search frames four heads at a time, so long rows and slow cells are theirs sooner.
+// Measured over synthetic batches, one family of crystals per row length (whole passes of four layers in us, several launches
+// / one; r: mean pairs per atom; r = 13: means of five batches each).
+// Training step as a graph, 64 angle bins (16 within a percent): r = 7: 5016 items 617/610, 5984 636/647, 9040 793/811; r =
+// 10: 5016 605/596, 6008 656/673, 8968 778/801; r = 13: 4936 695/679, 5792 741/724, 6184 728/724, 6568 720/722, 7016 792/803;
+// r = 17: 3968 591/557, 6016 673/670, 7936 748/759; r = 29: 4928 684/683, 6048 745/746, 10 080 986/996; r = 43: 3840 668/649,
+// 5120 744/750; r = 78: 600 649/647, 4200 872/873, 4800 880/906; r = 120 to 137: 960 748/758, 1920 878/901, 7680 1454/1505.
+// Distances alone: r = 7: 9040 539/535, 9992 551/556; r = 10: 10 032 561/557, 11 040 583/587; r = 13: 10 040 631/625, 10 992
+// 607/617; r = 17: 4992 465/455, 6016 484/482, 7936 527/535; r = 29: 4928 502/494, 6048 527/534; r = 43: 5120 558/550, 6080
+// 559/562; r = 78: 3000 582/581, 6000 689/714; r = 137: 2880 792/799, 7680 1002/1070.
+// Inference, where the histogram serves the projection alone: the wavefront of an item makes the product with the head's
+// weights itself, which saves the launch of the products and a round trip of the histogram but reads the weights (46 KB at 64
+// bins) once per item instead of once per 16.  64 bins: r = 7: 5016 260/203, 9992 328/306, 11 000 355/339, 12 016 373/389; r
+// = 10: 5016 263/201, 10 032 330/312, 11 040 347/341; r = 13: 8016 326/319, 10 040 398/378, 10 992 394/407; r = 17: 8960
+// 341/306, 9984 362/370, 12 032 399/439; r = 43: 5120 308/251, 9920 435/403; r = 78: 4800 385/348, 10 200 571/561; r = 137:
+// 4800 500/469, 5760 544/560, 7680 673/647, 11 520 850/872.  16 bins the same lines (r = 7: 9992 347/314, 12 016 387/399).
+// Distances alone: r = 6: 11 992 205/199, 16 000 228/228; r = 10: 12 008 219/214, 16 040 245/245; r = 13: 10 040 230/212, 10
+// 992 224/221, 12 016 227/227, 15 984 247/260; r = 17: 8960 206/193, 9984 214/214, 12 032 235/259; r = 43: 9920 260/256; r =
+// 78: 10 200 343/336; r = 137: 4800 331/297, 6720 363/367, 7680 374/401.
+// (Single batches, whose slowest cell may end last, scatter about these by a few percent.)
+int64_t item_pass_max(const cfh_params* p, int64_t N, int64_t E, bool lean) {
+    const bool angles = p->angle_bins > 0;
+    if (lean) return E > 100 * N ? 5120 : (angles || E > 12 * N ? 10240 : 16384);
+    if (E > 64 * N) return 0;
+    return angles ? (E > 32 * N ? 4096 : E > 12 * N ? 6144 : 5120) : (E > 16 * N ? 5120 : 10240);
 }
 template <typename Kern>
 int launch_item_pass(Kern kern, const cfh::CoreArgs& C, bool search, const float* wcat, hipStream_t st, const char* what) {
@@ -1706,7 +1712,7 @@ int launch_item_pass(Kern kern, const cfh::CoreArgs& C, bool search, const float
     return finish_launch(what);
 }
 #define CFH_ITEM_PASS(...) launch_item_pass(cfh::item_pass_kernel<__VA_ARGS__>, C, search, nullptr, st, what)
-#define CFH_ITEM_PASS_LEAN(...) launch_item_pass(cfh::item_pass_kernel<__VA_ARGS__, true>, C, search, project ? wcat : nullptr, st, what)
+#define CFH_ITEM_PASS_LEAN(...) launch_item_pass(cfh::item_pass_kernel<__VA_ARGS__, true>, C, search, wcat, st, what)
 #define CFH_CORE_FWD(...) launch_core(cfh::fused_core_fwd_kernel<__VA_ARGS__>, C, st, what)
 #define CFH_CORE_FWD_LEAN(...) launch_core(cfh::fused_core_fwd_kernel<__VA_ARGS__, true>, C, st, what)
 #define CFH_CORE_BWD(...) launch_core(cfh::fused_core_bwd_kernel<__VA_ARGS__>, C, st, what)
@@ -1762,8 +1768,7 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
     const cfh::WcatArgs WA{W_dist, W_axis1, W_axis2, W_axis3, hw, p->dist_coef, p->angle_coef,
                            p->angle_wscale, wcat};
     // (the word of the noise's seed is copied and advanced by the launch that makes the records)
-    const bool project_by_item = lean && item_project(p, N, E);
-    const bool one_launch = (N * p->num_heads <= item_pass_max(p, N, E) || project_by_item) && !(search && p->symm_break_noise > 0.0f && C.K.seed_dev);
+    const bool one_launch = N * p->num_heads <= item_pass_max(p, N, E, lean) && !(search && p->symm_break_noise > 0.0f && C.K.seed_dev);
     if (one_launch) {
         if (!wcat_made) {
             TimedScope timed("core_prepare", st);
@@ -1826,7 +1831,6 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
         C.slow_wgs = slow_wave_count(N, p->num_heads);
     }
     C.slow_flag = cfh::REC_BOX_LISTED;
-    const bool project = one_launch && project_by_item;
     const char* what = one_launch ? "item_pass" : "fused_core_forward";
     if (lean) {
         if (p->angle_bins == cfh::NBINS)        // moments around the nodes of inference
@@ -1837,7 +1841,7 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
         if (one_launch) { CFH_CORE_DISPATCH(CFH_ITEM_PASS); }
         else { CFH_CORE_DISPATCH(CFH_CORE_FWD); }
     }
-    if (rc || project) return rc;
+    if (rc || (one_launch && lean)) return rc;
     {
         TimedScope timed("core_project", st);
         project_launch(hw, hist, wcat, out, N, p->num_heads, st);

@@ -592,7 +592,7 @@ def test_largest_weights(N):
 
 
 # Inference of few items: the product of an item's histogram with the weights by its own wavefront.  One atom, a few, either side
-# of the item counts where a launch of its own makes it (10 240 with an angle encoding, 16 384 without).
+# of the item counts where a launch of its own makes it for short rows (10 240 with an angle encoding, 16 384 without).
 @pytest.mark.parametrize("bins,B,atoms", [(64, 1, 1), (64, 3, 7), (64, 64, 10), (64, 1280, 1), (64, 1281, 1), (16, 1, 1), (16, 24, 8),
                                           (16, 1280, 1), (16, 1281, 1), (0, 1, 1), (0, 24, 8), (0, 2048, 1), (0, 2049, 1)])
 def test_products_of_few_items(bins, B, atoms):
@@ -611,10 +611,14 @@ def test_products_of_few_items(bins, B, atoms):
     assert Hh.rel_err(out, kept.double()) < 5e-6
 
 
-# Either side of the item counts up to which a layer's items take one launch: 7168 with an angle encoding, 10 240 without (crystals
-# of 8 atoms), and 5120 for rows of more than 24 pairs on average (crystals of 25); inference, with the product: 10 240 and 16 384.
+# Either side of the item counts up to which a layer's items take one launch, crystals of as many atoms as the row has pairs.  With
+# everything kept: 5120 with an angle encoding (8 atoms), 6144 from 13 atoms on, 4096 from 33, none from 65; 10 240 without (8
+# atoms), 5120 from 17 atoms on.  Inference: 10 240 (8, 24 and 40 atoms), 16 384 without an angle encoding for up to 12 atoms, 5120
+# from 101 atoms on.  (And counts between them.)
 @pytest.mark.parametrize("bins,atoms,B", [(64, 8, 112), (16, 8, 112), (0, 8, 160), (64, 25, 25), (0, 25, 25), (64, 24, 37), (64, 8, 160),
-                                          (0, 8, 256)])
+                                          (0, 8, 256), (64, 8, 80), (16, 8, 80), (64, 24, 32), (16, 13, 59), (64, 40, 12), (64, 65, 2),
+                                          (0, 65, 2), (0, 24, 53), (64, 24, 53), (64, 40, 32), (0, 12, 170), (0, 13, 98), (64, 101, 6),
+                                          (0, 101, 6)])
 def test_item_counts_of_one_launch(bins, atoms, B):
     """The crystals of a batch are answered alike in a batch of one more (no frame changes: the same operations per item, sums of
     the layers' rows in other tiles)."""
