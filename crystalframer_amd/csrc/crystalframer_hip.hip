@@ -1703,6 +1703,10 @@ int64_t item_pass_max(const cfh_params* p, int64_t N, int64_t E, bool lean) {
     if (E > 64 * N) return 0;
     return angles ? (E > 32 * N ? 4096 : E > 12 * N ? 6144 : 5120) : (E > 16 * N ? 5120 : 10240);
 }
+// (the word of the noise's seed is copied and advanced by the launch that makes the records)
+bool one_launch_form(const cfh_params* p, int64_t N, int64_t E, bool search, bool lean) {
+    return N * p->num_heads <= item_pass_max(p, N, E, lean) && !(search && p->symm_break_noise > 0.0f && p->noise_seed_dev);
+}
 template <typename Kern>
 int launch_item_pass(Kern kern, const cfh::CoreArgs& C, bool search, const float* wcat, hipStream_t st, const char* what) {
     {
@@ -1737,7 +1741,9 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
     if ((rc = check_core_sizes(p, N, E))) return rc;
     if (N == 0) return CFH_OK;
     const bool has_ang = p->angle_bins > 0;
-    if (!qs || !k || !v || !W_dist || (!lean && (!z || !prob)) || !hist || !out)
+    const bool search = has_ang && search_frames != 0;
+    const bool one_launch = one_launch_form(p, N, E, search, lean);
+    if (!qs || !k || !v || !W_dist || (!lean && (!z || !prob)) || (!hist && !(lean && one_launch)) || !out)
         return fail(CFH_EINVAL, "qs, k, v, W_dist, z, prob, hist and out must not be NULL");
     if (has_ang && (!W_axis1 || !W_axis2 || !W_axis3 || !frames))
         return fail(CFH_EINVAL, "the angle encoding needs W_axis1..3 and frames");
@@ -1751,7 +1757,6 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
     C.K.heads = heads;
     C.K.contiguous_neighbours = 1;
     const CoreBuffers buf = fill_core(C, p, L, qs, k, v, rvlen != nullptr, cache, workspace);
-    const bool search = has_ang && search_frames != 0;
     if (buf.table && !buf.table_ready) {
         TimedScope timed("core_tables", st);
         hipLaunchKernelGGL(cfh::sorted_shifts_kernel, dim3((unsigned)B), dim3(cfh::FC_TCAP), 0, st, tvecs, C.table_R,
@@ -1767,8 +1772,6 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
     const int hw = cfh::core_hist_words(p->angle_bins, lean);
     const cfh::WcatArgs WA{W_dist, W_axis1, W_axis2, W_axis3, hw, p->dist_coef, p->angle_coef,
                            p->angle_wscale, wcat};
-    // (the word of the noise's seed is copied and advanced by the launch that makes the records)
-    const bool one_launch = N * p->num_heads <= item_pass_max(p, N, E, lean) && !(search && p->symm_break_noise > 0.0f && C.K.seed_dev);
     if (one_launch) {
         if (!wcat_made) {
             TimedScope timed("core_prepare", st);

@@ -693,6 +693,7 @@ __global__ __launch_bounds__(WAVE * CORE_WPB) void frame_axes_kernel(const CoreA
     const int wv = (int)(threadIdx.x >> 6), lane = (int)threadIdx.x & (WAVE - 1);
     const int blk = (int)blockIdx.x;
     if (blk >= slow_blocks && blk < slow_blocks + quad_blocks) {
+        static_assert(CORE_WPB == 1, "a workgroup is a wavefront: its place is that of its atom and heads");
         frame_quad_body(C, shared[wv].quad, die_order(blk - slow_blocks, quad_blocks, CORE_DIE_SHIFT - 2), lane);      // (two workgroups: an atom's)
         return;
     }

@@ -127,7 +127,10 @@ void model_buffers(const cfh_model* m, const cfh_model_batch* b, ModelBuffers& M
                 L.h = b->keep ? c.take<float>(N * F) : (split ? c.take<float>(F / 128 * N * D) : nullptr);
                 L.frames = c.take<float>(9 * N * H);
                 if (b->keep) { L.z = c.take<float>(E * H); L.prob = c.take<float>(E * H); }
-                L.hist = c.take<float>(H * N * hw);
+                // (inference in one launch per layer keeps the histograms in LDS)
+                bool hist = b->keep != 0;
+                for (int k = 0; k < m->layers; k++) hist |= !one_launch_form(&m->layer[k].core, b->N, b->E, ang > 0, true);
+                L.hist = hist ? c.take<float>(H * N * hw) : nullptr;
                 L.out = c.take<float>(N * D);
                 L.records = c.take<uint32_t>(N * H * cfh::REC_WORDS);
             }
