@@ -591,6 +591,42 @@ def test_largest_weights(N):
     assert torch.isfinite(kept).all() and Hh.rel_err(out, kept.double()) < 2e-6      # (sums of up to 512 products)
 
 
+# Two launches, one, 32 rows per workgroup
+@pytest.mark.parametrize("N", [33, 2065, 4129])
+def test_bridges_of_inference_use_all_bits_of_their_operands(N):
+    """Against float64, with weights large enough that every product shows in the output: 4 to 5e-7 in 2-norm with float32 sums, 2.3
+    to 2.8e-6 when one operand is the sum of two bfloat16 numbers instead of three (looked at with the oracle)."""
+    from crystalframer_amd import synthetic
+    from oracle import cpu_model
+    model, cb = _one_layer_of_atoms(N)
+    names = ["input_embeddings.weight"] + ["encoder.layers.0." + n + ".weight" for n in ("self_attn.out_proj", "linear1", "linear2")]
+    names.append("encoder.layers.0.self_attn.v_proj_weight")
+    with torch.no_grad():
+        for n in names[1:]:
+            model.get_parameter(n).mul_(3.0)
+        cb.x.copy_(torch.rand(cb.x.shape, generator=torch.Generator().manual_seed(N)) - 0.5)
+        model.eval()
+        out = model(cb).cpu().double()
+    some = slice(N - 33, N)
+    one = torch.ones(33, dtype=torch.long)
+    part = synthetic.CrystalBatch(cb.x[some].cpu(), cb.pos[some].cpu(), torch.arange(33), cb.trans_vec[some].cpu(), one, zero_based=True)
+    sd = {n: t.detach().cpu().double() for n, t in model.state_dict().items()}
+
+    def oracle(sd, x):
+        batch = synthetic.CrystalBatch(x, part.pos, part.batch, part.trans_vec, one, zero_based=True)
+        return cpu_model.model_forward(sd, batch, model.params, dtype=torch.float64, windows="full")
+
+    def two_parts(t):
+        first = t.float().bfloat16().float()
+        return first.double() + (t.float() - first).bfloat16().double()
+
+    ref = oracle(sd, part.x)
+    off = lambda t: float((t - ref).norm() / ref.norm())  # noqa: E731
+    short = [off(oracle({**sd, n: two_parts(sd[n])}, part.x)) for n in names] + [off(oracle(sd, two_parts(part.x).float()))]
+    assert min(short) > 2e-6
+    assert off(out[some]) < 1e-6
+
+
 # Inference of few items: the product of an item's histogram with the weights by its own wavefront.  One atom, a few, either side
 # of the item counts where a launch of its own makes it for short rows (10 240 with an angle encoding, 16 384 without).
 @pytest.mark.parametrize("bins,B,atoms", [(64, 1, 1), (64, 3, 7), (64, 64, 10), (64, 1280, 1), (64, 1281, 1), (16, 1, 1), (16, 24, 8),
