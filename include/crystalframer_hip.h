@@ -276,6 +276,7 @@ int cfh_fused_dpa_forward(const float* q, const float* k, const float* v, const 
  * n x n block of every crystal with rows and columns in atom order (cfh_pair_layout_check), which
  * is what lets gk and gv be summed without atomics and without the transposed copies the
  * reference makes.
+ * Other pairs are safe but not summed: an atom outside such a block gets zeros in gk and gv.
  * Replaces FusedDotProductAttentionCUDA.backward: kernels irregular_transpose, fused_dpa_bwd and
  * fused_dpa_bwd_q (models/cuda_funcs/fused_dpa.py:65-170).
  */
