@@ -538,7 +538,8 @@ __device__ __forceinline__ RecordHead record_head(const KernelArgs& P, int it, i
     if (R.bx.over && P.status) atomicOr(P.status, 1);
     R.boxw = (uint32_t)(R.bx.R1 | (R.bx.R2 << 8) | (R.bx.R3 << 16));
     if (P.heads) {
-        // (sizes that do not add up to the atoms and pairs of the batch: no pairs, and the status word says so)
+        // (fewer pairs or atoms stated than the sizes make: no pairs for the atoms whose rows pass the end, and the status word
+        // says so; that the sizes are those of `batch` is taken for granted, as by the arrays)
         if (R.e0 < 0 || R.npairs < 0 || R.npairs > P.E - R.e0 || R.j0 < 0 || R.npairs > P.N - R.j0) {
             if (P.status) atomicOr(P.status, 2);
             R.e0 = R.npairs = 0;
