@@ -210,8 +210,8 @@ constexpr int COL_GROUP = 4;     // = the lanes of a slot
 // both).  Rows of 137 pairs on average: 7680 items 14.0 and 15.0, 9600 18.9 and 25.0, 11 520 21.3 and 16.6, 30 720 50 and 32;
 // of 43: 7680 7.5 and 8.9, 10 240 9.9 and 9.4, 15 360 12.6 and 10.4; of 17: 16 384 8.8 and 9.1, 24 576 12.4 and 11.6; of 13.5:
 // 7432 5.0 and 6.2, 14 672 7.9 and 8.5, 17 112 9.4 and 9.4, 19 584 10.1 and 9.6, 39 216 17.4 and 15.9; of 7: 5632 4.9 and 5.5,
-// 22 528 9.6 and 10.1, 45 056 17.8 and 18.1.  Looking at the pairs first (those of a caller) takes 1.8 us more with four columns
-// and nothing with one: 19 584 items 11.4 and 10.1, so that rows of up to 24 pairs are left to one.
+// 22 528 9.6 and 10.1, 45 056 17.8 and 18.1.  Looking at the pairs (those of a caller) takes 1.8 us more with four columns and is
+// not needed with one: 19 584 items of the operators 10.6 with one and 11.3 with four, so that rows of up to 24 pairs take one.
 inline bool column_groups(const DpaArgs& P) {
     const int64_t N = P.N, E = P.E, items = N * P.H;
     return E > 24 * N ? items >= 10240 : !P.e_start && E > 10 * N && items >= 18432;
@@ -266,7 +266,7 @@ __global__ __launch_bounds__(WAVE * DPA_WAVES) void dpa_bwd_col_kernel(const Dpa
     for (int c = 0; c < GROUP; c++) gk[c] = gv[c] = make_float4(0.f, 0.f, 0.f, 0.f);
     if (n > 0) {
         const size_t eblock = (size_t)e0 - (size_t)col * n;    // first pair of the crystal
-        const int mine = GROUP == 1 ? col : min(col + qd, n - 1);                 // (past the last column: the last again, not written)
+        const int mine = GROUP == 1 ? col : min(col + qd, n - 1);      // (past the last column: the last again, not written)
         for (int ib = 0; ib < n; ib += DPA_SLOTS) {
             const int r = ib + slot;
             if (r < n) {                                       // (the same in the lanes of a slot)
