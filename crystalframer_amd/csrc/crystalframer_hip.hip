@@ -1555,7 +1555,7 @@ int cfh_adamw_step_batch(const cfh_adamw_job* jobs, int32_t njobs, float lr, flo
 // ---- fused attention core ----------------------------------------------------------------------------------------
 namespace {
 struct CoreLayout {
-    size_t items, sorted, near, wcat, gwcat, G, slow, total;
+    size_t items, sorted, near, wcat, gwcat, G, slow, tickets, total;
     int hw;
     int prep_blocks;      // blocks of 256 threads of the launch that makes the item records
 };
@@ -1582,6 +1582,8 @@ CoreLayout core_layout(const cfh_params* p, int64_t N, int64_t E, int64_t B, boo
     off += align256(((size_t)(backward ? (N + 15) / 16 + 1 : L.prep_blocks) +
                      (size_t)(backward ? ((N + 15) / 16 + cfh::SLOW_GB_BLOCKS) * 16 * p->num_heads
                                        : (int64_t)L.prep_blocks * cfh::SLOW_PREP_SLOTS)) * sizeof(int32_t));
+    L.tickets = off;
+    if (!backward) off += align256((size_t)cfh::sixteens((int)N) * p->num_heads * cfh::TICKET_STRIDE * sizeof(int32_t));
     L.total = off;
     return L;
 }
@@ -1663,16 +1665,30 @@ int launch_core(Kern kern, const cfh::CoreArgs& C, hipStream_t st, const char* w
     }
     return finish_launch(what);
 }
-// The slices of the sum over the words: 256 words per wavefront with all moments, 144 with the nodes of inference.
-void project_launch(int hw, const float* hist, const float* wcat, float* out, int64_t N, int H, hipStream_t st) {
-    const dim3 grid((unsigned)((N + 15) / 16), (unsigned)H);
-    auto launch = [&](auto kern, int waves) {
-        hipLaunchKernelGGL(kern, grid, dim3(cfh::WAVE * waves), 0, st, hist, wcat, out, (int)N, H);
-    };
-    if (hw == cfh::HW_ANG) launch(cfh::core_project_kernel<4, 16>, 4);
-    else if (hw == cfh::HW_LEAN) launch(cfh::core_project_kernel<5, 9>, 5);
-    else if (hw == cfh::HW_ANG16) launch(cfh::core_project_kernel<2, 4>, 2);
-    else launch(cfh::core_project_kernel<1, 4>, 1);
+// The products of the items from place `from` of the work order on (a multiple of 128; 0 where the histograms lie in the order
+// of the atoms).
+template <int HWK, bool PLACES>
+void project_launch(const cfh::CoreArgs& C, const float* wcat, int from, hipStream_t st) {
+    const int first = from / 128 * 8, N = C.K.N, last = PLACES ? cfh::sixteens(N) : (N + 15) / 16;
+    if (last > first)
+        hipLaunchKernelGGL((cfh::core_project_kernel<HWK, PLACES>), dim3((unsigned)(last - first), (unsigned)C.K.H),
+                           dim3(cfh::WAVE * cfh::ProjectSlices<HWK>::N), 0, st, C.hist, wcat, C.K.items, C.out, N, C.K.H, first);
+}
+// Inference in several launches per layer: the items up to this place of the work order (a multiple of 128) have their products
+// made in the main kernel (core_project_done).  The last fifth, at least 64 per compute unit (three times what is resident), is
+// left to a launch: a wavefront that makes products at the end of the main kernel has nobody left to hide behind, and the rows
+// written last are read back fast.  Whole passes of four layers, 64 bins, in us: all in a launch / left to it 32, 64, 140, 200 and
+// 300 per compute unit: 180 224 items 2992/2728, 2722, 2660, 2699, 2743; 132 000 items 2271/-, 2069, 2058, 2075, 2114; 90 112
+// items 1543/1420, 1393, 1414; 45 056 items 898/861, 852, 885; 76 736 items of long rows 1664/1620, 1587, 1599; 18 976 of long rows
+// 512/522, 509, 507.  16 bins (128 words): 90 112 items 1576/1551, 1549, 1557; 45 056 951/942, 942, 952.  Distances alone
+// (64 words) lose 10 us per layer to the tickets at 180 224 items.
+int products_in_place(const cfh_params* p, int64_t N, int hw) {
+    int cus = device_cus();
+    if (cus <= 0) cus = 256;
+    // (the offsets of the words within a head have 32 bits)
+    if (p->angle_bins == 0 || N * hw >= (int64_t)1 << 29) return 0;
+    const int64_t items = N * p->num_heads, left = items / 5 > 64 * (int64_t)cus ? items / 5 : 64 * (int64_t)cus;
+    return items > left ? (int)((items - left) / (128 * p->num_heads) * 128) : 0;
 }
 // Up to this many (atom, head) items the forward pass of a layer is one launch, one wavefront per item from the record to the
 // sums, instead of records, frame search and main kernel: about as many as are resident at once (19 to 23 per compute unit) and,
@@ -1780,6 +1796,10 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
         if (search) { C.K.q = qs; C.K.k = k; C.K.out_frame = frames; C.K.frames_to_records = 1; }
         else C.K.frames = has_ang ? frames : nullptr;
     } else {
+        if (lean && (C.ticket_items = products_in_place(p, N, hw)) > 0) {
+            C.K.tickets = C.tickets = reinterpret_cast<int32_t*>(ws + L.tickets);
+            C.wcat = wcat;
+        }
         const int prep_blocks = L.prep_blocks, wcat_blocks = wcat_made ? 0 : p->num_heads * cfh::DH;
         // records whose box is not the table's are listed by the launch that makes them and taken first by the main kernel
         if (buf.table) {
@@ -1847,7 +1867,11 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
     if (rc || (one_launch && lean)) return rc;
     {
         TimedScope timed("core_project", st);
-        project_launch(hw, hist, wcat, out, N, p->num_heads, st);
+        if (hw == cfh::HW_ANG) project_launch<cfh::HW_ANG, false>(C, wcat, 0, st);
+        else if (hw == cfh::HW_LEAN) project_launch<cfh::HW_LEAN, true>(C, wcat, C.ticket_items, st);
+        else if (hw == cfh::HW_DIST) project_launch<cfh::HW_DIST, false>(C, wcat, 0, st);
+        else if (lean) project_launch<cfh::HW_ANG16, true>(C, wcat, C.ticket_items, st);
+        else project_launch<cfh::HW_ANG16, false>(C, wcat, 0, st);
     }
     return finish_launch("fused_core_project");
 }

@@ -391,7 +391,9 @@ struct KernelArgs {
     unsigned long long* seed_snap;
     int32_t seed_advance;
     BasisConsts bc;
+    int32_t* tickets;             // words that the launch of the records clears, TICKET_STRIDE apart, one per (16 items, head); or null
 };
+constexpr int TICKET_STRIDE = 32;      // ints between two of them: a line each
 
 // Work distribution.  Wavefront w (= blockIdx.x) serves head w % H.  The items (atoms, visited in
 // `order`: descending neighbour count, i.e. longest first) of a head are dealt round-robin to NQUEUE
@@ -500,6 +502,14 @@ __device__ __forceinline__ int die_order(int b, int total, int shift) {
     if (b >= total - (total & (span - 1))) return b;
     return (((((b >> (shift + 3)) << 3) | (b & 7)) << shift)) | ((b >> 3) & ((1 << shift) - 1));
 }
+// Sixteen items of a head whose products with the weights are made together: every eighth place of 128 of the work order, the
+// atoms that die_order gives to one die.  How many there are for N atoms, which one a place belongs to, its rank among the
+// sixteen, and back.
+__host__ __device__ constexpr int sixteens(int N) { return (N + 127) / 128 * 8; }
+__device__ __forceinline__ int sixteen_of(int it) { return (it >> 7) * 8 + (it & 7); }
+__device__ __forceinline__ int sixteen_rank(int it) { return (it >> 3) & 15; }
+__device__ __forceinline__ int sixteen_place(int sixteen, int rank) { return (sixteen >> 3) * 128 + rank * 8 + (sixteen & 7); }
+__device__ __forceinline__ int sixteen_members(int sixteen, int N) { return max(0, min(16, (N - sixteen_place(sixteen, 0) + 7) >> 3)); }
 // Tables in the kernel arguments whose entries have ascending first numbers: the entry that number b (the same in all lanes)
 // belongs to, the last whose first(entry) is not above it.  Every lane looks at an entry of its own: one after the other, each
 // is a load that waits for the arguments' memory (25 entries: linear_wgrad_batch_kernel 69 -> 64 us, linear_wgrad_sum_kernel
@@ -588,6 +598,7 @@ __device__ __forceinline__ void prepare_items_block(const KernelArgs& P, int wit
         P.counters[idx * QSTRIDE] = 0;
         if (P.counters2) P.counters2[idx * QSTRIDE] = 0;
     }
+    if (P.tickets && idx < sixteens(P.N) * P.H) P.tickets[idx * TICKET_STRIDE] = 0;
     if (idx == 0 && with_query && P.seed_dev) {
         const unsigned long long s = *P.seed_dev;
         *P.seed_snap = s;

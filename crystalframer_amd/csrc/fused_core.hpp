@@ -122,7 +122,10 @@ struct CoreArgs {
     float* out;                   // (N,H,16) sum_j P_ij v_j (core_project_kernel adds W . hist)
     float* prob;                  // (E,H) P_ij
     float* z;                     // (E,H)
-    float* hist;                  // (H,N,hw)
+    float* hist;                  // (H,N,hw); inference with angles: (H, 16 sixteens(N), hw), row 16 sixteen_of(it) + rank
+    const float* wcat;            // (H,16,hw) weights of the products (with `tickets`)
+    int32_t* tickets;             // per (16 items, head) how many of them are done (core_project_done); or null
+    int32_t ticket_items;         // the places of the work order, from the start, that draw tickets
     // backward operands and results
     const float* go;              // (N,H,16) upstream gradient of out
     const float* outv;            // (N,H,16) the forward's final out
@@ -590,6 +593,119 @@ __device__ __forceinline__ float wave_sum4(const float (&v)[4], int lane) {
     s += dpp_move<0xB1>(s); s += dpp_move<0x4E>(s); s += dpp_move<0x141>(s);
     return s + dpp_move<0x128>(s);
 }
+// ---- products with the weights -----------------------------------------------------------------------------------
+// out (N,H,16) += Wcat_h (16, hw) . hist: sixteen items of a head through MFMA 16x16x4, the sum over the words in slices
+// that are added in a fixed order (256 words per slice with all moments, 144 with the nodes of inference), whichever
+// wavefront makes them: the result depends neither on timing nor on which of the two places below makes it.
+//   core_project_done     in the main kernel, by the wavefront that completes the sixteen;
+//   core_project_kernel   in a launch of its own, a workgroup per sixteen, a wavefront per slice.
+// The launch is bound by reading the histograms back: 519 MB (22 528 atoms, 720 words) in 131 us (4.0 TB/s).
+template <int HWK> struct ProjectSlices;
+template <> struct ProjectSlices<HW_ANG> { static constexpr int N = 4, UNITS = 16, BATCH = 8; };
+template <> struct ProjectSlices<HW_LEAN> { static constexpr int N = 5, UNITS = 9, BATCH = 5; };
+template <> struct ProjectSlices<HW_ANG16> { static constexpr int N = 2, UNITS = 4, BATCH = 4; };
+template <> struct ProjectSlices<HW_DIST> { static constexpr int N = 1, UNITS = 4, BATCH = 4; };
+// A slice: UNITS x 16 words, BATCH units' loads in flight together.  a(u): the four words of this lane's row of unit u; bp: its
+// weights.  The four lanes of a row read 64 consecutive bytes per load; which word of the sum a lane holds does not matter as
+// long as both operands agree.
+template <int UNITS, int BATCH, typename Load>
+__device__ __forceinline__ v4f_c project_slice(Load&& a, const float4* bp) {
+    v4f_c acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u0 = 0; u0 < UNITS; u0 += BATCH) {
+        float4 a4[BATCH], b4[BATCH];
+#pragma unroll
+        for (int u = 0; u < BATCH; u++)
+            if (u0 + u < UNITS) { a4[u] = a(u0 + u); b4[u] = bp[4 * (u0 + u)]; }
+        __builtin_amdgcn_sched_barrier(0);         // (all loads in flight before the first product)
+#pragma unroll
+        for (int u = 0; u < BATCH; u++) {
+            if (u0 + u >= UNITS) continue;
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[u].x, b4[u].x, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[u].y, b4[u].y, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[u].z, b4[u].z, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[u].w, b4[u].w, acc, 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    return acc;
+}
+
+// What wavefronts of other compute units and dies read in the same launch is written, and read, at device scope: the store goes
+// through to the memory behind the dies' L2s, the load takes nothing that an L1 or another die's L2 holds from before.  With
+// s_waitcnt between a wavefront's stores and its ticket, and a ticket that is drawn at device scope, whoever draws the last of
+// sixteen tickets reads what the other fifteen wrote; no cache is written back or emptied as a whole, which a fence of that
+// scope does (199 us for a launch of 2372 atoms' weight gradients with a fence before every ticket).
+constexpr int CPOL_DEVICE = 16;      // sc1
+typedef int v4i_c __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t device_rsrc(float* p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(p, 0, (int)bytes, 0x00027000);
+}
+__device__ __forceinline__ float4 load_device4(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+    const v4i_c v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, CPOL_DEVICE);
+    return make_float4(__int_as_float(v.x), __int_as_float(v.y), __int_as_float(v.z), __int_as_float(v.w));
+}
+__device__ __forceinline__ void store_device4(__amdgpu_buffer_rsrc_t r, uint32_t off, float4 v) {
+    const v4i_c w = {__float_as_int(v.x), __float_as_int(v.y), __float_as_int(v.z), __float_as_int(v.w)};
+    __builtin_amdgcn_raw_buffer_store_b128(w, r, (int)off, 0, CPOL_DEVICE);
+}
+__device__ __forceinline__ void store_device(float* p, float v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// A lane's row of the histograms and the atom it belongs to: rank (lane & 15) of the sixteen.  (A rank past the last member
+// takes the last.)
+struct ProjectRow { int atom; uint32_t row; };
+__device__ __forceinline__ ProjectRow project_row(const uint32_t* records, int sixteen, int members, int h, int H, int lane) {
+    const int rank = min(lane & 15, members - 1);
+    ProjectRow R;
+    R.atom = (int)records[((size_t)sixteen_place(sixteen, rank) * H + h) * REC_WORDS + REC_ATOM];
+    R.row = (uint32_t)(sixteen * 16 + rank);
+    return R;
+}
+// Rows of a head's histograms where they lie in the order of the sixteens.
+__host__ __device__ constexpr int project_rows(int N) { return 16 * sixteens(N); }
+
+// Inference of many items with the angle encoding: the item of this wavefront is done, its histogram row and its part of `out`
+// stored at device scope.  Draws the ticket of its sixteen; whoever draws the last one makes their products.  What is read so is
+// still in the dies' memory-side cache, and the product's 180 matrix instructions run beside the other wavefronts' vector ones: 22 528
+// atoms at 64 bins main kernel 393 us + products 131 in a launch of their own -> 449 + 30 (the last fifth, see products_in_place).
+// Sixteen items of ONE die: were they dealt over the dies, the one that happens to be behind would draw the last ticket of
+// nearly all, make the products alone and fall further behind (seven dies done after 416 us, the eighth after 1085).
+// Training, whose rows have 1024 words in the order of the atoms, keeps the launch: 18 976 items 80 us in two launches, 84 so.
+template <int HWK>
+__device__ __forceinline__ void core_project_done(const CoreArgs& C, int it, int h, int lane) {
+    using S = ProjectSlices<HWK>;
+    const int H = C.K.H, N = C.K.N, sixteen = sixteen_of(it), members = sixteen_members(sixteen, N);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    int ticket = 0;
+    if (lane == 0)
+        ticket = __hip_atomic_fetch_add(C.tickets + (sixteen * H + h) * TICKET_STRIDE, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__builtin_amdgcn_readfirstlane(ticket) != members - 1) return;
+    asm volatile("" ::: "memory");
+    const int col = lane & 15, kk = lane >> 4, rows = project_rows(N);
+    const ProjectRow R = project_row(C.K.items, sixteen, members, h, H, lane);
+    const __amdgpu_buffer_rsrc_t hist = device_rsrc(C.hist + (size_t)h * rows * HWK, (uint32_t)rows * (HWK * 4u));
+    uint32_t aoff = (R.row * HWK + 4u * kk) * 4u;
+    const float4* bp = reinterpret_cast<const float4*>(C.wcat + ((size_t)h * DH + col) * HWK) + kk;
+    v4f_c sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int s = 0; s < S::N; s++) {
+        const v4f_c acc = project_slice<S::UNITS, S::BATCH>([&](int u) { return load_device4(hist, aoff + 64u * u); }, bp);
+        if (s == 0) sum = acc;
+        else sum += acc;
+        aoff += 64u * S::UNITS;
+        bp += 4 * S::UNITS;
+    }
+    // component r of lane (kk, col): rank 4 kk + r, channel col
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        float* dst = C.out + ((size_t)__shfl(R.atom, 4 * kk + r) * H + h) * DH + col;
+        const float own = __hip_atomic_load(dst, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (4 * kk + r < members) *dst = own + sum[r];
+    }
+}
+
 // ANG: angle bins, 0 (distance encoding alone), 64 (moment series) or 16 (basis values added directly)
 // wid: this wavefront's (item, head)
 // wcat: not null: the wavefront makes the product of its histogram with the head's weights itself, the histogram stays in
@@ -606,6 +722,7 @@ __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLd
     constexpr bool VEC = HWL == HWK && HWK >= 4 * WAVE;      // clear, rescale and store four words per lane at a time
     constexpr int NW = VEC ? (HWK / 4 + WAVE - 1) / WAVE : 1;
     constexpr bool FULL = HWK % (4 * WAVE) == 0;
+    constexpr bool PLACES = LEAN && HAS_ANG;                 // histograms in the order of the sixteens
     float4* const tab = sh.tab;
     uint16_t* const list = sh.list;
     int32_t* const hist = sh.hist;
@@ -1000,12 +1117,17 @@ __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLd
             }
         } else {
             const float ox = rows8_sum(accv.x) * inv, oy = rows8_sum(accv.y) * inv;
-            if (lane < FC_GROUP) *reinterpret_cast<float2*>(C.out + ih * DH + 2 * sub) = make_float2(ox, oy);
+            if (lane < FC_GROUP) {
+                if (PLACES) { store_device(C.out + ih * DH + 2 * sub, ox); store_device(C.out + ih * DH + 2 * sub + 1, oy); }
+                else *reinterpret_cast<float2*>(C.out + ih * DH + 2 * sub) = make_float2(ox, oy);
+            }
         }
         if (!(LEAN && wcat)) {
             // all reads first (one LDS round trip instead of one per word), then store; a lane takes four
             // consecutive words at a time
-            float* dst = C.hist + ((size_t)h * P.N + i) * HWK;      // head-major: the rows of a head are contiguous
+            // head-major: the rows of a head are contiguous
+            float* dst = C.hist + (PLACES ? (size_t)h * project_rows(P.N) + sixteen_of(it_cur) * 16 + sixteen_rank(it_cur)
+                                          : (size_t)h * P.N + i) * HWK;
             if (ANG == SMALL_A) {
                 // distance bins as they are, every angle bin as the sum of its copies (integers: any order), zeros behind
                 for (int u = lane; u < HWK; u += WAVE) {
@@ -1015,17 +1137,22 @@ __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLd
 #pragma unroll
                         for (int c = 0; c < A16_COPIES; c++) sum += hist[HW_DIST + c * A16_STRIDE + (u - HW_DIST)];
                     }
-                    dst[u] = (float)sum * sc;
+                    if (PLACES) store_device(dst + u, (float)sum * sc);
+                    else dst[u] = (float)sum * sc;
                 }
             } else if (VEC) {
                 int4 hv[NW];
 #pragma unroll
                 for (int u = 0; u < NW; u++)
                     if (FULL || lane + WAVE * u < HWL / 4) hv[u] = reinterpret_cast<const int4*>(hist)[lane + WAVE * u];
+                const __amdgpu_buffer_rsrc_t words = device_rsrc(dst, HWK * 4u);
 #pragma unroll
                 for (int u = 0; u < NW; u++)
-                    if (FULL || lane + WAVE * u < HWL / 4) reinterpret_cast<float4*>(dst)[lane + WAVE * u] =
-                        make_float4((float)hv[u].x * sc, (float)hv[u].y * sc, (float)hv[u].z * sc, (float)hv[u].w * sc);
+                    if (FULL || lane + WAVE * u < HWL / 4) {
+                        const float4 v = make_float4((float)hv[u].x * sc, (float)hv[u].y * sc, (float)hv[u].z * sc, (float)hv[u].w * sc);
+                        if (PLACES) store_device4(words, 16u * (lane + WAVE * u), v);
+                        else reinterpret_cast<float4*>(dst)[lane + WAVE * u] = v;
+                    }
             } else {
                 for (int u = lane; u < HWK; u += WAVE) dst[u] = (float)hist[u] * sc;
             }
@@ -1042,6 +1169,7 @@ __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLd
                 }
             }
         }
+        if (PLACES && !own && it_cur < C.ticket_items) core_project_done<HWK>(C, it_cur, h, lane);
         CFH_PH_FLUSH(P.stats);
         if (P.stats && lane == 0) {
             atomicAdd(P.stats + STAT_FWD_EVAL, n_eval);
@@ -1062,48 +1190,37 @@ void fused_core_fwd_kernel(const CoreArgs C) {
     if (wid >= 0) fused_core_fwd_body<WL, ANG, COS_ABS, LEAN>(C, shared[threadIdx.x >> 6], wid);
 }
 
-// out (N,H,16) += Wcat_h (16, hw) . hist (H,N,hw): one workgroup of WAVES wavefronts per (16 atoms, head); each
-// wavefront takes UNITS x 16 words of the reduction index through MFMA 16x16x4 (the four lanes of a row read 64
-// consecutive bytes of it per load), the slices meet in LDS and are added in a fixed order by the first
-// wavefront (no atomics: the result does not depend on timing).  grid (ceil(N/16), H), block 64 * WAVES.
-// Bound by reading the histograms: 519 MB (22 528 atoms, 720 words) in 131 us (4.0 TB/s).  Measured at 640 words, 119 us: 129
-// with half of the loads ahead of the products; 115 with four tiles per workgroup and the weights in registers.
-template <int WAVES, int UNITS>
-__global__ __launch_bounds__(WAVE * WAVES) void core_project_kernel(const float* __restrict__ hist, const float* __restrict__ wcat,
-                                                                    float* __restrict__ out, int N, int H) {
-    constexpr int hw = WAVES * UNITS * 16;
-    __shared__ float part[WAVES][4][WAVE];
+// A workgroup per sixteen items and head, a wavefront per slice; the slices meet in LDS and the first wavefront adds them in
+// their order.  PLACES: histograms in the order of the sixteens, from sixteen `first` on; else in the order of the atoms,
+// sixteen consecutive ones.  grid (sixteens, H).
+template <int HWK, bool PLACES>
+__global__ __launch_bounds__(WAVE * ProjectSlices<HWK>::N) void core_project_kernel(const float* __restrict__ hist,
+        const float* __restrict__ wcat, const uint32_t* __restrict__ records, float* __restrict__ out, int N, int H, int first) {
+    using S = ProjectSlices<HWK>;
+    __shared__ float part[S::N][4][WAVE];
     const int lane = threadIdx.x & (WAVE - 1), wv = threadIdx.x >> 6, col = lane & 15, kk = lane >> 4;
-    const int h = blockIdx.y, i0 = blockIdx.x * 16;
-    const int row = min(i0 + col, N - 1);
-    // the four lanes (kk) of a row read 64 consecutive bytes per load; which word of the reduction index a lane
-    // holds does not matter as long as both operands agree
-    const float4* ap = reinterpret_cast<const float4*>(hist + ((size_t)h * N + row) * hw + wv * UNITS * 16) + kk;
-    const float4* bp = reinterpret_cast<const float4*>(wcat + ((size_t)h * DH + col) * hw + wv * UNITS * 16) + kk;
-    v4f_c acc = {0.f, 0.f, 0.f, 0.f};
-    float4 a4[UNITS], b4[UNITS];
-#pragma unroll
-    for (int u = 0; u < UNITS; u++) { a4[u] = ap[4 * u]; b4[u] = bp[4 * u]; }
-    __builtin_amdgcn_sched_barrier(0);         // (all loads in flight before the first product)
-#pragma unroll
-    for (int u = 0; u < UNITS; u++) {
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[u].x, b4[u].x, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[u].y, b4[u].y, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[u].z, b4[u].z, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[u].w, b4[u].w, acc, 0, 0, 0);
-    }
+    const int h = blockIdx.y, sixteen = first + (int)blockIdx.x;
+    const int members = PLACES ? sixteen_members(sixteen, N) : min(16, N - sixteen * 16);
+    if (members <= 0) return;
+    ProjectRow R;
+    if (PLACES) R = project_row(records, sixteen, members, h, H, lane);
+    else R.row = R.atom = min(sixteen * 16 + col, N - 1);
+    const float4* ap = reinterpret_cast<const float4*>(hist + ((size_t)h * (PLACES ? project_rows(N) : N) + R.row) * HWK +
+                                                       wv * S::UNITS * 16) + kk;
+    const float4* bp = reinterpret_cast<const float4*>(wcat + ((size_t)h * DH + col) * HWK + wv * S::UNITS * 16) + kk;
+    const v4f_c acc = project_slice<S::UNITS, S::UNITS>([&](int u) { return ap[4 * u]; }, bp);
 #pragma unroll
     for (int r = 0; r < 4; r++) part[wv][r][lane] = acc[r];
     __syncthreads();
     if (wv != 0) return;
-    // component r of lane (kk, col): atom 4 kk + r of the tile, channel col
+    // component r of lane (kk, col): rank 4 kk + r, channel col
 #pragma unroll
     for (int r = 0; r < 4; r++) {
         float sum = part[0][r][lane];
 #pragma unroll
-        for (int w = 1; w < WAVES; w++) sum += part[w][r][lane];
-        const int it = i0 + 4 * kk + r;
-        if (it < N) out[((size_t)it * H + h) * DH + col] += sum;
+        for (int w = 1; w < S::N; w++) sum += part[w][r][lane];
+        const int i = PLACES ? __shfl(R.atom, 4 * kk + r) : sixteen * 16 + 4 * kk + r;
+        if (4 * kk + r < members) out[((size_t)i * H + h) * DH + col] += sum;
     }
 }
 

@@ -130,7 +130,7 @@ void model_buffers(const cfh_model* m, const cfh_model_batch* b, ModelBuffers& M
                 // (inference in one launch per layer keeps the histograms in LDS)
                 bool hist = b->keep != 0;
                 for (int k = 0; k < m->layers; k++) hist |= !one_launch_form(&m->layer[k].core, b->N, b->E, ang > 0, true);
-                L.hist = hist ? c.take<float>(H * N * hw) : nullptr;
+                L.hist = hist ? c.take<float>(H * (size_t)(b->keep || ang == 0 ? N : cfh::project_rows((int)N)) * hw) : nullptr;
                 L.out = c.take<float>(N * D);
                 L.records = c.take<uint32_t>(N * H * cfh::REC_WORDS);
             }

@@ -647,6 +647,33 @@ def test_products_of_few_items(bins, B, atoms):
     assert Hh.rel_err(out, kept.double()) < 5e-6
 
 
+# Inference of many items with the angle encoding: the wavefront that completes sixteen items of a head makes their products, but
+# for the last items (a fifth, at least 16 384 on 256 compute units).  One atom short of the first 128 atoms whose products are
+# made so, exactly those, a last block of one atom and of 127, rows of mixed lengths, sixteen heads.
+@pytest.mark.parametrize("bins,B,atoms,width", [(64, 2175, (1, 1), 128), (64, 2176, (1, 1), 128), (16, 2177, (1, 1), 128),
+                                                (64, 2303, (1, 1), 128), (64, 4097, (1, 1), 128), (64, 640, (1, 9), 128),
+                                                (16, 700, (1, 9), 128), (64, 60, (30, 61), 128), (64, 1425, (1, 1), 256)])
+def test_products_by_the_wavefront_that_completes_sixteen_items(bins, B, atoms, width):
+    """Against the same pass with everything kept, whose products have a launch of their own (tolerance as above), and bit for bit
+    the same from call to call, on other crystals in between."""
+    from crystalframer_amd import params, synthetic
+    kw = dict(value_pe_angle_wscale=1.0, value_pe_dist_coef=1.5, value_pe_angle_coef=6.0) if bins == 16 else {}
+    mp = params.ModelParams(num_layers=1, value_pe_angle_real=bins, symm_break_noise=0.0, model_dim=width, head_num=width // 16,
+                            embedding_dim=[width], **kw)
+    make = lambda seed: synthetic.make_batch(B, atoms="uniform", atoms_lo=atoms[0], atoms_hi=atoms[1], len_lo=3.0, len_hi=9.0,  # noqa: E731
+                                             ang_lo=65.0, ang_hi=115.0, seed=seed)
+    model, cb = _model(mp, make(B))
+    other = make(B + 1).to("cuda")
+    model.eval()
+    kept = model(cb).detach()
+    with torch.no_grad():
+        out = model(cb)
+        for _ in range(3):
+            model(other)
+            assert torch.equal(model(cb), out)
+    assert Hh.rel_err(out, kept.double()) < 5e-6
+
+
 # Either side of the item counts up to which a layer's items take one launch, crystals of as many atoms as the row has pairs.  With
 # everything kept: 5120 with an angle encoding (8 atoms), 6144 from 13 atoms on, 4096 from 33, none from 65; 10 240 without (8
 # atoms), 5120 from 17 atoms on.  Inference: 10 240 (8, 24 and 40 atoms), 16 384 without an angle encoding for up to 12 atoms, 5120
