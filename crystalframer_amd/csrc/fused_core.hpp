@@ -572,18 +572,80 @@ __device__ __forceinline__ bool core_record_taken_elsewhere(const CoreArgs& C, u
 // =================================================================================================================
 // forward
 // =================================================================================================================
+// The distance bins of an item exist COPIES times in LDS, a copy per value of the lane's lowest bits, where there are many items:
+// most images of an item lie at nearly the same distance, a few bins of 64, and the lanes of an atomic instruction that meet on
+// a word go one after the other (inference of 180 224 items, 64 angle bins: LDS busy for 134 M clocks, 72 M of them such waits;
+// distances alone 78 M and 37 M).  4096 crystals, four layers, in us: 64 angle bins 1 copy 2650, 2 copies 2588, 4 (less LDS for
+// other wavefronts) 2655.  Rows of 40 to 200 pairs in
+// training lose 0.6 % with 2 copies, few items (item_pass_kernel) 0.5 to 1.3 %.
+constexpr int DIST_STRIDE = NBINS + 8;      // words from one copy to the next: other banks
+// An item's histogram in LDS: its words, then the further copies of its distance bins.
+template <int ANG, bool LEAN, int COPIES>
+struct CoreHist {
+    static constexpr int WORDS = LEAN && ANG == NBINS ? core_hist_words(ANG, LEAN) : core_hist_lds_words(ANG);
+    static constexpr int FIRST = WORDS + 8;      // (other banks than copy 0)
+    static constexpr int ALL = COPIES > 1 ? FIRST + (COPIES - 1) * DIST_STRIDE : WORDS;
+    static_assert(WORDS % 4 == 0 && ALL % 4 == 0 && (COPIES & (COPIES - 1)) == 0, "");
+    static constexpr __host__ __device__ int copy(int c) { return c == 0 ? 0 : FIRST + (c - 1) * DIST_STRIDE; }
+    // first word of the distance bins that this lane adds to
+    static __device__ __forceinline__ int dist_word(int lane) {
+        const int c = lane & (COPIES - 1);
+        return COPIES > 1 && c > 0 ? FIRST + (c - 1) * DIST_STRIDE : 0;
+    }
+    // word / four words with the copies of the distance bins added
+    static __device__ __forceinline__ int word(const int32_t* hist, int w) {
+        int v = hist[w];
+        if (COPIES > 1 && w < NBINS) {
+#pragma unroll
+            for (int c = 1; c < COPIES; c++) v += hist[copy(c) + w];
+        }
+        return v;
+    }
+    static __device__ __forceinline__ int4 word4(const int32_t* hist, int u) {
+        int4 v = reinterpret_cast<const int4*>(hist)[u];
+        if (COPIES > 1 && u < NBINS / 4) {
+#pragma unroll
+            for (int c = 1; c < COPIES; c++) {
+                const int4 w = reinterpret_cast<const int4*>(hist + copy(c))[u];
+                v.x += w.x; v.y += w.y; v.z += w.z; v.w += w.w;
+            }
+        }
+        return v;
+    }
+    static __device__ __forceinline__ void clear(int32_t* hist, int lane) {
+#pragma unroll
+        for (int u = 0; u < (ALL / 4 + WAVE - 1) / WAVE; u++)
+            if (ALL % (4 * WAVE) == 0 || lane + WAVE * u < ALL / 4) reinterpret_cast<int4*>(hist)[lane + WAVE * u] = make_int4(0, 0, 0, 0);
+    }
+    // times fac, rounded once per word: the copies are added up first
+    static __device__ __forceinline__ void rescale(int32_t* hist, float fac, int lane) {
+        constexpr int NU = (WORDS / 4 + WAVE - 1) / WAVE;
+        int4 v[NU];
+#pragma unroll
+        for (int u = 0; u < NU; u++)
+            if (WORDS % (4 * WAVE) == 0 || lane + WAVE * u < WORDS / 4) v[u] = word4(hist, lane + WAVE * u);
+        if (COPIES > 1 && lane < NBINS / 4) {
+#pragma unroll
+            for (int c = 1; c < COPIES; c++) reinterpret_cast<int4*>(hist + copy(c))[lane] = make_int4(0, 0, 0, 0);
+        }
+#pragma unroll
+        for (int u = 0; u < NU; u++)
+            if (WORDS % (4 * WAVE) == 0 || lane + WAVE * u < WORDS / 4) reinterpret_cast<int4*>(hist)[lane + WAVE * u] =
+                make_int4(rint_i((float)v[u].x * fac), rint_i((float)v[u].y * fac), rint_i((float)v[u].z * fac), rint_i((float)v[u].w * fac));
+    }
+};
 template <int HWK, int NLOGIT>
 struct CoreFwdShared {
     float4 tab[FC_TCAP];
     uint16_t list[FC_LISTCAP];
-    int32_t hist[HWK];
+    __attribute__((aligned(16))) int32_t hist[HWK];
     float4 pairA[FC_GROUP];      // rx, ry, rz, d2min
     float pairC[FC_GROUP];       // exp(logit - running max) / S in fixed-point units
     float logit_s[NLOGIT];       // logits of the row (rows of more pairs park them in the probability array)
 };
 // LEAN: inference, nothing is kept for a backward pass: fewer nodes for the moments; z and the probabilities are not written.
-template <int ANG, bool LEAN>
-using CoreFwdLds = CoreFwdShared<LEAN && ANG == NBINS ? core_hist_words(ANG, LEAN) : core_hist_lds_words(ANG), LEAN ? 4 : FC_LOGCAP>;
+template <int ANG, bool LEAN, int COPIES = 1>
+using CoreFwdLds = CoreFwdShared<CoreHist<ANG, LEAN, COPIES>::ALL, LEAN ? 4 : FC_LOGCAP>;
 // Sums of 4 values over the lanes of a wavefront: lane l gets the sum of value l / 16.
 __device__ __forceinline__ float wave_sum4(const float (&v)[4], int lane) {
     // each step halves the values a lane holds: it keeps one half and hands its partner the other
@@ -712,12 +774,13 @@ __device__ __forceinline__ void core_project_done(const CoreArgs& C, int it, int
 // LDS (LEAN only)
 // own: not null: the item's record and first operands, in registers
 struct CoreOwn { uint32_t rec; CorePrefetch pf; };
-template <int WL, int ANG, bool COS_ABS, bool LEAN>
-__device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLds<ANG, LEAN>& sh, int wid,
+template <int WL, int ANG, bool COS_ABS, bool LEAN, int COPIES = 1>
+__device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLds<ANG, LEAN, COPIES>& sh, int wid,
                                                     const float* __restrict__ wcat = nullptr, const CoreOwn* own = nullptr) {
     constexpr bool HAS_ANG = ANG > 0;
     constexpr int HWK = core_hist_words(ANG, LEAN);          // words per item in memory
-    constexpr int HWL = LEAN && ANG == NBINS ? HWK : core_hist_lds_words(ANG);      // ... and in LDS
+    using Hist = CoreHist<ANG, LEAN, COPIES>;
+    constexpr int HWL = Hist::WORDS;                         // ... and in LDS
     constexpr int NODES = LEAN ? LEAN_NODES : NBINS;
     constexpr bool VEC = HWL == HWK && HWK >= 4 * WAVE;      // clear, rescale and store four words per lane at a time
     constexpr int NW = VEC ? (HWK / 4 + WAVE - 1) / WAVE : 1;
@@ -743,13 +806,8 @@ __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLd
     const float INF = __builtin_inff();
 
     if (it_cur >= P.N) return;
-    if (VEC) {
-#pragma unroll
-        for (int u = 0; u < NW; u++)
-            if (FULL || lane + WAVE * u < HWL / 4) reinterpret_cast<int4*>(hist)[lane + WAVE * u] = make_int4(0, 0, 0, 0);
-    } else {
-        for (int u = lane; u < HWL; u += WAVE) hist[u] = 0;
-    }
+    Hist::clear(hist, lane);
+    const int dist0 = Hist::dist_word(lane);
     wave_sync();
 
     CFH_PH_DECL
@@ -871,11 +929,7 @@ __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLd
                         start = max(0, min(start, NBINS - WLr));
                         const float beta_c = ((float)(start + WLr / 2 + 1) - u) * bc.len_step;
                         const WindowSeed s = window_seed(beta_c, bc.len_step, w);
-#ifndef CFH_EXP_NOCONFLICT
-                        window_scatter_rn<WL>(hist + start, s, bc.len_cc, WLr);
-#else
-                        window_scatter_rn<WL>(hist + (start & 0) + lane, s, bc.len_cc, WLr);
-#endif
+                        window_scatter_rn<WL>(hist + dist0 + start, s, bc.len_cc, WLr);
                     }
                     if (HAS_ANG) {
                         if (d2 > 1e-5f) {       // the self image contributes to S and the distance encoding only
@@ -895,11 +949,7 @@ __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLd
                                 }
                                 const float mf = clampf(__builtin_rintf(uu), 0.0f, (float)(NODES - 1));
                                 const float eps = 2.0f * (uu - mf);
-#ifndef CFH_EXP_NOCONFLICT
                                 int32_t* hb = hist + HW_DIST + ax * NORD * NODES + (int)mf;
-#else
-                                int32_t* hb = hist + HW_DIST + ax * NORD * NBINS + ((int)mf & 0) + lane;
-#endif
                                 float val = w;
                                 atomicAdd(hb, rint_i(val));
 #pragma unroll
@@ -984,19 +1034,7 @@ __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLd
             if (gmax > m_run) {
                 if (m_run > -INF) {
                     const float fac = hw_exp2((m_run - gmax) * LOG2E);
-                    if (VEC) {
-                        int4 hv[NW];
-#pragma unroll
-                        for (int u = 0; u < NW; u++)
-                            if (FULL || lane + WAVE * u < HWL / 4) hv[u] = reinterpret_cast<const int4*>(hist)[lane + WAVE * u];
-#pragma unroll
-                        for (int u = 0; u < NW; u++)
-                            if (FULL || lane + WAVE * u < HWL / 4) reinterpret_cast<int4*>(hist)[lane + WAVE * u] =
-                                make_int4(rint_i((float)hv[u].x * fac), rint_i((float)hv[u].y * fac),
-                                          rint_i((float)hv[u].z * fac), rint_i((float)hv[u].w * fac));
-                    } else {
-                        for (int u = lane; u < HWL; u += WAVE) hist[u] = rint_i((float)hist[u] * fac);
-                    }
+                    Hist::rescale(hist, fac, lane);
                     accv.x *= fac; accv.y *= fac; Dl *= fac;
                 }
                 m_run = gmax;
@@ -1062,7 +1100,7 @@ __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLd
 #pragma unroll
                 for (int u = 0; u < NW; u++) {
                     int4 hv = make_int4(0, 0, 0, 0);
-                    if (FULL || lane + WAVE * u < HWL / 4) hv = reinterpret_cast<const int4*>(hist)[lane + WAVE * u];
+                    if (FULL || lane + WAVE * u < HWL / 4) hv = Hist::word4(hist, lane + WAVE * u);
                     word[4 * u] = (float)hv.x * sc; word[(4 * u + 1) % NV] = (float)hv.y * sc;
                     word[(4 * u + 2) % NV] = (float)hv.z * sc; word[(4 * u + 3) % NV] = (float)hv.w * sc;
                 }
@@ -1071,7 +1109,7 @@ __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLd
                 for (int u = 0; u < NV; u++) {
                     const int w = lane + WAVE * u;
                     int32_t sum = 0;
-                    if (ANG != SMALL_A || w < HW_DIST) sum = hist[w];
+                    if (ANG != SMALL_A || w < HW_DIST) sum = Hist::word(hist, w);
                     else if (w < HW_DIST + 3 * SMALL_A) {
 #pragma unroll
                         for (int c = 0; c < A16_COPIES; c++) sum += hist[HW_DIST + c * A16_STRIDE + (w - HW_DIST)];
@@ -1132,7 +1170,7 @@ __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLd
                 // distance bins as they are, every angle bin as the sum of its copies (integers: any order), zeros behind
                 for (int u = lane; u < HWK; u += WAVE) {
                     int32_t sum = 0;
-                    if (u < HW_DIST) sum = hist[u];
+                    if (u < HW_DIST) sum = Hist::word(hist, u);
                     else if (u < HW_DIST + 3 * SMALL_A) {
 #pragma unroll
                         for (int c = 0; c < A16_COPIES; c++) sum += hist[HW_DIST + c * A16_STRIDE + (u - HW_DIST)];
@@ -1144,7 +1182,7 @@ __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLd
                 int4 hv[NW];
 #pragma unroll
                 for (int u = 0; u < NW; u++)
-                    if (FULL || lane + WAVE * u < HWL / 4) hv[u] = reinterpret_cast<const int4*>(hist)[lane + WAVE * u];
+                    if (FULL || lane + WAVE * u < HWL / 4) hv[u] = Hist::word4(hist, lane + WAVE * u);
                 const __amdgpu_buffer_rsrc_t words = device_rsrc(dst, HWK * 4u);
 #pragma unroll
                 for (int u = 0; u < NW; u++)
@@ -1154,7 +1192,7 @@ __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLd
                         else reinterpret_cast<float4*>(dst)[lane + WAVE * u] = v;
                     }
             } else {
-                for (int u = lane; u < HWK; u += WAVE) dst[u] = (float)hist[u] * sc;
+                for (int u = lane; u < HWK; u += WAVE) dst[u] = (float)Hist::word(hist, u) * sc;
             }
         }
         if (LEAN) {}
@@ -1185,9 +1223,10 @@ __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLd
 template <int WL, int ANG, bool COS_ABS, bool LEAN = false>
 __global__ __launch_bounds__(WAVE * CORE_WPB) __attribute__((amdgpu_waves_per_eu(ANG > 0 ? 1 : 7)))
 void fused_core_fwd_kernel(const CoreArgs C) {
-    __shared__ CoreFwdLds<ANG, LEAN> shared[CORE_WPB];
+    constexpr int COPIES = LEAN && ANG == NBINS ? 2 : 1;
+    __shared__ CoreFwdLds<ANG, LEAN, COPIES> shared[CORE_WPB];
     const int wid = core_wave_record(C, (int)blockIdx.x * CORE_WPB + (int)(threadIdx.x >> 6), (int)threadIdx.x & (WAVE - 1));
-    if (wid >= 0) fused_core_fwd_body<WL, ANG, COS_ABS, LEAN>(C, shared[threadIdx.x >> 6], wid);
+    if (wid >= 0) fused_core_fwd_body<WL, ANG, COS_ABS, LEAN, COPIES>(C, shared[threadIdx.x >> 6], wid);
 }
 
 // A workgroup per sixteen items and head, a wavefront per slice; the slices meet in LDS and the first wavefront adds them in
