@@ -1733,6 +1733,27 @@ int launch_item_pass(Kern kern, const cfh::CoreArgs& C, bool search, const float
 }
 #define CFH_ITEM_PASS(...) launch_item_pass(cfh::item_pass_kernel<__VA_ARGS__>, C, search, nullptr, st, what)
 #define CFH_ITEM_PASS_LEAN(...) launch_item_pass(cfh::item_pass_kernel<__VA_ARGS__, true>, C, search, wcat, st, what)
+// Inference without the angle encoding: heads that share a wavefront of the main kernel (fused_core_fwd_heads_kernel; compiled for the
+// usual distance window of 11 bins).  Four halve the instructions of two but leave half the wavefronts, and the last of them, which
+// take the shortest rows, end alone: many items, or long rows, of which each keeps a wavefront busy for long.  Whole passes of four
+// layers in us, one head / two / four: r = 6 to 7 (pairs per atom): 21 600 items 288/269/276, 36 000 409/374/379, 72 000 511/443/435,
+// 147 456 896/750/713; 17 600 273/247/265, 26 400 352/313/324, 45 056 519/448/443, 90 112 728/588/570, 180 224 1315/1045/987; r = 13:
+// 12 920 245/255/297, 19 456 285/268/318, 30 400 374/329/355, 38 912 450/392/400, 77 824 830/716/697; r = 146: 13 440 554/492/532,
+// 30 720 1010/795/739, 96 000 (two layers) 1503/1154/990.
+int heads_per_wavefront(const cfh_params* p, int64_t N, int64_t E) {
+    if (p->angle_bins != 0 || p->num_heads % 4 != 0 || dist_window_dynamic(p) || p->window_mode != CFH_WINDOW_WIDE) return 1;
+    const int64_t items = N * p->num_heads;
+    return items >= (E > 64 * N ? 24576 : 45056) ? 4 : items >= 16384 ? 2 : 1;
+}
+template <int HEADS>
+int launch_core_heads(const cfh::CoreArgs& C, hipStream_t st, const char* what) {
+    {
+        TimedScope timed(what, st);
+        hipLaunchKernelGGL((cfh::fused_core_fwd_heads_kernel<11, HEADS>), dim3((unsigned)C.slow_wgs + (unsigned)C.K.N * (unsigned)C.K.H / HEADS),
+                           dim3(cfh::WAVE), 0, st, C);
+    }
+    return finish_launch(what);
+}
 #define CFH_CORE_FWD(...) launch_core(cfh::fused_core_fwd_kernel<__VA_ARGS__>, C, st, what)
 #define CFH_CORE_FWD_LEAN(...) launch_core(cfh::fused_core_fwd_kernel<__VA_ARGS__, true>, C, st, what)
 #define CFH_CORE_BWD(...) launch_core(cfh::fused_core_bwd_kernel<__VA_ARGS__>, C, st, what)
@@ -1855,10 +1876,13 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
     }
     C.slow_flag = cfh::REC_BOX_LISTED;
     const char* what = one_launch ? "item_pass" : "fused_core_forward";
+    const int nheads = lean && !one_launch && buf.table && buf.near && C.skip_log2 > 0.0f ? heads_per_wavefront(p, N, E) : 1;
     if (lean) {
         if (p->angle_bins == cfh::NBINS)        // moments around the nodes of inference
             C.K.bc.ang_inv_interval = (float)((double)C.K.bc.ang_inv_interval * cfh::LEAN_DEN / cfh::LEAN_NUM);
         if (one_launch) { CFH_CORE_DISPATCH(CFH_ITEM_PASS_LEAN); }
+        else if (nheads == 4) rc = launch_core_heads<4>(C, st, what);
+        else if (nheads == 2) rc = launch_core_heads<2>(C, st, what);
         else { CFH_CORE_DISPATCH(CFH_CORE_FWD_LEAN); }
     } else {
         if (one_launch) { CFH_CORE_DISPATCH(CFH_ITEM_PASS); }

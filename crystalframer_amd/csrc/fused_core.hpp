@@ -576,7 +576,7 @@ __device__ __forceinline__ bool core_record_taken_elsewhere(const CoreArgs& C, u
 // most images of an item lie at nearly the same distance, a few bins of 64, and the lanes of an atomic instruction that meet on
 // a word go one after the other (inference of 180 224 items, 64 angle bins: LDS busy for 134 M clocks, 72 M of them such waits;
 // distances alone 78 M and 37 M).  4096 crystals, four layers, in us: 64 angle bins 1 copy 2650, 2 copies 2588, 4 (less LDS for
-// other wavefronts) 2655.  Rows of 40 to 200 pairs in
+// other wavefronts) 2655; distances alone, four heads per wavefront, 1173, -, 1030.  Rows of 40 to 200 pairs in
 // training lose 0.6 % with 2 copies, few items (item_pass_kernel) 0.5 to 1.3 %.
 constexpr int DIST_STRIDE = NBINS + 8;      // words from one copy to the next: other banks
 // An item's histogram in LDS: its words, then the further copies of its distance bins.
@@ -1215,6 +1215,280 @@ __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLd
             atomicAdd(P.stats + STAT_FWD_PAIRS, (unsigned long long)npairs);
             atomicAdd(P.stats + STAT_FWD_SEEN, n_seen);
         }
+    }
+}
+
+// ---- inference without the angle encoding: several heads of an atom in one wavefront ------------------------------
+// Without frames nothing but a, q, k and v differs from head to head: the pairs' vectors and distances, the walk over the sorted
+// table, the list of the images and the ratios of the distance window are made once for HEADS items, the lanes of a row of eight
+// share out the heads for what is made once per (pair, head).  For items with the usual box, whose nearest images are known.
+// The kernel of one item per wavefront was bound by vector-instruction issue (138 M instructions for 180 224 items; four heads 69 M);
+// what bounds this one are LDS atomics and vector instructions alike (67 and 53 % with one copy of the bins).  4096 crystals,
+// four layers: 1306 us -> 1000.  With the angle encoding (built for 64 and 16 bins, two and four heads: 26 and 38 % fewer vector
+// instructions) the histograms leave room for too few wavefronts: 2650 -> 2654, 2830 us; training 1320 -> 1336, 1403.
+template <int HEADS>
+struct CoreHeadsShared {
+    using Hist = CoreHist<0, true, 4>;
+    struct Pair { float4 A; float C[HEADS]; };      // rx, ry, rz, d2min; per head exp(logit - running max) / S in fixed-point units
+    float4 tab[FC_TCAP];
+    uint16_t list[FC_LISTCAP];
+    __attribute__((aligned(16))) int32_t hist[HEADS][Hist::ALL];
+    __attribute__((aligned(16))) Pair pair[FC_GROUP];
+};
+__device__ __forceinline__ float rows8_max(float x) {
+    x = fmaxf(x, dpp_move<0x128>(x));          // row_ror 8: the other half of the 16-lane row
+    return -rows_min(-x);
+}
+// The records of HEADS heads of an item: words of heads 2 k, 2 k + 1 in the two halves of rec[k].
+template <int HEADS>
+struct HeadRecords {
+    uint32_t rec[HEADS / 2];
+    __device__ __forceinline__ void load(const KernelArgs& P, int it, int h0, int lane) {
+#pragma unroll
+        for (int k = 0; k < HEADS / 2; k++) rec[k] = P.items[((size_t)it * P.H + h0 + 2 * k) * REC_WORDS + lane];
+    }
+    __device__ __forceinline__ int word(int head, int w) const { return __builtin_amdgcn_readlane((int)rec[head >> 1], (head & 1) * REC_WORDS + w); }
+};
+template <int WL, int HEADS>
+__device__ __forceinline__ void fused_core_fwd_heads(const CoreArgs& C, CoreHeadsShared<HEADS>& sh, int h0, const HeadRecords<HEADS>& rec) {
+    static_assert(WL > 0 && (HEADS == 2 || HEADS == 4), "");
+    using Hist = typename CoreHeadsShared<HEADS>::Hist;
+    constexpr int LPH = FC_GROUP / HEADS;      // lanes of a row per head
+    constexpr int CH4 = HEADS / 2;             // 16-byte pieces of a head's 16 channels per lane
+    float4* const tab = sh.tab;
+    uint16_t* const list = sh.list;
+    const KernelArgs& P = C.K;
+    const BasisConsts bc = P.bc;
+    const int lane = threadIdx.x & (WAVE - 1), pr = lane >> 3, sub = lane & 7, H = P.H;
+    const int hs = sub / LPH, ck = sub % LPH;      // this lane's head and its part of the head's channels
+    const float prune = (P.prune_log2 > 0.0f) ? -P.prune_log2 : -3.0e38f;
+    const float INF = __builtin_inff();
+    const int i = rec.word(0, REC_ATOM), e0 = rec.word(0, REC_E0), npairs = rec.word(0, REC_NPAIRS), j0 = rec.word(0, REC_J0);
+    const int crystal = rec.word(0, REC_CRYSTAL);
+    const int s0 = 2 * C.table_R + 1, T = s0 * s0 * s0;
+    // operands of the pair served by this row, fetched one group ahead
+    float nrx = 0.f, nry = 0.f, nrz = 0.f, nnear = 0.f;
+    float4 nk[CH4], nv[CH4], q4[CH4];
+    auto fetch = [&](int g0) {
+        // (no branch per row: a row past the end re-reads the row's last pair; nothing of it is used)
+        const uint32_t el = (uint32_t)min(g0 + pr, npairs - 1);
+        const uint32_t e = min((uint32_t)e0 + el, (uint32_t)(P.E - 1));
+        const uint32_t jh = ((((uint32_t)j0 + el) * (uint32_t)H + (uint32_t)(h0 + hs)) * DH + 4u * CH4 * ck) * 4u;
+        const float3 r3 = load_at<float3>(P.rpos, e * 12u);
+        nrx = r3.x; nry = r3.y; nrz = r3.z;
+#pragma unroll
+        for (int c = 0; c < CH4; c++) { nk[c] = load_at<float4>(C.k, jh + 16u * c); nv[c] = load_at<float4>(C.v, jh + 16u * c); }
+        nnear = load_at<float>(C.pair_near, e * 8u);
+    };
+    float4 acc[CH4];                           // sum_j exp(logit_j - m_run) v_j of this lane's channels
+    {
+        const float4* src = C.sorted_tab + (size_t)crystal * FC_TCAP;
+        const float4 ta = src[lane], tb = src[lane + WAVE];
+        const uint32_t qo = (((uint32_t)i * (uint32_t)H + (uint32_t)(h0 + hs)) * DH + 4u * CH4 * ck) * 4u;
+#pragma unroll
+        for (int c = 0; c < CH4; c++) {
+            q4[c] = load_at<float4>(C.qs, qo + 16u * c);
+            acc[c] = nk[c] = nv[c] = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+        if (npairs > 0) fetch(0);
+#pragma unroll
+        for (int hh = 0; hh < HEADS; hh++) Hist::clear(sh.hist[hh], lane);
+        tab[lane] = ta;
+        tab[lane + WAVE] = tb;
+    }
+    float a2[HEADS], a_own = 0.0f, a2_far = -INF;      // a2_far: of the head that sees farthest
+#pragma unroll
+    for (int hh = 0; hh < HEADS; hh++) {
+        const float a = __int_as_float(rec.word(hh, REC_A));
+        a2[hh] = a * LOG2E;
+        a2_far = fmaxf(a2_far, a2[hh]);
+        a_own = hs == hh ? a : a_own;
+    }
+    const float cutS = C.skip_log2 * hw_rcp(-a2_far);      // (a bound with margins)
+    const int dist0 = Hist::dist_word(lane);
+    const float fixs = 1073741824.0f * hw_rcp((float)max(npairs, 1));      // (see fused_core_fwd_body)
+    float m_run = -INF, Dl = 0.0f;             // running maximum of the logits, share of the denominator: of this lane's head
+    unsigned long long n_eval = 0, n_seen = 0;
+    const bool count = P.stats != nullptr;
+    wave_sync();
+
+    for (int g0 = 0; g0 < npairs; g0 += FC_GROUP) {
+        const float rx = nrx, ry = nry, rz = nrz, d2min = nnear;
+        float4 k4[CH4], v4[CH4];
+#pragma unroll
+        for (int c = 0; c < CH4; c++) { k4[c] = nk[c]; v4[c] = nv[c]; }
+        if (g0 + FC_GROUP < npairs) fetch(g0 + FC_GROUP);
+        const bool active = g0 + pr < npairs;
+        // ---- one walk over the table: weights, normalisers, the images that any head keeps
+        const float rn = hw_sqrt(fmaf(rx, rx, fmaf(ry, ry, rz * rz)));
+        const float reach = fmaf(1.0001f, rn + hw_sqrt(d2min + cutS), 1e-4f);
+        const float lim = active ? fminf(reach, FC_REACH_ALL) : -1.0f;      // (lengths are >= 0; padding: +inf)
+        float Sb[HEADS];
+#pragma unroll
+        for (int hh = 0; hh < HEADS; hh++) Sb[hh] = 0.0f;
+        int nlist = 0;
+        {
+            float4 v = tab[sub];
+            for (int t0 = 0; t0 < T; t0 += FC_GROUP) {
+                const int t = t0 + sub;
+                const float4 vn = tab[min(t + FC_GROUP, FC_TCAP - 1)];      // the next step's entry, in flight meanwhile
+                const bool in = v.w <= lim;
+                const uint64_t inm = ballot(in);
+                if (inm == 0) break;                             // every row is past its reach (lengths ascend)
+                const float dx = rx + v.x, dy = ry + v.y, dz = rz + v.z;
+                const float de = in ? fmaf(dx, dx, fmaf(dy, dy, dz * dz)) - d2min : INF;      // (a < 0: weight 2^-inf = 0)
+                bool keep = false;
+#pragma unroll
+                for (int hh = 0; hh < HEADS; hh++) {
+                    const float ex = a2[hh] * de;
+                    Sb[hh] += hw_exp2(ex);
+                    keep = keep || ex >= prune;
+                    if (count) n_eval += __popcll(ballot(ex >= prune));
+                }
+                n_seen += (unsigned long long)(HEADS * __popcll(inm));
+                const uint64_t m = ballot(keep);
+                if (keep) list[nlist + lane_prefix(m)] = (uint16_t)((pr << FC_SHIFT) | t);
+                nlist += __popcll(m);
+                v = vn;
+            }
+        }
+        // ---- logits, running softmax: a lane per (pair, head, part of the channels)
+        float S = 0.0f;
+#pragma unroll
+        for (int hh = 0; hh < HEADS; hh++) { const float Sh = half_sum(Sb[hh]); S = hs == hh ? Sh : S; }
+        float qk = 0.0f;
+#pragma unroll
+        for (int c = 0; c < CH4; c++)
+            qk += fmaf(q4[c].x, k4[c].x, q4[c].y * k4[c].y) + fmaf(q4[c].z, k4[c].z, q4[c].w * k4[c].w);
+        qk += dpp_move<0xB1>(qk);
+        if (LPH == 4) qk += dpp_move<0x4E>(qk);
+        const float z = fmaf(hw_log2(S), LN2, a_own * d2min);
+        const float logit = active ? qk + z : -INF;
+        const float gmax = rows8_max(logit);
+        const bool grow = gmax > m_run;
+        const uint64_t rescaled = ballot(grow && m_run > -INF);
+        if (rescaled) {
+            const float fac = grow && m_run > -INF ? hw_exp2((m_run - gmax) * LOG2E) : 1.0f;
+#pragma unroll 1
+            for (int hh = 0; hh < HEADS; hh++)
+                if ((rescaled >> (hh * LPH)) & 1)
+                    Hist::rescale(sh.hist[hh], __int_as_float(__builtin_amdgcn_readlane(__float_as_int(fac), hh * LPH)), lane);
+#pragma unroll
+            for (int c = 0; c < CH4; c++) { acc[c].x *= fac; acc[c].y *= fac; acc[c].z *= fac; acc[c].w *= fac; }
+            Dl *= fac;
+        }
+        m_run = grow ? gmax : m_run;
+        const float ew = active ? hw_exp2((logit - m_run) * LOG2E) : 0.0f;
+#pragma unroll
+        for (int c = 0; c < CH4; c++) {
+            acc[c].x = fmaf(ew, v4[c].x, acc[c].x); acc[c].y = fmaf(ew, v4[c].y, acc[c].y);
+            acc[c].z = fmaf(ew, v4[c].z, acc[c].z); acc[c].w = fmaf(ew, v4[c].w, acc[c].w);
+        }
+        Dl += ew;
+        if (sub == 0 && active) sh.pair[pr].A = make_float4(rx, ry, rz, d2min);
+        if (ck == 0 && active) sh.pair[pr].C[hs] = ew * hw_rcp(S) * fixs;
+        wave_sync();
+        // ---- the images of the list, into every head's histogram (an image that only others keep is left out)
+        for (int base = 0; base < nlist; base += WAVE) {
+            const int idx = base + lane;
+            if (idx < nlist) {
+                const uint32_t ent = list[idx];
+                const float4 v = tab[ent & (FC_TCAP - 1)];
+                const auto& pp = sh.pair[ent >> FC_SHIFT];
+                const float4 pa = pp.A;
+                float pc[HEADS];
+#pragma unroll
+                for (int hh = 0; hh < HEADS; hh++) pc[hh] = pp.C[hh];
+                const float dx = pa.x + v.x, dy = pa.y + v.y, dz = pa.z + v.z;
+                const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+                const float de = d2 - pa.w;
+                const float u = hw_sqrt(d2) * bc.inv_interval;
+                int start = (int)(u - bc.start_off);          // truncation toward zero
+                start = max(0, min(start, NBINS - WL));
+                const float beta_c = ((float)(start + WL / 2 + 1) - u) * bc.len_step;
+                const WindowSeed s = window_seed(beta_c, bc.len_step, 1.0f);
+                float rr[WL / 2], rl[WL / 2];                 // from bin to bin outwards from the window's centre
+                rr[0] = s.rr; rl[0] = s.rl;
+#pragma unroll
+                for (int m = 1; m < WL / 2; m++) { rr[m] = rr[m - 1] * bc.len_cc; rl[m] = rl[m - 1] * bc.len_cc; }
+                start += dist0;
+#pragma unroll
+                for (int hh = 0; hh < HEADS; hh++) {
+                    const float ex = a2[hh] * de;
+                    if (ex >= prune) {
+                        const float gc = s.gc * (hw_exp2(ex) * pc[hh]);
+                        int32_t* const hb = sh.hist[hh] + start;
+                        atomicAdd(hb + WL / 2, rint_i(gc));
+                        float g = gc;
+#pragma unroll
+                        for (int m = 0; m < WL / 2; m++) { g *= rr[m]; atomicAdd(hb + WL / 2 + 1 + m, rint_i(g)); }
+                        g = gc;
+#pragma unroll
+                        for (int m = 0; m < WL / 2; m++) { g *= rl[m]; atomicAdd(hb + WL / 2 - 1 - m, rint_i(g)); }
+                    }
+                }
+            }
+        }
+        wave_sync();                      // list and pair data may be rewritten
+    }
+
+    // ---- the rows are complete: normalise and write
+    const float D = rows8_sum(Dl);
+    const float inv = D > 0.0f ? hw_rcp(D) : 0.0f;
+    const float sc_own = inv * hw_rcp(fixs);
+    {
+        float* const dst = C.out + ((size_t)i * H + h0) * DH;      // (the heads' channels are contiguous)
+#pragma unroll
+        for (int c = 0; c < CH4; c++) {
+            const float4 o = make_float4(rows8_sum(acc[c].x) * inv, rows8_sum(acc[c].y) * inv, rows8_sum(acc[c].z) * inv, rows8_sum(acc[c].w) * inv);
+            if (lane < FC_GROUP) reinterpret_cast<float4*>(dst)[sub * CH4 + c] = o;
+        }
+    }
+#pragma unroll
+    for (int hh = 0; hh < HEADS; hh++) {
+        const float sc = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sc_own), hh * LPH));
+        static_assert(HW_DIST == WAVE, "a word per lane");
+        C.hist[((size_t)(h0 + hh) * P.N + i) * HW_DIST + lane] = (float)Hist::word(sh.hist[hh], lane) * sc;
+    }
+    if (count && lane == 0) {
+        atomicAdd(P.stats + STAT_FWD_EVAL, n_eval);
+        atomicAdd(P.stats + STAT_FWD_RAW, (unsigned long long)HEADS * (unsigned long long)T * (unsigned long long)npairs);
+        atomicAdd(P.stats + STAT_FWD_PAIRS, (unsigned long long)HEADS * (unsigned long long)npairs);
+        atomicAdd(P.stats + STAT_FWD_SEEN, n_seen);
+    }
+}
+// The leading wavefronts take a listed record each, the others HEADS heads of an atom; where not all of those have the usual box,
+// one after the other (but the listed ones, as in the kernel of one item per wavefront).
+template <int WL, int HEADS>
+__global__ __launch_bounds__(WAVE) void fused_core_fwd_heads_kernel(const CoreArgs C) {
+    __shared__ union { CoreFwdLds<0, true> one; CoreHeadsShared<HEADS> several; } sh;
+    const KernelArgs& P = C.K;
+    const int lane = (int)threadIdx.x & (WAVE - 1), w = (int)blockIdx.x;
+    int wid, items = 1;
+    if (w < C.slow_wgs) {
+        wid = __builtin_amdgcn_readfirstlane(core_slow_record(C, w, lane));
+        if (wid < 0) return;
+    } else {
+        constexpr int shift = HEADS == 2 ? CORE_DIE_SHIFT - 1 : CORE_DIE_SHIFT - 2;      // (an atom's heads on one die)
+        wid = HEADS * __builtin_amdgcn_readfirstlane(die_order(w - C.slow_wgs, P.N * P.H / HEADS, shift));
+        const int it = div_heads(P, wid), h0 = wid - it * P.H;
+        if (it >= P.N) return;
+        HeadRecords<HEADS> rec;
+        rec.load(P, it, h0, lane);
+        const int usual = C.table_R | (C.table_R << 8) | (C.table_R << 16);
+        bool together = true;
+#pragma unroll
+        for (int hh = 0; hh < HEADS; hh++) together = together && rec.word(hh, REC_BOX) == usual && __int_as_float(rec.word(hh, REC_A)) < 0.0f;
+        if (together) {
+            fused_core_fwd_heads<WL, HEADS>(C, sh.several, h0, rec);
+            return;
+        }
+        items = HEADS;
+    }
+#pragma unroll 1
+    for (int k = 0; k < items; k++) {
+        wave_sync();
+        fused_core_fwd_body<WL, 0, false, true>(C, sh.one, wid + k);
     }
 }
 

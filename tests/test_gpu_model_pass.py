@@ -674,6 +674,31 @@ def test_products_by_the_wavefront_that_completes_sixteen_items(bins, B, atoms, 
     assert Hh.rel_err(out, kept.double()) < 5e-6
 
 
+# Inference without the angle encoding: one head of an atom per wavefront up to 16 383 items, two from there on, four from 45 056
+# (from 24 576 with rows of more than 64 pairs).  Either side of the lines; rows of one pair, of a whole group of eight, one more, of
+# several groups whose maximum grows, of more than 64; sixteen heads; a few cells so small that their box is not the usual one
+# (their heads one after the other).
+@pytest.mark.parametrize("B,atoms,width,small", [(2048, (1, 1), 128, 0), (5631, (1, 1), 128, 0), (5632, (1, 1), 128, 3), (704, (8, 8), 128, 0),
+                                                 (626, (9, 9), 128, 40), (300, (1, 60), 128, 7), (46, (67, 67), 128, 0), (45, (66, 68), 128, 0),
+                                                 (1024, (1, 1), 256, 0), (2816, (1, 1), 256, 5)])
+def test_heads_of_an_atom_in_one_wavefront(B, atoms, width, small):
+    """Against the same pass with everything kept, which takes one item per wavefront: the same operations per item but for images
+    lighter than 2^-32 of their pair's heaviest."""
+    from crystalframer_amd import params, synthetic
+    mp = params.ModelParams(num_layers=1, value_pe_angle_real=0, model_dim=width, head_num=width // 16, embedding_dim=[width])
+    cb = synthetic.make_batch(B, atoms="uniform", atoms_lo=atoms[0], atoms_hi=atoms[1], len_lo=4.0, len_hi=9.0, ang_lo=65.0, ang_hi=115.0,
+                              seed=B)
+    if small:
+        cb.trans_vec[torch.randperm(B, generator=torch.Generator().manual_seed(B))[:small]] *= 0.25
+    model, cb = _model(mp, cb)
+    model.eval()
+    kept = model(cb).detach()
+    with torch.no_grad():
+        out = model(cb)
+        assert torch.equal(model(cb), out)
+    assert Hh.rel_err(out, kept.double()) < 2e-6
+
+
 # Either side of the item counts up to which a layer's items take one launch, crystals of as many atoms as the row has pairs.  With
 # everything kept: 5120 with an angle encoding (8 atoms), 6144 from 13 atoms on, 4096 from 33, none from 65; 10 240 without (8
 # atoms), 5120 from 17 atoms on.  Inference: 10 240 (8, 24 and 40 atoms), 16 384 without an angle encoding for up to 12 atoms, 5120
