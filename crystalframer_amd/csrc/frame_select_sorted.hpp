@@ -31,10 +31,9 @@
 namespace cfh {
 
 constexpr int FQ_ROWS = 4;          // heads of an atom per wavefront, one per 16-lane row
-constexpr int FQ_STAGE = 16;        // pairs staged at a time (the rows of this search have no more)
 constexpr int FQ_PAIR_GROUP = 16;   // pairs of a row whose candidates are laid end to end at a time (one per lane of the row)
 constexpr int FQ_MAX_PAIRS = 16;    // longer rows go one item per wavefront: 64 lanes finish a long item sooner than 16
-static_assert(FQ_MAX_PAIRS <= FQ_STAGE && FQ_STAGE <= WAVE, "a row of the four-heads search is staged as a whole");
+static_assert(FQ_MAX_PAIRS == 16 && FQ_PAIR_GROUP == 16, "a lane per (head, pair) of the four-heads search");
 
 // Shifts t0 .. t0+cnt (cnt <= 128) of the box, sorted by length within the chunk: w = length with the position in the
 // chunk (loop order of the reference) in its low 7 bits, like the entries of the per-crystal tables.  Items whose box
@@ -384,7 +383,12 @@ __device__ __forceinline__ void frame_item_body(const CoreArgs& C, FrameShared& 
 // every row then lays its own candidates end to end and deals them to its 16 lanes, and keeps its own best.  The
 // loops run as long as the longest row needs (the four rows have the same pairs, so nearly the same lengths);
 // reductions stay inside a row (DPP).  Compared with one wavefront per item: a quarter of the staging work per item,
-// lanes filled by four short candidate lists instead of one, four independent items in flight per wavefront.
+// lanes filled by four short candidate lists instead of one, four independent items in flight per wavefront.  A lane is a
+// (head, pair): it makes the pair's q.k with the query of its own row, keeps what it knows of the pair in registers for both axes,
+// and a best candidate is a score and one key.  180 224 items of up to 10 pairs 139 -> 115 us, 18 976 of 1 to 60 pairs 30.3 -> 28.8
+// (before: q.k of the four heads one after the other with the query read across the rows, everything read back from LDS in each of
+// the three passes, a best candidate of three words).  Tried since: a wavefront for every four items that only pass through
+// (frame_axes_kernel), 115 -> 130, as a loop around the search of one item spills 110 scalar registers instead of 42.
 // Rows whose box is not the table's are left to frame_axes_sorted_kernel (unsorted_only).
 template <int CTRL>
 __device__ __forceinline__ float row_maxf_step(float x) { return fmaxf(x, dpp_move<CTRL>(x)); }
@@ -392,15 +396,26 @@ __device__ __forceinline__ float row_max(float x) {
     x = row_maxf_step<0xB1>(x); x = row_maxf_step<0x4E>(x); x = row_maxf_step<0x141>(x); x = row_maxf_step<0x140>(x);
     return x;
 }
-__device__ __forceinline__ void row_best(Best& b) {
-    best_dpp<0xB1>(b); best_dpp<0x4E>(b); best_dpp<0x141>(b); best_dpp<0x140>(b);
+// Best candidate of a row of at most 16 pairs: largest score, then lowest pair, then lowest translation -- the two in one key,
+// pair << FC_SHIFT | translation.
+struct BestKey { float score; int key; };
+constexpr int NO_KEY = 0x7fffffff;
+__device__ __forceinline__ bool better(float s1, int k1, float s2, int k2) { return s1 > s2 || (s1 == s2 && k1 < k2); }
+template <int CTRL>
+__device__ __forceinline__ void best_key_dpp(BestKey& b) {
+    const float os = dpp_move<CTRL>(b.score);
+    const int ok = dpp_movei<CTRL>(b.key);
+    if (better(os, ok, b.score, b.key)) { b.score = os; b.key = ok; }
+}
+__device__ __forceinline__ void row_best(BestKey& b) {
+    best_key_dpp<0xB1>(b); best_key_dpp<0x4E>(b); best_key_dpp<0x141>(b); best_key_dpp<0x140>(b);
 }
 
 struct FrameQuadShared {
     float4 tab[FC_TCAP];
-    float4 rp[FQ_STAGE];                 // staged pairs: rpos, d^2 of the nearest valid image (or -1)
-    float qk_s[FQ_ROWS][FQ_STAGE];       // q_h . k_j of the staged pairs, per row
-    float ph_s[2][FQ_ROWS][FQ_STAGE];    // phase of the tie-breaking noise of the staged pairs, per pass and row
+    float4 rp[FQ_MAX_PAIRS];             // pairs: rpos, d^2 of the nearest valid image (or -1)
+    float qk_s[FQ_ROWS][FQ_MAX_PAIRS];   // q_h . k_j, per row
+    float ph_s[FQ_ROWS][FQ_MAX_PAIRS];   // phase of the tie-breaking noise of the pass, per row
     uint32_t markw[FQ_ROWS][FQ_PAIR_GROUP * FC_TCAP / 32];      // per row: one bit per candidate, set where a pair's run begins
     uint32_t ent[FQ_ROWS][16];           // per row: the pairs that have candidates, in order: first candidate | pair << 16
 };
@@ -408,7 +423,7 @@ struct FrameQuadShared {
 __device__ __forceinline__ void frame_quad_body(const CoreArgs& C, FrameQuadShared& sh, int wid, int lane) {
     float4* const tab = sh.tab;
     float4* const rp = sh.rp;
-    float (*const qk_s)[FQ_STAGE] = sh.qk_s;
+    float (*const qk_s)[FQ_MAX_PAIRS] = sh.qk_s;
     uint32_t (*const markw)[FQ_PAIR_GROUP * FC_TCAP / 32] = sh.markw;
     uint32_t (*const ent)[16] = sh.ent;
 
@@ -465,195 +480,179 @@ __device__ __forceinline__ void frame_quad_body(const CoreArgs& C, FrameQuadShar
     }
     const float nz = noisy ? P.noise : 0.0f;
     const float sq_nz = sqrtf(nz);
+    // ---- stage: a lane per (head, pair).  What a lane knows of its own pair stays in registers, the candidates read the rest
+    const bool any = npairs > 0, pair_ok = mine && l16 < npairs;
+    float4 r4 = make_float4(0.f, 0.f, 0.f, -1.0f);
+    float myqk = 0.0f, phase0 = 0.0f, phase1 = 0.0f;
+    if (any) {
+        const int pj = min(l16, npairs - 1), e = e0 + pj;
+        const float4* kp = reinterpret_cast<const float4*>(C.k + ((size_t)(j0 + pj) * H + h_row) * DH);
+        float4 kv[DH / 4];
+#pragma unroll
+        for (int c4 = 0; c4 < DH / 4; c4++) kv[c4] = kp[c4];
+        r4.x = P.rpos[(size_t)e * 3 + 0]; r4.y = P.rpos[(size_t)e * 3 + 1]; r4.z = P.rpos[(size_t)e * 3 + 2];
+        if (C.pair_near) r4.w = C.pair_near[e].y;
+#pragma unroll
+        for (int c4 = 0; c4 < DH / 4; c4++) {
+            myqk = fmaf(q[4 * c4 + 0], kv[c4].x, myqk);
+            myqk = fmaf(q[4 * c4 + 1], kv[c4].y, myqk);
+            myqk = fmaf(q[4 * c4 + 2], kv[c4].z, myqk);
+            myqk = fmaf(q[4 * c4 + 3], kv[c4].w, myqk);
+        }
+        // the noise of a candidate is a hash of (pair, head, pass) shifted by the translation: the hash once per
+        // pair and pass here (three integer multiplications), not once per candidate
+        if (noisy) {
+            const uint32_t key = (uint32_t)(e * H + h_row);
+            phase0 = hash_uniform(seed_lo, seed_hi, key, 0u);
+            phase1 = hash_uniform(seed_hi, seed_lo, key, 1u);
+        }
+    }
+    if (row == 0) rp[l16] = r4;
+    qk_s[row][l16] = myqk;
     wave_sync();
     const float s1 = tab[1].w;          // shortest non-zero shift (entry 0 is the zero shift)
+    const float r2 = fmaf(r4.x, r4.x, fmaf(r4.y, r4.y, r4.z * r4.z));
+    const float r = hw_sqrt(r2);
+    // the pair's nearest valid image, when the batch's table of them is there: its d^2 lies in [dv_lo, dv_hi], its position in
+    // the sorted table is near_t
+    const bool near_known = r4.w >= 0.0f && r4.w < 1.0e37f;
+    const float dv_lo = __uint_as_float(__float_as_uint(r4.w) & ~(uint32_t)(FC_TCAP - 1));
+    const float dv_hi = dv_lo * (1.0f + 0x1p-15f);
+    const int near_t = (int)(__float_as_uint(r4.w) & (uint32_t)(FC_TCAP - 1));
 
     float f1x = 0.f, f1y = 0.f, f1z = 0.f, f2x = 0.f, f2y = 0.f, f2z = 0.f;
     unsigned long long n_seen = 0;
     for (int pass = 0; pass < 2; pass++) {
-        Best best;
-        best.score = -3.0e38f; best.e = 0x7fffffff; best.t = 0x7fffffff;
-        for (int sw = 0; sw < (pass == 1 ? 2 : 1); sw++) {
+        BestKey best;
+        best.score = -3.0e38f; best.key = NO_KEY;
+        wave_sync();
+        if (noisy) sh.ph_s[row][l16] = pass == 0 ? phase0 : phase1;
+        wave_sync();
+        for (int sw = 0; any && sw < (pass == 1 ? 2 : 1); sw++) {
             const float bound = (pass == 1 && sw == 1) ? row_max(best.score) : -3.0e38f;      // per row
-            for (int pb = 0; pb < npairs; pb += FQ_STAGE) {
-                const int nst = min(FQ_STAGE, npairs - pb);
-                if (npairs > FQ_STAGE || (pass == 0 && sw == 0)) {
-                    // ---- stage: lane = pair; q.k for the four heads with the query channels read across the rows
-                    wave_sync();
-                    float4 r4 = make_float4(0.f, 0.f, 0.f, -1.0f);
-                    const bool have = lane < nst;
-                    const int e = e0 + pb + min(lane, nst - 1);
-                    if (have) {
-                        r4.x = P.rpos[(size_t)e * 3 + 0]; r4.y = P.rpos[(size_t)e * 3 + 1]; r4.z = P.rpos[(size_t)e * 3 + 2];
-                        if (C.pair_near) r4.w = C.pair_near[e].y;
-                    }
-                    if (lane < FQ_STAGE) rp[lane] = r4;
-#pragma unroll 1
-                    for (int r = 0; r < FQ_ROWS; r++) {
-                        const int hr = min(hg * FQ_ROWS + r, H - 1);
-                        const float4* kp = reinterpret_cast<const float4*>(C.k + ((size_t)(j0 + pb + min(lane, nst - 1)) * H + hr) * DH);
-                        float acc = 0.0f;
-#pragma unroll
-                        for (int c4 = 0; c4 < DH / 4; c4++) {
-                            const float4 kv = kp[c4];
-                            acc = fmaf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(q[4 * c4 + 0]), r * 16)), kv.x, acc);
-                            acc = fmaf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(q[4 * c4 + 1]), r * 16)), kv.y, acc);
-                            acc = fmaf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(q[4 * c4 + 2]), r * 16)), kv.z, acc);
-                            acc = fmaf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(q[4 * c4 + 3]), r * 16)), kv.w, acc);
-                        }
-                        if (lane < FQ_STAGE) qk_s[r][lane] = acc;
-                    }
-                    // the noise of a candidate is a hash of (pair, head, pass) shifted by the translation: the hash once per
-                    // pair and pass here (three integer multiplications), not once per candidate
-                    if (noisy) {
-                        const uint32_t key = (uint32_t)((e0 + pb + min(l16, nst - 1)) * H + h_row);
-                        sh.ph_s[0][row][l16] = hash_uniform(seed_lo, seed_hi, key, 0u);
-                        sh.ph_s[1][row][l16] = hash_uniform(seed_hi, seed_lo, key, 1u);
-                    }
-                    wave_sync();
+            if (pass == 1 && sw == 0 && C.pair_near) {
+                // ---- lower bound of the second axis' best score: every pair's nearest valid image, one per lane
+                // (the same arithmetic as in the loop over candidates below, which meets this image again)
+                const float4 v = tab[near_known ? near_t : 0];
+                const int t = (int)(__float_as_uint(v.w) & (uint32_t)(FC_TCAP - 1));
+                const float dx = r4.x + v.x, dy = r4.y + v.y, dz = r4.z + v.z;
+                const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+                const float rinv = hw_rsq(d2);
+                const float ac = fabsf((dx * f1x + dy * f1y + dz * f1z) * rinv);
+                float score = fmaf(a, d2, myqk) + hw_log2(fmaxf(1.0f - ac, 1e-5f)) * LN2;
+                if (noisy) {
+                    const float un = __builtin_amdgcn_fractf(fmaf((float)t, 0.61803399f, phase1));
+                    score += (un - 0.5f) * P.noise;
                 }
-                for (int pc = 0; pc < nst; pc += 16) {
-                    // ---- this row's 16 pairs: how far each has to look, its candidates end to end
-                    const int pj = pc + l16;
-                    const bool pair_ok = mine && pj < nst;
-                    const float4 r4 = rp[min(pj, nst - 1)];
-                    const float myqk = qk_s[row][min(pj, nst - 1)];
-                    const float r2 = fmaf(r4.x, r4.x, fmaf(r4.y, r4.y, r4.z * r4.z));
-                    const float r = hw_sqrt(r2);
-                    // the pair's nearest valid image, when the batch's table of them is there: its d^2 lies in
-                    // [dv_lo, dv_hi], its position in the sorted table is near_t
-                    const bool near_known = r4.w >= 0.0f && r4.w < 1.0e37f;
-                    const float dv_lo = __uint_as_float(__float_as_uint(r4.w) & ~(uint32_t)(FC_TCAP - 1));
-                    const float dv_hi = dv_lo * (1.0f + 0x1p-15f);
-                    const int near_t = (int)(__float_as_uint(r4.w) & (uint32_t)(FC_TCAP - 1));
-                    if (pass == 1 && sw == 0 && C.pair_near) {
-                        // ---- lower bound of the second axis' best score: every pair's nearest valid image, one per lane
-                        // (the same arithmetic as in the loop over candidates below, which meets this image again)
-                        const float4 v = tab[near_known ? near_t : 0];
-                        const int t = (int)(__float_as_uint(v.w) & (uint32_t)(FC_TCAP - 1));
-                        const float dx = r4.x + v.x, dy = r4.y + v.y, dz = r4.z + v.z;
-                        const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-                        const float rinv = hw_rsq(d2);
-                        const float ac = fabsf((dx * f1x + dy * f1y + dz * f1z) * rinv);
-                        float score = fmaf(a, d2, myqk) + hw_log2(fmaxf(1.0f - ac, 1e-5f)) * LN2;
-                        if (noisy) {
-                            const float phase = sh.ph_s[1][row][min(pj, nst - 1)];
-                            const float un = __builtin_amdgcn_fractf(fmaf((float)t, 0.61803399f, phase));
-                            score += (un - 0.5f) * P.noise;
-                        }
-                        const int e = e0 + pb + pj;
-                        if (pair_ok && near_known && d2 > 1e-5f && ac < 0.9999f && better(score, e, t, best.score, best.e, best.t)) {
-                            best.score = score; best.e = e; best.t = t;
-                        }
-                        n_seen += (unsigned long long)__popcll(ballot(pair_ok));
-                        continue;
-                    }
-                    float reach;
-                    if (sw == 0) {
-                        reach = near_known ? fmaf(1.0001f, r + hw_sqrt(dv_hi + nz), 1e-3f)
-                                           : fmaf(1.0001f, fmaf(2.0f, r, (r2 > 1e-5f ? 0.0f : s1) + sq_nz), 1e-3f);
-                    } else if (bound > -1.0e38f) {
-                        const float need = (bound - myqk - 0.5f * nz) * inv_a;
-                        reach = need >= 0.0f ? fmaf(1.0001f, r + hw_sqrt(need), 1e-3f) : -1.0f;
-                    } else {
-                        reach = 3.0e38f;
-                    }
-                    int cnt;
-                    {
-                        int lo = 0, hi = FC_TCAP;
-#pragma unroll
-                        for (int s = 0; s < 8; s++) {      // the count is one of 0 .. 128: eight halvings
-                            const int mid = min((lo + hi) >> 1, FC_TCAP - 1);
-                            const bool le = lo < hi && tab[mid].w <= reach;
-                            lo = le ? mid + 1 : lo;
-                            hi = le ? hi : mid;
-                        }
-                        cnt = pair_ok ? min(lo, bx.T) : 0;
-                    }
-                    if (pass == 0 && C.pair_near) {
-                        // First axis: no candidate of a pair scores above hi (its nearest valid image with the noise at
-                        // its most favourable), and its nearest valid image scores at least lo.  A pair whose hi stays
-                        // below the best lo of the row cannot hold the maximum: its candidates are left out.  (The
-                        // margins cover the rounding of d^2 in the table of nearest images and of the scores.)
-                        const float hi = near_known ? fmaf(a, dv_lo - 0.5f * nz, myqk) : 3.0e38f;
-                        const float lo_s = near_known ? fmaf(a, dv_hi + 0.5f * nz, myqk) : -3.0e38f;
-                        const float mg = 2e-6f * (fabsf(myqk) + fabsf(a) * (dv_hi + nz)) + 1e-30f;
-                        const float lb = row_max(pair_ok ? lo_s - mg : -3.0e38f);
-                        if (!(hi + mg >= lb)) cnt = 0;
-                    }
-                    int incl = cnt;                        // inclusive prefix within the row
-                    incl += dpp_movei<0x111>(incl);
-                    incl += dpp_movei<0x112>(incl);
-                    incl += dpp_movei<0x114>(incl);
-                    incl += dpp_movei<0x118>(incl);
-                    const int t0 = __builtin_amdgcn_readlane(incl, 15), t1 = __builtin_amdgcn_readlane(incl, 31);
-                    const int t2 = __builtin_amdgcn_readlane(incl, 47), t3 = __builtin_amdgcn_readlane(incl, 63);
-                    const int total = row == 0 ? t0 : row == 1 ? t1 : row == 2 ? t2 : t3;
-                    const int longest = max(max(t0, t1), max(t2, t3));
-                    // Which pair a candidate belongs to, without a search: a bit per candidate marks where the run of a
-                    // pair begins, so the pair of candidate c is the number of marks up to c (a population count of
-                    // the 16 marks of the step plus what the steps before counted) into the list of the pairs that
-                    // have candidates.  One read of the marks and one of that list per step, instead of four dependent
-                    // reads of a bisection: the step's latency was what the wavefronts waited for.
-                    const uint32_t nzrow = (uint32_t)(ballot(cnt > 0) >> (16 * row)) & 0xffffu;
-                    const int kslot = __popc(nzrow & ((1u << l16) - 1u));
-                    const int first = incl - cnt;
-                    wave_sync();                           // the readers of the marks and the list are done
-#pragma unroll
-                    for (int u = 0; u < FQ_PAIR_GROUP * FC_TCAP / 32 / 16; u++) markw[row][l16 + 16 * u] = 0u;
-                    wave_sync();
-                    if (cnt > 0) {
-                        ent[row][kslot] = (uint32_t)first | ((uint32_t)l16 << 16);
-                        atomicOr(&markw[row][first >> 5], 1u << (first & 31));
-                    }
-                    wave_sync();
-                    n_seen += (unsigned long long)(t0 + t1 + t2 + t3);
-                    int carry = 0;                         // marks in the steps before this one (the same in a row)
-                    for (int base = 0; base < longest; base += 16) {
-                        const int c = base + l16;
-                        const bool in = c < total;
-                        const uint32_t m16 = (markw[row][base >> 5] >> (base & 16)) & 0xffffu;
-                        const int kk = carry + __popc(m16 & ((2u << l16) - 1u)) - 1;
-                        carry += __popc(m16);
-                        const uint32_t en = ent[row][in ? kk : 0];
-                        const int pl = in ? (int)(en >> 16) : 0;
-                        const float4 v = tab[in ? c - (int)(en & 0xffffu) : 0];
-                        const int ps = min(pc + pl, nst - 1);
-                        const float4 cq = rp[ps];
-                        const float cqk = qk_s[row][ps];
-                        const int e = e0 + pb + pc + pl;
-                        const int t = (int)(__float_as_uint(v.w) & (uint32_t)(FC_TCAP - 1));
-                        const float dx = cq.x + v.x, dy = cq.y + v.y, dz = cq.z + v.z;
-                        const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-                        float score = fmaf(a, d2, cqk);
-                        bool ok = in && d2 > 1e-5f;
-                        if (pass == 1) {
-                            const float rinv = hw_rsq(d2);
-                            const float ac = fabsf((dx * f1x + dy * f1y + dz * f1z) * rinv);
-                            score += hw_log2(fmaxf(1.0f - ac, 1e-5f)) * LN2;
-                            ok = ok && ac < 0.9999f;
-                        }
-                        if (noisy) {
-                            const float phase = sh.ph_s[pass][row][ps];
-                            const float un = __builtin_amdgcn_fractf(fmaf((float)t, 0.61803399f, phase));
-                            if (pass == 0) score = fmaf(a, d2 + (un - 0.5f) * P.noise, cqk);
-                            else score += (un - 0.5f) * P.noise;
-                        }
-                        if (ok && better(score, e, t, best.score, best.e, best.t)) {
-                            best.score = score; best.e = e; best.t = t;
-                        }
-                    }
+                const int key = (l16 << FC_SHIFT) | t;
+                if (pair_ok && near_known && d2 > 1e-5f && ac < 0.9999f && better(score, key, best.score, best.key)) {
+                    best.score = score; best.key = key;
                 }
+                n_seen += (unsigned long long)__popcll(ballot(pair_ok));
+                continue;
+            }
+            // ---- how far this lane's pair has to look, its row's candidates end to end
+            float reach;
+            if (sw == 0) {
+                reach = near_known ? fmaf(1.0001f, r + hw_sqrt(dv_hi + nz), 1e-3f)
+                                   : fmaf(1.0001f, fmaf(2.0f, r, (r2 > 1e-5f ? 0.0f : s1) + sq_nz), 1e-3f);
+            } else if (bound > -1.0e38f) {
+                const float need = (bound - myqk - 0.5f * nz) * inv_a;
+                reach = need >= 0.0f ? fmaf(1.0001f, r + hw_sqrt(need), 1e-3f) : -1.0f;
+            } else {
+                reach = 3.0e38f;
+            }
+            int cnt;
+            {
+                int lo = 0, hi = FC_TCAP;
+#pragma unroll
+                for (int s = 0; s < 8; s++) {      // the count is one of 0 .. 128: eight halvings
+                    const int mid = min((lo + hi) >> 1, FC_TCAP - 1);
+                    const bool le = lo < hi && tab[mid].w <= reach;
+                    lo = le ? mid + 1 : lo;
+                    hi = le ? hi : mid;
+                }
+                cnt = pair_ok ? min(lo, bx.T) : 0;
+            }
+            if (pass == 0 && C.pair_near) {
+                // First axis: no candidate of a pair scores above hi (its nearest valid image with the noise at
+                // its most favourable), and its nearest valid image scores at least lo.  A pair whose hi stays
+                // below the best lo of the row cannot hold the maximum: its candidates are left out.  (The
+                // margins cover the rounding of d^2 in the table of nearest images and of the scores.)
+                const float hi = near_known ? fmaf(a, dv_lo - 0.5f * nz, myqk) : 3.0e38f;
+                const float lo_s = near_known ? fmaf(a, dv_hi + 0.5f * nz, myqk) : -3.0e38f;
+                const float mg = 2e-6f * (fabsf(myqk) + fabsf(a) * (dv_hi + nz)) + 1e-30f;
+                const float lb = row_max(pair_ok ? lo_s - mg : -3.0e38f);
+                if (!(hi + mg >= lb)) cnt = 0;
+            }
+            int incl = cnt;                        // inclusive prefix within the row
+            incl += dpp_movei<0x111>(incl);
+            incl += dpp_movei<0x112>(incl);
+            incl += dpp_movei<0x114>(incl);
+            incl += dpp_movei<0x118>(incl);
+            const int t0 = __builtin_amdgcn_readlane(incl, 15), t1 = __builtin_amdgcn_readlane(incl, 31);
+            const int t2 = __builtin_amdgcn_readlane(incl, 47), t3 = __builtin_amdgcn_readlane(incl, 63);
+            const int total = row == 0 ? t0 : row == 1 ? t1 : row == 2 ? t2 : t3;
+            const int longest = max(max(t0, t1), max(t2, t3));
+            // Which pair a candidate belongs to, without a search: a bit per candidate marks where the run of a
+            // pair begins, so the pair of candidate c is the number of marks up to c (a population count of
+            // the 16 marks of the step plus what the steps before counted) into the list of the pairs that
+            // have candidates.  One read of the marks and one of that list per step, instead of four dependent
+            // reads of a bisection: the step's latency was what the wavefronts waited for.
+            const uint32_t nzrow = (uint32_t)(ballot(cnt > 0) >> (16 * row)) & 0xffffu;
+            const int kslot = __popc(nzrow & ((1u << l16) - 1u));
+            const int first = incl - cnt;
+            wave_sync();                           // the readers of the marks and the list are done
+#pragma unroll
+            for (int u = 0; u < FQ_PAIR_GROUP * FC_TCAP / 32 / 16; u++) markw[row][l16 + 16 * u] = 0u;
+            wave_sync();
+            if (cnt > 0) {
+                ent[row][kslot] = (uint32_t)first | ((uint32_t)l16 << 16);
+                atomicOr(&markw[row][first >> 5], 1u << (first & 31));
+            }
+            wave_sync();
+            n_seen += (unsigned long long)(t0 + t1 + t2 + t3);
+            int carry = 0;                         // marks in the steps before this one (the same in a row)
+            for (int base = 0; base < longest; base += 16) {
+                const int c = base + l16;
+                const bool in = c < total;
+                const uint32_t m16 = (markw[row][base >> 5] >> (base & 16)) & 0xffffu;
+                const int kk = carry + __popc(m16 & ((2u << l16) - 1u)) - 1;
+                carry += __popc(m16);
+                const uint32_t en = ent[row][in ? kk : 0];
+                const int pl = in ? (int)(en >> 16) : 0;
+                const float4 v = tab[in ? c - (int)(en & 0xffffu) : 0];
+                const float4 cq = rp[pl];
+                const float cqk = qk_s[row][pl];
+                const int t = (int)(__float_as_uint(v.w) & (uint32_t)(FC_TCAP - 1));
+                const float dx = cq.x + v.x, dy = cq.y + v.y, dz = cq.z + v.z;
+                const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+                float score = fmaf(a, d2, cqk);
+                bool ok = in && d2 > 1e-5f;
+                if (pass == 1) {
+                    const float rinv = hw_rsq(d2);
+                    const float ac = fabsf((dx * f1x + dy * f1y + dz * f1z) * rinv);
+                    score += hw_log2(fmaxf(1.0f - ac, 1e-5f)) * LN2;
+                    ok = ok && ac < 0.9999f;
+                }
+                if (noisy) {
+                    const float un = __builtin_amdgcn_fractf(fmaf((float)t, 0.61803399f, sh.ph_s[row][pl]));
+                    if (pass == 0) score = fmaf(a, d2 + (un - 0.5f) * P.noise, cqk);
+                    else score += (un - 0.5f) * P.noise;
+                }
+                const int key = (pl << FC_SHIFT) | t;
+                if (ok && better(score, key, best.score, best.key)) { best.score = score; best.key = key; }
             }
         }
         row_best(best);
         float vx = 0.f, vy = 0.f, vz = 0.f;
-        if (best.e != 0x7fffffff) {
+        if (best.key != NO_KEY) {
             float sx, sy, sz;
-            shift_of(best.t, bx, L, sx, sy, sz);
-            vx = P.rpos[(size_t)best.e * 3 + 0] + sx;
-            vy = P.rpos[(size_t)best.e * 3 + 1] + sy;
-            vz = P.rpos[(size_t)best.e * 3 + 2] + sz;
+            shift_of(best.key & (FC_TCAP - 1), bx, L, sx, sy, sz);
+            const float4 cq = rp[best.key >> FC_SHIFT];
+            vx = cq.x + sx;
+            vy = cq.y + sy;
+            vz = cq.z + sz;
             unit_vector(vx, vy, vz);
         }
         if (pass == 0) { f1x = vx; f1y = vy; f1z = vz; }
