@@ -1723,11 +1723,21 @@ int64_t item_pass_max(const cfh_params* p, int64_t N, int64_t E, bool lean) {
 bool one_launch_form(const cfh_params* p, int64_t N, int64_t E, bool search, bool lean) {
     return N * p->num_heads <= item_pass_max(p, N, E, lean) && !(search && p->symm_break_noise > 0.0f && p->noise_seed_dev);
 }
+// Inference of very few items with the angle encoding: four more wavefronts per item make its product with the weights, which they
+// have asked for by then (2.1 us of the 13.9 that the item's own wavefront takes for one crystal of 8 atoms).  Up to three items per
+// compute unit: a fourth workgroup of five wavefronts there waits.  Whole passes of four layers in us, own wavefront / helpers: 64
+// items 135/131, 232 163/160, 456 182/176, 608 172/168, 760 168/162, 836 168/185; 16 bins 64 items 140/137, 456 188/185.  (Distances
+// alone, 64 words per item: no difference.)
+bool products_by_helpers(const cfh_params* p, int64_t N) {
+    int cus = device_cus();
+    if (cus <= 0) cus = 256;
+    return p->angle_bins > 0 && !dist_window_dynamic(p) && p->window_mode == CFH_WINDOW_WIDE && N * p->num_heads <= 3 * (int64_t)cus;
+}
 template <typename Kern>
-int launch_item_pass(Kern kern, const cfh::CoreArgs& C, bool search, const float* wcat, hipStream_t st, const char* what) {
+int launch_item_pass(Kern kern, const cfh::CoreArgs& C, bool search, const float* wcat, hipStream_t st, const char* what, int waves = 1) {
     {
         TimedScope timed(what, st);
-        hipLaunchKernelGGL(kern, dim3((unsigned)C.K.N * (unsigned)C.K.H), dim3(cfh::WAVE), 0, st, C, search ? 1 : 0, wcat);
+        hipLaunchKernelGGL(kern, dim3((unsigned)C.K.N * (unsigned)C.K.H), dim3(cfh::WAVE * waves), 0, st, C, search ? 1 : 0, wcat);
     }
     return finish_launch(what);
 }
@@ -1754,6 +1764,9 @@ int launch_core_heads(const cfh::CoreArgs& C, hipStream_t st, const char* what) 
     }
     return finish_launch(what);
 }
+#define CFH_HELPERS(ANG)                                                                                  \
+    (p->cos_abs ? launch_item_pass(cfh::item_pass_kernel<11, ANG, true, true, 4>, C, search, wcat, st, what, 5)      \
+                : launch_item_pass(cfh::item_pass_kernel<11, ANG, false, true, 4>, C, search, wcat, st, what, 5))
 #define CFH_CORE_FWD(...) launch_core(cfh::fused_core_fwd_kernel<__VA_ARGS__>, C, st, what)
 #define CFH_CORE_FWD_LEAN(...) launch_core(cfh::fused_core_fwd_kernel<__VA_ARGS__, true>, C, st, what)
 #define CFH_CORE_BWD(...) launch_core(cfh::fused_core_bwd_kernel<__VA_ARGS__>, C, st, what)
@@ -1880,7 +1893,8 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
     if (lean) {
         if (p->angle_bins == cfh::NBINS)        // moments around the nodes of inference
             C.K.bc.ang_inv_interval = (float)((double)C.K.bc.ang_inv_interval * cfh::LEAN_DEN / cfh::LEAN_NUM);
-        if (one_launch) { CFH_CORE_DISPATCH(CFH_ITEM_PASS_LEAN); }
+        if (one_launch && products_by_helpers(p, N)) { rc = p->angle_bins == cfh::SMALL_A ? CFH_HELPERS(cfh::SMALL_A) : CFH_HELPERS(cfh::NBINS); }
+        else if (one_launch) { CFH_CORE_DISPATCH(CFH_ITEM_PASS_LEAN); }
         else if (nheads == 4) rc = launch_core_heads<4>(C, st, what);
         else if (nheads == 2) rc = launch_core_heads<2>(C, st, what);
         else { CFH_CORE_DISPATCH(CFH_CORE_FWD_LEAN); }

@@ -706,13 +706,24 @@ __global__ __launch_bounds__(WAVE * CORE_WPB) void frame_axes_kernel(const CoreA
 // launches of their own each of the three is a chain of dependent steps behind a launch that fills a fraction of the chip.
 // One crystal of 8 atoms: 22 us in three launches, 17 in one; a whole call of four layers 185 -> 173.  The record in registers
 // and the sums' first operands asked for ahead of the search, instead of both through memory: 153 -> 149.
-template <int WL, int ANG, bool COS_ABS, bool LEAN = false>
-__global__ __launch_bounds__(WAVE) void item_pass_kernel(const CoreArgs C, int search, const float* __restrict__ wcat) {
+// HELPERS (inference): further wavefronts of the workgroup, four channels each, that ask for the weights of the product at the start
+// of the kernel and make it when the item's wavefront is done.
+template <int WL, int ANG, bool COS_ABS, bool LEAN = false, int HELPERS = 0>
+__global__ __launch_bounds__(WAVE * (1 + HELPERS)) void item_pass_kernel(const CoreArgs C, int search, const float* __restrict__ wcat) {
+    static_assert(HELPERS == 0 || (LEAN && HELPERS * 4 == DH), "");
     __shared__ union { FrameShared frame; CoreFwdLds<ANG, LEAN> core; } sh;
     const KernelArgs& P = C.K;
-    const int wid = (int)blockIdx.x, lane = (int)threadIdx.x;
+    const int wid = (int)blockIdx.x, lane = (int)threadIdx.x & (WAVE - 1);
     const int it = div_heads(P, wid), h = wid - it * P.H;
     if (it >= P.N) return;
+    if (HELPERS > 0 && threadIdx.x >= WAVE) {
+        const int c0 = 4 * ((int)(threadIdx.x >> 6) - 1);
+        CoreProductWeights<core_hist_words(ANG, LEAN)> W;
+        W.load(wcat, h, c0, lane);
+        __syncthreads();
+        W.product(sh.core.hist, sh.core.tab, C.out, h, P.H, c0, lane);
+        return;
+    }
     // (the record stays in registers, and what the sums need first is asked for ahead of the search; a backward pass reads the
     // record from memory)
     CoreOwn own;
@@ -723,7 +734,8 @@ __global__ __launch_bounds__(WAVE) void item_pass_kernel(const CoreArgs C, int s
         __threadfence_block();
     }
     if (!LEAN && lane < REC_WORDS) P.items[((size_t)it * P.H + h) * REC_WORDS + lane] = own.rec;
-    fused_core_fwd_body<WL, ANG, COS_ABS, LEAN>(C, sh.core, wid, wcat, &own);
+    fused_core_fwd_body<WL, ANG, COS_ABS, LEAN, 1, (HELPERS > 0)>(C, sh.core, wid, wcat, &own);
+    if (HELPERS > 0) __syncthreads();
 }
 
 }  // namespace cfh

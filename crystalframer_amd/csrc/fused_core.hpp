@@ -774,7 +774,9 @@ __device__ __forceinline__ void core_project_done(const CoreArgs& C, int it, int
 // LDS (LEAN only)
 // own: not null: the item's record and first operands, in registers
 struct CoreOwn { uint32_t rec; CorePrefetch pf; };
-template <int WL, int ANG, bool COS_ABS, bool LEAN, int COPIES = 1>
+// HAND_OVER (LEAN only): the histogram stays in LDS as float32 words, with the item's part of `out` and its atom in front of the
+// table, for other wavefronts of the workgroup (core_product_words)
+template <int WL, int ANG, bool COS_ABS, bool LEAN, int COPIES = 1, bool HAND_OVER = false>
 __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLds<ANG, LEAN, COPIES>& sh, int wid,
                                                     const float* __restrict__ wcat = nullptr, const CoreOwn* own = nullptr) {
     constexpr bool HAS_ANG = ANG > 0;
@@ -1089,7 +1091,7 @@ __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLd
         const float D = uniform_f(wave_sum(Dl));
         const float inv = D > 0.0f ? hw_rcp(D) : 0.0f;
         const float sc = inv * hw_rcp(fixs);
-        if (LEAN && wcat) {
+        if (LEAN && (HAND_OVER || wcat)) {
             // Four words per lane at a time (fewer words: one).  A loop over the channels, four at a time with their loads in
             // flight together: a wavefront runs through this once, and fetching the instructions of all sixteen took longer than
             // the loop's waits for weights (a layer's launch of 64 items 20.0 us, in the loop 18.2; whole calls of 4872 items 272 and
@@ -1118,6 +1120,17 @@ __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLd
                 }
             }
             const float ox = rows8_sum(accv.x) * inv, oy = rows8_sum(accv.y) * inv;      // (the same in every 8-lane row)
+            if (HAND_OVER) {
+                wave_sync();
+#pragma unroll
+                for (int u = 0; u < NV; u++) {
+                    const int w = VEC ? 4 * (lane + WAVE * (u >> 2)) + (u & 3) : lane + WAVE * u;
+                    if (w < HWK) hist[w] = __float_as_int(word[u]);
+                }
+                if (lane < FC_GROUP) reinterpret_cast<float2*>(tab)[lane] = make_float2(ox, oy);
+                if (lane == 0) tab[4].x = __int_as_float(i);
+                return;
+            }
             const float* Wh = wcat + (size_t)h * DH * HWK;
             float* const dst = C.out + ih * DH;
 #pragma unroll 1
@@ -1217,6 +1230,55 @@ __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLd
         }
     }
 }
+
+// The product of four channels (from c0 on) of a handed-over item with the weights, which wait in registers: the same sums as the
+// item's own wavefront makes.
+template <int HWK>
+struct CoreProductWeights {
+    static constexpr bool VEC = HWK >= 4 * WAVE;
+    static constexpr int NW = VEC ? (HWK / 4 + WAVE - 1) / WAVE : 1, NV = VEC ? 4 * NW : HWK / WAVE;
+    float w[4][NV];
+    __device__ __forceinline__ void load(const float* __restrict__ wcat, int h, int c0, int lane) {
+        const float* Wh = wcat + ((size_t)h * DH + c0) * HWK;
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+#pragma unroll
+            for (int u = 0; u < (VEC ? NW : NV); u++) {
+                if (VEC) {      // (a lane past the end reads the last words; its own are zero)
+                    const float4 t = *reinterpret_cast<const float4*>(Wh + c * HWK + 4 * min(lane + WAVE * u, HWK / 4 - 1));
+                    w[c][4 * u] = t.x; w[c][(4 * u + 1) % NV] = t.y; w[c][(4 * u + 2) % NV] = t.z; w[c][(4 * u + 3) % NV] = t.w;
+                } else {
+                    w[c][u] = Wh[c * HWK + lane + WAVE * u];
+                }
+            }
+    }
+    __device__ __forceinline__ void product(const int32_t* hist, const float4* tab, float* out, int h, int H, int c0, int lane) const {
+        float word[NV], v[4];
+#pragma unroll
+        for (int u = 0; u < (VEC ? NW : NV); u++) {
+            if (VEC) {
+                int4 t = make_int4(0, 0, 0, 0);
+                if (lane + WAVE * u < HWK / 4) t = reinterpret_cast<const int4*>(hist)[lane + WAVE * u];
+                word[4 * u] = __int_as_float(t.x); word[(4 * u + 1) % NV] = __int_as_float(t.y);
+                word[(4 * u + 2) % NV] = __int_as_float(t.z); word[(4 * u + 3) % NV] = __int_as_float(t.w);
+            } else {
+                word[u] = __int_as_float(hist[lane + WAVE * u]);
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            v[c] = lane == ((c0 + c) >> 1) ? reinterpret_cast<const float*>(tab)[c0 + c] : 0.0f;
+#pragma unroll
+            for (int u = 0; u < (VEC ? NW : NV); u++)
+                v[c] = VEC ? fmaf(word[4 * u], w[c][4 * u], fmaf(word[(4 * u + 1) % NV], w[c][(4 * u + 1) % NV],
+                             fmaf(word[(4 * u + 2) % NV], w[c][(4 * u + 2) % NV], fmaf(word[(4 * u + 3) % NV], w[c][(4 * u + 3) % NV], v[c]))))
+                           : fmaf(word[u], w[c][u], v[c]);
+        }
+        const float sum = wave_sum4(v, lane);
+        const int i = __float_as_int(tab[4].x);
+        if ((lane & 15) == 0) out[((size_t)i * H + h) * DH + c0 + (lane >> 4)] = sum;
+    }
+};
 
 // ---- inference without the angle encoding: several heads of an atom in one wavefront ------------------------------
 // Without frames nothing but a, q, k and v differs from head to head: the pairs' vectors and distances, the walk over the sorted

@@ -647,6 +647,27 @@ def test_products_of_few_items(bins, B, atoms):
     assert Hh.rel_err(out, kept.double()) < 5e-6
 
 
+# Very few items (up to 768 on 256 compute units): further wavefronts of an item's workgroup make the product.  One atom, rows of
+# several groups of eight pairs whose maximum grows, either side of the line, the absolute value of the cosine, sixteen heads.
+@pytest.mark.parametrize("bins,B,atoms,width,cos_abs", [(64, 1, 1, 128, 0), (64, 2, 43, 128, 0), (64, 96, 1, 128, 0), (64, 97, 1, 128, 0),
+                                                        (16, 1, 1, 128, 1), (16, 12, 8, 128, 0), (64, 3, 16, 256, 1)])
+def test_products_by_further_wavefronts_of_an_item(bins, B, atoms, width, cos_abs):
+    """Against the same pass with everything kept (tolerance as above), which has a launch of its own for the products."""
+    from crystalframer_amd import params, synthetic
+    kw = dict(value_pe_angle_wscale=1.0, value_pe_dist_coef=1.5, value_pe_angle_coef=6.0) if bins == 16 else {}
+    mp = params.ModelParams(num_layers=2, value_pe_angle_real=bins, symm_break_noise=0.0, model_dim=width, head_num=width // 16,
+                            embedding_dim=[width], cos_abs=cos_abs, **kw)
+    cb = synthetic.make_batch(B, atoms="uniform", atoms_lo=atoms, atoms_hi=atoms, len_lo=3.0, len_hi=9.0, ang_lo=65.0,
+                              ang_hi=115.0, seed=B)
+    model, cb = _model(mp, cb)
+    model.eval()
+    kept = model(cb).detach()
+    with torch.no_grad():
+        out = model(cb)
+        assert torch.equal(model(cb), out)
+    assert Hh.rel_err(out, kept.double()) < 1e-5
+
+
 # Inference of many items with the angle encoding: the wavefront that completes sixteen items of a head makes their products, but
 # for the last items (a fifth, at least 16 384 on 256 compute units).  One atom short of the first 128 atoms whose products are
 # made so, exactly those, a last block of one atom and of 127, rows of mixed lengths, sixteen heads.
