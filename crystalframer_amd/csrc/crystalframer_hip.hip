@@ -1857,7 +1857,7 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
             if (F.sorted_tab) {
                 // four heads of an atom per wavefront for the items with the usual box and short rows, the others one
                 // by one, all in one launch
-                const unsigned item_blocks = ((unsigned)N * (unsigned)p->num_heads + cfh::CORE_WPB - 1) / cfh::CORE_WPB;
+                const unsigned items = (unsigned)N * (unsigned)p->num_heads;
                 const unsigned quad_waves = (unsigned)N * (unsigned)((p->num_heads + cfh::FQ_ROWS - 1) / cfh::FQ_ROWS);
                 const unsigned quad_blocks = (quad_waves + cfh::CORE_WPB - 1) / cfh::CORE_WPB;
                 if (F.K.slow_count) {
@@ -1866,10 +1866,20 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
                     F.slow_wgs = slow_wave_count(N, p->num_heads);
                 }
                 const unsigned slow_blocks = ((unsigned)F.slow_wgs + cfh::CORE_WPB - 1) / cfh::CORE_WPB;
+                // Whole blocks of pairs in work order: the rows of more than FQ_MAX_PAIRS pairs come first, and there are at most
+                // (E - N) / FQ_MAX_PAIRS of them, as every atom has one pair at least.  Where many items are left behind them,
+                // they are looked at four at a time.
+                int64_t long_rows = order && E >= N ? (E - N) / cfh::FQ_MAX_PAIRS : N;
+                if (long_rows > N) long_rows = N;
+                const unsigned singles = (unsigned)long_rows * (unsigned)p->num_heads;
                 {
                     TimedScope timed("frame_axes", st);
-                    hipLaunchKernelGGL(cfh::frame_axes_kernel, dim3(slow_blocks + quad_blocks + item_blocks),
-                                       dim3(cfh::WAVE * cfh::CORE_WPB), 0, st, F, (int)slow_blocks, (int)quad_blocks);
+                    if (items - singles >= 49152)
+                        hipLaunchKernelGGL(cfh::frame_axes_kernel<4>, dim3(slow_blocks + quad_blocks + singles + (items - singles + 3) / 4),
+                                           dim3(cfh::WAVE * cfh::CORE_WPB), 0, st, F, (int)slow_blocks, (int)quad_blocks, (int)singles);
+                    else
+                        hipLaunchKernelGGL(cfh::frame_axes_kernel<1>, dim3(slow_blocks + quad_blocks + items),
+                                           dim3(cfh::WAVE * cfh::CORE_WPB), 0, st, F, (int)slow_blocks, (int)quad_blocks, 0);
                 }
                 if ((rc = finish_launch("frame_axes"))) return rc;
             } else if ((rc = launch_core(cfh::frame_axes_sorted_kernel, F, st, "frame_axes"))) return rc;

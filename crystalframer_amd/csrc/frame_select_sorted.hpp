@@ -387,8 +387,7 @@ __device__ __forceinline__ void frame_item_body(const CoreArgs& C, FrameShared& 
 // (head, pair): it makes the pair's q.k with the query of its own row, keeps what it knows of the pair in registers for both axes,
 // and a best candidate is a score and one key.  180 224 items of up to 10 pairs 139 -> 115 us, 18 976 of 1 to 60 pairs 30.3 -> 28.8
 // (before: q.k of the four heads one after the other with the query read across the rows, everything read back from LDS in each of
-// the three passes, a best candidate of three words).  Tried since: a wavefront for every four items that only pass through
-// (frame_axes_kernel), 115 -> 130, as a loop around the search of one item spills 110 scalar registers instead of 42.
+// the three passes, a best candidate of three words).
 // Rows whose box is not the table's are left to frame_axes_sorted_kernel (unsorted_only).
 template <int CTRL>
 __device__ __forceinline__ float row_maxf_step(float x) { return fmaxf(x, dpp_move<CTRL>(x)); }
@@ -683,23 +682,55 @@ __global__ __launch_bounds__(WAVE * CORE_WPB) void frame_axes_sorted_kernel(cons
 //   1. one per listed record with a box of their own, by rank over the lists (made by the launch that wrote the
 //      records; no record of that rank: the wavefront ends): several sorted chunks, the longest of the launch;
 //   2. the four-heads search over all atoms;
-//   3. one per item, for the items that neither of the two takes (usual box, longer rows: they are at the start of the
-//      work order, so the wavefronts that find nothing to do come last and only pass through).
+//   3. REST = 1: one per item, for the items that neither of the two takes (usual box, longer rows: they are at the start of the
+//      work order, so the wavefronts that find nothing to do come last and only pass through);
+//      else one per item for the first `items` places, where the long rows are, and one per REST items behind them, for whatever
+//      is left there (a box of its own of a rank past the leading wavefronts, a >= 0).
 // With the items of (3) and their many passing wavefronts in front, the four-heads search started after a third of
 // the launch's time, and the records with a box of their own, scattered over the work order, later still.
-__global__ __launch_bounds__(WAVE * CORE_WPB) void frame_axes_kernel(const CoreArgs C, int slow_blocks, int quad_blocks) {
+// REST: a wavefront that passes through takes its turn at the dispatcher all the same, 115 us for 180 224 items of up to 10 pairs
+// where 83 are left without them; REST 4 99.7, 8 97.6, 16 101.  But the loop keeps more alive: 18 976 items of 1 to 60 pairs 28.8 us
+// with REST 1, 30.4 with 4, 30 720 long rows 145 and 150.
+template <int REST>
+__global__ __launch_bounds__(WAVE * CORE_WPB) void frame_axes_kernel(const CoreArgs C, int slow_blocks, int quad_blocks, int items) {
     __shared__ union { FrameShared item; FrameQuadShared quad; } shared[CORE_WPB];
-    const int wv = (int)(threadIdx.x >> 6), lane = (int)threadIdx.x & (WAVE - 1);
-    const int blk = (int)blockIdx.x;
+    static_assert(CORE_WPB == 1, "a workgroup is a wavefront: its place is that of its items");
+    const int lane = (int)threadIdx.x & (WAVE - 1);
+    int blk = (int)blockIdx.x;
     if (blk >= slow_blocks && blk < slow_blocks + quad_blocks) {
-        static_assert(CORE_WPB == 1, "a workgroup is a wavefront: its place is that of its atom and heads");
-        frame_quad_body(C, shared[wv].quad, die_order(blk - slow_blocks, quad_blocks, CORE_DIE_SHIFT - 2), lane);      // (two workgroups: an atom's)
+        frame_quad_body(C, shared[0].quad, die_order(blk - slow_blocks, quad_blocks, CORE_DIE_SHIFT - 2), lane);      // (two workgroups: an atom's)
         return;
     }
     const bool listed = blk < slow_blocks;
-    const int wid = listed ? core_slow_record(C, blk * CORE_WPB + wv, lane) : (blk - slow_blocks - quad_blocks) * CORE_WPB + wv;
-    if (wid < 0) return;
-    frame_item_body(C, shared[wv].item, wid, lane, !listed, !listed && slow_blocks > 0);
+    int wid = blk - slow_blocks - quad_blocks;
+    if (listed) {
+        wid = core_slow_record(C, blk, lane);
+        if (wid < 0) return;
+    }
+    if (REST == 1) {
+        frame_item_body(C, shared[0].item, wid, lane, !listed, !listed && slow_blocks > 0);
+        return;
+    }
+    uint32_t todo = 1;
+    if (!listed && wid >= items) {
+        const int last = C.K.N * C.K.H - 1;
+        wid = items + (wid - items) * REST;
+        const uint32_t* rec = C.K.items + (size_t)min(wid + (lane & (REST - 1)), last) * REC_WORDS;
+        const uint4 w = *reinterpret_cast<const uint4*>(rec);
+        const bool quad = (int)(w.w & 0x00ffffffu) == (C.table_R | (C.table_R << 8) | (C.table_R << 16)) &&
+                          __uint_as_float(rec[REC_A]) < 0.0f && (int)w.z <= FQ_MAX_PAIRS;
+        todo = (uint32_t)ballot(lane < REST && wid + lane <= last && !quad);
+    }
+    // (the arguments are read from memory again for every item: kept over the loop they are put away at the start of every
+    // wavefront, the four-heads ones too: 185 us)
+    typedef const __attribute__((address_space(4))) CoreArgs ArgsInMemory;
+    ArgsInMemory* args = (ArgsInMemory*)__builtin_amdgcn_kernarg_segment_ptr();
+#pragma unroll 1
+    for (; todo; todo &= todo - 1) {
+        asm volatile("" : "+s"(args));
+        wave_sync();
+        frame_item_body(*(const CoreArgs*)args, shared[0].item, wid + (int)__builtin_ctz(todo), lane, !listed, !listed && slow_blocks > 0);
+    }
 }
 
 // Everything of an item in one wavefront, for few items: its record, the search for its frame, the lattice sums.  In
