@@ -1654,6 +1654,11 @@ int slow_wave_count(int64_t N, int H) {
     const int64_t w = (N * H / 16 + 7) / 8 * 8;
     return (int)(w < 256 ? 256 : w);
 }
+// Wavefronts of a kernel that are resident at once, so many per compute unit.
+unsigned resident_waves(int per_cu) {
+    const int cus = device_cus();
+    return (unsigned)(per_cu * (cus > 0 ? cus : 256));
+}
 // one wavefront (= workgroup) per (item, head); the hardware deals them to the compute units as slots free up
 template <typename Kern>
 int launch_core(Kern kern, const cfh::CoreArgs& C, hipStream_t st, const char* what) {
@@ -1759,8 +1764,9 @@ template <int HEADS>
 int launch_core_heads(const cfh::CoreArgs& C, hipStream_t st, const char* what) {
     {
         TimedScope timed(what, st);
-        hipLaunchKernelGGL((cfh::fused_core_fwd_heads_kernel<11, HEADS>), dim3((unsigned)C.slow_wgs + (unsigned)C.K.N * (unsigned)C.K.H / HEADS),
-                           dim3(cfh::WAVE), 0, st, C);
+        const unsigned rest = resident_waves(16);
+        hipLaunchKernelGGL((cfh::fused_core_fwd_heads_kernel<11, HEADS>), dim3((unsigned)C.slow_wgs + (unsigned)C.K.N * (unsigned)C.K.H / HEADS + rest),
+                           dim3(cfh::WAVE), 0, st, C, (int)rest);
     }
     return finish_launch(what);
 }
@@ -1867,19 +1873,19 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
                 }
                 const unsigned slow_blocks = ((unsigned)F.slow_wgs + cfh::CORE_WPB - 1) / cfh::CORE_WPB;
                 // Whole blocks of pairs in work order: the rows of more than FQ_MAX_PAIRS pairs come first, and there are at most
-                // (E - N) / FQ_MAX_PAIRS of them, as every atom has one pair at least.  Where many items are left behind them,
-                // they are looked at four at a time.
+                // (E - N) / FQ_MAX_PAIRS of them, as every atom has one pair at least.  Where many items are left behind them, they
+                // have no wavefronts of their own.
                 int64_t long_rows = order && E >= N ? (E - N) / cfh::FQ_MAX_PAIRS : N;
                 if (long_rows > N) long_rows = N;
-                const unsigned singles = (unsigned)long_rows * (unsigned)p->num_heads;
+                const unsigned singles = (unsigned)long_rows * (unsigned)p->num_heads, rest = resident_waves(24);
                 {
                     TimedScope timed("frame_axes", st);
                     if (items - singles >= 49152)
-                        hipLaunchKernelGGL(cfh::frame_axes_kernel<4>, dim3(slow_blocks + quad_blocks + singles + (items - singles + 3) / 4),
-                                           dim3(cfh::WAVE * cfh::CORE_WPB), 0, st, F, (int)slow_blocks, (int)quad_blocks, (int)singles);
+                        hipLaunchKernelGGL(cfh::frame_axes_kernel<true>, dim3(slow_blocks + quad_blocks + singles + rest),
+                                           dim3(cfh::WAVE * cfh::CORE_WPB), 0, st, F, (int)slow_blocks, (int)quad_blocks, (int)singles, (int)rest);
                     else
-                        hipLaunchKernelGGL(cfh::frame_axes_kernel<1>, dim3(slow_blocks + quad_blocks + items),
-                                           dim3(cfh::WAVE * cfh::CORE_WPB), 0, st, F, (int)slow_blocks, (int)quad_blocks, 0);
+                        hipLaunchKernelGGL(cfh::frame_axes_kernel<false>, dim3(slow_blocks + quad_blocks + items),
+                                           dim3(cfh::WAVE * cfh::CORE_WPB), 0, st, F, (int)slow_blocks, (int)quad_blocks, 0, 0);
                 }
                 if ((rc = finish_launch("frame_axes"))) return rc;
             } else if ((rc = launch_core(cfh::frame_axes_sorted_kernel, F, st, "frame_axes"))) return rc;

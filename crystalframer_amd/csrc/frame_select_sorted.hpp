@@ -682,21 +682,23 @@ __global__ __launch_bounds__(WAVE * CORE_WPB) void frame_axes_sorted_kernel(cons
 //   1. one per listed record with a box of their own, by rank over the lists (made by the launch that wrote the
 //      records; no record of that rank: the wavefront ends): several sorted chunks, the longest of the launch;
 //   2. the four-heads search over all atoms;
-//   3. REST = 1: one per item, for the items that neither of the two takes (usual box, longer rows: they are at the start of the
-//      work order, so the wavefronts that find nothing to do come last and only pass through);
-//      else one per item for the first `items` places, where the long rows are, and one per REST items behind them, for whatever
-//      is left there (a box of its own of a rank past the leading wavefronts, a >= 0).
+//   3. one per item, for the items that neither of the two takes (usual box, longer rows: they are at the start of the
+//      work order, so the wavefronts that find nothing to do come last and only pass through).
 // With the items of (3) and their many passing wavefronts in front, the four-heads search started after a third of
 // the launch's time, and the records with a box of their own, scattered over the work order, later still.
-// REST: a wavefront that passes through takes its turn at the dispatcher all the same, 115 us for 180 224 items of up to 10 pairs
-// where 83 are left without them; REST 4 99.7, 8 97.6, 16 101.  But the loop keeps more alive: 18 976 items of 1 to 60 pairs 28.8 us
-// with REST 1, 30.4 with 4, 30 720 long rows 145 and 150.
-template <int REST>
-__global__ __launch_bounds__(WAVE * CORE_WPB) void frame_axes_kernel(const CoreArgs C, int slow_blocks, int quad_blocks, int items) {
+// REST: (3) for the `items` first places alone, where the long rows are, and behind them
+//   4. `rest` wavefronts, as many as are resident, that look at every rest-th place each for whatever is left there (a box of its
+//      own of a rank past the leading wavefronts, a >= 0, a long row out of order).
+// A wavefront that passes through takes its turn at the dispatcher all the same: 180 224 items of up to 10 pairs 115 us, 83 without
+// those wavefronts, with REST 103.  But the loop over the places keeps more alive: 18 976 items of 1 to 60 pairs 28.8 us and
+// 30.4, 30 720 long rows 145 and 150.  (Four neighbouring places per wavefront: 100 us, but in a batch of nothing but cells
+// with a box of their own, 82 000 items, 916 -> 1422.)
+template <bool REST>
+__global__ __launch_bounds__(WAVE * CORE_WPB) void frame_axes_kernel(const CoreArgs C, int slow_blocks, int quad_blocks, int items, int rest) {
     __shared__ union { FrameShared item; FrameQuadShared quad; } shared[CORE_WPB];
     static_assert(CORE_WPB == 1, "a workgroup is a wavefront: its place is that of its items");
     const int lane = (int)threadIdx.x & (WAVE - 1);
-    int blk = (int)blockIdx.x;
+    const int blk = (int)blockIdx.x;
     if (blk >= slow_blocks && blk < slow_blocks + quad_blocks) {
         frame_quad_body(C, shared[0].quad, die_order(blk - slow_blocks, quad_blocks, CORE_DIE_SHIFT - 2), lane);      // (two workgroups: an atom's)
         return;
@@ -707,29 +709,34 @@ __global__ __launch_bounds__(WAVE * CORE_WPB) void frame_axes_kernel(const CoreA
         wid = core_slow_record(C, blk, lane);
         if (wid < 0) return;
     }
-    if (REST == 1) {
+    if (!REST) {
         frame_item_body(C, shared[0].item, wid, lane, !listed, !listed && slow_blocks > 0);
         return;
     }
-    uint32_t todo = 1;
-    if (!listed && wid >= items) {
-        const int last = C.K.N * C.K.H - 1;
-        wid = items + (wid - items) * REST;
-        const uint32_t* rec = C.K.items + (size_t)min(wid + (lane & (REST - 1)), last) * REC_WORDS;
-        const uint4 w = *reinterpret_cast<const uint4*>(rec);
-        const bool quad = (int)(w.w & 0x00ffffffu) == (C.table_R | (C.table_R << 8) | (C.table_R << 16)) &&
-                          __uint_as_float(rec[REC_A]) < 0.0f && (int)w.z <= FQ_MAX_PAIRS;
-        todo = (uint32_t)ballot(lane < REST && wid + lane <= last && !quad);
-    }
+    const bool several = !listed && wid >= items;
     // (the arguments are read from memory again for every item: kept over the loop they are put away at the start of every
     // wavefront, the four-heads ones too: 185 us)
     typedef const __attribute__((address_space(4))) CoreArgs ArgsInMemory;
     ArgsInMemory* args = (ArgsInMemory*)__builtin_amdgcn_kernarg_segment_ptr();
 #pragma unroll 1
-    for (; todo; todo &= todo - 1) {
-        asm volatile("" : "+s"(args));
-        wave_sync();
-        frame_item_body(*(const CoreArgs*)args, shared[0].item, wid + (int)__builtin_ctz(todo), lane, !listed, !listed && slow_blocks > 0);
+    for (; wid < C.K.N * C.K.H; wid += rest * WAVE) {
+        uint64_t todo = 1;
+        if (several) {      // places wid, wid + rest, ...
+            const int total = C.K.N * C.K.H;
+            const int64_t place = (int64_t)wid + (int64_t)lane * rest;
+            const uint32_t* rec = C.K.items + (size_t)min(place, (int64_t)total - 1) * REC_WORDS;
+            const uint4 w = *reinterpret_cast<const uint4*>(rec);
+            const bool quad = (int)(w.w & 0x00ffffffu) == (C.table_R | (C.table_R << 8) | (C.table_R << 16)) &&
+                              __uint_as_float(rec[REC_A]) < 0.0f && (int)w.z <= FQ_MAX_PAIRS;
+            todo = ballot(place < total && !quad);
+        }
+#pragma unroll 1
+        for (; todo; todo &= todo - 1) {
+            asm volatile("" : "+s"(args));
+            wave_sync();
+            frame_item_body(*(const CoreArgs*)args, shared[0].item, wid + (int)__builtin_ctzll(todo) * rest, lane, !listed, !listed && slow_blocks > 0);
+        }
+        if (!several) return;
     }
 }
 

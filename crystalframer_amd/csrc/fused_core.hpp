@@ -1519,38 +1519,51 @@ __device__ __forceinline__ void fused_core_fwd_heads(const CoreArgs& C, CoreHead
         atomicAdd(P.stats + STAT_FWD_SEEN, n_seen);
     }
 }
-// The leading wavefronts take a listed record each, the others HEADS heads of an atom; where not all of those have the usual box,
-// one after the other (but the listed ones, as in the kernel of one item per wavefront).
+// The leading wavefronts take a listed record each, the next ones HEADS heads of an atom (where some of those are listed, the others
+// one after the other), and the `rest` last ones the listed records that are left, by rank, each every rest-th of them.  (Records
+// with a box of their own have 16 wavefronts per compute unit here and 28 in the kernel of one item per wavefront: a batch of nothing
+// but such cells, 82 000 items, takes 1.26 times as long; the leading wavefronts are enough for one item in sixteen.)
 template <int WL, int HEADS>
-__global__ __launch_bounds__(WAVE) void fused_core_fwd_heads_kernel(const CoreArgs C) {
+__global__ __launch_bounds__(WAVE) void fused_core_fwd_heads_kernel(const CoreArgs C, int rest) {
     __shared__ union { CoreFwdLds<0, true> one; CoreHeadsShared<HEADS> several; } sh;
     const KernelArgs& P = C.K;
     const int lane = (int)threadIdx.x & (WAVE - 1), w = (int)blockIdx.x;
-    int wid, items = 1;
-    if (w < C.slow_wgs) {
-        wid = __builtin_amdgcn_readfirstlane(core_slow_record(C, w, lane));
-        if (wid < 0) return;
-    } else {
+    const int groups = P.N * P.H / HEADS;
+    const bool by_rank = w < C.slow_wgs || w >= C.slow_wgs + groups;
+    int wid = 0, rank = w < C.slow_wgs ? w : w - groups;
+    uint32_t left = 1;                 // heads of this wavefront's own that are not listed
+    if (!by_rank) {
         constexpr int shift = HEADS == 2 ? CORE_DIE_SHIFT - 1 : CORE_DIE_SHIFT - 2;      // (an atom's heads on one die)
-        wid = HEADS * __builtin_amdgcn_readfirstlane(die_order(w - C.slow_wgs, P.N * P.H / HEADS, shift));
+        wid = HEADS * __builtin_amdgcn_readfirstlane(die_order(w - C.slow_wgs, groups, shift));
         const int it = div_heads(P, wid), h0 = wid - it * P.H;
         if (it >= P.N) return;
         HeadRecords<HEADS> rec;
         rec.load(P, it, h0, lane);
         const int usual = C.table_R | (C.table_R << 8) | (C.table_R << 16);
+        left = 0;
         bool together = true;
 #pragma unroll
-        for (int hh = 0; hh < HEADS; hh++) together = together && rec.word(hh, REC_BOX) == usual && __int_as_float(rec.word(hh, REC_A)) < 0.0f;
+        for (int hh = 0; hh < HEADS; hh++) {
+            const int box = rec.word(hh, REC_BOX);
+            together = together && box == usual && __int_as_float(rec.word(hh, REC_A)) < 0.0f;
+            left |= ((uint32_t)box & REC_BOX_LISTED) != 0u ? 0u : 1u << hh;
+        }
         if (together) {
             fused_core_fwd_heads<WL, HEADS>(C, sh.several, h0, rec);
             return;
         }
-        items = HEADS;
     }
 #pragma unroll 1
-    for (int k = 0; k < items; k++) {
+    for (; left; left &= left - 1) {
+        int item = wid + __builtin_ctz(left);
+        if (by_rank) {
+            item = __builtin_amdgcn_readfirstlane(core_slow_record(C, rank, lane));
+            if (item < 0) return;
+            if (rank >= C.slow_wgs) left = 3;      // (another rank behind this one)
+            rank += rest;
+        }
         wave_sync();
-        fused_core_fwd_body<WL, 0, false, true>(C, sh.one, wid + k);
+        fused_core_fwd_body<WL, 0, false, true>(C, sh.one, item);
     }
 }
 
