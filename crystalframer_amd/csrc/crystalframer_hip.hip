@@ -1858,7 +1858,7 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
             {
                 TimedScope timed("core_prepare", st);
                 hipLaunchKernelGGL(cfh::core_prepare_wcat_kernel, dim3(prep_blocks + wcat_blocks), dim3(256), 0, st,
-                                   F.K, 1, prep_blocks, WA);
+                                   F.K, 2, prep_blocks, WA);
             }
             if (F.sorted_tab) {
                 // four heads of an atom per wavefront for the items with the usual box and short rows, the others one

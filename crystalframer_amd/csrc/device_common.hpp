@@ -590,6 +590,7 @@ __device__ __forceinline__ uint32_t make_record_lane(const KernelArgs& P, int it
          : lane == 31 ? (uint32_t)R.b : 0u;
 }
 
+// with_query: 1 the query in the record, 2 the search reads it where it is.
 // One thread per (item, head): builds the records, clears the work queues of the launch and (backward)
 // the weight-gradient outputs that the reduction after the main kernel adds into.
 __device__ __forceinline__ void prepare_items_block(const KernelArgs& P, int with_query, int block) {
@@ -619,7 +620,7 @@ __device__ __forceinline__ void prepare_items_block(const KernelArgs& P, int wit
         slow = P.slow_count != nullptr && !(R.bx.R1 == P.slow_R && R.bx.R2 == P.slow_R && R.bx.R3 == P.slow_R);
         const float* L = P.tvecs + (size_t)R.b * 9;
         float q[DH] = {};
-        if (with_query) {
+        if (with_query == 1) {
             const float4* src = reinterpret_cast<const float4*>(P.q + ((size_t)R.i * P.H + h) * DH);
 #pragma unroll
             for (int c = 0; c < DH / 4; c++) {
@@ -664,7 +665,9 @@ __device__ __forceinline__ void prepare_items_block(const KernelArgs& P, int wit
         uint32_t* rec = P.items + (size_t)idx * REC_WORDS;
         *reinterpret_cast<uint4*>(rec) = make_uint4((uint32_t)R.i, (uint32_t)R.e0, (uint32_t)R.npairs, R.boxw);
 #pragma unroll
-        for (int u = 0; u < 7; u++) reinterpret_cast<float4*>(rec)[1 + u] = tail[u];
+        for (int u = 0; u < 7; u++)      // (words 16 .. 27: query or frames only; 180 224 records of
+                                         // distances alone without them 12.2 us -> 9.9, with a frame search 14.4 -> 11.6)
+            if (u < 3 || u == 6 || with_query == 1 || P.frames) reinterpret_cast<float4*>(rec)[1 + u] = tail[u];
     }
 }
 __global__ __launch_bounds__(256) void prepare_items_kernel(const KernelArgs P, int with_query) {

@@ -121,8 +121,9 @@ __device__ __forceinline__ void frame_item_body(const CoreArgs& C, FrameShared& 
         const Lattice L = item.L;
         const Box bx = item.bx;
         float qi[DH];
+        const uint32_t query = own ? rec_cur : __float_as_uint(P.q[((size_t)i * H + h) * DH + (lane & (DH - 1))]);
 #pragma unroll
-        for (int c = 0; c < DH; c++) qi[c] = rec_f(rec_cur, REC_QUERY + c);
+        for (int c = 0; c < DH; c++) qi[c] = rec_f(query, own ? REC_QUERY + c : c);
         const bool sorted = C.sorted_tab != nullptr && bx.R1 == C.table_R && bx.R2 == C.table_R && bx.R3 == C.table_R &&
                             a < 0.0f;
         if (others_only && sorted && item.npairs <= FQ_MAX_PAIRS) return;      // searched four heads at a time
@@ -459,7 +460,7 @@ __device__ __forceinline__ void frame_quad_body(const CoreArgs& C, FrameQuadShar
     const float inv_a = a < 0.0f ? hw_rcp(a) : 0.0f;      // (for a reach with margins: the hardware reciprocal will do)
     float q[DH];
     {
-        const float4* qp = reinterpret_cast<const float4*>(rec + REC_QUERY);
+        const float4* qp = reinterpret_cast<const float4*>(P.q + ((size_t)i * H + h_row) * DH);
 #pragma unroll
         for (int c4 = 0; c4 < DH / 4; c4++) {
             const float4 v = qp[c4];
