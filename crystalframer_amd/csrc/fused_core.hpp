@@ -1088,6 +1088,15 @@ __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLd
 
         // ---- the row is complete: normalise and write
         CFH_PH(7);
+        auto count_item = [&] {
+            CFH_PH_FLUSH(P.stats);
+            if (P.stats && lane == 0) {
+                atomicAdd(P.stats + STAT_FWD_EVAL, n_eval);
+                atomicAdd(P.stats + STAT_FWD_RAW, (unsigned long long)bx.T * (unsigned long long)npairs);
+                atomicAdd(P.stats + STAT_FWD_PAIRS, (unsigned long long)npairs);
+                atomicAdd(P.stats + STAT_FWD_SEEN, n_seen);
+            }
+        };
         const float D = uniform_f(wave_sum(Dl));
         const float inv = D > 0.0f ? hw_rcp(D) : 0.0f;
         const float sc = inv * hw_rcp(fixs);
@@ -1129,6 +1138,7 @@ __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLd
                 }
                 if (lane < FC_GROUP) reinterpret_cast<float2*>(tab)[lane] = make_float2(ox, oy);
                 if (lane == 0) tab[4].x = __int_as_float(i);
+                count_item();
                 return;
             }
             const float* Wh = wcat + (size_t)h * DH * HWK;
@@ -1221,13 +1231,7 @@ __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLd
             }
         }
         if (PLACES && !own && it_cur < C.ticket_items) core_project_done<HWK>(C, it_cur, h, lane);
-        CFH_PH_FLUSH(P.stats);
-        if (P.stats && lane == 0) {
-            atomicAdd(P.stats + STAT_FWD_EVAL, n_eval);
-            atomicAdd(P.stats + STAT_FWD_RAW, (unsigned long long)bx.T * (unsigned long long)npairs);
-            atomicAdd(P.stats + STAT_FWD_PAIRS, (unsigned long long)npairs);
-            atomicAdd(P.stats + STAT_FWD_SEEN, n_seen);
-        }
+        count_item();
     }
 }
 

@@ -668,6 +668,36 @@ def test_products_by_further_wavefronts_of_an_item(bins, B, atoms, width, cos_ab
     assert Hh.rel_err(out, kept.double()) < 1e-5
 
 
+# Every form of inference counts its terms: with further wavefronts for the product, one launch without, several launches with the
+# products in the main kernel, two and four heads per wavefront.
+@pytest.mark.parametrize("bins,B,atoms", [(64, 1, 8), (16, 3, 8), (64, 120, 1), (0, 3, 8), (64, 2200, 1), (0, 2100, 1), (0, 5700, 1)])
+def test_inference_counts_its_terms(bins, B, atoms):
+    """The same pairs as a pass that keeps everything, and its images within 0.1 % (its inputs differ in their last bits, which
+    moves an image across the threshold of a pair now and then)."""
+    from crystalframer_amd import _lib, params, synthetic
+    from crystalframer_amd.cuda_funcs import KernelManager as KM
+    kw = dict(value_pe_angle_wscale=1.0, value_pe_dist_coef=1.5, value_pe_angle_coef=6.0) if bins == 16 else {}
+    mp = params.ModelParams(num_layers=1, value_pe_angle_real=bins, symm_break_noise=0.0, **kw)
+    cb = synthetic.make_batch(B, atoms="uniform", atoms_lo=atoms, atoms_hi=atoms, len_lo=3.0, len_hi=9.0, ang_lo=65.0,
+                              ang_hi=115.0, seed=B)
+    model, cb = _model(mp, cb)
+    model.eval()
+    saved, counts = KM.COLLECT_STATS, []
+    KM.COLLECT_STATS = True
+    try:
+        for keep in (True, False):
+            _lib.read_stats(torch.device("cuda:0"), reset=True)
+            with torch.set_grad_enabled(keep):
+                model(cb)
+            counts.append(_lib.read_stats(torch.device("cuda:0"), reset=True))
+    finally:
+        KM.COLLECT_STATS = saved
+    kept, lean = counts
+    assert lean["fwd_pairs"] == kept["fwd_pairs"] == 8 * B * atoms * atoms
+    for name in ("fwd_evaluated", "fwd_in_box", "fwd_visited"):
+        assert kept[name] > 0 and abs(lean[name] - kept[name]) <= (1e-3 if name != "fwd_visited" else 0.5) * kept[name], name
+
+
 # Inference of many items with the angle encoding: the wavefront that completes sixteen items of a head makes their products, but
 # for the last items (a fifth, at least 16 384 on 256 compute units).  One atom short of the first 128 atoms whose products are
 # made so, exactly those, a last block of one atom and of 127, rows of mixed lengths, sixteen heads.
