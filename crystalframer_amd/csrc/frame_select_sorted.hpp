@@ -774,7 +774,6 @@ __global__ __launch_bounds__(WAVE * (1 + HELPERS)) void item_pass_kernel(const C
     }
     if (!LEAN && lane < REC_WORDS) P.items[((size_t)it * P.H + h) * REC_WORDS + lane] = own.rec;
     fused_core_fwd_body<WL, ANG, COS_ABS, LEAN, 1, (HELPERS > 0)>(C, sh.core, wid, wcat, &own);
-    if (HELPERS > 0) __syncthreads();
 }
 
 }  // namespace cfh

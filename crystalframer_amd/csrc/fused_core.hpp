@@ -775,7 +775,7 @@ __device__ __forceinline__ void core_project_done(const CoreArgs& C, int it, int
 // own: not null: the item's record and first operands, in registers
 struct CoreOwn { uint32_t rec; CorePrefetch pf; };
 // HAND_OVER (LEAN only): the histogram stays in LDS as float32 words, with the item's part of `out` and its atom in front of the
-// table, for other wavefronts of the workgroup (core_product_words)
+// table, for other wavefronts of the workgroup (CoreProductWeights), which wait at a barrier until it is there
 template <int WL, int ANG, bool COS_ABS, bool LEAN, int COPIES = 1, bool HAND_OVER = false>
 __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLds<ANG, LEAN, COPIES>& sh, int wid,
                                                     const float* __restrict__ wcat = nullptr, const CoreOwn* own = nullptr) {
@@ -1138,6 +1138,7 @@ __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLd
                 }
                 if (lane < FC_GROUP) reinterpret_cast<float2*>(tab)[lane] = make_float2(ox, oy);
                 if (lane == 0) tab[4].x = __int_as_float(i);
+                __syncthreads();      // (the statistics wait, not the product)
                 count_item();
                 return;
             }
