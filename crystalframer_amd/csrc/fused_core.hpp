@@ -328,7 +328,7 @@ __global__ __launch_bounds__(256) void core_wcat_kernel(const WcatArgs A) { core
 // following H * 16 those of core_wcat_kernel.
 __global__ __launch_bounds__(256) void core_prepare_wcat_kernel(const KernelArgs P, int with_query, int prep_blocks,
                                                                 const WcatArgs A) {
-    if ((int)blockIdx.x < prep_blocks) prepare_items_block(P, with_query, (int)blockIdx.x);
+    if ((int)blockIdx.x < prep_blocks) prepare_items_block<true>(P, with_query, (int)blockIdx.x);
     else core_wcat_block(A, (int)blockIdx.x - prep_blocks);
 }
 constexpr int CORE_GW_SLICES = 8;      // at most this many slices of the atoms per job (copies of the scratch)
