@@ -1659,6 +1659,16 @@ unsigned resident_waves(int per_cu) {
     const int cus = device_cus();
     return (unsigned)(per_cu * (cus > 0 ? cus : 256));
 }
+// Workgroups of a kernel that are resident on the device at once (asked of the runtime once per kernel).
+template <auto KERN>
+unsigned resident_workgroups(int threads) {
+    static const int per_cu = [threads] {
+        int n = 0;
+        return hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, KERN, threads, 0) == hipSuccess && n > 0 ? n : 16;
+    }();
+    const int cus = device_cus();
+    return (unsigned)(per_cu * (cus > 0 ? cus : 256));
+}
 // one wavefront (= workgroup) per (item, head); the hardware deals them to the compute units as slots free up
 template <typename Kern>
 int launch_core(Kern kern, const cfh::CoreArgs& C, hipStream_t st, const char* what) {
@@ -1855,6 +1865,21 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
             F.K.q = qs; F.K.k = k; F.K.out_frame = frames;
             F.K.counters2 = reinterpret_cast<int32_t*>(ws + QUEUE_OFFSET + QUEUE_SET_BYTES);
             F.K.frames_to_records = 1;
+            // Whole blocks of pairs in work order: the rows of more than FQ_MAX_PAIRS pairs come first, and there are at most
+            // (E - N) / FQ_MAX_PAIRS of them, as every atom has one pair at least.  Where a third of the items or more lie behind
+            // them, those have no wavefronts of their own: what the four-heads search leaves of them is listed.  Whole passes of four
+            // layers, 64 bins, in us, a wavefront each / from the lists.  r (pairs per atom) = 3: 31 992 items 487/476, 127 992
+            // 1668/1602; r = 7: 14 160 492/484, 40 520 816/808, 80 904 1474/1445; r = 8: 32 704 721/711, 130 744 2004/1970; r = 10:
+            // 20 600 493/491, 128 040 2060/2032; r = 11: 19 624 519/516, 62 936 1182/1161, 127 880 2178/2164; r = 12, a third
+            // behind: 19 968 526/525, 63 936 1246/1231, 127 968 2215/2224; r = 14, a fifth: 20 000 539/543, 129 288 2450/2481; r =
+            // 16: 19 752 595/600, 128 000 2739/2777.  With cells whose box is not the usual one, r = 7: one in a hundred 14 160
+            // 595/578, 80 904 2964/2837; one in ten 1346/1321, 4227/4088; all 2121/2019, 10 608/10 242.
+            const unsigned items = (unsigned)N * (unsigned)p->num_heads;
+            int64_t long_rows = order && E >= N ? (E - N) / cfh::FQ_MAX_PAIRS : N;
+            if (long_rows > N) long_rows = N;
+            const unsigned singles = (unsigned)long_rows * (unsigned)p->num_heads;
+            const bool from_lists = F.sorted_tab && F.K.slow_count && 3 * (uint64_t)(items - singles) >= items;
+            if (from_lists) { F.K.list_pairs = cfh::FQ_MAX_PAIRS; F.K.list_from = (int32_t)long_rows; }
             {
                 TimedScope timed("core_prepare", st);
                 hipLaunchKernelGGL(cfh::core_prepare_wcat_kernel, dim3(prep_blocks + wcat_blocks), dim3(256), 0, st,
@@ -1863,7 +1888,6 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
             if (F.sorted_tab) {
                 // four heads of an atom per wavefront for the items with the usual box and short rows, the others one
                 // by one, all in one launch
-                const unsigned items = (unsigned)N * (unsigned)p->num_heads;
                 const unsigned quad_waves = (unsigned)N * (unsigned)((p->num_heads + cfh::FQ_ROWS - 1) / cfh::FQ_ROWS);
                 const unsigned quad_blocks = (quad_waves + cfh::CORE_WPB - 1) / cfh::CORE_WPB;
                 if (F.K.slow_count) {
@@ -1872,15 +1896,10 @@ int fused_core_forward_impl(const cfh_params* p, const float* qs, const float* k
                     F.slow_wgs = slow_wave_count(N, p->num_heads);
                 }
                 const unsigned slow_blocks = ((unsigned)F.slow_wgs + cfh::CORE_WPB - 1) / cfh::CORE_WPB;
-                // Whole blocks of pairs in work order: the rows of more than FQ_MAX_PAIRS pairs come first, and there are at most
-                // (E - N) / FQ_MAX_PAIRS of them, as every atom has one pair at least.  Where many items are left behind them, they
-                // have no wavefronts of their own.
-                int64_t long_rows = order && E >= N ? (E - N) / cfh::FQ_MAX_PAIRS : N;
-                if (long_rows > N) long_rows = N;
-                const unsigned singles = (unsigned)long_rows * (unsigned)p->num_heads, rest = resident_waves(24);
                 {
                     TimedScope timed("frame_axes", st);
-                    if (items - singles >= 49152)
+                    const unsigned rest = resident_workgroups<cfh::frame_axes_kernel<true>>(cfh::WAVE * cfh::CORE_WPB);
+                    if (from_lists)
                         hipLaunchKernelGGL(cfh::frame_axes_kernel<true>, dim3(slow_blocks + quad_blocks + singles + rest),
                                            dim3(cfh::WAVE * cfh::CORE_WPB), 0, st, F, (int)slow_blocks, (int)quad_blocks, (int)singles, (int)rest);
                     else

@@ -377,6 +377,8 @@ struct KernelArgs {
     int32_t* slow_list;           // (blocks, SLOW_PREP_SLOTS) records whose box is not the usual one, for the launches that
                                   // follow to take first
     int32_t slow_R;               // half-width of the usual box
+    int32_t list_pairs;           // > 0: listed as well what the four-heads frame search leaves: rows of more pairs from place
+    int32_t list_from;            // list_from of the work order on, and a >= 0
     unsigned long long* stats;    // optional running totals (see STAT_* below); never reset by a launch
     int32_t* status;              // word of the workspace header (bits, never cleared): 1 a box was cut back to RMAX;
                                   // 2 the pairs of an atom are not the consecutive neighbours j0, j0 + 1, ...
@@ -620,7 +622,9 @@ __device__ __forceinline__ void prepare_items_block(const KernelArgs& P, int wit
     if (valid) {
         const int it = idx / P.H, h = idx - it * P.H;
         R = record_head(P, it, h);
-        slow = P.slow_count != nullptr && !(R.bx.R1 == P.slow_R && R.bx.R2 == P.slow_R && R.bx.R3 == P.slow_R);
+        slow = P.slow_count != nullptr &&
+               (!(R.bx.R1 == P.slow_R && R.bx.R2 == P.slow_R && R.bx.R3 == P.slow_R) ||
+                (P.list_pairs > 0 && (!(R.a < 0.0f) || (R.npairs > P.list_pairs && it >= P.list_from))));
         const float* L = P.tvecs + (size_t)R.b * 9;
         float q[DH] = {};
         if (with_query == 1) {

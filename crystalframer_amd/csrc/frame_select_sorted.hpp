@@ -85,10 +85,10 @@ struct FrameShared {
 };
 // one wavefront, one item: wid = item * H + head.  `others_only`: only the items that the four-heads-per-wavefront
 // search leaves out (box not the table's, or more pairs than it takes).
-// `skip_listed`: the records listed for the first wavefronts of the launch are theirs.
+// `skip_listed`: 1 the records listed for the first wavefronts of the launch are theirs, 2 no listed record is taken here.
 // `own`: not null: the item's record, in registers; the frames go into it instead of memory (`keep`: as well).
 __device__ __forceinline__ void frame_item_body(const CoreArgs& C, FrameShared& sh, int wid, int lane, bool others_only,
-                                                bool skip_listed, uint32_t* own = nullptr, bool keep = true) {
+                                                int skip_listed, uint32_t* own = nullptr, bool keep = true) {
     float4* const tab = sh.tab;
     float4* const pq = sh.pq;
     uint32_t* const markw = sh.markw;
@@ -110,8 +110,8 @@ __device__ __forceinline__ void frame_item_body(const CoreArgs& C, FrameShared& 
     {
         const uint32_t rec_cur = own ? *own : load_record_lane(P, it_cur, h, lane);
         if (skip_listed && ((uint32_t)__builtin_amdgcn_readlane((int)rec_cur, REC_BOX) & REC_BOX_LISTED) != 0u &&
-            core_slow_rank(C, wid, lane) < C.slow_wgs)
-            return;      // (a listed record of higher rank stays here)
+            (skip_listed == 2 || core_slow_rank(C, wid, lane) < C.slow_wgs))
+            return;      // (1: a listed record of higher rank stays here)
         const Item item = unpack_item(rec_cur);
         const int crystal = __builtin_amdgcn_readlane((int)rec_cur, REC_CRYSTAL);
         const int j0 = __builtin_amdgcn_readlane((int)rec_cur, REC_J0);
@@ -389,7 +389,7 @@ __device__ __forceinline__ void frame_item_body(const CoreArgs& C, FrameShared& 
 // and a best candidate is a score and one key.  180 224 items of up to 10 pairs 139 -> 115 us, 18 976 of 1 to 60 pairs 30.3 -> 28.8
 // (before: q.k of the four heads one after the other with the query read across the rows, everything read back from LDS in each of
 // the three passes, a best candidate of three words).
-// Rows whose box is not the table's are left to frame_axes_sorted_kernel (unsorted_only).
+// Rows whose box is not the table's are left to frame_item_body.
 template <int CTRL>
 __device__ __forceinline__ float row_maxf_step(float x) { return fmaxf(x, dpp_move<CTRL>(x)); }
 __device__ __forceinline__ float row_max(float x) {
@@ -676,7 +676,7 @@ __device__ __forceinline__ void frame_quad_body(const CoreArgs& C, FrameQuadShar
 __global__ __launch_bounds__(WAVE * CORE_WPB) void frame_axes_sorted_kernel(const CoreArgs C) {
     __shared__ FrameShared shared[CORE_WPB];
     frame_item_body(C, shared[threadIdx.x >> 6], (int)blockIdx.x * CORE_WPB + (int)(threadIdx.x >> 6),
-                    (int)threadIdx.x & (WAVE - 1), false, false);
+                    (int)threadIdx.x & (WAVE - 1), false, 0);
 }
 
 // Both ways in one launch, the slowest work first.  Wavefronts in the order of the grid:
@@ -687,13 +687,14 @@ __global__ __launch_bounds__(WAVE * CORE_WPB) void frame_axes_sorted_kernel(cons
 //      work order, so the wavefronts that find nothing to do come last and only pass through).
 // With the items of (3) and their many passing wavefronts in front, the four-heads search started after a third of
 // the launch's time, and the records with a box of their own, scattered over the work order, later still.
-// REST: (3) for the `items` first places alone, where the long rows are, and behind them
-//   4. `rest` wavefronts, as many as are resident, that look at every rest-th place each for whatever is left there (a box of its
-//      own of a rank past the leading wavefronts, a >= 0, a long row out of order).
+// REST: (3) for the `items` first places alone, where the long rows are, and for unlisted ones only; whatever else the four-heads search
+// leaves is listed, too, and behind them come
+//   4. `rest` wavefronts, as many as are resident, that take the listed records past the leading wavefronts: the first by their own
+//      rank, the next ones as they come from a counter, until there are no more.
 // A wavefront that passes through takes its turn at the dispatcher all the same: 180 224 items of up to 10 pairs 115 us, 83 without
-// those wavefronts, with REST 103.  But the loop over the places keeps more alive: 18 976 items of 1 to 60 pairs 28.8 us and
-// 30.4, 30 720 long rows 145 and 150.  (Four neighbouring places per wavefront: 100 us, but in a batch of nothing but cells
-// with a box of their own, 82 000 items, 916 -> 1422.)
+// those wavefronts, with REST 99.  In a batch of nothing but cells with a box of their own (180 816 items) 1781 us with a wavefront
+// for each, with REST 1661; half of them so 747 and 686.  (NQUEUE counters, a die's wavefronts two of them: the atomics on one
+// counter took 14 ns each, 1301 us for the half.  The places dealt out beforehand: 2189 and 894.)
 template <bool REST>
 __global__ __launch_bounds__(WAVE * CORE_WPB) void frame_axes_kernel(const CoreArgs C, int slow_blocks, int quad_blocks, int items, int rest) {
     __shared__ union { FrameShared item; FrameQuadShared quad; } shared[CORE_WPB];
@@ -706,38 +707,32 @@ __global__ __launch_bounds__(WAVE * CORE_WPB) void frame_axes_kernel(const CoreA
     }
     const bool listed = blk < slow_blocks;
     int wid = blk - slow_blocks - quad_blocks;
-    if (listed) {
-        wid = core_slow_record(C, blk, lane);
-        if (wid < 0) return;
-    }
     if (!REST) {
-        frame_item_body(C, shared[0].item, wid, lane, !listed, !listed && slow_blocks > 0);
+        if (listed && (wid = core_slow_record(C, blk, lane)) < 0) return;
+        frame_item_body(C, shared[0].item, wid, lane, !listed, !listed && slow_blocks > 0 ? 1 : 0);
         return;
     }
     const bool several = !listed && wid >= items;
+    int rank = listed ? blk : slow_blocks + wid - items;
+    SlowRuns runs{0, 0};
+    if (listed || several) runs = core_slow_runs(C, lane);
     // (the arguments are read from memory again for every item: kept over the loop they are put away at the start of every
     // wavefront, the four-heads ones too: 185 us)
     typedef const __attribute__((address_space(4))) CoreArgs ArgsInMemory;
     ArgsInMemory* args = (ArgsInMemory*)__builtin_amdgcn_kernarg_segment_ptr();
 #pragma unroll 1
-    for (; wid < C.K.N * C.K.H; wid += rest * WAVE) {
-        uint64_t todo = 1;
-        if (several) {      // places wid, wid + rest, ...
-            const int total = C.K.N * C.K.H;
-            const int64_t place = (int64_t)wid + (int64_t)lane * rest;
-            const uint32_t* rec = C.K.items + (size_t)min(place, (int64_t)total - 1) * REC_WORDS;
-            const uint4 w = *reinterpret_cast<const uint4*>(rec);
-            const bool quad = (int)(w.w & 0x00ffffffu) == (C.table_R | (C.table_R << 8) | (C.table_R << 16)) &&
-                              __uint_as_float(rec[REC_A]) < 0.0f && (int)w.z <= FQ_MAX_PAIRS;
-            todo = ballot(place < total && !quad);
+    for (;;) {
+        asm volatile("" : "+s"(args));
+        const CoreArgs& A = *(const CoreArgs*)args;
+        if (listed || several) {
+            wid = __builtin_amdgcn_readfirstlane(core_slow_record(A, runs, rank, lane));
+            if (wid < 0) return;
         }
-#pragma unroll 1
-        for (; todo; todo &= todo - 1) {
-            asm volatile("" : "+s"(args));
-            wave_sync();
-            frame_item_body(*(const CoreArgs*)args, shared[0].item, wid + (int)__builtin_ctzll(todo) * rest, lane, !listed, !listed && slow_blocks > 0);
-        }
+        wave_sync();
+        frame_item_body(A, shared[0].item, wid, lane, !listed && !several, listed || several ? 0 : 2);
         if (!several) return;
+        const int q = blk & (NQUEUE - 1);
+        rank = slow_blocks + rest + queue_draw(A.K.counters + q * QSTRIDE) * NQUEUE + q;
     }
 }
 
@@ -769,7 +764,7 @@ __global__ __launch_bounds__(WAVE * (1 + HELPERS)) void item_pass_kernel(const C
     own.rec = make_record_lane(P, it, h, lane, search != 0);
     own.pf = core_prefetch(C, own.rec, it, h, lane);
     if (ANG > 0 && search) {
-        frame_item_body(C, sh.frame, wid, lane, false, false, &own.rec, !LEAN);
+        frame_item_body(C, sh.frame, wid, lane, false, 0, &own.rec, !LEAN);
         __threadfence_block();
     }
     if (!LEAN && lane < REC_WORDS) P.items[((size_t)it * P.H + h) * REC_WORDS + lane] = own.rec;

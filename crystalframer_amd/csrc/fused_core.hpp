@@ -522,15 +522,22 @@ __device__ __forceinline__ void core_store_table(const CoreItem& ci, const CoreP
 // the same in all lanes.  Two levels, so that the wavefront waits for memory twice whatever the number of lists: every
 // lane adds the counts of its own run of consecutive lists (loads that do not depend on each other), a prefix sum over
 // the lanes names the run that holds rank r, and a second prefix sum over the counts of that run names the list.
-__device__ __forceinline__ int core_slow_record(const CoreArgs& C, int r, int lane) {
+struct SlowRuns { int mine, incl; };      // records of this lane's run of lists; of the runs up to and with it
+__device__ __forceinline__ SlowRuns core_slow_runs(const CoreArgs& C, int lane) {
     const int n = C.slow_lists;
     const int run = (n + WAVE - 1) / WAVE;
-    int mine = 0;
-    for (int k = 0; k < run; k++) mine += lane * run + k < n ? C.K.slow_count[lane * run + k] : 0;
-    const int incl = wave_scan_incl(mine);
-    if (r >= __builtin_amdgcn_readlane(incl, WAVE - 1)) return -1;
-    const int seg = __builtin_amdgcn_readfirstlane(__ffsll((unsigned long long)ballot(incl > r)) - 1);
-    int base = __builtin_amdgcn_readlane(incl - mine, seg);
+    SlowRuns R;
+    R.mine = 0;
+    for (int k = 0; k < run; k++) R.mine += lane * run + k < n ? C.K.slow_count[lane * run + k] : 0;
+    R.incl = wave_scan_incl(R.mine);
+    return R;
+}
+__device__ __forceinline__ int core_slow_record(const CoreArgs& C, const SlowRuns& R, int r, int lane) {
+    const int n = C.slow_lists;
+    const int run = (n + WAVE - 1) / WAVE;
+    if (r >= __builtin_amdgcn_readlane(R.incl, WAVE - 1)) return -1;
+    const int seg = __builtin_amdgcn_readfirstlane(__ffsll((unsigned long long)ballot(R.incl > r)) - 1);
+    int base = __builtin_amdgcn_readlane(R.incl - R.mine, seg);
     for (int k0 = 0; k0 < run; k0 += WAVE) {
         const int li = seg * run + k0 + lane;
         const int c = (k0 + lane < run && li < n) ? C.K.slow_count[li] : 0;
@@ -544,6 +551,9 @@ __device__ __forceinline__ int core_slow_record(const CoreArgs& C, int r, int la
         base += tot;
     }
     return -1;
+}
+__device__ __forceinline__ int core_slow_record(const CoreArgs& C, int r, int lane) {
+    return core_slow_record(C, core_slow_runs(C, lane), r, lane);
 }
 // Which record a wavefront of a main kernel starts with: the first slow_wgs wavefronts a listed one (-1: none left),
 // the others the records in work order.

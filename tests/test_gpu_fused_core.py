@@ -232,6 +232,85 @@ def test_sorted_frame_search_equals_the_box_search_at_batch_256(noise):
     assert float((n - 1).abs().max()) < 1e-5
 
 
+def _joined(*parts, seed=5):
+    """One problem of the crystals of several batches."""
+    from crystalframer_amd import synthetic
+    sizes = torch.cat([c.sizes for c in parts])
+    batch = torch.repeat_interleave(torch.arange(len(sizes)), sizes)
+    return Hh.problem_from_batch(synthetic.CrystalBatch(torch.cat([c.x for c in parts]), torch.cat([c.pos for c in parts]), batch,
+                                                        torch.cat([c.trans_vec for c in parts]), sizes, zero_based=True), seed=seed)
+
+
+def _cells(B, lo, hi, narrow=False, seed=1):
+    """Crystals of lo to hi atoms; narrow: every half-width of their boxes is at least 3 for most widths."""
+    from crystalframer_amd import synthetic
+    edge = dict(len_lo=1.9, len_hi=2.4) if narrow else dict(len_lo=4.0, len_hi=9.0)
+    return synthetic.make_batch(B, atoms="uniform", atoms_lo=lo, atoms_hi=hi, ang_lo=65.0, ang_hi=115.0, seed=seed, **edge)
+
+
+def _left_behind(P):
+    """Places of the work order behind those that rows of more than 16 pairs can have."""
+    return P.N - min(P.N, (P.E - P.N) // 16)
+
+
+# Where a third of the items or more lie behind the places that long rows can have, what the four-heads search leaves is taken from the
+# lists: by the leading wavefronts (a sixteenth of the items, at least 256), by the resident ones behind them (at most 24 per compute
+# unit), and what is left from their counters.  Fewer listed records than leading wavefronts, up to two per resident one and more
+# than that; long rows, listed and not, in front of short ones; a last list and a last run of lists of other lengths.
+@pytest.mark.parametrize("noise", [0.0, 1e-5])
+@pytest.mark.parametrize("name", ["few", "one_each", "a_few_more", "two_each", "many", "long_rows", "long_narrow_rows"])
+def test_frames_of_many_items_equal_the_box_search(name, noise):
+    import crystalframer_amd as cf
+    KM = cf.KernelManager
+    KM.SYMM_BREAK_NOISE, KM.NOISE_SEED, KM.NOISE_SEED_DEVICE = noise, 7, None
+    P = dict(few=lambda: _joined(_cells(2000, 1, 3), _cells(9, 1, 2, True)),
+             one_each=lambda: _joined(_cells(817, 1, 1, True)),
+             a_few_more=lambda: _joined(_cells(829, 1, 1, True)),
+             two_each=lambda: _joined(_cells(1700, 1, 1, True)),
+             many=lambda: _joined(_cells(1801, 1, 3, True), _cells(1200, 1, 6)),
+             long_rows=lambda: _joined(_cells(24, 17, 40), _cells(2, 17, 40, True), _cells(4200, 1, 3), _cells(700, 1, 2, True)),
+             long_narrow_rows=lambda: _joined(_cells(9, 17, 30, True), _cells(1, 70, 70, True), _cells(2500, 1, 2, True)))[name]()
+    assert 3 * _left_behind(P) >= P.N and 8 * P.N > 6144
+    listed = int((TO.translation_ranges(P.a, P.rvlen, P.batch, CUT).reshape(-1, 3) != 2).any(-1).sum())
+    lead = max(256, (P.N * 8 // 16 + 7) // 8 * 8)
+    resident = 24 * torch.cuda.get_device_properties(0).multi_processor_count
+    least = dict(few=1, one_each=lead + 1, a_few_more=lead + 1, two_each=lead + resident + 1, many=lead + 2 * resident,
+                 long_rows=lead + 1, long_narrow_rows=lead + 2 * resident)[name]
+    assert least <= listed and (name != "few" or listed < lead)
+    if "long" in name:
+        assert P.E > P.N + 16 * 100      # more than a hundred places for long rows
+    fr, ref = _frames_both_ways(P)
+    assert torch.equal(fr, ref)
+
+
+def test_frames_of_many_items_whose_width_is_not_negative():
+    """a = 0 and a > 0 (the farthest images win) in a few items of a large batch, the fixed box: neither the four-heads search nor
+    a box of their own takes them."""
+    P = _joined(_cells(3001, 1, 3))
+    assert 3 * _left_behind(P) >= P.N
+    pick = torch.randperm(P.N * 8, generator=torch.Generator().manual_seed(3))[:900]
+    P.a.view(-1)[pick[:450]] = 0.0
+    P.a.view(-1)[pick[450:]] = 0.01
+    fr, ref = _frames_both_ways(P, cutoff=None)
+    assert torch.equal(fr, ref)
+
+
+def test_frames_of_many_items_in_a_work_order_of_the_callers_own(monkeypatch):
+    """The shortest rows first: the long ones lie behind the places that are theirs otherwise."""
+    from crystalframer_amd import cuda_funcs as F
+    own = F.edge_schedule
+
+    def shortest_first(edges, N):
+        e_start, order = own(edges, N)
+        return e_start, order.flip(0).contiguous()
+    P = _joined(_cells(15, 17, 40), _cells(2400, 1, 3), _cells(300, 1, 2, True))
+    assert 3 * _left_behind(P) >= P.N
+    _, ref = _frames_both_ways(P)
+    monkeypatch.setattr(F, "edge_schedule", shortest_first)
+    _, fr, _ = run_core(P, frames="search", need_grad=False)
+    assert torch.equal(fr, ref)
+
+
 @pytest.mark.parametrize("noise", [0.0, 1e-5])
 def test_sorted_frame_search_mixed_boxes_fixed_box_and_long_rows(noise):
     """Small cells (boxes wider than the table's: whole-box scan in chunks), the fixed box without a cutoff, rows

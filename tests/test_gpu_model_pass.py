@@ -725,32 +725,6 @@ def test_products_by_the_wavefront_that_completes_sixteen_items(bins, B, atoms, 
     assert Hh.rel_err(out, kept.double()) < 5e-6
 
 
-# Frames of many items (49 152 and more behind the rows of over 16 pairs): four items per wavefront are looked at for what the search
-# of four heads leaves.  Cells so small that their box is not the usual one, more of them than the leading wavefronts take (a
-# sixteenth of the items), alone and beside long rows; the last wavefront with fewer than four items.
-@pytest.mark.parametrize("B,atoms,small", [(6147, 1, 2000), (6149, 1, 6149), (3100, 2, 40), (390, 17, 250)])
-def test_frames_of_many_items(B, atoms, small):
-    """The crystals of a large batch are answered as in batches small enough to search one item at a time."""
-    from crystalframer_amd import params, synthetic
-    mp = params.ModelParams(num_layers=1, symm_break_noise=0.0)
-    cb = synthetic.make_batch(B, atoms="uniform", atoms_lo=atoms, atoms_hi=atoms, len_lo=4.0, len_hi=9.0, ang_lo=65.0, ang_hi=115.0,
-                              seed=B)
-    frac = torch.linalg.solve(cb.trans_vec[cb.batch].double().transpose(1, 2), cb.pos.double()[:, :, None])
-    cb.trans_vec[torch.randperm(B, generator=torch.Generator().manual_seed(B))[:small]] *= 0.3
-    cb.pos[:] = (cb.trans_vec[cb.batch].double().transpose(1, 2) @ frac)[:, :, 0].float()
-    part = lambda b0, b1: synthetic.CrystalBatch(cb.x[atoms * b0:atoms * b1], cb.pos[atoms * b0:atoms * b1],  # noqa: E731
-                                                 cb.batch[atoms * b0:atoms * b1] - b0, cb.trans_vec[b0:b1], cb.sizes[b0:b1], zero_based=True)
-    model, _ = _model(mp, part(0, 20))
-    model.eval()
-    step = 600 // atoms
-    with torch.no_grad():
-        out = model(cb.to("cuda"))
-        want = torch.cat([model(part(b, min(B, b + step)).to("cuda")) for b in range(0, B, step)])
-    # (a near tie between two candidates falls either way with the last bit of the inputs, which depend on the rows beside them)
-    off = ((out - want).abs() / want.abs().max()).flatten()
-    assert (off > 5e-6).float().mean() < 2e-3 and off.median() < 1e-6
-
-
 # Inference without the angle encoding: one head of an atom per wavefront up to 16 383 items, two from there on, four from 45 056
 # (from 24 576 with rows of more than 64 pairs).  Either side of the lines; rows of one pair, of a whole group of eight, one more, of
 # several groups whose maximum grows, of more than 64; sixteen heads; a few cells so small that their box is not the usual one
