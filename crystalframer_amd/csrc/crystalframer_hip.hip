@@ -1654,11 +1654,6 @@ int slow_wave_count(int64_t N, int H) {
     const int64_t w = (N * H / 16 + 7) / 8 * 8;
     return (int)(w < 256 ? 256 : w);
 }
-// Wavefronts of a kernel that are resident at once, so many per compute unit.
-unsigned resident_waves(int per_cu) {
-    const int cus = device_cus();
-    return (unsigned)(per_cu * (cus > 0 ? cus : 256));
-}
 // Workgroups of a kernel that are resident on the device at once (asked of the runtime once per kernel).
 template <auto KERN>
 unsigned resident_workgroups(int threads) {
@@ -1774,7 +1769,7 @@ template <int HEADS>
 int launch_core_heads(const cfh::CoreArgs& C, hipStream_t st, const char* what) {
     {
         TimedScope timed(what, st);
-        const unsigned rest = resident_waves(16);
+        const unsigned rest = resident_workgroups<cfh::fused_core_fwd_heads_kernel<11, HEADS>>(cfh::WAVE);
         hipLaunchKernelGGL((cfh::fused_core_fwd_heads_kernel<11, HEADS>), dim3((unsigned)C.slow_wgs + (unsigned)C.K.N * (unsigned)C.K.H / HEADS + rest),
                            dim3(cfh::WAVE), 0, st, C, (int)rest);
     }

@@ -783,12 +783,14 @@ __device__ __forceinline__ void core_project_done(const CoreArgs& C, int it, int
 // wcat: not null: the wavefront makes the product of its histogram with the head's weights itself, the histogram stays in
 // LDS (LEAN only)
 // own: not null: the item's record and first operands, in registers
+// given: the item is this wavefront's, listed or not
 struct CoreOwn { uint32_t rec; CorePrefetch pf; };
 // HAND_OVER (LEAN only): the histogram stays in LDS as float32 words, with the item's part of `out` and its atom in front of the
 // table, for other wavefronts of the workgroup (CoreProductWeights), which wait at a barrier until it is there
 template <int WL, int ANG, bool COS_ABS, bool LEAN, int COPIES = 1, bool HAND_OVER = false>
 __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLds<ANG, LEAN, COPIES>& sh, int wid,
-                                                    const float* __restrict__ wcat = nullptr, const CoreOwn* own = nullptr) {
+                                                    const float* __restrict__ wcat = nullptr, const CoreOwn* own = nullptr,
+                                                    bool given = false) {
     constexpr bool HAS_ANG = ANG > 0;
     constexpr int HWK = core_hist_words(ANG, LEAN);          // words per item in memory
     using Hist = CoreHist<ANG, LEAN, COPIES>;
@@ -825,7 +827,7 @@ __device__ __forceinline__ void fused_core_fwd_body(const CoreArgs& C, CoreFwdLd
     CFH_PH_DECL
     {
         const uint32_t rec_cur = own ? own->rec : load_record_lane(P, it_cur, h, lane);
-        if (!own && core_record_taken_elsewhere(C, rec_cur, wid, lane)) return;
+        if (!own && !given && core_record_taken_elsewhere(C, rec_cur, wid, lane)) return;
         const CorePrefetch pf = own ? own->pf : core_prefetch(C, rec_cur, it_cur, h, lane);
         CFH_PH(0);
         const CoreItem ci = core_unpack(C, rec_cur, true);
@@ -1535,18 +1537,24 @@ __device__ __forceinline__ void fused_core_fwd_heads(const CoreArgs& C, CoreHead
     }
 }
 // The leading wavefronts take a listed record each, the next ones HEADS heads of an atom (where some of those are listed, the others
-// one after the other), and the `rest` last ones the listed records that are left, by rank, each every rest-th of them.  (Records
-// with a box of their own have 16 wavefronts per compute unit here and 28 in the kernel of one item per wavefront: a batch of nothing
-// but such cells, 82 000 items, takes 1.26 times as long; the leading wavefronts are enough for one item in sixteen.)
+// one after the other), and the `rest` last ones, as many as are resident, the listed records that are left: the first by their own
+// rank, the next ones as they come from NQUEUE counters, until there are no more (they wait at the list for what they take next,
+// where a wavefront per item waits for its turn at the dispatcher).
+// Records with a box of their own have 18 wavefronts per compute unit here (LDS) and 28 in the kernel of one item per wavefront.
+// Whole passes of four layers in us, that kernel / this one: nothing but such cells, 22 000 items 999/1004, 66 000 items 2601/2655
+// (dealt out beforehand and looked up in the lists twice, at 16 per compute unit: 3111); half of them so 1611/1576; one in ten 851/766;
+// ordinary cells, 180 224 items, 1305/960.  Five wavefronts per SIMD with four heads: 96 registers instead of 103, 1036 -> 1017 for the
+// ordinary cells of another machine.  Two records per draw: 22 000 items 1005 -> 1059.
 template <int WL, int HEADS>
-__global__ __launch_bounds__(WAVE) void fused_core_fwd_heads_kernel(const CoreArgs C, int rest) {
+__global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(HEADS == 4 ? 5 : 1)))
+void fused_core_fwd_heads_kernel(const CoreArgs C, int rest) {
     __shared__ union { CoreFwdLds<0, true> one; CoreHeadsShared<HEADS> several; } sh;
     const KernelArgs& P = C.K;
     const int lane = (int)threadIdx.x & (WAVE - 1), w = (int)blockIdx.x;
     const int groups = P.N * P.H / HEADS;
     const bool by_rank = w < C.slow_wgs || w >= C.slow_wgs + groups;
     int wid = 0, rank = w < C.slow_wgs ? w : w - groups;
-    uint32_t left = 1;                 // heads of this wavefront's own that are not listed
+    uint32_t left = 0;                 // heads of this wavefront's own that are not listed
     if (!by_rank) {
         constexpr int shift = HEADS == 2 ? CORE_DIE_SHIFT - 1 : CORE_DIE_SHIFT - 2;      // (an atom's heads on one die)
         wid = HEADS * __builtin_amdgcn_readfirstlane(die_order(w - C.slow_wgs, groups, shift));
@@ -1555,7 +1563,6 @@ __global__ __launch_bounds__(WAVE) void fused_core_fwd_heads_kernel(const CoreAr
         HeadRecords<HEADS> rec;
         rec.load(P, it, h0, lane);
         const int usual = C.table_R | (C.table_R << 8) | (C.table_R << 16);
-        left = 0;
         bool together = true;
 #pragma unroll
         for (int hh = 0; hh < HEADS; hh++) {
@@ -1568,17 +1575,26 @@ __global__ __launch_bounds__(WAVE) void fused_core_fwd_heads_kernel(const CoreAr
             return;
         }
     }
+    SlowRuns runs{0, 0};
+    if (by_rank) runs = core_slow_runs(C, lane);
 #pragma unroll 1
-    for (; left; left &= left - 1) {
-        int item = wid + __builtin_ctz(left);
+    for (;;) {
+        int item;
         if (by_rank) {
-            item = __builtin_amdgcn_readfirstlane(core_slow_record(C, rank, lane));
+            item = __builtin_amdgcn_readfirstlane(core_slow_record(C, runs, rank, lane));
             if (item < 0) return;
-            if (rank >= C.slow_wgs) left = 3;      // (another rank behind this one)
-            rank += rest;
+        } else {
+            if (left == 0) return;
+            item = wid + __builtin_ctz(left);
+            left &= left - 1;
         }
         wave_sync();
-        fused_core_fwd_body<WL, 0, false, true>(C, sh.one, item);
+        fused_core_fwd_body<WL, 0, false, true>(C, sh.one, item, nullptr, nullptr, true);
+        if (w < C.slow_wgs) return;
+        if (by_rank) {
+            const int q = w & (NQUEUE - 1);
+            rank = C.slow_wgs + rest + queue_draw(P.counters + q * QSTRIDE) * NQUEUE + q;
+        }
     }
 }
 

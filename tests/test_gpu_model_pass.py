@@ -750,6 +750,43 @@ def test_heads_of_an_atom_in_one_wavefront(B, atoms, width, small):
     assert Hh.rel_err(out, kept.double()) < 2e-6
 
 
+# ... and many such cells: fewer of them than the leading wavefronts (a sixteenth of the items, at least 256), up to one and two for each
+# of the resident wavefronts behind (at most 24 per compute unit), and more, which come from their counters; every head of a cell
+# listed or only some (atoms differ in their widths); ordinary cells in front and behind.  {crystals: (from atoms, to atoms, narrow)}
+@pytest.mark.parametrize("heads,width,parts", [(2, 128, [(2100, 1, 1, False), (20, 1, 2, True)]), (2, 128, [(2050, 1, 1, True)]),
+                                               (2, 128, [(1500, 1, 2, True), (300, 1, 6, False), (200, 1, 2, True)]),
+                                               (2, 128, [(1100, 2, 2, True)]), (4, 128, [(5700, 1, 1, True)]), (4, 256, [(2817, 1, 1, True)]),
+                                               (4, 128, [(900, 1, 3, True), (3000, 1, 3, False), (1, 17, 17, True)]),
+                                               (4, 128, [(20, 17, 30, True), (3500, 1, 3, True)])])
+def test_many_cells_with_a_box_of_their_own_beside_several_heads_per_wavefront(heads, width, parts):
+    """Against the same pass with everything kept (one item per wavefront; tolerance as above), bit for bit the same from call to call
+    with other crystals in between, whose histograms lie where a record that nobody took would find its own."""
+    from crystalframer_amd import params, synthetic
+    mp = params.ModelParams(num_layers=1, value_pe_angle_real=0, model_dim=width, head_num=width // 16, embedding_dim=[width])
+
+    def make(seed):
+        cells = [synthetic.make_batch(B, atoms="uniform", atoms_lo=lo, atoms_hi=hi, ang_lo=65.0, ang_hi=115.0, seed=seed + k,
+                                      **(dict(len_lo=1.9, len_hi=2.4) if narrow else dict(len_lo=4.0, len_hi=9.0)))
+                 for k, (B, lo, hi, narrow) in enumerate(parts)]
+        sizes = torch.cat([c.sizes for c in cells])
+        return synthetic.CrystalBatch(torch.cat([c.x for c in cells]), torch.cat([c.pos for c in cells]),
+                                      torch.repeat_interleave(torch.arange(len(sizes)), sizes), torch.cat([c.trans_vec for c in cells]),
+                                      sizes, zero_based=True)
+    model, cb = _model(mp, make(1))
+    other = make(50).to("cuda")
+    items = cb.pos.shape[0] * width // 16
+    assert (45056 if heads == 4 else 16384) <= items and (heads == 4 or items < 45056)
+    model.eval()
+    kept = model(cb).detach()
+    with torch.no_grad():
+        model(other)
+        out = model(cb)
+        for _ in range(2):
+            model(other)
+            assert torch.equal(model(cb), out)
+    assert Hh.rel_err(out, kept.double()) < 2e-6
+
+
 # Either side of the item counts up to which a layer's items take one launch, crystals of as many atoms as the row has pairs.  With
 # everything kept: 5120 with an angle encoding (8 atoms), 6144 from 13 atoms on, 4096 from 33, none from 65; 10 240 without (8
 # atoms), 5120 from 17 atoms on.  Inference: 10 240 (8, 24 and 40 atoms), 16 384 without an angle encoding for up to 12 atoms, 5120
